@@ -6,6 +6,7 @@ cannot be found or built, or a call reports a non-zero status, an exception is r
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import itertools
 import math
@@ -121,6 +122,8 @@ _lock = threading.Lock()
 def load() -> ctypes.CDLL:
     """Load libhawk_hip.so, building it first only if no built library is present."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -168,8 +171,39 @@ def require_cuda(*tensors: torch.Tensor) -> torch.device:
     return dev
 
 
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """``torch.cuda.device(dev)``, or nothing at all where that device is current already (the
+    switch costs 3 us of host time per call, more than the launch it guards)."""
+    return _SAME_DEVICE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
 def stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    if dev.index is None:
+        return torch.cuda.current_stream(dev).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
+def launches_directly(*tensors) -> bool:
+    """Whether a kernel can be launched on these tensors without going through its
+    ``torch.library`` op.  The op exists for tracing (``torch.compile``, fake tensors, dispatch
+    modes) and for the error that differentiating through it raises; its wrapper costs about 25 us
+    of host time per call, as much as a small scan takes on the GPU.  Plain CUDA tensors outside
+    any of that need none of it: same launch function, same results."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
+        return False
+    if torch._C._len_torch_dispatch_stack() != 0:
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN_TENSORS or not t.is_cuda or (grad and t.requires_grad):
+            return False
+    return True
 
 
 def ptr(t):
@@ -281,7 +315,7 @@ _decode_captured: dict = {}   # (device, stream, capture id) -> counters of laun
 
 def _capture_id(dev: torch.device) -> int:
     cid = ctypes.c_ulonglong(0)
-    with torch.cuda.device(dev):
+    with on_device(dev):
         check("hawk_stream_capture_id", load().hawk_stream_capture_id(stream_ptr(dev), ctypes.byref(cid)))
     return cid.value
 

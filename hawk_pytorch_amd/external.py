@@ -34,7 +34,7 @@ def _launch_conv_fwd(x, w, b, state, out_dtype) -> torch.Tensor:
     W = w.shape[0]
     y = _lib.activation_empty((B, T, D), out_dtype, dev)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_conv1d_fwd(
             x.data_ptr(), w.data_ptr(), b.data_ptr(), _lib.ptr(state), y.data_ptr(),
             B, T, D, W, _lib.dtype_code(x.dtype), _lib.dtype_code(out_dtype), _lib.stream_ptr(dev),
@@ -54,7 +54,7 @@ def _launch_conv_bwd(grad_y, x, w):
     lib = _lib.load()
     nbytes = lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_conv1d_bwd(
             grad_y.data_ptr(), x.data_ptr(), w.data_ptr(), dx.data_ptr(), dw.data_ptr(), db.data_ptr(),
             B, T, D, W, _lib.dtype_code(x.dtype), _lib.dtype_code(grad_y.dtype),
@@ -92,6 +92,19 @@ def _(grad_y, x, w):
     )
 
 
+def _conv1d_fwd(x, w, b, state, out_fp32: bool):
+    tensors = (x, w, b) if state is None else (x, w, b, state)
+    if _lib.launches_directly(*tensors):
+        return _launch_conv_fwd(x, w, b, state, torch.float32 if out_fp32 else torch.bfloat16)
+    return _conv1d_fwd_op(x, w, b, state, out_fp32)
+
+
+def _conv1d_bwd(grad_y, x, w):
+    if _lib.launches_directly(grad_y, x, w):
+        return _launch_conv_bwd(grad_y, x, w)
+    return _conv1d_bwd_op(grad_y, x, w)
+
+
 class _TemporalConv(Function):
     """y = causal depthwise conv(x; w, b) with zero history; hand-written backward."""
 
@@ -100,7 +113,7 @@ class _TemporalConv(Function):
         xc = x if x.is_contiguous() else x.contiguous()
         ctx.save_for_backward(xc, w)
         ctx.in_dtype = x.dtype
-        return _conv1d_fwd_op(xc, w, b, None, out_fp32)
+        return _conv1d_fwd(xc, w, b, None, out_fp32)
 
     @staticmethod
     def backward(ctx, grad_y):  # type: ignore[override]
@@ -108,7 +121,7 @@ class _TemporalConv(Function):
         if grad_y.dtype not in (torch.bfloat16, torch.float32):
             grad_y = grad_y.float()
         gy = grad_y if grad_y.is_contiguous() else grad_y.contiguous()
-        dx, dw, db = _conv1d_bwd_op(gy, xc, w)
+        dx, dw, db = _conv1d_bwd(gy, xc, w)
         return dx, dw, db, None
 
 
@@ -132,7 +145,7 @@ def temporal_conv1d(x, w, b, out_dtype: Optional[torch.dtype] = None, state=None
     if state is not None:
         assert state.shape == (x.shape[0], W - 1, D)
         xc = x if x.is_contiguous() else x.contiguous()
-        return _conv1d_fwd_op(xc, w32, b32, state.to(x.dtype), out_dtype == torch.float32)
+        return _conv1d_fwd(xc, w32, b32, state.to(x.dtype), out_dtype == torch.float32)
     return _TemporalConv.apply(x, w32, b32, out_dtype == torch.float32)
 
 
@@ -192,7 +205,7 @@ def temporal_conv1d_step(conv_state, x_new, w, b, out_dtype: Optional[torch.dtyp
         out_dtype = torch.promote_types(conv_state.dtype, w.dtype)
     y = torch.empty((B, D), dtype=out_dtype, device=dev)
     w32, b32 = _lib.dense16(w.detach().float()), _lib.dense16(b.detach().float())
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = _lib.load().hawk_conv1d_step(
             conv_state.data_ptr(), xn.data_ptr(), w32.data_ptr(), b32.data_ptr(), y.data_ptr(),
             B, D, W, _lib.dtype_code(conv_state.dtype), _lib.dtype_code(out_dtype), _lib.stream_ptr(dev),
@@ -214,7 +227,7 @@ def rglru_step(x, x_rg_lru, a_rg_lru, a_param, recc_state):
     xs = [_lib.dense16(t.reshape(B, D).to(run_dtype)) for t in (x, x_rg_lru, a_rg_lru)]
     lam = _lib.dense16(a_param.detach().float())
     h = torch.empty((B, D), dtype=run_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = _lib.load().hawk_rglru_step(
             xs[0].data_ptr(), xs[1].data_ptr(), xs[2].data_ptr(), lam.data_ptr(),
             recc_state.data_ptr(), h.data_ptr(), B, D,
@@ -244,7 +257,7 @@ def rglru_step_gated(x, x_rg_lru, a_rg_lru, a_param, recc_state, y, bias_i=None,
         y2 = y2.contiguous()
     ldy = y2.stride(0) if B > 1 else D
     out = torch.empty((B, D), dtype=run_dtype, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = _lib.load().hawk_rglru_step_gated(
             xs[0].data_ptr(), xs[1].data_ptr(), xs[2].data_ptr(), _lib.ptr(biases[0]), _lib.ptr(biases[1]),
             lam.data_ptr(), y2.data_ptr(), ldy, recc_state.data_ptr(), None, out.data_ptr(), B, D,
@@ -308,7 +321,7 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     lam = _lib.dense16(a_param.detach().float())
     out = torch.empty((B, D), dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         # counters that let several workgroups share a block's output columns
         nws = lib.hawk_decode_core_workspace_bytes(B, D, input_gate.num_blocks)
         ws = _lib.decode_workspace(dev, nws)
@@ -405,7 +418,7 @@ def _launch_gate_fwd(x, w_i, b_i, w_a, b_a, out_bf16: bool):
     out_dtype = torch.bfloat16 if out_bf16 else torch.float32
     xg = _lib.activation_empty(x.shape, out_dtype, dev)
     ag = _lib.activation_empty(x.shape, out_dtype, dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = _lib.load().hawk_gate_proj_fwd(
             x2.data_ptr(), w_i.data_ptr(), b_i.data_ptr(), w_a.data_ptr(), b_a.data_ptr(), xg.data_ptr(),
             ag.data_ptr(), M, D, nb, _lib.dtype_code(x2.dtype), _lib.dtype_code(w_i.dtype),
@@ -431,7 +444,7 @@ def _launch_gate_bwd(x, d_xg, d_ag, w_i, w_a, addend=None):
     db_a = torch.empty(D, dtype=torch.float32, device=dev)
     nbytes = lib.hawk_gate_proj_bwd_weights_workspace_bytes(M, D, nb)
     ws = _gate_workspace(dev, nbytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.stream_ptr(dev)
         status = lib.hawk_gate_proj_bwd_input(
             g_i.data_ptr(), g_a.data_ptr(), w_i.data_ptr(), w_a.data_ptr(), _lib.ptr(addend), dx.data_ptr(), M, D, nb,
@@ -479,6 +492,19 @@ def _(x, d_xg, d_ag, w_i, w_a, addend=None):
     )
 
 
+def gate_proj_fwd(x, w_i, b_i, w_a, b_a, out_bf16: bool):
+    if _lib.launches_directly(x, w_i, b_i, w_a, b_a):
+        return _launch_gate_fwd(x, w_i, b_i, w_a, b_a, out_bf16)
+    return _gate_proj_fwd_op(x, w_i, b_i, w_a, b_a, out_bf16)
+
+
+def gate_proj_bwd(x, d_xg, d_ag, w_i, w_a, addend=None):
+    tensors = (x, d_xg, d_ag, w_i, w_a) if addend is None else (x, d_xg, d_ag, w_i, w_a, addend)
+    if _lib.launches_directly(*tensors):
+        return _launch_gate_bwd(x, d_xg, d_ag, w_i, w_a, addend)
+    return _gate_proj_bwd_op(x, d_xg, d_ag, w_i, w_a, addend)
+
+
 # The projection kernels round fp32 weights to bf16 as they load them, every workgroup for
 # itself, and moving 512 KiB instead of 256 KiB per workgroup through its L1 makes the forward
 # 8 us and the input gradient 13 us longer at a block width of 256.  From this many rows on,
@@ -494,7 +520,7 @@ def kernel_weights(w_i: torch.Tensor, w_a: torch.Tensor, rows: int):
             # both gates in one launch
             wi, wa = _lib.dense16(w_i.detach()), _lib.dense16(w_a.detach())
             both = torch.empty((2, nb, bw, bw), dtype=torch.bfloat16, device=w_i.device)
-            with torch.cuda.device(w_i.device):
+            with _lib.on_device(w_i.device):
                 _lib.check("hawk_gate_weights_to_bf16", _lib.load().hawk_gate_weights_to_bf16(
                     wi.data_ptr(), wa.data_ptr(), both[0].data_ptr(), both[1].data_ptr(), nb, bw,
                     _lib.stream_ptr(w_i.device)))
@@ -512,14 +538,14 @@ class _GateProjection(Function):
         ctx.param_dtypes = (w_i.dtype, b_i.dtype, w_a.dtype, b_a.dtype)
         w_i, w_a = kernel_weights(w_i, w_a, xc.numel() // xc.shape[-1])
         ctx.save_for_backward(xc, w_i, w_a)
-        return _gate_proj_fwd_op(xc, w_i, b_i.float().reshape(-1), w_a, b_a.float().reshape(-1), out_bf16)
+        return gate_proj_fwd(xc, w_i, b_i.float().reshape(-1), w_a, b_a.float().reshape(-1), out_bf16)
 
     @staticmethod
     def backward(ctx, d_xg, d_ag):  # type: ignore[override]
         x, w_i, w_a = ctx.saved_tensors
         gdt = torch.bfloat16 if (d_xg.dtype == torch.bfloat16 and d_ag.dtype == torch.bfloat16) else torch.float32
         d_xg, d_ag = (g.to(gdt).contiguous() for g in (d_xg, d_ag))
-        dx, dw_i, db_i, dw_a, db_a = _gate_proj_bwd_op(x, d_xg, d_ag, w_i, w_a)
+        dx, dw_i, db_i, dw_a, db_a = gate_proj_bwd(x, d_xg, d_ag, w_i, w_a)
         nb, bw, _ = w_i.shape
         dts = ctx.param_dtypes
         return (dx, dw_i.to(dts[0]), db_i.reshape(nb, bw).to(dts[1]), dw_a.to(dts[2]),

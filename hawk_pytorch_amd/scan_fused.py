@@ -54,7 +54,7 @@ def _launch_scan_fwd(x, x_rg_lru, a_rg_lru, a_param, h_bf16: bool) -> torch.Tens
     h = _lib.activation_empty((b, sq, d), out_dtype, dev)
     nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
     ws = _lib.scan_workspace(dev, nbytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_rglru_scan_fwd_mixed(
             x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), h.data_ptr(),
             b, sq, d, in_code, _lib.dtype_code(out_dtype), ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
@@ -75,7 +75,7 @@ def _launch_scan_bwd(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out):
     dlam = torch.empty(d, dtype=torch.float32, device=dev)
     nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
     ws = _lib.scan_workspace(dev, nbytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_rglru_scan_bwd_mixed(
             x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(),
             h_saved.data_ptr(), grad_out.data_ptr(), dx.data_ptr(), dxg.data_ptr(), dag.data_ptr(),
@@ -122,6 +122,15 @@ def _(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out):
     return e(), e(), e(), torch.empty(x.shape[-1], dtype=torch.float32, device=x.device)
 
 
+def _scan_fwd(x, x_rg_lru, a_rg_lru, a_param, h_bf16: bool):
+    launch = _launch_scan_fwd if _lib.launches_directly(x, x_rg_lru, a_rg_lru, a_param) else _rglru_scan_fwd_op
+    return launch(x, x_rg_lru, a_rg_lru, a_param, h_bf16)
+
+
+def _scan_bwd(*tensors):
+    return (_launch_scan_bwd if _lib.launches_directly(*tensors) else _rglru_scan_bwd_op)(*tensors)
+
+
 # ---------------------------------------------------------------------------------------
 # Upstream-shaped host wrappers
 # ---------------------------------------------------------------------------------------
@@ -158,7 +167,7 @@ def sequential_scan_forward(
     a_param = a_param.float().contiguous()
     h_bf16 = out_dtype == torch.bfloat16 or (out_dtype is None and x.dtype == torch.bfloat16)
     assert out_dtype in (None, x.dtype, torch.bfloat16), f"unsupported h dtype {out_dtype} for {x.dtype} inputs"
-    return _rglru_scan_fwd_op(x, x_rg_lru, a_rg_lru, a_param, h_bf16)
+    return _scan_fwd(x, x_rg_lru, a_rg_lru, a_param, h_bf16)
 
 
 def sequential_scan_backward(
@@ -192,7 +201,7 @@ def sequential_scan_backward(
         x_saved, x_rg_lru_saved, a_rg_lru_saved, h_saved, grad_out
     )
     a_param_saved = a_param_saved.float().contiguous()
-    return _rglru_scan_bwd_op(x_saved, x_rg_lru_saved, a_rg_lru_saved, a_param_saved, h_saved, grad_out)
+    return _scan_bwd(x_saved, x_rg_lru_saved, a_rg_lru_saved, a_param_saved, h_saved, grad_out)
 
 
 def _common_input_dtype(*tensors: torch.Tensor) -> torch.dtype:
@@ -275,7 +284,7 @@ def _launch_scan_gated_fwd(x, x_rg_lru, a_rg_lru, a_param, y, h_bf16: bool, want
     h_last = torch.empty((b, 1, d) if want_last else (0,), dtype=out_dtype, device=dev)
     nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
     ws = _lib.scan_workspace(dev, nbytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_rglru_scan_gated_fwd(
             x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), y.data_ptr(), ldy,
             h.data_ptr() if want_h else None, out.data_ptr(), h_last.data_ptr() if want_last else None,
@@ -304,7 +313,7 @@ def _launch_scan_gated_bwd(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out)
     dlam = torch.empty(d, dtype=torch.float32, device=dev)
     nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
     ws = _lib.scan_workspace(dev, nbytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         status = lib.hawk_rglru_scan_gated_bwd(
             x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), y.data_ptr(), ldy,
             h_saved.data_ptr(), grad_out.data_ptr(), dx.data_ptr(), dxg.data_ptr(), dag.data_ptr(),
@@ -363,6 +372,16 @@ def _(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out):
     )
 
 
+def _scan_gated_fwd(x, x_rg_lru, a_rg_lru, a_param, y, h_bf16: bool, want_h: bool, want_last: bool):
+    direct = _lib.launches_directly(x, x_rg_lru, a_rg_lru, a_param, y)
+    launch = _launch_scan_gated_fwd if direct else _rglru_scan_gated_fwd_op
+    return launch(x, x_rg_lru, a_rg_lru, a_param, y, h_bf16, want_h, want_last)
+
+
+def _scan_gated_bwd(*tensors):
+    return (_launch_scan_gated_bwd if _lib.launches_directly(*tensors) else _rglru_scan_gated_bwd_op)(*tensors)
+
+
 class GatedDiagonalRecurrence(Function):
     """(out, h_last) = (gelu(y) * h, h[:, -1:]) with h = scan(x, x_rg_lru, a_rg_lru, a_param).
 
@@ -383,7 +402,7 @@ class GatedDiagonalRecurrence(Function):
         lam = a_param.float().contiguous()
         h_bf16 = autocast or in_dtype == torch.bfloat16
         want_h = any(ctx.needs_input_grad[:5])
-        out, h, h_last = _rglru_scan_gated_fwd_op(xc, xgc, agc, lam, y, h_bf16, want_h, bool(want_last))
+        out, h, h_last = _scan_gated_fwd(xc, xgc, agc, lam, y, h_bf16, want_h, bool(want_last))
         if want_h:
             ctx.save_for_backward(xc, xgc, agc, a_param, y, h)
         ctx.y_dtype = y.dtype
@@ -399,7 +418,7 @@ class GatedDiagonalRecurrence(Function):
             grad_out = grad_out.contiguous()
         if grad_out.dtype != h_saved.dtype:
             grad_out = grad_out.to(h_saved.dtype)
-        dx, dxg, dag, dlam, dy = _rglru_scan_gated_bwd_op(
+        dx, dxg, dag, dlam, dy = _scan_gated_bwd(
             x, x_rg_lru, a_rg_lru, a_param.float().contiguous(), y, h_saved, grad_out
         )
         if dy.dtype != ctx.y_dtype:
@@ -427,17 +446,17 @@ def fused_linear_scan_gated(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state
 class RecurrentCore(Function):
     @staticmethod
     def forward(ctx, u, w_i, b_i, w_a, b_a, a_param, y, want_last):
-        from .external import _gate_proj_fwd_op, kernel_weights  # deferred: external imports nothing from here
+        from .external import gate_proj_fwd, kernel_weights  # deferred: external imports nothing from here
 
         assert u.dtype == torch.bfloat16, "the fused core runs on bf16 activations"
         uc = u if u.is_contiguous() else u.contiguous()
         lam = a_param.float().contiguous()
         ctx.dtypes = (w_i.dtype, b_i.dtype, w_a.dtype, b_a.dtype, a_param.dtype, y.dtype)
         w_i, w_a = kernel_weights(w_i, w_a, uc.numel() // uc.shape[-1])
-        xg, ag = _gate_proj_fwd_op(uc, w_i, b_i.float().reshape(-1), w_a, b_a.float().reshape(-1), True)
+        xg, ag = gate_proj_fwd(uc, w_i, b_i.float().reshape(-1), w_a, b_a.float().reshape(-1), True)
         _check_shapes(uc, xg, ag, a_param)
         want_h = any(ctx.needs_input_grad[:7])
-        out, h, h_last = _rglru_scan_gated_fwd_op(uc, xg, ag, lam, y, True, want_h, bool(want_last))
+        out, h, h_last = _scan_gated_fwd(uc, xg, ag, lam, y, True, want_h, bool(want_last))
         if want_h:
             ctx.save_for_backward(uc, xg, ag, h, y, w_i, w_a, a_param)
         ctx.mark_non_differentiable(h_last)
@@ -445,13 +464,13 @@ class RecurrentCore(Function):
 
     @staticmethod
     def backward(ctx, grad_out, _grad_last):  # type: ignore[override]
-        from .external import _gate_proj_bwd_op
+        from .external import gate_proj_bwd
 
         u, xg, ag, h, y, w_i, w_a, a_param = ctx.saved_tensors
         go = grad_out if grad_out.dtype == h.dtype else grad_out.to(h.dtype)
         go = go if go.is_contiguous() else go.contiguous()
-        du_scan, d_xg, d_ag, dlam, dy = _rglru_scan_gated_bwd_op(u, xg, ag, a_param.float().contiguous(), y, h, go)
-        du, dw_i, db_i, dw_a, db_a = _gate_proj_bwd_op(u, d_xg, d_ag, w_i, w_a, du_scan)
+        du_scan, d_xg, d_ag, dlam, dy = _scan_gated_bwd(u, xg, ag, a_param.float().contiguous(), y, h, go)
+        du, dw_i, db_i, dw_a, db_a = gate_proj_bwd(u, d_xg, d_ag, w_i, w_a, du_scan)
         nb, bw, _ = w_i.shape
         t = ctx.dtypes
         return (du, dw_i.to(t[0]), db_i.reshape(nb, bw).to(t[1]), dw_a.to(t[2]), db_a.reshape(nb, bw).to(t[3]),
@@ -505,7 +524,7 @@ def _launch_block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, want_h: 
     lib = _lib.load()
     ws = _lib.scan_workspace(dev, lib.hawk_scan_workspace_bytes(B, T, D, code))
     y_ptr = xy.data_ptr() + D * xy.element_size()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         st = _lib.stream_ptr(dev)
         if W == 4 and T >= _FUSED_CONV_MIN_T:
             # conv + both projections, then the gated scan: one host call
@@ -552,7 +571,7 @@ def _launch_block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out):
     ws = _lib.scan_workspace(dev, lib.hawk_scan_workspace_bytes(B, T, D, code))
     gws = _gate_workspace(dev, lib.hawk_gate_proj_bwd_weights_workspace_bytes(M, D, nb))
     cws = torch.empty(lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         # scan (with the output gate) -> projections' input gradient onto the scan's, in place ->
         # conv -> projections' weight gradients, and one launch for the three closing reductions
         _lib.check("hawk_block_core_bwd", lib.hawk_block_core_bwd(
@@ -600,6 +619,16 @@ def _(xy, u, xg, ag, h, conv_w, w_i, w_a, a_param, grad_out):
             f(nb, bw, bw), f(D), f(nb, bw, bw), f(D), f(D))
 
 
+def _block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h: bool, want_last: bool):
+    direct = _lib.launches_directly(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param)
+    launch = _launch_block_core_fwd if direct else _block_core_fwd_op
+    return launch(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h, want_last)
+
+
+def _block_core_bwd(*tensors):
+    return (_launch_block_core_bwd if _lib.launches_directly(*tensors) else _block_core_bwd_op)(*tensors)
+
+
 class BlockCore(Function):
     @staticmethod
     def forward(ctx, xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_last):
@@ -613,7 +642,7 @@ class BlockCore(Function):
         cw = conv_w.float().contiguous()
         w_i16, w_a16 = kernel_weights(w_i, w_a, B * T)
         want_h = any(ctx.needs_input_grad[:8])
-        out, u, xg, ag, h, h_last = _block_core_fwd_op(
+        out, u, xg, ag, h, h_last = _block_core_fwd(
             xy, cw, conv_b.float().contiguous(), w_i16, b_i.float().reshape(-1), w_a16, b_a.float().reshape(-1),
             lam, want_h, bool(want_last))
         if want_h:
@@ -626,7 +655,7 @@ class BlockCore(Function):
         xy, u, xg, ag, h, cw, w_i, w_a, lam = ctx.saved_tensors
         go = grad_out if grad_out.dtype == torch.bfloat16 else grad_out.to(torch.bfloat16)
         go = go if go.is_contiguous() else go.contiguous()
-        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = _block_core_bwd_op(xy, u, xg, ag, h, cw, w_i, w_a, lam, go)
+        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = _block_core_bwd(xy, u, xg, ag, h, cw, w_i, w_a, lam, go)
         nb, bw, _ = w_i.shape
         t = ctx.dtypes
         return (d_xy, dcw.to(t[0]), dcb.to(t[1]), dw_i.to(t[2]), db_i.reshape(nb, bw).to(t[3]), dw_a.to(t[4]),
