@@ -84,6 +84,20 @@ SIGNATURES = {
         [_c_void_p] * 2 + [ctypes.c_longlong] + [_c_void_p] * 8 + [ctypes.c_longlong] + [_c_void_p] * 2
         + [_c_int] * 7 + [_c_void_p, _c_size_t, _c_void_p],
     ),
+    "hawk_decode_linear_supported": (_c_int, [_c_int] * 3),
+    "hawk_decode_linear_workspace_bytes": (_c_size_t, [_c_int] * 3),
+    "hawk_decode_linear": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),
+    "hawk_decode_layer_supported": (_c_int, [_c_int] * 4),
+    "hawk_decode_layer_workspace_bytes": (_c_size_t, [_c_int] * 5),
+    "hawk_decode_norm_linear": (
+        _c_int,
+        [_c_void_p] * 2 + [ctypes.c_float] + [_c_void_p] * 2 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p],
+    ),
+    "hawk_decode_layer_tail": (
+        _c_int,
+        [_c_void_p] * 4 + [ctypes.c_float] + [_c_void_p] * 3 + [ctypes.c_float] + [_c_void_p] * 2 + [_c_int] * 5
+        + [_c_void_p, _c_size_t, _c_void_p],
+    ),
     "hawk_gate_proj_fwd": (_c_int, [_c_void_p] * 7 + [_c_int] * 6 + [_c_void_p]),
     "hawk_conv_gate_proj_fwd": (
         _c_int, [_c_void_p, ctypes.c_longlong] + [_c_void_p] * 9 + [_c_int] * 6 + [_c_void_p]
@@ -189,6 +203,14 @@ def stream_ptr(dev: torch.device) -> int:
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
+def transforms_active() -> bool:
+    """Whether anything watches or rewrites operator calls: dispatch and function modes, functorch's
+    transforms (vmap, grad, jvp), forward-mode differentiation."""
+    return (torch._C._len_torch_dispatch_stack() != 0 or torch._C._len_torch_function_stack() != 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0)
+
+
 def launches_directly(*tensors) -> bool:
     """Whether a kernel can be launched on these tensors without going through its
     ``torch.library`` op.  The op exists for tracing (``torch.compile``, fake tensors, dispatch
@@ -197,7 +219,7 @@ def launches_directly(*tensors) -> bool:
     any of that need none of it: same launch function, same results."""
     if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
         return False
-    if torch._C._len_torch_dispatch_stack() != 0:
+    if transforms_active():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
@@ -344,6 +366,28 @@ def decode_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     return ws
 
 
+_decode_layer_workspaces: dict = {}
+_MAX_DECODE_LAYER_WORKSPACES = 16   # streams; the oldest is dropped first
+
+
+def decode_layer_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
+    """Scratch of a decode step's layers, one buffer per (device, stream): calls on a stream are
+    ordered, and nothing is kept in it from one call to the next.  A graph being recorded gets its
+    own, from its own memory."""
+    if torch.cuda.is_current_stream_capturing():
+        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    key = (_device_index(dev), stream_ptr(dev))
+    with _lock:
+        ws = _decode_layer_workspaces.get(key)
+        if ws is None or ws.numel() < nbytes:
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            _decode_layer_workspaces.pop(key, None)
+            while len(_decode_layer_workspaces) >= _MAX_DECODE_LAYER_WORKSPACES:
+                _decode_layer_workspaces.pop(next(iter(_decode_layer_workspaces)))
+            _decode_layer_workspaces[key] = ws
+    return ws
+
+
 def release_workspaces() -> None:
     """Drop every cached scan and decode workspace (they are re-created on demand)."""
     with _lock:
@@ -351,6 +395,7 @@ def release_workspaces() -> None:
         _captured.clear()
         _decode_workspaces.clear()
         _decode_captured.clear()
+        _decode_layer_workspaces.clear()
 
 
 def _flag_of(ws: torch.Tensor, dev: torch.device) -> int:

@@ -304,6 +304,64 @@ int hawk_decode_core_step(void* conv_state, const void* x_new, long long ldx, co
                                     stream);
 }
 
+int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }
+
+size_t hawk_decode_linear_workspace_bytes(int M, int N, int K) {
+    return hawk::decode_linear_supported(M, N, K) ? hawk::decode_linear_workspace_bytes(M, N, K) : 0;
+}
+
+int hawk_decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* workspace_device,
+                       size_t workspace_bytes, void* stream) {
+    if (!x || !w || !out) return HAWK_ERR_NULL_POINTER;
+    if (!hawk::decode_linear_supported(M, N, K)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(x) || !aligned16(w) || !aligned16(out)) return HAWK_ERR_ALIGNMENT;
+    const size_t need = hawk::decode_linear_workspace_bytes(M, N, K);
+    if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;
+    if (!aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    return hawk::decode_linear(x, w, out, M, N, K, workspace_device, as_stream(stream));
+}
+
+int hawk_decode_layer_supported(int M, int H, int R, int I) {
+    return (hawk::decode_norm_supported(H) && hawk::decode_linear_supported(M, H, R) &&
+            hawk::decode_linear_supported(M, I, H) && hawk::decode_linear_supported(M, H, I))
+               ? 1 : 0;
+}
+
+size_t hawk_decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next) {
+    if (!hawk_decode_layer_supported(M, H, R, I) || !hawk::decode_linear_supported(M, n_next, H)) return 0;
+    return hawk::decode_layer_workspace_bytes(M, H, R, I, n_next);
+}
+
+int hawk_decode_norm_linear(void* hidden, const void* norm_w, float eps, const void* w, void* out, int M, int N, int H,
+                            void* workspace_device, size_t workspace_bytes, void* stream) {
+    if (!hidden || !norm_w || !w || !out) return HAWK_ERR_NULL_POINTER;
+    if (!hawk::decode_norm_supported(H) || !hawk::decode_linear_supported(M, N, H)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(hidden) || !aligned16(norm_w) || !aligned16(w) || !aligned16(out)) return HAWK_ERR_ALIGNMENT;
+    const size_t need = ((size_t)M * H * 2 + 255) / 256 * 256 + hawk::decode_linear_workspace_bytes(M, N, H);
+    if (!workspace_device || workspace_bytes < need) return HAWK_ERR_WORKSPACE;
+    if (!aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    return hawk::decode_norm_linear(hidden, norm_w, eps, w, out, M, N, H, workspace_device, as_stream(stream));
+}
+
+int hawk_decode_layer_tail(const void* gated, const void* w_resid, void* hidden, const void* norm_w, float eps,
+                           const void* w_gate_up, const void* w_down, const void* next_norm_w, float next_eps,
+                           const void* w_next, void* next_out, int M, int H, int R, int I, int n_next,
+                           void* workspace_device, size_t workspace_bytes, void* stream) {
+    if (!gated || !w_resid || !hidden || !norm_w || !w_gate_up || !w_down || !next_norm_w || !w_next || !next_out)
+        return HAWK_ERR_NULL_POINTER;
+    if (!hawk_decode_layer_supported(M, H, R, I) || !hawk::decode_linear_supported(M, n_next, H))
+        return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(gated) || !aligned16(w_resid) || !aligned16(hidden) || !aligned16(norm_w) ||
+        !aligned16(w_gate_up) || !aligned16(w_down) || !aligned16(next_norm_w) || !aligned16(w_next) ||
+        !aligned16(next_out))
+        return HAWK_ERR_ALIGNMENT;
+    if (!workspace_device || workspace_bytes < hawk::decode_layer_workspace_bytes(M, H, R, I, n_next))
+        return HAWK_ERR_WORKSPACE;
+    if (!aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    return hawk::decode_layer_tail(gated, w_resid, hidden, norm_w, eps, w_gate_up, w_down, next_norm_w, next_eps,
+                                   w_next, next_out, M, H, R, I, n_next, workspace_device, as_stream(stream));
+}
+
 int hawk_gate_proj_fwd(const void* x, const void* w_i, const float* b_i, const void* w_a, const float* b_a,
                        void* x_rg_lru, void* a_rg_lru, int M, int D, int num_blocks, int x_dtype, int w_dtype,
                        int out_dtype, void* stream) {

@@ -1,0 +1,602 @@
+// Decode step around the recurrent core: the dense projections of a layer for a handful of rows
+// (one new token per sequence), with the norms, residual adds and the gated GELU in the same
+// kernels.  Upstream runs them as library GEMMs with eager kernels in between
+// (hawk/hawk.py:53-58, :70-86, :163-203, :222-243, :284-303).
+//
+// With up to 256 rows a projection is a pass over its weights: 2560 x 15360 bf16 weights are
+// 79 MB, 14 us at the rate a large copy reaches, and their 20 GFLOP at 256 rows are half of that
+// on the matrix cores.  What the kernel must do is keep enough weight bytes in flight and touch
+// every byte in as few places as possible:
+//   * a workgroup of four waves owns MT rows x 64 output columns; the weights are read once per
+//     MT rows, in full 128-byte lines, through registers into LDS;
+//   * the waves split K, not the tile: wave w multiplies the w-th 16 of every 64 input channels for
+//     the whole tile, so each staged byte is read from LDS exactly once.  With the tile split over
+//     the waves instead every weight byte is read by as many waves as there are row blocks;
+//   * the four partial tiles meet in LDS at the end and leave in whole rows;
+//   * projections with few columns also split K over workgroups and leave fp32 partial sums, which
+//     the kernel that follows (residual add + norm) adds up in a fixed order on its way.
+// All sums are fp32, in an order that depends on the shape alone, and values are rounded to bf16 where
+// the separate operations round them, so both routes differ by the order of the sums only.
+#include "hawk_scan.h"
+
+#include <stdint.h>
+
+#include "hawk_device.h"
+
+namespace hawk {
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kWaves = 4;
+constexpr int kThreads = kWaves * kWave;
+constexpr int kNT = 64;          // output columns of a workgroup
+constexpr int kKT = 64;          // input channels of a step: 128 bytes of a row
+constexpr int kRowBytes = kKT * 2;
+
+enum Epilogue { kStoreBf16 = 0, kStorePartial = 1, kStoreGelu = 2 };
+
+inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+
+// 16-byte piece `c` of row `r` of a staged tile.  The pieces of a row are permuted by the row's
+// number, so that the 8 rows one LDS cycle reads the same piece of cover all banks.
+__device__ __forceinline__ int piece_offset(int r, int c) { return r * kRowBytes + ((c ^ (r & 7)) << 4); }
+
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// One thread's share of a finished row: 8 adjacent columns a, c, or 4 gate columns a and the up
+// columns c beside them.
+template <int EPI>
+__device__ __forceinline__ void store_columns(void* out, f32x4 a, f32x4 c, int split, int m, int n, int M, int N) {
+    if constexpr (EPI == kStorePartial) {
+        float* o = static_cast<float*>(out) + ((size_t)split * M + m) * N + n;
+        *reinterpret_cast<f32x4*>(o) = a;
+        *reinterpret_cast<f32x4*>(o + 4) = c;
+    } else if constexpr (EPI == kStoreBf16) {
+        const u32x4 r = {pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w), pack_bf16x2(c.x, c.y), pack_bf16x2(c.z, c.w)};
+        *reinterpret_cast<u32x4*>(static_cast<bf16_t*>(out) + (size_t)m * N + n) = r;
+    } else {
+        // rounded where the separate operations round: the projection, the GELU, the product
+        float g[4], u[4];
+        unpack(u32x2{pack_bf16x2(a.x, a.y), pack_bf16x2(a.z, a.w)}, g);
+        unpack(u32x2{pack_bf16x2(c.x, c.y), pack_bf16x2(c.z, c.w)}, u);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) g[v] = gelu_times(g[v], 1.0f);
+        unpack(u32x2{pack_bf16x2(g[0], g[1]), pack_bf16x2(g[2], g[3])}, g);
+        const u32x2 r = {pack_bf16x2(g[0] * u[0], g[1] * u[1]), pack_bf16x2(g[2] * u[2], g[3] * u[3])};
+        *reinterpret_cast<u32x2*>(static_cast<bf16_t*>(out) + (size_t)m * N + n) = r;
+    }
+}
+
+template <int MT>
+struct GemmLds {
+    static constexpr int kStage = (MT + kNT) * kRowBytes;
+    static constexpr int kSums = kWaves * 32 * kNT * 4;      // the waves' sums of 32 rows
+    static constexpr int kBytes = 2 * kStage > kSums ? 2 * kStage : kSums;
+};
+
+// out = x w^T for x [M, K] and w [N, K], both bf16 with dense rows; K a multiple of DEPTH * 64, N of 8.
+//   kStoreBf16     out [M, N] bf16
+//   kStorePartial  out [splits, M, N] fp32, split s over its share of K
+//   kStoreGelu     w [2 N, K] holds gate rows, then up rows; out [M, N] bf16 = gelu(gate) * up
+// DEPTH: tiles kept in flight in registers.
+template <int MT, int DEPTH, int EPI>
+__global__ __launch_bounds__(kThreads, 3) void decode_gemm_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
+    int ntiles, int mtiles, int splits) {
+    constexpr int MB = MT / 32;
+    constexpr int XP = MT / 32;               // 16-byte loads per thread and step for x; the weights take two
+    static_assert(DEPTH == 2 || DEPTH == 4, "an even number of steps per turn of the loop");
+    __shared__ __align__(16) unsigned char smem[GemmLds<MT>::kBytes];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+
+    // The row tiles of one weight tile sit 8 workgroups apart: on the same XCD, at the same time,
+    // so the second one finds the weights in that XCD's L2.
+    const int b = (int)blockIdx.x;
+    const int group = b / (8 * mtiles), in_group = b - group * 8 * mtiles;
+    const int mt = in_group / 8;
+    const int item = group * 8 + (in_group & 7);
+    if (item >= ntiles * splits) return;      // the grid is padded to whole groups of 8
+    const int split = item / ntiles;
+    const int nt = item - split * ntiles;
+    const int m0 = mt * MT, n0 = nt * (EPI == kStoreGelu ? kNT / 2 : kNT);
+
+    // this split's share of K, in turns of DEPTH steps
+    const int turns = K / (DEPTH * kKT);
+    const int turn0 = (int)((long long)turns * split / splits);
+    const int turn1 = (int)((long long)turns * (split + 1) / splits);
+    const int steps = (turn1 - turn0) * DEPTH;
+    const uint32_t k_bytes0 = (uint32_t)turn0 * DEPTH * kRowBytes;
+    const uint32_t row_bytes = (uint32_t)K * 2u;
+    // rows past M and weight rows past N read as zeros (range check of the buffer resources)
+    const rsrc_t bx = make_rsrc(x + (size_t)m0 * K, (uint32_t)min(MT, M - m0) * row_bytes);
+    const int n1 = EPI == kStoreGelu ? N + n0 : n0 + 32;            // first row of the tile's second half
+    const int rows0 = min(32, N - n0), rows1 = EPI == kStoreGelu ? rows0 : max(min(32, N - n1), 0);
+    const rsrc_t bw0 = make_rsrc(w + (size_t)n0 * K, (uint32_t)rows0 * row_bytes);
+    const rsrc_t bw1 = make_rsrc(rows1 > 0 ? w + (size_t)n1 * K : w, (uint32_t)rows1 * row_bytes);
+
+    const int lr = tid / 8, lc = tid & 7;     // a load covers 32 rows of 128 bytes
+    const uint32_t lane_bytes = (uint32_t)lr * row_bytes + (uint32_t)lc * 16u;
+    const int piece = piece_offset(lr, lc);   // (rows 32 apart have the same permutation)
+
+    u32x4 rx[DEPTH][XP], rw[DEPTH][2];
+    auto load = [&](int slot, int step) {
+        const uint32_t k = k_bytes0 + (uint32_t)min(step, steps - 1) * kRowBytes;
+        // The loads keep this order, here and in front of the loop: the compiler counts them to know
+        // which have arrived, and where two orders meet it waits for all of the younger step too.
+#pragma unroll
+        for (int p = 0; p < XP; ++p) {
+            rx[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        bx, lane_bytes + p * 32u * row_bytes + k, 0, kAuxDefault));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        rw[slot][0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(bw0, lane_bytes + k, 0, kAuxDefault));
+        __builtin_amdgcn_sched_barrier(0);
+        rw[slot][1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(bw1, lane_bytes + k, 0, kAuxDefault));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto stage = [&](int slot, int buf) {
+        unsigned char* s = smem + buf * GemmLds<MT>::kStage;
+#pragma unroll
+        for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(s + p * 32 * kRowBytes + piece) = rx[slot][p];
+        *reinterpret_cast<u32x4*>(s + MT * kRowBytes + piece) = rw[slot][0];
+        *reinterpret_cast<u32x4*>(s + (MT + 32) * kRowBytes + piece) = rw[slot][1];
+    };
+
+    f32x16 acc[MB][2];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[mb][nh][i] = 0.0f;
+
+    // operand of this wave: 16 input channels = two 16-byte pieces of every row
+    const int op = piece_offset(lane & 31, 2 * wv + (lane >> 5));
+
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load(d, d);
+    stage(0, 0);
+    load(0, DEPTH);
+    lds_barrier();
+    for (int t = 0; t < steps; t += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            // buffer d & 1 holds step t + d; the next step's tile is written beside it, its slot
+            // asks for the tile DEPTH steps on, and the products hide both
+            const unsigned char* s = smem + (d & 1) * GemmLds<MT>::kStage;
+            bf16x8 fw[2], fx[MB];
+#pragma unroll
+            for (int nh = 0; nh < 2; ++nh)
+                fw[nh] = *reinterpret_cast<const bf16x8*>(s + (MT + 32 * nh) * kRowBytes + op);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) fx[mb] = *reinterpret_cast<const bf16x8*>(s + 32 * mb * kRowBytes + op);
+            stage((d + 1) % DEPTH, (d + 1) & 1);
+            load((d + 1) % DEPTH, t + d + 1 + DEPTH);
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int nh = 0; nh < 2; ++nh)
+                    acc[mb][nh] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[nh], fx[mb], acc[mb][nh], 0, 0, 0);
+            lds_barrier();
+        }
+    }
+
+    // The waves' sums of 32 rows at a time meet in LDS: [wave][row][16 pieces of 4 columns], pieces
+    // permuted by the row like the staged tiles; then 8 threads finish one row.
+    const int er = tid / 8, ec = tid & 7;
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+        if (mb > 0) lds_barrier();
+#pragma unroll
+        for (int nh = 0; nh < 2; ++nh)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int r = lane & 31, c = nh * 8 + 2 * g + (lane >> 5);
+                const f32x4 v = {acc[mb][nh][4 * g], acc[mb][nh][4 * g + 1], acc[mb][nh][4 * g + 2],
+                                 acc[mb][nh][4 * g + 3]};
+                *reinterpret_cast<f32x4*>(smem + ((wv * 32 + r) * 16 + (c ^ (r & 7))) * 16) = v;
+            }
+        lds_barrier();
+        const int m = m0 + mb * 32 + er;
+        f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f}, c = a;
+        // kStoreGelu: 4 gate columns and the up columns beside them; else 8 adjacent columns
+        const int pa = EPI == kStoreGelu ? ec : 2 * ec, pc = EPI == kStoreGelu ? 8 + ec : 2 * ec + 1;
+#pragma unroll
+        for (int q = 0; q < kWaves; ++q) {
+            a += *reinterpret_cast<const f32x4*>(smem + ((q * 32 + er) * 16 + (pa ^ (er & 7))) * 16);
+            c += *reinterpret_cast<const f32x4*>(smem + ((q * 32 + er) * 16 + (pc ^ (er & 7))) * 16);
+        }
+        const int n = n0 + (EPI == kStoreGelu ? 4 : 8) * ec;
+        if (m < M && n < N) {
+            store_columns<EPI>(out, a, c, split, m, n, M, N);
+        }
+    }
+}
+
+// The same products for more than 64 rows, in tiles of 128 rows x NT columns.  Here the bytes that
+// pass from the L2s into the compute units set the pace, not HBM: one compute unit takes in about
+// 23 bytes per clock (counters: 77 cache lines in flight at 430 clocks each, the L1 stalled on
+// pending misses for half of the time, LDS and matrix cores below 40 %), so the tile is as square as
+// the number of workgroups allows: 256 rows x 15360 columns x 2560 take 43 us in tiles of 128 x 64, 39 in
+// tiles of 256 x 64 and 36.5 in tiles of 128 x 128.  (Eight waves instead of four and loads four
+// steps ahead instead of two changed nothing; neither did starting at different places of K.)  The waves split the tile 2 x 2; what that reads from LDS more than
+// once stays below what arrives from the L1.
+template <int NT>
+struct WideLds {
+    static constexpr int kStage = (128 + NT) * kRowBytes;
+    static constexpr int kBytes = 2 * kStage > 128 * NT * 4 ? 2 * kStage : 128 * NT * 4;
+};
+
+template <int NT, int DEPTH, int EPI>
+__global__ __launch_bounds__(kThreads, NT >= 128 ? 1 : 2) void decode_gemm_wide_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
+    int ntiles, int mtiles, int splits) {
+    constexpr int MT = 128;
+    constexpr int XP = MT / 32, WP = NT / 32, NB = NT / 64;
+    constexpr int NC = EPI == kStoreGelu ? NT / 2 : NT;       // output columns of a tile
+    __shared__ __align__(16) unsigned char smem[WideLds<NT>::kBytes];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int wm = wv & 1, wn = wv >> 1;
+
+    // row tiles of one weight tile 8 workgroups apart, as above
+    const int b = (int)blockIdx.x;
+    const int group = b / (8 * mtiles), in_group = b - group * 8 * mtiles;
+    const int item = group * 8 + (in_group & 7);
+    if (item >= ntiles * splits) return;
+    const int split = item / ntiles;
+    const int nt = item - split * ntiles;
+    const int m0 = in_group / 8 * MT, n0 = nt * NC;
+
+    const int turns = K / (DEPTH * kKT);
+    const int turn0 = (int)((long long)turns * split / splits);
+    const int turn1 = (int)((long long)turns * (split + 1) / splits);
+    const int steps = (turn1 - turn0) * DEPTH;
+    const uint32_t k_bytes0 = (uint32_t)turn0 * DEPTH * kRowBytes;
+    const uint32_t row_bytes = (uint32_t)K * 2u;
+
+    // rows past M and weight rows past N read as zeros
+    const rsrc_t bx = make_rsrc(x + (size_t)m0 * K, (uint32_t)min(MT, M - m0) * row_bytes);
+    const uint32_t w_bytes = (uint32_t)min(NC, N - n0) * row_bytes;
+    const rsrc_t bw = make_rsrc(w + (size_t)n0 * K, w_bytes);
+    const rsrc_t bup = make_rsrc(EPI == kStoreGelu ? w + (size_t)(N + n0) * K : w, w_bytes);
+
+    const int lr = tid / 8, lc = tid & 7;
+    const uint32_t lane_bytes = (uint32_t)lr * row_bytes + (uint32_t)lc * 16u;
+    const int piece = piece_offset(lr, lc);
+
+    u32x4 rx[DEPTH][XP], rw[DEPTH][WP];
+    auto load = [&](int slot, int step) {
+        const uint32_t k = k_bytes0 + (uint32_t)min(step, steps - 1) * kRowBytes;
+#pragma unroll
+        for (int p = 0; p < XP; ++p) {
+            rx[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        bx, lane_bytes + p * 32u * row_bytes + k, 0, kAuxDefault));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int p = 0; p < WP; ++p) {
+            const bool up = EPI == kStoreGelu && p >= WP / 2;
+            const uint32_t off = lane_bytes + (uint32_t)(up ? p - WP / 2 : p) * 32u * row_bytes + k;
+            rw[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(up ? bup : bw, off, 0,
+                                                                                          kAuxDefault));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto stage = [&](int slot, int buf) {
+        unsigned char* s = smem + buf * WideLds<NT>::kStage + piece;
+#pragma unroll
+        for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(s + p * 32 * kRowBytes) = rx[slot][p];
+#pragma unroll
+        for (int p = 0; p < WP; ++p) *reinterpret_cast<u32x4*>(s + (MT + p * 32) * kRowBytes) = rw[slot][p];
+    };
+
+    f32x16 acc[2][NB];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.0f;
+
+    const int xrow = wm * 64 + (lane & 31), wrow = MT + wn * (NT / 2) + (lane & 31);
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) load(d, d);
+    stage(0, 0);
+    load(0, DEPTH);
+    lds_barrier();
+    for (int t = 0; t < steps; t += DEPTH) {
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            const unsigned char* s = smem + (d & 1) * WideLds<NT>::kStage;
+            stage((d + 1) % DEPTH, (d + 1) & 1);
+            load((d + 1) % DEPTH, t + d + 1 + DEPTH);
+#pragma unroll
+            for (int ks = 0; ks < kKT / 16; ++ks) {
+                bf16x8 fx[2], fw[NB];
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+                    fx[mb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(xrow + 32 * mb, 2 * ks + (lane >> 5)));
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb)
+                    fw[nb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(wrow + 32 * nb, 2 * ks + (lane >> 5)));
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[nb], fx[mb], acc[mb][nb], 0, 0, 0);
+            }
+            lds_barrier();
+        }
+    }
+
+    // the tile through LDS, [128 rows][NT / 4 pieces of 4 columns] with the pieces permuted by the row,
+    // so that it leaves in whole rows
+    constexpr int PR = NT / 4;
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int r = wm * 64 + mb * 32 + (lane & 31);
+                const int c = (wn * (NT / 2) + nb * 32) / 4 + 2 * g + (lane >> 5);
+                const f32x4 v = {acc[mb][nb][4 * g], acc[mb][nb][4 * g + 1], acc[mb][nb][4 * g + 2],
+                                 acc[mb][nb][4 * g + 3]};
+                *reinterpret_cast<f32x4*>(smem + (r * PR + (c ^ (r & 7))) * 16) = v;
+            }
+    lds_barrier();
+    constexpr int CPT = EPI == kStoreGelu ? 4 : 8;            // output columns per thread
+    constexpr int TPR = NC / CPT;                             // threads per row
+    const int ec = tid % TPR;
+    const int n = n0 + CPT * ec;
+#pragma unroll
+    for (int r = tid / TPR; r < MT; r += kThreads / TPR) {
+        const int m = m0 + r;
+        const int pa = EPI == kStoreGelu ? ec : 2 * ec, pc = EPI == kStoreGelu ? PR / 2 + ec : 2 * ec + 1;
+        const f32x4 a = *reinterpret_cast<const f32x4*>(smem + (r * PR + (pa ^ (r & 7))) * 16);
+        const f32x4 c = *reinterpret_cast<const f32x4*>(smem + (r * PR + (pc ^ (r & 7))) * 16);
+        if (m < M && n < N) store_columns<EPI>(out, a, c, split, m, n, M, N);
+    }
+}
+
+// out = the sum of S partial sums [S, n], rounded once: the last step of a product split over K whose
+// output is read as bf16.
+template <int S>
+__global__ __launch_bounds__(256) void sum_partial_kernel(const float* __restrict__ partial, bf16_t* __restrict__ out,
+                                                          size_t n) {
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (at >= n) return;
+    f32x4 part[S][2];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        part[s][0] = *reinterpret_cast<const f32x4*>(partial + s * n + at);
+        part[s][1] = *reinterpret_cast<const f32x4*>(partial + s * n + at + 4);
+    }
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        v[k] = part[0][k / 4][k % 4];
+#pragma unroll
+        for (int s = 1; s < S; ++s) v[k] += part[s][k / 4][k % 4];
+    }
+    u32x4 r;
+    pack(v, r);
+    *reinterpret_cast<u32x4*>(out + at) = r;
+}
+
+int sum_partial(const float* partial, int splits, void* out, size_t n, hipStream_t st) {
+    const dim3 grid((unsigned)((n / 8 + 255) / 256));
+    bf16_t* o = static_cast<bf16_t*>(out);
+    switch (splits) {
+#define HAWK_SUM(S) \
+    case S: hipLaunchKernelGGL((sum_partial_kernel<S>), grid, dim3(256), 0, st, partial, o, n); break;
+        HAWK_SUM(2) HAWK_SUM(3) HAWK_SUM(4) HAWK_SUM(5) HAWK_SUM(6) HAWK_SUM(7) HAWK_SUM(8)
+#undef HAWK_SUM
+        default: return HAWK_ERR_BAD_SHAPE;
+    }
+    return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
+}
+
+// hidden += the sum of S partial sums, then out = hidden / rms(hidden) * weight; the sum, the new hidden
+// state and the result are each rounded to bf16 once, as the separate operations round them
+// (hawk/hawk.py:53-58, :236-241).  One workgroup per row, 8 channels per thread: latency is all it
+// costs, so every load of a thread is in flight before the first is used (S is a template
+// parameter for that: with a loop over the partial sums their round trips added up, 7.8 against
+// 4.9 us at 128 rows of 2560 and 8 of them).
+constexpr int kNormMaxThreads = 1024;
+
+template <int S>
+__global__ __launch_bounds__(kNormMaxThreads) void add_norm_kernel(bf16_t* __restrict__ hidden,
+                                                                   const float* __restrict__ partial,
+                                                                   const bf16_t* __restrict__ weight, float eps,
+                                                                   bf16_t* __restrict__ out, int M, int D) {
+    __shared__ float s_sum[kNormMaxThreads / kWave];
+    const int m = (int)blockIdx.x, c = 8 * (int)threadIdx.x;
+    const bool on = c < D;
+    const size_t at = (size_t)m * D + (on ? c : 0);
+    const u32x4 h = load_raw<bf16_t, 8>(hidden + at);
+    const u32x4 wraw = load_raw<bf16_t, 8>(weight + (on ? c : 0));
+    f32x4 part[S > 0 ? S : 1][2];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const float* p = partial + (size_t)s * M * D + at;
+        part[s][0] = *reinterpret_cast<const f32x4*>(p);
+        part[s][1] = *reinterpret_cast<const f32x4*>(p + 4);
+    }
+    float v[8], sq = 0.0f;
+    unpack(h, v);
+    if constexpr (S > 0) {
+        float add[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            add[k] = part[0][k / 4][k % 4];
+#pragma unroll
+            for (int s = 1; s < S; ++s) add[k] += part[s][k / 4][k % 4];
+        }
+        u32x4 r;
+        pack(add, r);        // rounded where a separate projection rounds its output
+        unpack(r, add);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v[k] += add[k];
+        pack(v, r);
+        if (on) *reinterpret_cast<u32x4*>(hidden + at) = r;
+        unpack(r, v);     // the norm sees the hidden state as it is kept
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) sq = fmaf(v[k], v[k], sq);
+    if (!on) sq = 0.0f;
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+    if ((threadIdx.x & (kWave - 1)) == 0) s_sum[threadIdx.x / kWave] = sq;
+    __syncthreads();
+    float total = 0.0f;
+    for (int k = 0; k < (int)blockDim.x / kWave; ++k) total += s_sum[k];
+    const float scale = 1.0f / sqrtf(total / (float)D + eps);
+    float g[8];
+    unpack(wraw, g);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) g[k] *= v[k] * scale;
+    u32x4 r;
+    pack(g, r);
+    if (on) *reinterpret_cast<u32x4*>(out + at) = r;
+}
+
+int add_norm(void* hidden, const float* partial, int splits, const void* weight, float eps, void* out, int M, int D,
+             hipStream_t st) {
+    const dim3 grid((unsigned)M), block((unsigned)(ceil_div(D / 8, kWave) * kWave));
+    bf16_t* h = static_cast<bf16_t*>(hidden);
+    const bf16_t* w = static_cast<const bf16_t*>(weight);
+    bf16_t* o = static_cast<bf16_t*>(out);
+    switch (splits) {
+#define HAWK_NORM(S) \
+    case S: hipLaunchKernelGGL((add_norm_kernel<S>), grid, block, 0, st, h, partial, w, eps, o, M, D); break;
+        HAWK_NORM(0) HAWK_NORM(1) HAWK_NORM(2) HAWK_NORM(3) HAWK_NORM(4) HAWK_NORM(5) HAWK_NORM(6) HAWK_NORM(7) HAWK_NORM(8)
+#undef HAWK_NORM
+        default: return HAWK_ERR_BAD_SHAPE;
+    }
+    return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
+}
+
+// How a product is cut: rows and columns of a tile, tiles in flight, workgroups along K.
+struct Cut {
+    int mt, nt, depth, splits;
+};
+// Workgroups a product that is split over K is cut into: one per compute unit.  Measured on a layer
+// of 2560 x 7680 (four products, two norms): 240 gives 49 / 53 / 63 / 82 / 104 us at 1 / 32 / 64 / 128 /
+// 256 rows, 320 gives 52 / 59 / 71 / 95 / 121 (the partial sums of more splits cost more than the
+// second workgroup on a compute unit brings), 160 gives 49 / 55 / 67 / 84 / 114.
+constexpr int kSplitWorkgroups = 240;
+// Tiles of 128 x 128 from this many of them on; with fewer, part of the chip would be idle.
+constexpr int kMinWideTiles = 200;
+
+Cut cut_for(int M, int N, int K, bool gelu, bool may_split) {
+    Cut c;
+    c.mt = M <= 32 ? 32 : (M <= 64 ? 64 : 128);
+    c.nt = kNT;
+    c.depth = K % (4 * kKT) == 0 ? 4 : 2;
+    c.splits = 1;
+    const int mtiles = ceil_div(M, c.mt), cols = gelu ? 2 * N : N;
+    if (c.mt == 128) {
+        if (!may_split && ceil_div(cols, 128) * mtiles >= kMinWideTiles) c.nt = 128;
+        else c.depth = 2;
+    }
+    if (may_split) {
+        const int tiles = ceil_div(cols, c.nt) * mtiles, turns = K / (c.depth * kKT);
+        int s = kSplitWorkgroups / tiles;
+        if (s > kDecodeMaxSplits) s = kDecodeMaxSplits;
+        if (s > turns / 2) s = turns / 2;    // shorter loops are all filling of the pipeline
+        c.splits = s < 1 ? 1 : s;
+    }
+    return c;
+}
+
+template <int EPI>
+int gemm(const void* x, const void* w, void* out, int M, int N, int K, const Cut& c, hipStream_t st) {
+    const int ntiles = ceil_div(N, EPI == kStoreGelu ? c.nt / 2 : c.nt), mtiles = ceil_div(M, c.mt);
+    const dim3 grid((unsigned)(ceil_div(ntiles * c.splits, 8) * 8 * mtiles));
+    const bf16_t* xp = static_cast<const bf16_t*>(x);
+    const bf16_t* wp = static_cast<const bf16_t*>(w);
+#define HAWK_GEMM(KERNEL, TILE, DEPTH)                                                                                      \
+    hipLaunchKernelGGL((KERNEL<TILE, DEPTH, EPI>), grid, dim3(kThreads), 0, st, xp, wp, out, M, N, K, ntiles, mtiles, \
+                       c.splits)
+    if (c.mt == 32) {
+        if (c.depth == 4) HAWK_GEMM(decode_gemm_kernel, 32, 4);
+        else HAWK_GEMM(decode_gemm_kernel, 32, 2);
+    } else if (c.mt == 64) {
+        if (c.depth == 4) HAWK_GEMM(decode_gemm_kernel, 64, 4);
+        else HAWK_GEMM(decode_gemm_kernel, 64, 2);
+    } else if (c.nt == 64) {
+        HAWK_GEMM(decode_gemm_wide_kernel, 64, 2);
+    } else {
+        if (c.depth == 4) HAWK_GEMM(decode_gemm_wide_kernel, 128, 4);
+        else HAWK_GEMM(decode_gemm_wide_kernel, 128, 2);
+    }
+#undef HAWK_GEMM
+    return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
+}
+
+}  // namespace
+
+bool decode_linear_supported(int M, int N, int K) {
+    return M >= 1 && M <= kDecodeMaxRows && N >= 8 && N % 8 == 0 && N <= (1 << 20) && K >= 2 * kKT &&
+           K % (2 * kKT) == 0 && K <= 65536;
+}
+bool decode_norm_supported(int D) { return D >= 8 && D % 8 == 0 && D <= 8 * kNormMaxThreads; }
+
+// The workspace of a layer: normed rows, the MLP's product, partial sums.
+size_t decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next) {
+    const size_t a = (size_t)cut_for(M, H, R, false, true).splits * H, b = (size_t)cut_for(M, H, I, false, true).splits * H;
+    const size_t c = (size_t)cut_for(M, n_next, H, false, true).splits * n_next;
+    const size_t most = a > b ? (a > c ? a : c) : (b > c ? b : c);
+    return align256((size_t)M * H * 2) + align256((size_t)M * I * 2) + align256(most * M * sizeof(float));
+}
+
+size_t decode_linear_workspace_bytes(int M, int N, int K) {
+    const Cut c = cut_for(M, N, K, false, true);
+    return c.splits > 1 ? (size_t)c.splits * M * N * sizeof(float) : 0;
+}
+
+int decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* ws, hipStream_t st) {
+    const Cut c = cut_for(M, N, K, false, true);
+    if (c.splits == 1) return gemm<kStoreBf16>(x, w, out, M, N, K, cut_for(M, N, K, false, false), st);
+    if (int rc = gemm<kStorePartial>(x, w, ws, M, N, K, c, st)) return rc;
+    return sum_partial(static_cast<const float*>(ws), c.splits, out, (size_t)M * N, st);
+}
+
+int decode_norm_linear(void* hidden, const void* norm_w, float eps, const void* w, void* out, int M, int N, int H,
+                       void* ws, hipStream_t st) {
+    if (int rc = add_norm(hidden, nullptr, 0, norm_w, eps, ws, M, H, st)) return rc;
+    return decode_linear(ws, w, out, M, N, H, static_cast<char*>(ws) + align256((size_t)M * H * 2), st);
+}
+
+int decode_layer_tail(const void* gated, const void* w_resid, void* hidden, const void* norm_w, float eps,
+                      const void* w_gate_up, const void* w_down, const void* next_norm_w, float next_eps,
+                      const void* w_next, void* next_out, int M, int H, int R, int I, int n_next, void* ws,
+                      hipStream_t st) {
+    char* p = static_cast<char*>(ws);
+    void* normed = p;
+    void* act = p + align256((size_t)M * H * 2);
+    float* partial = reinterpret_cast<float*>(p + align256((size_t)M * H * 2) + align256((size_t)M * I * 2));
+    const Cut resid = cut_for(M, H, R, false, true), down = cut_for(M, H, I, false, true);
+    if (int rc = gemm<kStorePartial>(gated, w_resid, partial, M, H, R, resid, st)) return rc;
+    if (int rc = add_norm(hidden, partial, resid.splits, norm_w, eps, normed, M, H, st)) return rc;
+    if (int rc = gemm<kStoreGelu>(normed, w_gate_up, act, M, I, H, cut_for(M, I, H, true, false), st)) return rc;
+    if (int rc = gemm<kStorePartial>(act, w_down, partial, M, H, I, down, st)) return rc;
+    if (int rc = add_norm(hidden, partial, down.splits, next_norm_w, next_eps, normed, M, H, st)) return rc;
+    return decode_linear(normed, w_next, next_out, M, n_next, H, partial, st);
+}
+
+}  // namespace hawk

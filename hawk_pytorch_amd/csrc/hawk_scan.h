@@ -101,6 +101,22 @@ int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, 
                    int D, int nb, int W, void* scan_ws, size_t scan_ws_bytes, void* gate_ws, size_t gate_ws_bytes,
                    void* conv_ws, size_t conv_ws_bytes, hipStream_t st);
 
+// hawk_decode.hip
+// x w^T for up to kDecodeMaxRows rows; see include/hawk_hip.h for the operands
+constexpr int kDecodeMaxRows = 256;
+constexpr int kDecodeMaxSplits = 8;
+bool decode_linear_supported(int M, int N, int K);
+bool decode_norm_supported(int D);
+size_t decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next);
+size_t decode_linear_workspace_bytes(int M, int N, int K);
+int decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* ws, hipStream_t st);
+int decode_norm_linear(void* hidden, const void* norm_w, float eps, const void* w, void* out, int M, int N, int H,
+                       void* ws, hipStream_t st);
+int decode_layer_tail(const void* gated, const void* w_resid, void* hidden, const void* norm_w, float eps,
+                      const void* w_gate_up, const void* w_down, const void* next_norm_w, float next_eps,
+                      const void* w_next, void* next_out, int M, int H, int R, int I, int n_next, void* ws,
+                      hipStream_t st);
+
 // hawk_probe.hip
 bool stream_probe_shape_ok(size_t bytes, size_t row_pitch, int shape);
 int stream_probe(const void* const* reads, int n_reads, void* const* writes, int n_writes, size_t bytes,

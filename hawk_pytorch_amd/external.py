@@ -312,13 +312,12 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     if ldx % 8 != 0 or xn.data_ptr() % 16 != 0:
         xn, ldx = _lib.dense16(xn.contiguous()), D
     y2, ldy = rows(y)
-    w32, b32 = _lib.dense16(conv.w.detach().float()), _lib.dense16(conv.b.detach().float())
+    w32, b32, b_i, b_a, lam = (
+        t if t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+        else _lib.dense16(t.detach().float()) for t in (conv.w, conv.b, input_gate.b, a_gate.b, a_param))
     w_i, w_a = _lib.dense16(input_gate.w.detach()), _lib.dense16(a_gate.w.detach())
     if w_a.dtype != w_i.dtype:
         w_a = w_a.to(w_i.dtype)
-    b_i = _lib.dense16(input_gate.b.detach().float().reshape(D))
-    b_a = _lib.dense16(a_gate.b.detach().float().reshape(D))
-    lam = _lib.dense16(a_param.detach().float())
     out = torch.empty((B, D), dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
     with _lib.on_device(dev):
@@ -334,6 +333,51 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
         )
     _lib.check("hawk_decode_core_step_ws", status)
     return out.reshape(shape)
+
+
+# ---------------------------------------------------------------------------------------
+# The dense part of a decode step: the layers' projections, norms, residual adds and gated GELU for
+# up to 256 rows (hawk/hawk.py:53-58, :70-86, :163-166, :198-203, :222-243, :284-303 upstream).
+# ---------------------------------------------------------------------------------------
+def decode_layers_supported(M: int, H: int, R: int, inter: int, vocab: int) -> bool:
+    lib = _lib.load()
+    return bool(lib.hawk_decode_layer_supported(M, H, R, inter) and lib.hawk_decode_linear_supported(M, 2 * R, H)
+                and lib.hawk_decode_linear_supported(M, vocab, H))
+
+
+class DecodeLayers:
+    """The launches of one decode step around the recurrent cores, on one hidden state [M, H] (bf16,
+    updated in place).  All weights are plain dense bf16 CUDA tensors of the step's device."""
+
+    def __init__(self, hidden: torch.Tensor, R: int, inter: int, vocab: int):
+        self.hidden = hidden
+        self.M, self.H = hidden.shape
+        self.R, self.inter = R, inter
+        dev = self.dev = hidden.device
+        self.lib = _lib.load()
+        nbytes = max(self.lib.hawk_decode_layer_workspace_bytes(self.M, self.H, R, inter, n) for n in (2 * R, vocab))
+        self.ws = _lib.decode_layer_workspace(dev, nbytes)
+        self.stream = _lib.stream_ptr(dev)
+
+    def first(self, norm_w: torch.Tensor, eps: float, w: torch.Tensor) -> torch.Tensor:
+        """rmsnorm(hidden) w^T"""
+        out = torch.empty((self.M, w.shape[0]), dtype=torch.bfloat16, device=self.dev)
+        with _lib.on_device(self.dev):
+            _lib.check("hawk_decode_norm_linear", self.lib.hawk_decode_norm_linear(
+                self.hidden.data_ptr(), norm_w.data_ptr(), eps, w.data_ptr(), out.data_ptr(), self.M, w.shape[0],
+                self.H, self.ws.data_ptr(), self.ws.numel(), self.stream))
+        return out
+
+    def tail(self, gated, w_resid, norm_w, eps, w_gate_up, w_down, next_norm_w, next_eps, w_next) -> torch.Tensor:
+        """What follows a layer's recurrent core, up to the next layer's input projection (or the head)."""
+        out = torch.empty((self.M, w_next.shape[0]), dtype=torch.bfloat16, device=self.dev)
+        with _lib.on_device(self.dev):
+            _lib.check("hawk_decode_layer_tail", self.lib.hawk_decode_layer_tail(
+                gated.data_ptr(), w_resid.data_ptr(), self.hidden.data_ptr(), norm_w.data_ptr(), eps,
+                w_gate_up.data_ptr(), w_down.data_ptr(), next_norm_w.data_ptr(), next_eps, w_next.data_ptr(),
+                out.data_ptr(), self.M, self.H, self.R, self.inter, w_next.shape[0], self.ws.data_ptr(),
+                self.ws.numel(), self.stream))
+        return out
 
 
 # ---------------------------------------------------------------------------------------

@@ -27,12 +27,15 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import _lib
 from .cache import RNNCache
 from .external import (
     BlockDiagonalLinear,
     Conv1D,
+    DecodeLayers,
     decode_core_step,
     decode_core_supported,
+    decode_layers_supported,
     gate_projections,
     gate_projections_supported,
     rglru_step,
@@ -140,10 +143,36 @@ class Hawk(nn.Module):
         lecun_init(self.input_xy.weight, self.config.hidden_size)
         nn.init.zeros_(self.resid_proj.weight)
 
+    def step(self, xy: torch.Tensor, layer_past: RNNCache) -> torch.Tensor:
+        """One new token per batch row on a warm cache: the input projection's output [B, 1, 2R] to the
+        output projection's input [B, 1, R]; updates the cache."""
+        branch, gate_branch = xy.chunk(2, dim=-1)
+        layer_past.own_buffers()
+        fused_gates = self.config.fused_gates and gate_projections_supported(branch, self.rg_lru_input_gate)
+        layer_past.current_cache_size = 1
+        if (fused_gates and self.config.fused_epilogue and self.config.fused_decode_core
+                and decode_core_supported(branch, self.conv1d, self.rg_lru_input_gate, layer_past.conv_state)):
+            return decode_core_step(layer_past.conv_state, branch, self.conv1d, self.rg_lru_input_gate,
+                                    self.rg_lru_a_gate, self.rg_lru_a_param, layer_past.recc_state, gate_branch)
+        if fused_gates:
+            u = temporal_conv1d_step(layer_past.conv_state, branch, self.conv1d.w, self.conv1d.b, torch.bfloat16)
+            xg, ag = gate_projections(u, self.rg_lru_input_gate, self.rg_lru_a_gate, torch.bfloat16)
+            bias_i = bias_a = None  # already added by the projection kernel
+        else:
+            u = self.conv1d.step(layer_past.conv_state, branch)
+            xg = self.rg_lru_input_gate(u, add_bias=False)
+            ag = self.rg_lru_a_gate(u, add_bias=False)
+            bias_i, bias_a = self.rg_lru_input_gate.b, self.rg_lru_a_gate.b
+        if self.config.fused_epilogue:
+            return rglru_step_gated(u, xg, ag, self.rg_lru_a_param, layer_past.recc_state, gate_branch,
+                                    bias_i=bias_i, bias_a=bias_a)
+        if bias_i is not None:
+            xg, ag = xg + bias_i.reshape(-1), ag + bias_a.reshape(-1)
+        return F.gelu(gate_branch) * rglru_step(u, xg, ag, self.rg_lru_a_param, layer_past.recc_state)
+
     def forward(self, x: torch.Tensor, layer_past: Optional[RNNCache]) -> Tuple[torch.Tensor, Optional[RNNCache]]:
         warm = self.use_cache and layer_past is not None and layer_past.current_cache_size > 0
         xy = self.input_xy(x)
-        branch, gate_branch = xy.chunk(2, dim=-1)
 
         if warm:
             # One new token per batch row.  (Upstream accepts more and silently keeps only the
@@ -155,73 +184,63 @@ class Hawk(nn.Module):
                     f"a warm cache takes one new token per call, got {x.shape[1]}; "
                     "feed longer inputs with a fresh RNNCache (prefill)"
                 )
-            layer_past.own_buffers()
-            fused_gates = self.config.fused_gates and gate_projections_supported(branch, self.rg_lru_input_gate)
-            gate_branch = gate_branch[:, -1:, :]
-            layer_past.current_cache_size = 1
-            if (fused_gates and self.config.fused_epilogue and self.config.fused_decode_core
-                    and decode_core_supported(branch, self.conv1d, self.rg_lru_input_gate, layer_past.conv_state)):
-                gated = decode_core_step(layer_past.conv_state, branch[:, -1:, :], self.conv1d,
-                                         self.rg_lru_input_gate, self.rg_lru_a_gate, self.rg_lru_a_param,
-                                         layer_past.recc_state, gate_branch)
-                return self.resid_proj(gated), layer_past
-            if fused_gates:
-                u = temporal_conv1d_step(layer_past.conv_state, branch[:, -1:, :], self.conv1d.w, self.conv1d.b,
-                                         torch.bfloat16)
-                xg, ag = gate_projections(u, self.rg_lru_input_gate, self.rg_lru_a_gate, torch.bfloat16)
-                bias_i = bias_a = None  # already added by the projection kernel
-            else:
-                u = self.conv1d.step(layer_past.conv_state, branch[:, -1:, :])
-                xg = self.rg_lru_input_gate(u, add_bias=False)
-                ag = self.rg_lru_a_gate(u, add_bias=False)
-                bias_i, bias_a = self.rg_lru_input_gate.b, self.rg_lru_a_gate.b
-            if self.config.fused_epilogue:
-                gated = rglru_step_gated(u, xg, ag, self.rg_lru_a_param, layer_past.recc_state, gate_branch,
-                                         bias_i=bias_i, bias_a=bias_a)
-                return self.resid_proj(gated), layer_past
-            if bias_i is not None:
-                xg, ag = xg + bias_i.reshape(-1), ag + bias_a.reshape(-1)
-            h = rglru_step(u, xg, ag, self.rg_lru_a_param, layer_past.recc_state)
-            cache = layer_past
-        else:
-            if self.use_cache:
-                assert layer_past is not None, "use_cache=True needs one RNNCache per layer in layer_past"
-                layer_past.seed_conv_state(branch)
-            cache = layer_past if self.use_cache else None
-            if self.config.fused_gates and gate_projections_supported(branch, self.rg_lru_input_gate):
-                if (self.config.fused_epilogue and self.config.fused_block_core and block_core_layout_ok(xy)):
-                    # conv, projections, scan and output gate as one autograd node on xy itself
-                    gated, h_last = recurrent_block_core(xy, self.conv1d, self.rg_lru_input_gate,
-                                                         self.rg_lru_a_gate, self.rg_lru_a_param,
-                                                         return_last_state=True)
-                    if self.use_cache:
-                        layer_past.update_cache(h_last)
-                    return self.resid_proj(gated), cache
-                # bf16 end to end: upstream's gate einsums (under autocast) and its scan
-                # (cast_inputs, hawk/scan_fused.py:428) round the conv output to bf16 anyway
-                u = temporal_conv1d(branch, self.conv1d.w, self.conv1d.b, torch.bfloat16)
-                if self.config.fused_epilogue:
-                    # projections, scan and output gate as one autograd node
-                    gated, h_last = recurrent_core(u, self.rg_lru_input_gate, self.rg_lru_a_gate,
-                                                   self.rg_lru_a_param, gate_branch, return_last_state=True)
-                    if self.use_cache:
-                        layer_past.update_cache(h_last)
-                    return self.resid_proj(gated), cache
-                xg, ag = gate_projections(u, self.rg_lru_input_gate, self.rg_lru_a_gate, torch.bfloat16)
-            else:
-                u = self.conv1d(branch)
-                xg, ag = self.rg_lru_input_gate(u), self.rg_lru_a_gate(u)
-            gates = (xg, ag, self.rg_lru_a_param.float())
-            if self.config.fused_epilogue:
-                gated, h_last = fused_linear_scan_gated(u, *gates, gate_branch, return_last_state=True)
+            return self.resid_proj(self.step(xy, layer_past)), layer_past
+        branch, gate_branch = xy.chunk(2, dim=-1)
+        if self.use_cache:
+            assert layer_past is not None, "use_cache=True needs one RNNCache per layer in layer_past"
+            layer_past.seed_conv_state(branch)
+        cache = layer_past if self.use_cache else None
+        if self.config.fused_gates and gate_projections_supported(branch, self.rg_lru_input_gate):
+            if (self.config.fused_epilogue and self.config.fused_block_core and block_core_layout_ok(xy)):
+                # conv, projections, scan and output gate as one autograd node on xy itself
+                gated, h_last = recurrent_block_core(xy, self.conv1d, self.rg_lru_input_gate,
+                                                     self.rg_lru_a_gate, self.rg_lru_a_param,
+                                                     return_last_state=True)
                 if self.use_cache:
                     layer_past.update_cache(h_last)
                 return self.resid_proj(gated), cache
-            h = fused_linear_scan(u, *gates)
+            # bf16 end to end: upstream's gate einsums (under autocast) and its scan
+            # (cast_inputs, hawk/scan_fused.py:428) round the conv output to bf16 anyway
+            u = temporal_conv1d(branch, self.conv1d.w, self.conv1d.b, torch.bfloat16)
+            if self.config.fused_epilogue:
+                # projections, scan and output gate as one autograd node
+                gated, h_last = recurrent_core(u, self.rg_lru_input_gate, self.rg_lru_a_gate,
+                                               self.rg_lru_a_param, gate_branch, return_last_state=True)
+                if self.use_cache:
+                    layer_past.update_cache(h_last)
+                return self.resid_proj(gated), cache
+            xg, ag = gate_projections(u, self.rg_lru_input_gate, self.rg_lru_a_gate, torch.bfloat16)
+        else:
+            u = self.conv1d(branch)
+            xg, ag = self.rg_lru_input_gate(u), self.rg_lru_a_gate(u)
+        gates = (xg, ag, self.rg_lru_a_param.float())
+        if self.config.fused_epilogue:
+            gated, h_last = fused_linear_scan_gated(u, *gates, gate_branch, return_last_state=True)
             if self.use_cache:
-                layer_past.update_cache(h[:, -1:, :])
+                layer_past.update_cache(h_last)
+            return self.resid_proj(gated), cache
+        h = fused_linear_scan(u, *gates)
+        if self.use_cache:
+            layer_past.update_cache(h[:, -1:, :])
 
         return self.resid_proj(F.gelu(gate_branch) * h), cache
+
+
+def _plain(module: Optional[nn.Module], cls: type) -> bool:
+    """Exactly this class, and a call of it runs this class's forward and nothing else."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and module._compiled_call_impl is None)
+
+
+def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.device) -> Optional[torch.Tensor]:
+    """The weight of a plain module if a kernel can read it as it is: bf16, dense, aligned."""
+    if not _plain(module, cls):
+        return None
+    w = module._parameters.get("weight")
+    if (type(w) is not nn.Parameter or w.dtype != torch.bfloat16 or w.shape != shape or w.device != dev
+            or not w.is_contiguous() or w.data_ptr() % 16 != 0 or module._parameters.get("bias") is not None):
+        return None
+    return w
 
 
 class RNNLayer(nn.Module):
@@ -240,6 +259,22 @@ class RNNLayer(nn.Module):
         hidden_states = hidden_states + mixed
         hidden_states = hidden_states + self.mlp(self.post_recurrent_norm(hidden_states))
         return hidden_states, cache
+
+    def decode_weights(self, H: int, R: int, inter: int, dev: torch.device):
+        """(norm, eps, input, output, norm, eps, gate and up, down) weights of this layer as the decode
+        kernels take them, or None if something here is not what the constructor put there."""
+        m = self._modules
+        recc, mlp, n1, n2 = m.get("recc"), m.get("mlp"), m.get("input_norm"), m.get("post_recurrent_norm")
+        if not (_plain(self, RNNLayer) and _plain(recc, Hawk) and _plain(mlp, MLP) and recc.use_cache):
+            return None
+        ws = (_dense_weight(n1, RMSNorm, (H,), dev), _dense_weight(n2, RMSNorm, (H,), dev),
+              _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev),
+              _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev),
+              _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev),
+              _dense_weight(mlp._modules.get("resid_proj"), nn.Linear, (H, inter), dev))
+        if any(w is None for w in ws):
+            return None
+        return ws[0], n1.eps, ws[2], ws[3], ws[1], n2.eps, ws[4], ws[5]
 
 
 class HawkModel(nn.Module):
@@ -272,6 +307,42 @@ class HawkModel(nn.Module):
             for _ in self.layers
         ]
 
+    def _decode_step(self, input_ids, layer_past) -> Optional[torch.Tensor]:
+        """Logits of one token per sequence on warm caches through the decode kernels, or None where
+        they do not apply (nothing has been touched then): bf16 weights in the modules that the
+        constructor made, up to 256 rows, no gradients, nothing that records or rewrites operator calls."""
+        cfg = self.config
+        if (torch.is_grad_enabled() or not isinstance(input_ids, torch.Tensor) or input_ids.ndim != 2
+                or input_ids.shape[1] != 1 or not input_ids.is_cuda or not (cfg.fused_gates and cfg.fused_epilogue)
+                or any(p is None or p.current_cache_size <= 0 for p in layer_past)
+                or not _lib.launches_directly(input_ids) or nn.modules.module._has_any_global_hook()
+                or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
+                or not _plain(self.embed_tokens, nn.Embedding)):
+            return None
+        dev = input_ids.device
+        M, H, R, inter = input_ids.shape[0], cfg.hidden_size, cfg.recurrent_size, cfg.intermediate_size
+        if M < 1 or not decode_layers_supported(M, H, R, inter, cfg.vocab_size):
+            return None
+        embed = self.embed_tokens.weight
+        norm = _dense_weight(self.norm, RMSNorm, (H,), dev)
+        head = _dense_weight(self.lm_head, nn.Linear, (cfg.vocab_size, H), dev)
+        weights = [layer.decode_weights(H, R, inter, dev) if type(layer) is RNNLayer else None
+                   for layer in self.layers]
+        if (norm is None or head is None or not weights or any(w is None for w in weights)
+                or embed.dtype != torch.bfloat16 or embed.device != dev or embed.shape[1] != H):
+            return None
+
+        hidden = self.embed_tokens(input_ids).reshape(M, H)   # a tensor of this call's own
+        run = DecodeLayers(hidden, R, inter, cfg.vocab_size)
+        xy = run.first(weights[0][0], weights[0][1], weights[0][2])
+        for i, (layer, past) in enumerate(zip(self.layers, layer_past)):
+            _, _, _, w_out, norm_w, eps, w_gate_up, w_down = weights[i]
+            gated = layer.recc.step(xy.reshape(M, 1, 2 * R), past)
+            gated = _lib.dense16(gated if gated.dtype == torch.bfloat16 else gated.to(torch.bfloat16))
+            following = weights[i + 1][:3] if i + 1 < len(weights) else (norm, self.norm.eps, head)
+            xy = run.tail(gated, w_out, norm_w, eps, w_gate_up, w_down, *following)
+        return xy.reshape(M, 1, cfg.vocab_size)
+
     def forward(
         self,
         input_ids: Optional[torch.LongTensor] = None,
@@ -281,6 +352,11 @@ class HawkModel(nn.Module):
         if layer_past is None:
             layer_past = [None] * len(self.layers)
         assert isinstance(layer_past, list) and len(layer_past) == len(self.layers)
+
+        if self.use_cache:
+            logits = self._decode_step(input_ids, layer_past)
+            if logits is not None:
+                return logits, list(layer_past)
 
         hidden_states = self.embed_tokens(input_ids)
         caches = []

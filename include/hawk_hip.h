@@ -298,6 +298,45 @@ int hawk_decode_core_step_ws(void* conv_state, const void* x_new, long long ldx,
                              int dtype, int w_dtype, int state_dtype, void* workspace_device,
                              size_t workspace_bytes, void* stream);
 
+/* Dense projections of a decode step: out [M, N] = x [M, K] w^T for up to 256 rows, bf16 with
+ * fp32 sums, w [N, K] as torch.nn.Linear keeps it (upstream: the Linear calls of
+ * hawk/hawk.py:70-86, :163-203, :284-303 on one token per sequence).  K must be a multiple of
+ * 128 (at most 65536) and N of 8; all tensors dense and 16-byte aligned.  The workspace (16-byte
+ * aligned, contents irrelevant, NULL where the size query says 0) holds the partial sums of
+ * products that are split over K. */
+int hawk_decode_linear_supported(int M, int N, int K);
+size_t hawk_decode_linear_workspace_bytes(int M, int N, int K);
+int hawk_decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* workspace_device,
+                       size_t workspace_bytes, void* stream);
+
+/* 1 if the two calls below serve a layer: M rows, hidden size H (a multiple of 128, at most
+ * 8192), recurrent size R and intermediate size I (multiples of 128). */
+int hawk_decode_layer_supported(int M, int H, int R, int I);
+size_t hawk_decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next);
+
+/* out [M, N] = rmsnorm(hidden) w^T: the norm in front of the first layer and its input
+ * projection (hawk/hawk.py:53-58, :163-166).  hidden [M, H] and norm_w [H] bf16; the workspace
+ * takes M * H bf16 values, rounded up to 256 bytes, and hawk_decode_linear_workspace_bytes(M, N, H)
+ * behind them (hawk_decode_layer_workspace_bytes(M, H, R, I, N) is enough). */
+int hawk_decode_norm_linear(void* hidden, const void* norm_w, float eps, const void* w, void* out, int M,
+                            int N, int H, void* workspace_device, size_t workspace_bytes, void* stream);
+
+/* What follows the recurrent core of a layer in a decode step, up to the next layer's core
+ * (hawk/hawk.py:198-203, :222-243, and :163-166 of the next layer or :284-303):
+ *   hidden += gated w_resid^T
+ *   hidden += (gelu(g) * u) w_down^T with [g, u] = rmsnorm(hidden; norm_w) w_gate_up^T
+ *   next_out [M, n_next] = rmsnorm(hidden; next_norm_w) w_next^T
+ * gated [M, R]; hidden [M, H] in place; w_resid [H, R]; w_gate_up [2 I, H] (gate rows first);
+ * w_down [H, I]; w_next [n_next, H]; everything bf16, dense and 16-byte aligned, sums in fp32,
+ * every projection, the GELU, the product, the additions and the norms rounded to bf16 as the
+ * separate operations round them.  The workspace holds hawk_decode_layer_workspace_bytes(M, H, R, I, n_next) bytes
+ * (16-byte aligned, contents irrelevant); calls in order on one stream can share it.  Results are a
+ * function of the operands alone (fixed summation order). */
+int hawk_decode_layer_tail(const void* gated, const void* w_resid, void* hidden, const void* norm_w,
+                           float eps, const void* w_gate_up, const void* w_down, const void* next_norm_w,
+                           float next_eps, const void* w_next, void* next_out, int M, int H, int R, int I,
+                           int n_next, void* workspace_device, size_t workspace_bytes, void* stream);
+
 /* Both gate logits of M = B*T tokens in one pass over x:
  *   x_rg_lru[m, h*bw+j] = b_i[h*bw+j] + sum_i x[m, h*bw+i] w_i[h, i, j]     (same for a_rg_lru)
  * Replaces the two BlockDiagonalLinear calls of hawk/hawk.py:181-182 (einsum + bias,
