@@ -84,6 +84,17 @@ SIGNATURES = {
         [_c_void_p] * 2 + [ctypes.c_longlong] + [_c_void_p] * 8 + [ctypes.c_longlong] + [_c_void_p] * 2
         + [_c_int] * 7 + [_c_void_p, _c_size_t, _c_void_p],
     ),
+    "hawk_cast": (
+        _c_int, [ctypes.POINTER(_c_void_p)] * 2 + [ctypes.POINTER(ctypes.c_ulonglong)] + [_c_int] * 2 + [_c_void_p]
+    ),
+    "hawk_add_norm_fwd": (_c_int, [_c_void_p] * 3 + [ctypes.c_float] + [_c_void_p] * 3 + [_c_int] * 2 + [_c_void_p]),
+    "hawk_add_norm_bwd_workspace_bytes": (_c_size_t, [_c_int] * 2),
+    "hawk_add_norm_bwd": (_c_int, [_c_void_p] * 8 + [_c_int] * 2 + [_c_void_p, _c_size_t, _c_void_p]),
+    "hawk_gelu_mul_fwd": (_c_int, [_c_void_p] * 2 + [_c_int] * 2 + [_c_void_p]),
+    "hawk_gelu_mul_bwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 2 + [_c_void_p]),
+    "hawk_cross_entropy_fwd": (_c_int, [_c_void_p] * 5 + [_c_int] * 3 + [_c_void_p]),
+    "hawk_cross_entropy_bwd": (_c_int, [_c_void_p] * 6 + [_c_int] * 3 + [_c_void_p]),
+    "hawk_embedding_bwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p]),
     "hawk_decode_linear_supported": (_c_int, [_c_int] * 3),
     "hawk_decode_linear_workspace_bytes": (_c_size_t, [_c_int] * 3),
     "hawk_decode_linear": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),

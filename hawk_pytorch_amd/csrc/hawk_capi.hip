@@ -304,6 +304,83 @@ int hawk_decode_core_step(void* conv_state, const void* x_new, long long ldx, co
                                     stream);
 }
 
+int hawk_cast(const void* const* src, void* const* dst, const unsigned long long* counts, int n, int to_bf16,
+              void* stream) {
+    if (!src || !dst || !counts) return HAWK_ERR_NULL_POINTER;
+    if (n < 1 || n > hawk::kCastSegments) return HAWK_ERR_BAD_SHAPE;
+    for (int k = 0; k < n; ++k) {
+        if (!src[k] || !dst[k]) return HAWK_ERR_NULL_POINTER;
+        if (counts[k] % 4 != 0) return HAWK_ERR_BAD_SHAPE;
+        if (!aligned16(src[k]) || !aligned16(dst[k])) return HAWK_ERR_ALIGNMENT;
+    }
+    return hawk::cast_arrays(src, dst, counts, n, to_bf16 != 0, as_stream(stream));
+}
+
+int hawk_add_norm_fwd(const float* hidden, const void* delta, const float* weight, float eps, float* sum, void* out,
+                      float* rstd, int rows, int D, void* stream) {
+    if (!hidden || !weight || !out || !rstd || (delta && !sum)) return HAWK_ERR_NULL_POINTER;
+    if (rows < 1 || !hawk::train_norm_supported(D)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(hidden) || !aligned16(delta) || !aligned16(weight) || !aligned16(sum) || !aligned16(out))
+        return HAWK_ERR_ALIGNMENT;
+    return hawk::add_norm_fwd(hidden, delta, weight, eps, sum, out, rstd, rows, D, as_stream(stream));
+}
+
+size_t hawk_add_norm_bwd_workspace_bytes(int rows, int D) {
+    return rows >= 1 && hawk::train_norm_supported(D) ? hawk::add_norm_bwd_workspace_bytes(rows, D) : 0;
+}
+
+int hawk_add_norm_bwd(const void* dout, const float* sum, const float* rstd, const float* weight,
+                      const float* d_direct, float* d_sum, void* d_delta, float* dweight, int rows, int D,
+                      void* workspace_device, size_t workspace_bytes, void* stream) {
+    if (!dout || !sum || !rstd || !weight || !d_sum || !dweight) return HAWK_ERR_NULL_POINTER;
+    if (rows < 1 || !hawk::train_norm_supported(D)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(dout) || !aligned16(sum) || !aligned16(weight) || !aligned16(d_direct) || !aligned16(d_sum) ||
+        !aligned16(d_delta) || !aligned16(workspace_device))
+        return HAWK_ERR_ALIGNMENT;
+    if (!workspace_device || workspace_bytes < hawk::add_norm_bwd_workspace_bytes(rows, D)) return HAWK_ERR_WORKSPACE;
+    return hawk::add_norm_bwd(dout, sum, rstd, weight, d_direct, d_sum, d_delta, dweight, rows, D, workspace_device,
+                              as_stream(stream));
+}
+
+int hawk_gelu_mul_fwd(const void* gate_up, void* act, int rows, int I, void* stream) {
+    if (!gate_up || !act) return HAWK_ERR_NULL_POINTER;
+    if (rows < 1 || I < 8 || I % 8 != 0) return HAWK_ERR_BAD_SHAPE;
+    if ((long long)rows * (I / 8) > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(gate_up) || !aligned16(act)) return HAWK_ERR_ALIGNMENT;
+    return hawk::gelu_mul_fwd(gate_up, act, rows, I, as_stream(stream));
+}
+
+int hawk_gelu_mul_bwd(const void* gate_up, const void* dact, void* d_gate_up, int rows, int I, void* stream) {
+    if (!gate_up || !dact || !d_gate_up) return HAWK_ERR_NULL_POINTER;
+    if (rows < 1 || I < 8 || I % 8 != 0) return HAWK_ERR_BAD_SHAPE;
+    if ((long long)rows * (I / 8) > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(gate_up) || !aligned16(dact) || !aligned16(d_gate_up)) return HAWK_ERR_ALIGNMENT;
+    return hawk::gelu_mul_bwd(gate_up, dact, d_gate_up, rows, I, as_stream(stream));
+}
+
+int hawk_cross_entropy_fwd(const void* logits, const long long* labels, float* lse, float* loss, float* mean, int B,
+                           int T, int V, void* stream) {
+    if (!logits || !labels || !lse || !loss || !mean) return HAWK_ERR_NULL_POINTER;
+    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(logits)) return HAWK_ERR_ALIGNMENT;
+    return hawk::cross_entropy_fwd(logits, labels, lse, loss, mean, B * T, T, V, as_stream(stream));
+}
+
+int hawk_cross_entropy_bwd(const void* logits, const long long* labels, const float* lse, const float* mean,
+                           const float* dloss, void* dlogits, int B, int T, int V, void* stream) {
+    if (!logits || !labels || !lse || !mean || !dloss || !dlogits) return HAWK_ERR_NULL_POINTER;
+    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(logits) || !aligned16(dlogits)) return HAWK_ERR_ALIGNMENT;
+    return hawk::cross_entropy_bwd(logits, labels, lse, mean, dloss, dlogits, B * T, T, V, as_stream(stream));
+}
+
+int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D, void* stream) {
+    if (!ids || !dout || !dweight) return HAWK_ERR_NULL_POINTER;
+    if (rows < 1 || rows > hawk::kEmbeddingMaxRows || V < 1 || D < 8 || D % 8 != 0) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(dout)) return HAWK_ERR_ALIGNMENT;
+    return hawk::embedding_bwd(ids, dout, dweight, rows, V, D, as_stream(stream));
+}
+
 int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }
 
 size_t hawk_decode_linear_workspace_bytes(int M, int N, int K) {

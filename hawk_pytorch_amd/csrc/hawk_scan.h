@@ -117,6 +117,25 @@ int decode_layer_tail(const void* gated, const void* w_resid, void* hidden, cons
                       const void* w_next, void* next_out, int M, int H, int R, int I, int n_next, void* ws,
                       hipStream_t st);
 
+// hawk_train.hip
+constexpr int kCastSegments = 8;
+constexpr int kEmbeddingMaxRows = 8192;   // a list of them is kept in LDS
+int cast_arrays(const void* const* src, void* const* dst, const unsigned long long* counts, int n, bool to_bf16,
+                hipStream_t st);
+bool train_norm_supported(int D);
+int add_norm_fwd(const float* hidden, const void* delta, const float* weight, float eps, float* sum, void* out,
+                 float* rstd, int rows, int D, hipStream_t st);
+size_t add_norm_bwd_workspace_bytes(int rows, int D);
+int add_norm_bwd(const void* dout, const float* sum, const float* rstd, const float* weight, const float* d_direct,
+                 float* d_sum, void* d_delta, float* dweight, int rows, int D, void* ws, hipStream_t st);
+int gelu_mul_fwd(const void* gu, void* act, long long rows, int I, hipStream_t st);
+int gelu_mul_bwd(const void* gu, const void* dact, void* dgu, long long rows, int I, hipStream_t st);
+int cross_entropy_fwd(const void* logits, const long long* labels, float* lse, float* loss, float* mean, int rows,
+                      int T, int V, hipStream_t st);
+int cross_entropy_bwd(const void* logits, const long long* labels, const float* lse, const float* mean,
+                      const float* dloss, void* dlogits, int rows, int T, int V, hipStream_t st);
+int embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D, hipStream_t st);
+
 // hawk_probe.hip
 bool stream_probe_shape_ok(size_t bytes, size_t row_pitch, int shape);
 int stream_probe(const void* const* reads, int n_reads, void* const* writes, int n_writes, size_t bytes,

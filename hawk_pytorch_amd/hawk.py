@@ -27,7 +27,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from . import _lib
+from . import _lib, train_fused
 from .cache import RNNCache
 from .external import (
     BlockDiagonalLinear,
@@ -232,15 +232,22 @@ def _plain(module: Optional[nn.Module], cls: type) -> bool:
             and not module._forward_pre_hooks and module._compiled_call_impl is None)
 
 
-def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.device) -> Optional[torch.Tensor]:
-    """The weight of a plain module if a kernel can read it as it is: bf16, dense, aligned."""
-    if not _plain(module, cls):
-        return None
-    w = module._parameters.get("weight")
-    if (type(w) is not nn.Parameter or w.dtype != torch.bfloat16 or w.shape != shape or w.device != dev
-            or not w.is_contiguous() or w.data_ptr() % 16 != 0 or module._parameters.get("bias") is not None):
+def _dense_param(module: Optional[nn.Module], name: str, shape, dtype: torch.dtype,
+                 dev: torch.device) -> Optional[torch.Tensor]:
+    """A module's parameter if a kernel can read it as it is: of this type and shape, dense, aligned."""
+    w = module._parameters.get(name)
+    if (type(w) is not nn.Parameter or w.dtype != dtype or w.shape != shape or w.device != dev
+            or not w.is_contiguous() or w.data_ptr() % 16 != 0):
         return None
     return w
+
+
+def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.device,
+                  dtype: torch.dtype = torch.bfloat16) -> Optional[torch.Tensor]:
+    """The weight of a plain module without a bias, as above."""
+    if not _plain(module, cls) or module._parameters.get("bias") is not None:
+        return None
+    return _dense_param(module, "weight", shape, dtype, dev)
 
 
 class RNNLayer(nn.Module):
@@ -275,6 +282,32 @@ class RNNLayer(nn.Module):
         if any(w is None for w in ws):
             return None
         return ws[0], n1.eps, ws[2], ws[3], ws[1], n2.eps, ws[4], ws[5]
+
+
+    def train_weights(self, cfg: HawkConfig, dev: torch.device):
+        """(eps, eps, parameters) of this layer in the order of train_fused.layer, or None if something
+        here is not what the constructor put there."""
+        m = self._modules
+        recc, mlp, n1, n2 = m.get("recc"), m.get("mlp"), m.get("input_norm"), m.get("post_recurrent_norm")
+        if not (_plain(self, RNNLayer) and _plain(recc, Hawk) and _plain(mlp, MLP) and not recc.use_cache):
+            return None
+        conv, gi, ga = (recc._modules.get(k) for k in ("conv1d", "rg_lru_input_gate", "rg_lru_a_gate"))
+        if not (_plain(conv, Conv1D) and _plain(gi, BlockDiagonalLinear) and _plain(ga, BlockDiagonalLinear)):
+            return None
+        H, R, inter, nb = cfg.hidden_size, cfg.recurrent_size, cfg.intermediate_size, cfg.num_blocks
+        f32, bw = torch.float32, R // nb
+        ws = (_dense_weight(n1, RMSNorm, (H,), dev, f32), _dense_weight(n2, RMSNorm, (H,), dev, f32),
+              _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev, f32),
+              _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev, f32),
+              _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev, f32),
+              _dense_weight(mlp._modules.get("resid_proj"), nn.Linear, (H, inter), dev, f32),
+              _dense_param(conv, "w", (cfg.conv_width, R), f32, dev), _dense_param(conv, "b", (R,), f32, dev),
+              _dense_param(gi, "w", (nb, bw, bw), f32, dev), _dense_param(gi, "b", (nb, bw), f32, dev),
+              _dense_param(ga, "w", (nb, bw, bw), f32, dev), _dense_param(ga, "b", (nb, bw), f32, dev),
+              _dense_param(recc, "rg_lru_a_param", (R,), f32, dev))
+        if any(w is None for w in ws):
+            return None
+        return n1.eps, n2.eps, ws
 
 
 class HawkModel(nn.Module):
@@ -343,6 +376,50 @@ class HawkModel(nn.Module):
             xy = run.tail(gated, w_out, norm_w, eps, w_gate_up, w_down, *following)
         return xy.reshape(M, 1, cfg.vocab_size)
 
+    def _train_step(self, input_ids, labels) -> Optional[torch.Tensor]:
+        """The loss of fp32 parameters under bf16 autocast, with one autograd node for the embedding, for
+        each layer and for the head, or None where that does not apply: in the modules that the
+        constructor made, all of a node's parameters trained (or no gradients at all), nothing that
+        records or rewrites operator calls.  A layer to which it does not apply is called as a module."""
+        cfg = self.config
+        if (not isinstance(input_ids, torch.Tensor) or not isinstance(labels, torch.Tensor) or input_ids.ndim != 2
+                or labels.shape != input_ids.shape or not input_ids.is_cuda or labels.device != input_ids.device
+                or input_ids.dtype != torch.int64 or labels.dtype != torch.int64 or input_ids.numel() == 0
+                or not input_ids.is_contiguous() or not labels.is_contiguous()
+                or not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") != torch.bfloat16
+                or not _lib.launches_directly(input_ids, labels) or nn.modules.module._has_any_global_hook()):
+            return None
+        H, V, dev, f32 = cfg.hidden_size, cfg.vocab_size, input_ids.device, torch.float32
+        rows, emb = input_ids.numel(), self.embed_tokens
+        grad = torch.is_grad_enabled()
+        norm, head = _dense_weight(self.norm, RMSNorm, (H,), dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H),
+                                                                                     dev, f32)
+        if (H % 8 != 0 or H > 4096 or V % 8 != 0 or norm is None or head is None or rows * V >= 1 << 40
+                or (grad and not (norm.requires_grad and head.requires_grad))):
+            return None
+        table = _dense_param(emb, "weight", (V, H), f32, dev) if _plain(emb, nn.Embedding) else None
+        if (table is not None and rows <= train_fused.EMBEDDING_MAX_ROWS and emb.padding_idx is None
+                and emb.max_norm is None and not emb.scale_grad_by_freq and not emb.sparse):
+            hidden = train_fused.embedding(input_ids, table)
+        else:
+            hidden = emb(input_ids)
+        kernels = (cfg.fused_gates and cfg.fused_epilogue and cfg.fused_block_core and cfg.intermediate_size % 8 == 0
+                   and cfg.recurrent_size % cfg.num_blocks == 0 and 1 <= cfg.conv_width <= 8
+                   and cfg.recurrent_size // cfg.num_blocks in (32, 64, 128, 256)
+                   and rows * max(cfg.intermediate_size, cfg.recurrent_size) < 1 << 31)
+        delta = None
+        for layer in self.layers:
+            weights = layer.train_weights(cfg, dev) if kernels and type(layer) is RNNLayer else None
+            if (weights is None or hidden.dtype != f32 or not hidden.is_contiguous()
+                    or (grad and not all(p.requires_grad for p in weights[2]))):
+                hidden, _ = layer(hidden if delta is None else hidden + delta, layer_past=None)
+                delta = None
+            else:
+                hidden, delta = train_fused.layer(hidden, delta, *weights)
+        if hidden.dtype != f32 or not hidden.is_contiguous():
+            hidden = hidden.float().contiguous()
+        return train_fused.loss(hidden, delta, self.norm.eps, norm, head, labels)
+
     def forward(
         self,
         input_ids: Optional[torch.LongTensor] = None,
@@ -357,6 +434,10 @@ class HawkModel(nn.Module):
             logits = self._decode_step(input_ids, layer_past)
             if logits is not None:
                 return logits, list(layer_past)
+        elif labels is not None and all(past is None for past in layer_past):
+            loss = self._train_step(input_ids, labels)
+            if loss is not None:
+                return loss
 
         hidden_states = self.embed_tokens(input_ids)
         caches = []

@@ -619,13 +619,13 @@ def _(xy, u, xg, ag, h, conv_w, w_i, w_a, a_param, grad_out):
             f(nb, bw, bw), f(D), f(nb, bw, bw), f(D), f(D))
 
 
-def _block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h: bool, want_last: bool):
+def block_core_forward(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h: bool, want_last: bool):
     direct = _lib.launches_directly(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param)
     launch = _launch_block_core_fwd if direct else _block_core_fwd_op
     return launch(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h, want_last)
 
 
-def _block_core_bwd(*tensors):
+def block_core_backward(*tensors):
     return (_launch_block_core_bwd if _lib.launches_directly(*tensors) else _block_core_bwd_op)(*tensors)
 
 
@@ -642,7 +642,7 @@ class BlockCore(Function):
         cw = conv_w.float().contiguous()
         w_i16, w_a16 = kernel_weights(w_i, w_a, B * T)
         want_h = any(ctx.needs_input_grad[:8])
-        out, u, xg, ag, h, h_last = _block_core_fwd(
+        out, u, xg, ag, h, h_last = block_core_forward(
             xy, cw, conv_b.float().contiguous(), w_i16, b_i.float().reshape(-1), w_a16, b_a.float().reshape(-1),
             lam, want_h, bool(want_last))
         if want_h:
@@ -655,7 +655,7 @@ class BlockCore(Function):
         xy, u, xg, ag, h, cw, w_i, w_a, lam = ctx.saved_tensors
         go = grad_out if grad_out.dtype == torch.bfloat16 else grad_out.to(torch.bfloat16)
         go = go if go.is_contiguous() else go.contiguous()
-        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = _block_core_bwd(xy, u, xg, ag, h, cw, w_i, w_a, lam, go)
+        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = block_core_backward(xy, u, xg, ag, h, cw, w_i, w_a, lam, go)
         nb, bw, _ = w_i.shape
         t = ctx.dtypes
         return (d_xy, dcw.to(t[0]), dcb.to(t[1]), dw_i.to(t[2]), db_i.reshape(nb, bw).to(t[3]), dw_a.to(t[4]),

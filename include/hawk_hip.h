@@ -298,6 +298,42 @@ int hawk_decode_core_step_ws(void* conv_state, const void* x_new, long long ldx,
                              int dtype, int w_dtype, int state_dtype, void* workspace_device,
                              size_t workspace_bytes, void* stream);
 
+/* Training pass around the recurrent core (upstream: RMSNorm, MLP, RNNLayer and HawkModel.forward,
+ * hawk/hawk.py:53-58, :70-86, :222-303), values rounded to bf16 where bf16 autocast rounds them.  All
+ * tensors dense and 16-byte aligned; sums in fp32, in a fixed order.
+ *
+ * hawk_cast: n (at most 8) arrays of counts[k] elements (multiples of 4), fp32 -> bf16 or back, in one
+ * launch; src, dst and counts are host arrays. */
+int hawk_cast(const void* const* src, void* const* dst, const unsigned long long* counts, int n,
+              int to_bf16, void* stream);
+/* sum = hidden + delta; out = sum * rstd * weight with rstd = 1 / sqrt(mean(sum^2) + eps).  hidden, sum
+ * [rows, D] fp32; delta [rows, D] bf16 or NULL (then sum is not written and may be NULL); weight [D]
+ * fp32; out [rows, D] bf16; rstd [rows] fp32.  D a multiple of 8, at most 4096. */
+int hawk_add_norm_fwd(const float* hidden, const void* delta, const float* weight, float eps, float* sum,
+                      void* out, float* rstd, int rows, int D, void* stream);
+/* d_sum = d_direct + the gradient of out reaching sum (fp32; d_direct may be NULL), d_delta its bf16
+ * rounding (or NULL), dweight [D] fp32. */
+size_t hawk_add_norm_bwd_workspace_bytes(int rows, int D);
+int hawk_add_norm_bwd(const void* dout, const float* sum, const float* rstd, const float* weight,
+                      const float* d_direct, float* d_sum, void* d_delta, float* dweight, int rows, int D,
+                      void* workspace_device, size_t workspace_bytes, void* stream);
+/* act [rows, I] = gelu(g) * u for rows [g, u] of 2 I channels, and the gradient of those rows; bf16, I
+ * a multiple of 8. */
+int hawk_gelu_mul_fwd(const void* gate_up, void* act, int rows, int I, void* stream);
+int hawk_gelu_mul_bwd(const void* gate_up, const void* dact, void* d_gate_up, int rows, int I, void* stream);
+/* Mean next-token cross entropy of bf16 logits [B * T, V] (V a multiple of 8): row (b, t) against
+ * labels[b, t + 1] (int64, [B, T]); the last row of a sequence and rows with label -100 do not count; a
+ * label outside [0, V) makes the loss NaN.  lse, loss: [B * T] fp32 scratch (lse is read by the
+ * backward); mean: [2] fp32, the mean loss and the number of counted rows. */
+int hawk_cross_entropy_fwd(const void* logits, const long long* labels, float* lse, float* loss, float* mean,
+                           int B, int T, int V, void* stream);
+int hawk_cross_entropy_bwd(const void* logits, const long long* labels, const float* lse, const float* mean,
+                           const float* dloss, void* dlogits, int B, int T, int V, void* stream);
+/* dweight [V, D] fp32, zeroed by the caller: row id += the rows of dout [rows, D] fp32 whose token is id,
+ * in their order.  rows at most 8192, D a multiple of 8; tokens outside [0, V) add nothing. */
+int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D,
+                       void* stream);
+
 /* Dense projections of a decode step: out [M, N] = x [M, K] w^T for up to 256 rows, bf16 with
  * fp32 sums, w [N, K] as torch.nn.Linear keeps it (upstream: the Linear calls of
  * hawk/hawk.py:70-86, :163-203, :284-303 on one token per sequence).  K must be a multiple of

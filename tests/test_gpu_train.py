@@ -1,0 +1,203 @@
+"""The kernels around the recurrent core in a training pass (hawk_train.hip) against 64-bit references,
+and the model's loss and gradients with one autograd node per layer against the modules' own."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import hawk_pytorch_amd as hk
+from hawk_pytorch_amd import train_fused
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda", 0)
+EPS32 = 2.0 ** -24
+
+
+def _gen(seed):
+    return torch.Generator("cuda").manual_seed(seed)
+
+
+def _randn(gen, *shape, dtype=torch.float32):
+    return torch.randn(*shape, generator=gen, device=DEV).to(dtype)
+
+
+def _close(got, want, bound):
+    assert bool(((got.double() - want).abs() <= bound).all())
+
+
+# channel counts: one lane, a ragged group, either side of each number of groups per lane; rows: fewer than
+# a workgroup's waves, a remainder, more than the backward's grid holds at once
+@pytest.mark.parametrize("rows,D", [(1, 8), (5, 504), (3, 512), (7, 520), (9, 1032), (2600, 1024), (6, 2056), (13, 4096)])
+@pytest.mark.parametrize("with_delta", [True, False])
+def test_add_norm(rows, D, with_delta):
+    gen = _gen(rows + D)
+    hidden, w = _randn(gen, rows, D), _randn(gen, D) * 0.1 + 1
+    delta = _randn(gen, rows, D, dtype=torch.bfloat16) if with_delta else None
+    dout, direct = _randn(gen, rows, D, dtype=torch.bfloat16), _randn(gen, rows, D)
+    total, out, rstd = train_fused._add_norm(hidden, delta, w, 1e-6)
+    want = hidden + delta.float() if with_delta else hidden
+    assert torch.equal(total, want)
+    x, wd, dy = want.double().requires_grad_(), w.double().requires_grad_(), dout.double()
+    y = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-6) * wd
+    _close(out, y.detach(), 2.0 ** -8 * y.detach().abs() + 1e-6)
+    dx, dw = torch.autograd.grad(y, (x, wd), dy)
+    d_sum, d_delta, dweight = train_fused._add_norm_backward(dout, total, rstd, w, direct, with_delta)
+    want_d = dx + direct.double()
+    # sums of D (rows) products in fp32, over terms whose sizes the second factors bound
+    _close(d_sum, want_d, 64 * EPS32 * (want_d.abs() + dx.abs().mean(-1, keepdim=True) + (dy * wd).abs().detach() + 1))
+    scale = (dy * x.detach()).abs().mul(rstd.double()[:, None]).sum(0)
+    _close(dweight, dw, (rows + 64) * EPS32 * scale + 1e-12)
+    if with_delta:
+        assert torch.equal(d_delta, d_sum.bfloat16())
+
+
+@pytest.mark.parametrize("rows,inter", [(1, 8), (3, 264), (257, 1024)])
+def test_gelu_mul_rounds_like_the_separate_operations(rows, inter):
+    from hawk_pytorch_amd import _lib
+
+    gen = _gen(inter)
+    gu = _randn(gen, rows, 2 * inter, dtype=torch.bfloat16) * 2
+    dact = _randn(gen, rows, inter, dtype=torch.bfloat16)
+    act, dgu = torch.empty_like(dact), torch.empty_like(gu)
+    st = _lib.stream_ptr(DEV)
+    train_fused._check("hawk_gelu_mul_fwd", gu.data_ptr(), act.data_ptr(), rows, inter, st)
+    train_fused._check("hawk_gelu_mul_bwd", gu.data_ptr(), dact.data_ptr(), dgu.data_ptr(), rows, inter, st)
+    leaf = gu.clone().requires_grad_()
+    gate, up = leaf.chunk(2, dim=-1)
+    want = F.gelu(gate) * up
+    want.backward(dact)
+    # values next to a rounding boundary may fall to either side of it, at each of two roundings
+    for got, ref in ((act, want.detach()), (dgu, leaf.grad)):
+        ref = ref.double()
+        _close(got, ref, 2.0 ** -7 * ref.abs() + 1e-6)
+
+
+@pytest.mark.parametrize("B,T,V", [(1, 2, 8), (2, 5, 1000), (3, 4, 4104), (2, 3, 32000), (1, 4, 40008)])
+def test_cross_entropy(B, T, V):
+    gen = _gen(V)
+    H = 64
+    hidden, norm, head = _randn(gen, B, T, H), torch.ones(H, device=DEV), _randn(gen, V, H)
+    labels = torch.randint(0, V, (B, T), generator=gen, device=DEV)
+    labels[0, T - 1] = V - 1
+    if T > 3:
+        labels[-1, 1] = -100
+    hidden.requires_grad_(), head.requires_grad_()
+    loss = train_fused.loss(hidden, None, 1e-6, norm, head, labels)
+    # the logits as they were rounded, then everything in 64 bits
+    x = F.rms_norm(hidden.detach(), (H,), norm, 1e-6).bfloat16()
+    logits = torch.mm(x.view(-1, H), head.detach().bfloat16().t()).view(B, T, V)
+    l64 = logits[:, :-1].double().requires_grad_()
+    want = F.cross_entropy(l64.reshape(-1, V), labels[:, 1:].reshape(-1))
+    assert abs(float(loss.detach()) - float(want.detach())) < 1e-5 * max(1.0, float(want.detach()))
+    d64, = torch.autograd.grad(want, l64)
+    d_head, = torch.autograd.grad(loss, head)
+    want_head = d64.reshape(-1, V).t() @ x[:, :-1].reshape(-1, H).double()
+    # the gradient of the logits and the product are rounded to bf16
+    bound = 2.0 ** -8 * (d64.abs().reshape(-1, V).t() @ x[:, :-1].reshape(-1, H).double().abs()) + 2.0 ** -8 * want_head.abs()
+    _close(d_head, want_head, bound + 1e-9)
+
+
+def test_cross_entropy_of_infinite_logits_and_uncounted_rows():
+    B, T, V, H = 1, 4, 16, 8
+    norm = torch.ones(H, device=DEV)
+    labels = torch.randint(0, V, (B, T), generator=_gen(0), device=DEV)
+    hidden, head = torch.ones(B, T, H, device=DEV), torch.zeros(V, H, device=DEV)
+    none = train_fused.loss(hidden, None, 1e-6, norm, head, torch.full_like(labels, -100))
+    assert bool(torch.isnan(none))                       # a mean over nothing, as F.cross_entropy returns
+    head[3] = -float("inf")                              # a logit of -inf is a probability of zero
+    labels.fill_(2)
+    assert abs(float(train_fused.loss(hidden, None, 1e-6, norm, head, labels)) - float(torch.tensor(15.0).log())) < 1e-5
+    labels.fill_(3)
+    assert float(train_fused.loss(hidden, None, 1e-6, norm, head, labels)) == float("inf")
+    labels.fill_(V)                                      # not a token
+    assert bool(torch.isnan(train_fused.loss(hidden, None, 1e-6, norm, head, labels)))
+
+
+@pytest.mark.parametrize("rows,V,D", [(1, 5, 8), (130, 7, 264), (2048, 50, 512), (8192, 3, 1032)])
+def test_embedding_gradient(rows, V, D):
+    gen = _gen(rows)
+    ids = torch.randint(0, V, (1, rows), generator=gen, device=DEV)
+    ids[0, 0] = V - 1
+    weight, d = _randn(gen, V, D).requires_grad_(), _randn(gen, 1, rows, D)
+    out = train_fused.embedding(ids, weight)
+    assert torch.equal(out, F.embedding(ids, weight))
+    got, = torch.autograd.grad(out, weight, d)
+    want = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, ids[0], d[0].double())
+    scale = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, ids[0], d[0].double().abs())
+    _close(got, want, rows * EPS32 * scale)
+
+
+def _model(vocab=1000, D=256, inter=520, layers=2, nb=4, **kw):
+    torch.manual_seed(6)
+    model = hk.HawkModel(hk.HawkConfig(vocab_size=vocab, hidden_size=D, intermediate_size=inter, num_hidden_layers=layers,
+                                       recurrent_size=D, num_blocks=nb, **kw)).cuda()
+    for layer in model.layers:
+        torch.nn.init.normal_(layer.recc.resid_proj.weight, std=0.02)
+        torch.nn.init.normal_(layer.mlp.resid_proj.weight, std=0.02)
+    torch.nn.init.normal_(model.lm_head.weight, std=0.02)
+    return model
+
+
+def _grads(model, ids, labels, **kw):
+    model.zero_grad(set_to_none=True)
+    with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+        loss = model(ids, labels)
+    grads = torch.autograd.grad(loss, [p for p in model.parameters() if p.requires_grad], **kw)
+    return loss.detach(), grads
+
+
+# more tokens than the embedding kernel takes, a short sequence, a narrow conv
+@pytest.mark.parametrize("B,T,kw", [(1, 64, {}), (3, 331, {}), (2, 5, {}), (5, 1700, {}), (2, 100, dict(conv_width=2))])
+def test_model_training_pass_on_both_routes(B, T, kw, monkeypatch):
+    """A hook on a layer's MLP sends that layer through its modules; the rest stays on the kernels."""
+    model = _model(**kw)
+    ids = torch.randint(0, 1000, (B, T), generator=_gen(B), device=DEV)
+    labels = ids.clone()
+    labels[0, 1] = -100
+    nodes, real = [], train_fused.layer
+    monkeypatch.setattr(train_fused, "layer", lambda *a: (nodes.append(1), real(*a))[1])
+    loss, grads = _grads(model, ids, labels)
+    assert len(nodes) == 2
+    hooks = [layer.mlp.register_forward_hook(lambda *a: None) for layer in model.layers]
+    hooks.append(model.norm.register_forward_hook(lambda *a: None))
+    want_loss, want = _grads(model, ids, labels)
+    assert len(nodes) == 2
+    hooks[0].remove()
+    mixed_loss, mixed = _grads(model, ids, labels)
+    for h in hooks:
+        h.remove()
+    # rounded to bf16 at the same places; a value on a boundary that falls to the other side is 2^-8 off,
+    # and travels through both layers
+    for got_loss, got in ((loss, grads), (mixed_loss, mixed)):
+        assert abs(float(got_loss) - float(want_loss)) < 1e-3
+        for g, w in zip(got, want):
+            assert g.dtype == w.dtype and g.shape == w.shape
+            assert float((g - w).norm()) <= 2e-2 * float(w.norm())
+    with torch.no_grad(), torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+        assert torch.equal(model(ids, labels), loss)
+
+
+def test_second_derivatives_frozen_parameters_and_saved_tensor_hooks():
+    model = _model(layers=1)
+    ids = torch.randint(0, 1000, (1, 40), generator=_gen(1), device=DEV)
+    _, want = _grads(model, ids, ids)
+    _, recorded = _grads(model, ids, ids, create_graph=True)
+    names = [n for n, _ in model.named_parameters()]
+    for n, g, w in zip(names, recorded, want):
+        assert float((g.detach() - w).norm()) <= 2e-2 * float(w.norm()), n
+    # a gradient of a gradient that does not pass through the recurrent core
+    k = names.index("lm_head.weight")
+    second, = torch.autograd.grad(recorded[k].square().sum(), [model.norm.weight])
+    assert bool(torch.isfinite(second).all()) and float(second.abs().max()) > 0
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(1), t)[1], lambda t: t):
+        _, hooked = _grads(model, ids, ids)
+    assert packed and all(torch.equal(a, b) for a, b in zip(hooked, want))
+    model.layers[0].mlp.gate_up_proj.weight.requires_grad_(False)
+    model.embed_tokens.weight.requires_grad_(False)
+    _, frozen = _grads(model, ids, ids)
+    rest = [w for n, w in zip(names, want) if n not in ("layers.0.mlp.gate_up_proj.weight", "embed_tokens.weight")]
+    assert len(frozen) == len(rest)
+    for g, w in zip(frozen, rest):
+        assert float((g - w).norm()) <= 2e-2 * float(w.norm())
