@@ -97,13 +97,13 @@ class _Layer(Function):
         H = hidden.shape[-1]
         total = hidden if delta is None else hidden + delta
         xy = F.linear(F.rms_norm(total, (H,), n1, eps1), w_in)
-        gated = BlockCore.apply(xy, cw, cb, wi, bi, wa, ba, lam, False)[0]
+        gated = BlockCore.apply(xy, cw, cb, wi, bi, wa, ba, lam, False, torch.is_grad_enabled())[0]
         total = total + F.linear(gated, w_out)
         gate, up = F.linear(F.rms_norm(total, (H,), n2, eps2), w_gu).chunk(2, dim=-1)
         return total, F.linear(F.gelu(gate) * up, w_dn)
 
     @staticmethod
-    def forward(ctx, eps1, eps2, hidden, delta, n1, n2, w_in, w_out, w_gu, w_dn, cw, cb, wi, bi, wa, ba, lam):
+    def forward(ctx, recorded, eps1, eps2, hidden, delta, n1, n2, w_in, w_out, w_gu, w_dn, cw, cb, wi, bi, wa, ba, lam):
         B, T, H = hidden.shape
         rows, R, inter = B * T, w_out.shape[1], w_dn.shape[1]
         dev = hidden.device
@@ -111,7 +111,7 @@ class _Layer(Function):
         total1, x1, rstd1 = _add_norm(hidden.view(rows, H), None if delta is None else delta.view(rows, H), n1, eps1)
         xy = torch.mm(x1, w_in16.t()).view(B, T, 2 * R)
         wi16, wa16 = kernel_weights(wi, wa, rows)
-        grad = any(ctx.needs_input_grad)
+        grad = recorded and any(ctx.needs_input_grad)
         gated, u, xg, ag, h, _ = block_core_forward(xy, cw, cb, wi16, bi.reshape(-1), wa16, ba.reshape(-1), lam, grad,
                                                     False)
         mixed = torch.mm(gated.view(rows, R), w_out16.t())
@@ -134,8 +134,8 @@ class _Layer(Function):
         inputs = saved[:15]
         if torch.is_grad_enabled():
             grads = _replayed(lambda *a: _Layer.plain(*ctx.eps, *a), inputs, (d_total, d_out),
-                              ctx.needs_input_grad[2:])
-            return (None, None) + grads
+                              ctx.needs_input_grad[3:])
+            return (None, None, None) + grads
         hidden, delta, n1, n2 = inputs[:4]
         cw, wi, bi, lam = inputs[8], inputs[10], inputs[11], inputs[14]
         (w_in16, w_out16, w_gu16, w_dn16, wi16, wa16, total1, x1, rstd1, xy, u, xg, ag, h, gated, total2, x2, rstd2,
@@ -166,7 +166,7 @@ class _Layer(Function):
         shape = (B, T, H)
         grads = (d_hidden.view(shape), None if d_delta is None else d_delta.view(shape), d_n1, d_n2, d_in_w, d_out_w,
                  d_gu_w, d_dn, dcw, dcb, dwi, dbi.view(bi.shape), dwa, dba.view(bi.shape), dlam)
-        return (None, None) + tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad[2:]))
+        return (None, None, None) + tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad[3:]))
 
 
 class _Loss(Function):
@@ -245,7 +245,7 @@ def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 def layer(hidden, delta: Optional[torch.Tensor], eps1: float, eps2: float, params) -> Tuple[torch.Tensor, torch.Tensor]:
-    return _Layer.apply(eps1, eps2, hidden, delta, *params)
+    return _Layer.apply(torch.is_grad_enabled(), eps1, eps2, hidden, delta, *params)
 
 
 def loss(hidden, delta, eps: float, norm, head, labels) -> torch.Tensor:

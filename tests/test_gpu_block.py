@@ -161,3 +161,41 @@ def test_backward_without_bias_gradients_and_with_misaligned_weight_gradients():
     torch.cuda.synchronize()
     assert torch.equal(dwi.view(nb, bw, bw), ref[3]) and torch.equal(dwa.view(nb, bw, bw), ref[5])
     assert torch.equal(dbi, ref[4]) and torch.equal(dba, ref[6])
+
+
+def test_core_without_gradients_writes_no_states_and_gives_the_same_values():
+    """Under no_grad the scan's states stay unwritten, whatever the parameters ask for; same outputs bit for
+    bit.  Gradients enabled but asked of nothing: the same."""
+    import hawk_pytorch_amd as hk
+    from hawk_pytorch_amd import scan_fused
+
+    torch.manual_seed(0)
+    D, nb = 256, 4
+    conv = hk.Conv1D(D, 4, w_init_variance_scale=1.0).cuda()
+    gates = [hk.BlockDiagonalLinear(D, nb, device="cuda") for _ in range(2)]
+    lam = torch.nn.Parameter(hk.rnn_param_init(torch.empty(D, device="cuda"), 0.9, 0.999))
+    sizes, real = [], scan_fused._launch_block_core_fwd
+
+    def spy(*args):
+        got = real(*args)
+        sizes.append(got[4].numel())
+        return got
+
+    for B, T in [(2, 300), (1, 33), (3, 7)]:
+        xy = torch.randn(B, T, 2 * D, device="cuda").bfloat16()
+        try:
+            scan_fused._launch_block_core_fwd = spy
+            want, want_last = hk.recurrent_block_core(xy, conv, *gates, lam, return_last_state=True)
+            with torch.no_grad():
+                got, last = hk.recurrent_block_core(xy, conv, *gates, lam, return_last_state=True)
+                alone = hk.recurrent_block_core(xy, conv, *gates, lam)
+        finally:
+            scan_fused._launch_block_core_fwd = real
+        assert sizes[-3:] == [B * T * D, 0, 0]
+        assert want.requires_grad and not got.requires_grad
+        assert torch.equal(got, want) and torch.equal(last, want_last) and torch.equal(alone, want)
+        x, xg, ag, y = (torch.randn(B, T, D, device="cuda").bfloat16() for _ in range(4))
+        want, want_last = hk.fused_linear_scan_gated(x, xg, ag, lam, y, return_last_state=True)
+        with torch.no_grad():
+            got, last = hk.fused_linear_scan_gated(x, xg, ag, lam, y, return_last_state=True)
+        assert torch.equal(got, want) and torch.equal(last, want_last)
