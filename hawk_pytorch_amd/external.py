@@ -299,10 +299,16 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     )
     assert recc_state.numel() == B * D and recc_state.is_contiguous()
     assert x_new.dtype == torch.bfloat16 and conv_state.dtype == torch.bfloat16, "the fused step runs on bf16"
-    dev = _lib.require_cuda(conv_state, x_new, conv.w, input_gate.w, a_gate.w, a_param, recc_state, y)
+    conv_w, w_i, w_a = conv.w, input_gate.w, a_gate.w
+    dev, index = x_new.device, x_new.get_device()
+    for t in (conv_state, conv_w, w_i, w_a, a_param, recc_state, y):
+        if index < 0 or t.get_device() != index:
+            _lib.require_cuda(conv_state, x_new, conv_w, w_i, w_a, a_param, recc_state, y)   # says which
 
     def rows(t):
-        """[B, D] view with unit column stride and its row stride, copying only if it must."""
+        """[B, D] rows with unit column stride and the distance between them, copying only if it must."""
+        if t.dtype == torch.bfloat16 and t.ndim == 3 and t.shape[1] == 1 and t.stride(2) == 1 and t.stride(0) >= D:
+            return t, (t.stride(0) if B > 1 else D)
         t2 = t.reshape(B, D) if t.dtype == torch.bfloat16 else t.reshape(B, D).to(torch.bfloat16)
         if t2.stride(1) != 1 or (B > 1 and t2.stride(0) < D):
             t2 = t2.contiguous()
@@ -314,11 +320,11 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     y2, ldy = rows(y)
     w32, b32, b_i, b_a, lam = (
         t if t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-        else _lib.dense16(t.detach().float()) for t in (conv.w, conv.b, input_gate.b, a_gate.b, a_param))
-    w_i, w_a = _lib.dense16(input_gate.w.detach()), _lib.dense16(a_gate.w.detach())
+        else _lib.dense16(t.detach().float()) for t in (conv_w, conv.b, input_gate.b, a_gate.b, a_param))
+    w_i, w_a = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else _lib.dense16(t.detach()) for t in (w_i, w_a))
     if w_a.dtype != w_i.dtype:
-        w_a = w_a.to(w_i.dtype)
-    out = torch.empty((B, D), dtype=torch.bfloat16, device=dev)
+        w_a = w_a.detach().to(w_i.dtype)
+    out = torch.empty(shape, dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
     with _lib.on_device(dev):
         # counters that let several workgroups share a block's output columns
@@ -332,7 +338,7 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
             _lib.stream_ptr(dev),
         )
     _lib.check("hawk_decode_core_step_ws", status)
-    return out.reshape(shape)
+    return out
 
 
 # ---------------------------------------------------------------------------------------
