@@ -95,6 +95,9 @@ SIGNATURES = {
     "hawk_cross_entropy_fwd": (_c_int, [_c_void_p] * 5 + [_c_int] * 3 + [_c_void_p]),
     "hawk_cross_entropy_bwd": (_c_int, [_c_void_p] * 6 + [_c_int] * 3 + [_c_void_p]),
     "hawk_embedding_bwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p]),
+    "hawk_weight_grad_supported": (_c_int, [_c_int] * 3),
+    "hawk_weight_grad_workspace_bytes": (_c_size_t, [_c_int] * 3),
+    "hawk_weight_grad": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),
     "hawk_decode_linear_supported": (_c_int, [_c_int] * 3),
     "hawk_decode_linear_workspace_bytes": (_c_size_t, [_c_int] * 3),
     "hawk_decode_linear": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),

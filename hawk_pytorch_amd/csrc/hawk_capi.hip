@@ -381,6 +381,22 @@ int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, 
     return hawk::embedding_bwd(ids, dout, dweight, rows, V, D, as_stream(stream));
 }
 
+int hawk_weight_grad_supported(int rows, int N, int K) { return hawk::weight_grad_supported(rows, N, K) ? 1 : 0; }
+
+size_t hawk_weight_grad_workspace_bytes(int rows, int N, int K) {
+    return hawk::weight_grad_supported(rows, N, K) ? hawk::weight_grad_workspace_bytes(rows, N, K) : 0;
+}
+
+int hawk_weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K, void* workspace_device,
+                     size_t workspace_bytes, void* stream) {
+    if (!dy || !x || !dw) return HAWK_ERR_NULL_POINTER;
+    if (!hawk::weight_grad_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(dy) || !aligned16(x) || !aligned16(dw) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    const size_t need = hawk::weight_grad_workspace_bytes(rows, N, K);
+    if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;
+    return hawk::weight_grad(dy, x, dw, rows, N, K, workspace_device, as_stream(stream));
+}
+
 int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }
 
 size_t hawk_decode_linear_workspace_bytes(int M, int N, int K) {

@@ -136,6 +136,11 @@ int cross_entropy_bwd(const void* logits, const long long* labels, const float* 
                       const float* dloss, void* dlogits, int rows, int T, int V, hipStream_t st);
 int embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D, hipStream_t st);
 
+// hawk_wgrad.hip
+bool weight_grad_supported(int rows, int N, int K);
+size_t weight_grad_workspace_bytes(int rows, int N, int K);
+int weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K, void* ws, hipStream_t st);
+
 // hawk_probe.hip
 bool stream_probe_shape_ok(size_t bytes, size_t row_pitch, int shape);
 int stream_probe(const void* const* reads, int n_reads, void* const* writes, int n_writes, size_t bytes,

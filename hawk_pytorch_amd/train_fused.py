@@ -73,6 +73,31 @@ def _add_norm_backward(dout, total, rstd, weight, d_direct, want_delta: bool):
     return d_sum, d_delta, dweight
 
 
+def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """dy^T x of [n, N] and [n, K]: fp32 by the kernel that splits the rows, where the result is at most 128 of
+    its tiles; from there on the library's product is as fast or faster, in bf16."""
+    n, N = dy.shape
+    K = x.shape[1]
+    lib = _lib.load()
+    if -(-N // 128) * -(-K // 128) > 128 or not lib.hawk_weight_grad_supported(n, N, K):
+        return torch.mm(dy.t(), x)
+    dev = dy.device
+    dw = torch.empty((N, K), dtype=_F32, device=dev)
+    nbytes = lib.hawk_weight_grad_workspace_bytes(n, N, K)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    with _lib.on_device(dev):
+        _check("hawk_weight_grad", dy.data_ptr(), x.data_ptr(), dw.data_ptr(), n, N, K, _lib.ptr(ws), nbytes,
+               _lib.stream_ptr(dev))
+    return dw
+
+
+def _all_fp32(tensors):
+    """The tensors, those in bf16 converted by one launch."""
+    narrow = [t for t in tensors if t.dtype != _F32]
+    wide = iter(_cast(narrow, _F32) if narrow else ())
+    return [t if t.dtype == _F32 else next(wide) for t in tensors]
+
+
 def _replayed(fn, inputs, grads, needs):
     """Gradients of fn(*inputs) as a differentiable graph, for a backward pass that is itself recorded."""
     wanted = [t for t, need in zip(inputs, needs) if need]
@@ -146,23 +171,23 @@ class _Layer(Function):
         dev = hidden.device
         d_total, d_out = _dense(d_total, _F32).view(rows, H), _dense(d_out, _BF16).view(rows, H)
         d_act = torch.mm(d_out, w_dn16)
-        d_dn = torch.mm(d_out.t(), act)
+        d_dn = _weight_grad(d_out, act)
         d_gu = torch.empty_like(gu)
         with _lib.on_device(dev):
             _check("hawk_gelu_mul_bwd", gu.data_ptr(), d_act.data_ptr(), d_gu.data_ptr(), rows, inter,
                    _lib.stream_ptr(dev))
         d_x2 = torch.mm(d_gu, w_gu16)
-        d_gu_w = torch.mm(d_gu.t(), x2)
+        d_gu_w = _weight_grad(d_gu, x2)
         d_total, d_mixed, d_n2 = _add_norm_backward(d_x2, total2, rstd2, n2, d_total, True)
         d_gated = torch.mm(d_mixed, w_out16)
-        d_out_w = torch.mm(d_mixed.t(), gated.view(rows, R))
+        d_out_w = _weight_grad(d_mixed, gated.view(rows, R))
         d_xy, dcw, dcb, dwi, dbi, dwa, dba, dlam = block_core_backward(xy, u, xg, ag, h, cw, wi16, wa16, lam,
                                                                        d_gated.view(B, T, R))
         d_xy = d_xy.view(rows, 2 * R)
         d_x1 = torch.mm(d_xy, w_in16)
-        d_in_w = torch.mm(d_xy.t(), x1)
+        d_in_w = _weight_grad(d_xy, x1)
         d_hidden, d_delta, d_n1 = _add_norm_backward(d_x1, total1, rstd1, n1, d_total, delta is not None)
-        d_in_w, d_out_w, d_gu_w, d_dn = _cast([d_in_w, d_out_w, d_gu_w, d_dn], _F32)
+        d_in_w, d_out_w, d_gu_w, d_dn = _all_fp32([d_in_w, d_out_w, d_gu_w, d_dn])
         shape = (B, T, H)
         grads = (d_hidden.view(shape), None if d_delta is None else d_delta.view(shape), d_n1, d_n2, d_in_w, d_out_w,
                  d_gu_w, d_dn, dcw, dcb, dwi, dbi.view(bi.shape), dwa, dba.view(bi.shape), dlam)

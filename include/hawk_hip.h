@@ -334,6 +334,14 @@ int hawk_cross_entropy_bwd(const void* logits, const long long* labels, const fl
 int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D,
                        void* stream);
 
+/* dw [N, K] fp32 = dy^T x for dy [rows, N] and x [rows, K] bf16: the weight gradient of a linear layer, summed
+ * in fp32 in a fixed order.  Dense and 16-byte aligned, N and K multiples of 8, rows * N and rows * K below
+ * 2^30.  The workspace (NULL where the query says 0) takes partial results. */
+int hawk_weight_grad_supported(int rows, int N, int K);
+size_t hawk_weight_grad_workspace_bytes(int rows, int N, int K);
+int hawk_weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K,
+                     void* workspace_device, size_t workspace_bytes, void* stream);
+
 /* Dense projections of a decode step: out [M, N] = x [M, K] w^T for up to 256 rows, bf16 with
  * fp32 sums, w [N, K] as torch.nn.Linear keeps it (upstream: the Linear calls of
  * hawk/hawk.py:70-86, :163-203, :284-303 on one token per sequence).  K must be a multiple of

@@ -201,3 +201,16 @@ def test_second_derivatives_frozen_parameters_and_saved_tensor_hooks():
     assert len(frozen) == len(rest)
     for g, w in zip(frozen, rest):
         assert float((g - w).norm()) <= 2e-2 * float(w.norm())
+
+
+# a single value, ragged edges of a tile in all three sizes, rows that end inside a step, one and several splits
+@pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (64, 128, 128), (77, 136, 120), (513, 264, 136), (1024, 128, 256),
+                                      (2047, 1024, 512), (4593, 8, 1032), (130, 2048, 1024)])
+def test_weight_gradient(rows, N, K):
+    gen = _gen(rows)
+    dy, x = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, rows, K, dtype=torch.bfloat16)
+    got = train_fused._weight_grad(dy, x)
+    assert got.dtype == torch.float32
+    want = dy.double().t() @ x.double()
+    _close(got, want, (rows + 8) * EPS32 * (dy.double().abs().t() @ x.double().abs()))   # fp32 sums of exact products
+    assert torch.equal(train_fused._weight_grad(dy, x), got)
