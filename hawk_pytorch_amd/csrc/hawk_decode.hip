@@ -15,6 +15,9 @@
 //   * the four partial tiles meet in LDS at the end and leave in whole rows;
 //   * projections with few columns also split K over workgroups and leave fp32 partial sums, which
 //     the kernel that follows (residual add + norm) adds up in a fixed order on its way.
+// A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 49 / 53 / 63 /
+// 82 / 104 us at 1 / 32 / 64 / 128 / 256 rows with cold weights (157 MB); the library's four products alone
+// took 121 us at 256 rows, with the norms, additions, GELU and product around them 149.
 // All sums are fp32, in an order that depends on the shape alone, and values are rounded to bf16 where
 // the separate operations round them, so both routes differ by the order of the sums only.
 #include "hawk_scan.h"

@@ -17,7 +17,8 @@ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------------------
 // Conversions of up to kCastSegments arrays in one launch: a layer's four weights to bf16 in front of
-// its forward, their gradients to fp32 behind its backward (a launch each otherwise).
+// its forward, their gradients to fp32 behind its backward.  Bound by memory; a launch each (4 us with
+// the gap) is what it spares: 6.5 us for the 2.4 M weights of a layer of 512 x 1024.
 // ---------------------------------------------------------------------------------------
 constexpr int kCastThreads = 256;
 struct CastTask {
@@ -47,7 +48,10 @@ __global__ __launch_bounds__(kCastThreads) void cast_kernel(CastTask t) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Residual add + RMSNorm.  A wave owns a row; a lane owns Q groups of 8 adjacent channels.
+// Residual add + RMSNorm.  A wave owns a row, so its sum is a few shuffles and rows need no barrier; a lane
+// owns Q groups of 8 adjacent channels (16 bytes of bf16).  Memory and, at a few thousand rows,
+// latency bound.  2048 rows of 512: forward 5.2 us (add, norm and conversion to bf16 apart 12.8),
+// backward 6.2 + 3.0 for the weight's sums (conversion, two norm kernels, weight sums and add apart 25).
 // ---------------------------------------------------------------------------------------
 constexpr int kNormWaves = 4;
 
@@ -186,7 +190,9 @@ __global__ __launch_bounds__(kColsumThreads) void norm_weight_kernel(ColsumTask 
 }
 
 // ---------------------------------------------------------------------------------------
-// act = gelu(gate) * up on rows [gate, up] of 2 I channels, and its gradient in the same layout.
+// act = gelu(gate) * up on rows [gate, up] of 2 I channels, and its gradient in the same layout, 16 bytes
+// per lane and access.  Memory bound: 2048 rows of 2 x 1024 forward 4.8 us (GELU and product apart 13),
+// backward 6.3 (two products, GELU gradient and concatenation apart 33).
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void gelu_mul_fwd_kernel(const bf16_t* __restrict__ gu, bf16_t* __restrict__ act,
                                                            size_t groups, int per_row) {
@@ -249,7 +255,9 @@ __global__ __launch_bounds__(256) void gelu_mul_bwd_kernel(const bf16_t* __restr
 // Next-token cross entropy on bf16 logits [B T, V]: row (b, t) is scored against labels[b, t + 1], the
 // last row of a sequence and rows whose label is -100 count for nothing.  The forward reads the logits
 // once (running maximum and sum), the backward reads them once more and writes their gradient; as
-// fp32 log-probabilities the same rows were written and read six times over in 32 bits.
+// fp32 log-probabilities the same rows were written and read six times over in 32 bits.  A workgroup
+// per row; the exponentials of 512 threads keep up with memory: 46 us forward, 43 backward at 2048 rows of
+// 32000 (2.9 and 6.1 TB/s), 550 us before.
 // ---------------------------------------------------------------------------------------
 constexpr int kCeThreads = 512;
 constexpr long long kIgnoreIndex = -100;
@@ -374,7 +382,8 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(
 // id, in their order.  The workgroup of a token's first occurrence lists all of them (one wave, 64
 // positions per ballot) and adds the rows; the eight waves take an eighth of the list each, so that
 // one frequent token (padding) is not one wave's work.  Looking through all positions costs
-// every workgroup rows / 64 ballots, which is why the number of rows is limited.
+// every workgroup rows / 64 ballots, which is why the number of rows is limited.  2048 tokens of 512
+// channels: 23 us (the library's kernel 126).
 // ---------------------------------------------------------------------------------------
 constexpr int kEmbedWaves = 8;
 

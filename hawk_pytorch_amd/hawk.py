@@ -4,17 +4,22 @@ This is the harness that calls the hot path the way upstream's model does
 (hawk/hawk.py:89-303): same constructor arguments, same forward signatures, same
 parameter names and shapes (so an upstream ``state_dict`` loads unchanged), same
 zero-initialised output projections.  The dense projections and norms are ordinary
-PyTorch-ROCm modules (library GEMMs); the loss is plain ``F.cross_entropy``.
+PyTorch-ROCm modules (library GEMMs) and the loss is plain ``F.cross_entropy``, except on the two
+paths named last below.
 
-What differs from upstream is confined to the recurrent block:
+What differs from upstream is the recurrent block and how a whole pass is launched:
 
 * prefill and training call ``Conv1D`` and the scan from this package; with
   ``HawkConfig.fused_epilogue`` (default) the scan kernel also applies the block's gate,
   ``gelu(y) * h``, and its backward also produces the gate's gradient;
-* decode (``use_cache=True`` with a warm ``RNNCache``) issues two fused kernels per layer
-  (conv window roll + conv; gate biases + RG-LRU state update + output gate) instead of
-  about thirty eager ones, works for any batch size, and evaluates the two gate
-  projections once instead of twice.
+* decode (``use_cache=True`` with a warm ``RNNCache``) issues one fused kernel per layer for the
+  recurrent core, works for any batch size, and evaluates the two gate projections once instead
+  of twice;
+* a decode step of bf16 weights without gradients (``HawkModel._decode_step``) and a training pass of
+  fp32 weights under bf16 autocast (``HawkModel._train_step``) run the norms, residual additions, gated
+  GELU, loss and, in decode, the projections as this package's kernels, with the modules' parameters and
+  roundings.  Where a module is not what the constructor made, or something watches its call, the
+  modules run.
 """
 
 from __future__ import annotations
