@@ -380,28 +380,6 @@ def decode_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     return ws
 
 
-_decode_layer_workspaces: dict = {}
-_MAX_DECODE_LAYER_WORKSPACES = 16   # streams; the oldest is dropped first
-
-
-def decode_layer_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
-    """Scratch of a decode step's layers, one buffer per (device, stream): calls on a stream are
-    ordered, and nothing is kept in it from one call to the next.  A graph being recorded gets its
-    own, from its own memory."""
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    key = (_device_index(dev), stream_ptr(dev))
-    with _lock:
-        ws = _decode_layer_workspaces.get(key)
-        if ws is None or ws.numel() < nbytes:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-            _decode_layer_workspaces.pop(key, None)
-            while len(_decode_layer_workspaces) >= _MAX_DECODE_LAYER_WORKSPACES:
-                _decode_layer_workspaces.pop(next(iter(_decode_layer_workspaces)))
-            _decode_layer_workspaces[key] = ws
-    return ws
-
-
 def release_workspaces() -> None:
     """Drop every cached scan and decode workspace (they are re-created on demand)."""
     with _lock:
@@ -409,7 +387,6 @@ def release_workspaces() -> None:
         _captured.clear()
         _decode_workspaces.clear()
         _decode_captured.clear()
-        _decode_layer_workspaces.clear()
 
 
 def _flag_of(ws: torch.Tensor, dev: torch.device) -> int:

@@ -362,7 +362,9 @@ class DecodeLayers:
         dev = self.dev = hidden.device
         self.lib = _lib.load()
         nbytes = max(self.lib.hawk_decode_layer_workspace_bytes(self.M, self.H, R, inter, n) for n in (2 * R, vocab))
-        self.ws = _lib.decode_layer_workspace(dev, nbytes)
+        # one allocation per step, not a buffer kept per stream: a layer is several launches that hand
+        # values on in it, and two threads may issue steps to one stream
+        self.ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         self.stream = _lib.stream_ptr(dev)
 
     def first(self, norm_w: torch.Tensor, eps: float, w: torch.Tensor) -> torch.Tensor:
