@@ -234,7 +234,8 @@ class Hawk(nn.Module):
 def _plain(module: Optional[nn.Module], cls: type) -> bool:
     """Exactly this class, and a call of it runs this class's forward and nothing else."""
     return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
-            and not module._forward_pre_hooks and module._compiled_call_impl is None)
+            and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks
+            and module._compiled_call_impl is None)
 
 
 def _dense_param(module: Optional[nn.Module], name: str, shape, dtype: torch.dtype,

@@ -214,3 +214,18 @@ def test_weight_gradient(rows, N, K):
     want = dy.double().t() @ x.double()
     _close(got, want, (rows + 8) * EPS32 * (dy.double().abs().t() @ x.double().abs()))   # fp32 sums of exact products
     assert torch.equal(train_fused._weight_grad(dy, x), got)
+
+
+@pytest.mark.parametrize("where", ["layers.0", "layers.1.mlp", "layers.0.recc.input_xy", "norm", "lm_head", "embed_tokens"])
+def test_backward_hooks_of_modules_are_called(where):
+    """Full backward hooks and backward pre-hooks, on every kind of module a node would stand for."""
+    model = _model()
+    ids = torch.randint(0, 1000, (1, 40), generator=_gen(2), device=DEV)
+    module, called = model.get_submodule(where), []
+    handles = [module.register_full_backward_hook(lambda *a: called.append("hook")),
+               module.register_full_backward_pre_hook(lambda *a: called.append("pre"))]
+    with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+        model(ids, ids).backward()
+    assert sorted(called) == ["hook", "pre"]
+    for h in handles:
+        h.remove()
