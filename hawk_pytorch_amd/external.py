@@ -307,8 +307,9 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
 
     def rows(t):
         """[B, D] rows with unit column stride and the distance between them, copying only if it must."""
-        if t.dtype == torch.bfloat16 and t.ndim == 3 and t.shape[1] == 1 and t.stride(2) == 1 and t.stride(0) >= D:
+        if t.dtype == torch.bfloat16 and t.shape == (B, 1, D) and t.stride(2) == 1 and t.stride(0) >= D:
             return t, (t.stride(0) if B > 1 else D)
+        # any other shape of B * D elements is folded into rows; one of more or fewer raises here
         t2 = t.reshape(B, D) if t.dtype == torch.bfloat16 else t.reshape(B, D).to(torch.bfloat16)
         if t2.stride(1) != 1 or (B > 1 and t2.stride(0) < D):
             t2 = t2.contiguous()
@@ -318,9 +319,10 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     if ldx % 8 != 0 or xn.data_ptr() % 16 != 0:
         xn, ldx = _lib.dense16(xn.contiguous()), D
     y2, ldy = rows(y)
+    b_i, b_a = (t if t.numel() == D else t.reshape(D) for t in (input_gate.b, a_gate.b))   # (raises for another size)
     w32, b32, b_i, b_a, lam = (
         t if t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
-        else _lib.dense16(t.detach().float()) for t in (conv_w, conv.b, input_gate.b, a_gate.b, a_param))
+        else _lib.dense16(t.detach().float()) for t in (conv_w, conv.b, b_i, b_a, a_param))
     w_i, w_a = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else _lib.dense16(t.detach()) for t in (w_i, w_a))
     if w_a.dtype != w_i.dtype:
         w_a = w_a.detach().to(w_i.dtype)

@@ -446,3 +446,109 @@ def test_activation_placement_steps_through_the_kilobyte(monkeypatch):
     with pytest.raises(ValueError):
         _lib.activation_empty(shape, torch.bfloat16, "cpu")
     assert _lib.activation_empty((8, 64), torch.bfloat16, "cpu").numel() == 512   # small: the setting is not read
+
+
+class _RecordingLibrary:
+    """Stands for the loaded library in a test of argument handling: notes the calls, launches nothing."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        return lambda *a: (self.calls.append((name, a)), 0)[1]
+
+
+@pytest.fixture
+def decode_step_on_cpu(monkeypatch):
+    """decode_core_step on CPU tensors, up to the launch: returns (call, recorded launches)."""
+    import contextlib
+
+    from hawk_pytorch_amd import external
+
+    lib = _RecordingLibrary()
+    monkeypatch.setattr(_lib, "load", lambda: lib)
+    monkeypatch.setattr(_lib, "on_device", lambda dev: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream_ptr", lambda dev: 0)
+    monkeypatch.setattr(_lib, "require_cuda", lambda *t: t[0].device)
+    monkeypatch.setattr(_lib, "decode_workspace", lambda dev, n: torch.zeros(16, dtype=torch.uint8))
+
+    def call(B, D, x_new, y, **biases):
+        conv = hk.Conv1D(width=D, temporal_width=4)
+        gates = [hk.BlockDiagonalLinear(D, D // 64) for _ in range(2)]
+        for name, b in biases.items():
+            gates[name == "b_a"].b = torch.nn.Parameter(b)
+        lib.calls.clear()
+        with torch.no_grad():
+            return external.decode_core_step(torch.zeros(B, 3, D).bfloat16(), x_new, conv, gates[0], gates[1],
+                                             torch.zeros(D), torch.zeros(B, 1, D), y)
+
+    return call, lib.calls
+
+
+def _rows(*shape):
+    return torch.arange(math.prod(shape)).reshape(shape).bfloat16()
+
+
+@pytest.mark.parametrize("which", ["x_new", "y"])
+@pytest.mark.parametrize("make", [
+    lambda D: _rows(1, 1, D), lambda D: _rows(3, 1, D), lambda D: _rows(5, 1, D), lambda D: _rows(4, 1, 2 * D),
+    lambda D: _rows(8, 1, 2 * D)[:4], lambda D: _rows(4, 1, D + 64), lambda D: _rows(4, 1, D + 1),
+    lambda D: _rows(4, 1, D)[:, :, :64],
+], ids=["one row", "too few rows", "too many rows", "not chunked", "not chunked, a slice", "wider", "one wider", "narrower"])
+def test_decode_core_step_refuses_rows_of_another_shape(which, make, decode_step_on_cpu):
+    """The kernel reads B rows of D elements: an operand that holds others is refused before any launch."""
+    B, D = 4, 256
+    call, launches = decode_step_on_cpu
+    other = make(D)
+    with pytest.raises((RuntimeError, AssertionError)):
+        call(B, D, **{"x_new": _rows(B, 1, D), "y": _rows(B, 1, D), which: other})
+    assert not any(name == "hawk_decode_core_step_ws" for name, _ in launches)
+
+
+@pytest.mark.parametrize("make", [
+    lambda B, D: _rows(B, 1, D), lambda B, D: _rows(B, D), lambda B, D: _rows(B, 1, 2 * D)[:, :, D:],
+    lambda B, D: _rows(B, 1, D + 8)[:, :, :D], lambda B, D: _rows(B, 1, D + 3)[:, :, 3:], lambda B, D: _rows(B, 2 * D)[:, :D],
+    lambda B, D: _rows(1, B, D), lambda B, D: _rows(B // 2, 1, 2 * D) if B > 1 else _rows(1, 1, D),
+    lambda B, D: _rows(B // 2, 1, 3 * D)[:, :, :2 * D] if B > 1 else _rows(1, 1, D),
+    lambda B, D: _rows(1, 1, D).expand(B, 1, D), lambda B, D: _rows(D, 1, B).transpose(0, 2),
+    lambda B, D: _rows(B, 1, 2 * D)[:, :, ::2], lambda B, D: _rows(B, 2, D)[:, 1:], lambda B, D: _rows(B, 1, D).float(),
+], ids=["dense", "2-d", "half", "padded", "unaligned", "2-d half", "rows in the middle", "folded", "folded, padded",
+        "expanded", "transposed", "every other", "every other row", "fp32"])
+@pytest.mark.parametrize("B", [1, 4])
+def test_decode_core_step_hands_over_the_rows_it_was_given(B, make, decode_step_on_cpu, monkeypatch):
+    """Whatever the layout, the pointer and row distance that reach the library describe t.reshape(B, D)."""
+    import ctypes as c
+
+    D = 256
+    call, _ = decode_step_on_cpu
+    seen = []
+
+    def read(ptr, ld):
+        whole = (c.c_uint16 * ((B - 1) * ld + D)).from_address(ptr)
+        flat = torch.frombuffer(bytearray(whole), dtype=torch.bfloat16)
+        return flat.as_strided((B, D), (ld, 1)).clone()
+
+    real = _RecordingLibrary.__getattr__
+
+    def spy(self, name):
+        f = real(self, name)
+        if name != "hawk_decode_core_step_ws":
+            return f
+        return lambda *a: (seen.append((read(a[1], a[2]), read(a[10], a[11]))), f(*a))[1]
+
+    monkeypatch.setattr(_RecordingLibrary, "__getattr__", spy)
+    t = make(B, D)
+    for x_new, y in ((_rows(B, 1, D), t), (t.bfloat16(), _rows(B, 1, D))):
+        seen.clear()
+        assert call(B, D, x_new, y).shape == x_new.shape
+        (got_x, got_y), = seen
+        assert torch.equal(got_x, x_new.reshape(B, D)) and torch.equal(got_y, y.reshape(B, D).bfloat16())
+
+
+@pytest.mark.parametrize("which", ["b_i", "b_a"])
+@pytest.mark.parametrize("n", [64, 192, 320])
+def test_decode_core_step_refuses_biases_of_another_size(which, n, decode_step_on_cpu):
+    call, launches = decode_step_on_cpu
+    with pytest.raises(RuntimeError):
+        call(2, 256, _rows(2, 1, 256), _rows(2, 1, 256), **{which: torch.zeros(n)})
+    assert not any(name == "hawk_decode_core_step_ws" for name, _ in launches)
