@@ -256,6 +256,13 @@ def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.devi
     return _dense_param(module, "weight", shape, dtype, dev)
 
 
+def _node_input(hidden: torch.Tensor, shape, dev: torch.device) -> bool:
+    """Whether a training node can read a hidden state that a module returned: the kernels take its
+    pointer, and the labels are read by its rows, so nothing about it can be taken for granted."""
+    return (type(hidden) is torch.Tensor and hidden.dtype == torch.float32 and hidden.device == dev
+            and hidden.shape == shape and hidden.is_contiguous() and hidden.data_ptr() % 16 == 0)
+
+
 class RNNLayer(nn.Module):
     """Pre-norm residual layer: recurrent block, then MLP."""
 
@@ -414,17 +421,22 @@ class HawkModel(nn.Module):
                    and cfg.recurrent_size // cfg.num_blocks in (32, 64, 128, 256)
                    and rows * max(cfg.intermediate_size, cfg.recurrent_size) < 1 << 31)
         delta = None
+        shape = (*input_ids.shape, H)
         for layer in self.layers:
             weights = layer.train_weights(cfg, dev) if kernels and type(layer) is RNNLayer else None
-            if (weights is None or hidden.dtype != f32 or not hidden.is_contiguous()
+            if (weights is None or not _node_input(hidden, shape, dev)
                     or (grad and not all(p.requires_grad for p in weights[2]))):
                 hidden, _ = layer(hidden if delta is None else hidden + delta, layer_past=None)
                 delta = None
             else:
                 hidden, delta = train_fused.layer(hidden, delta, *weights)
-        if hidden.dtype != f32 or not hidden.is_contiguous():
-            hidden = hidden.float().contiguous()
+        if not _node_input(hidden, shape, dev):
+            return self._next_token_loss(self.norm(hidden if delta is None else hidden + delta), labels)
         return train_fused.loss(hidden, delta, self.norm.eps, norm, head, labels)
+
+    def _next_token_loss(self, hidden_states: torch.Tensor, labels: torch.Tensor) -> torch.Tensor:
+        logits = self.lm_head(hidden_states[..., :-1, :])
+        return F.cross_entropy(logits.reshape(-1, logits.size(-1)).float(), labels[..., 1:].reshape(-1))
 
     def forward(
         self,
@@ -455,6 +467,5 @@ class HawkModel(nn.Module):
         if self.use_cache:
             return self.lm_head(hidden_states), caches
         if labels is not None:
-            logits = self.lm_head(hidden_states[..., :-1, :])
-            return F.cross_entropy(logits.reshape(-1, logits.size(-1)).float(), labels[..., 1:].reshape(-1))
+            return self._next_token_loss(hidden_states, labels)
         return self.lm_head(hidden_states)

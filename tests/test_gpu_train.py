@@ -229,3 +229,48 @@ def test_backward_hooks_of_modules_are_called(where):
     assert sorted(called) == ["hook", "pre"]
     for h in handles:
         h.remove()
+
+
+class _Returns(torch.nn.Module):
+    """A layer of someone's own: the layer it wraps, and then something done to the hidden state."""
+
+    def __init__(self, layer, fn):
+        super().__init__()
+        self.layer, self.fn = layer, fn
+
+    def forward(self, hidden, layer_past=None):
+        hidden, cache = self.layer(hidden, layer_past=layer_past)
+        return self.fn(hidden), cache
+
+
+def _off_boundary(h):
+    return torch.cat([h.new_zeros(1), h.reshape(-1)])[1:].view(h.shape)
+
+
+@pytest.mark.parametrize("fn", [_off_boundary, lambda h: h.bfloat16(), lambda h: h.transpose(0, 1).contiguous().transpose(0, 1)],
+                         ids=["off a 16-byte boundary", "bf16", "transposed in memory"])
+@pytest.mark.parametrize("at", [0, 1])
+def test_hidden_states_that_the_nodes_cannot_read_take_the_modules(at, fn):
+    model = _model()
+    model.layers[at] = _Returns(model.layers[at], fn)
+    ids = torch.randint(0, 1000, (2, 40), generator=_gen(4), device=DEV)
+    loss, grads = _grads(model, ids, ids)
+    hooks = [m.register_forward_hook(lambda *a: None) for m in (model.norm, model.layers[1 - at])]
+    want_loss, want = _grads(model, ids, ids)
+    for h in hooks:
+        h.remove()
+    assert abs(float(loss) - float(want_loss)) < 1e-3
+    for g, w in zip(grads, want):
+        assert float((g - w).norm()) <= 2e-2 * float(w.norm())
+
+
+@pytest.mark.parametrize("fn", [lambda h: h[:, :-1].contiguous(), lambda h: torch.cat([h, h], dim=1), lambda h: h.cpu()],
+                         ids=["shorter", "longer", "on another device"])
+@pytest.mark.parametrize("at", [0, 1])
+def test_hidden_states_of_another_shape_or_device_are_refused(at, fn):
+    """As the modules refuse them: by the loss for want of as many labels, by an operator for the device."""
+    model = _model()
+    model.layers[at] = _Returns(model.layers[at], fn)
+    ids = torch.randint(0, 1000, (2, 40), generator=_gen(4), device=DEV)
+    with pytest.raises((ValueError, RuntimeError)):
+        _grads(model, ids, ids)

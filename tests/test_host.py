@@ -552,3 +552,21 @@ def test_decode_core_step_refuses_biases_of_another_size(which, n, decode_step_o
     with pytest.raises(RuntimeError):
         call(2, 256, _rows(2, 1, 256), _rows(2, 1, 256), **{which: torch.zeros(n)})
     assert not any(name == "hawk_decode_core_step_ws" for name, _ in launches)
+
+
+def test_training_nodes_take_only_hidden_states_their_kernels_can_read():
+    """What a layer that ran as a module returned is looked at before a node takes its pointer."""
+    from hawk_pytorch_amd.hawk import _node_input
+
+    cpu, shape = torch.device("cpu"), (2, 3, 8)
+    good = torch.zeros(shape)
+    assert _node_input(good, shape, cpu)
+    assert not _node_input(good, shape, torch.device("cuda", 0))                 # on another device
+    assert not _node_input(torch.zeros(shape, device="meta"), shape, cpu)
+    assert not _node_input(good[:, :2].contiguous(), shape, cpu)                 # fewer positions than labels
+    assert not _node_input(torch.zeros(2, 4, 8), shape, cpu)                     # more
+    assert not _node_input(good.view(6, 8), shape, cpu)
+    assert not _node_input(good.bfloat16(), shape, cpu)
+    assert not _node_input(torch.zeros(3, 2, 8).transpose(0, 1), shape, cpu)
+    assert not _node_input(torch.zeros(49)[1:].view(shape), shape, cpu)          # not on a 16-byte boundary
+    assert not _node_input(torch.nn.Parameter(good), shape, cpu)
