@@ -99,10 +99,16 @@ def _all_fp32(tensors):
 
 
 def _replayed(fn, inputs, grads, needs):
-    """Gradients of fn(*inputs) as a differentiable graph, for a backward pass that is itself recorded."""
-    wanted = [t for t, need in zip(inputs, needs) if need]
+    """Gradients of fn(*inputs) as a differentiable graph, for a backward pass that is itself recorded.
+
+    fn runs on aliases and the gradients are taken with respect to those.  The inputs themselves are still
+    part of the graph that made them: where one is used again further up (a head tied to the embedding, a
+    layer at two depths, one weight for both gates), a gradient with respect to the input would hold the
+    other uses' share too, which their own nodes return once more."""
     with torch.enable_grad(), torch.autocast(device_type="cuda", dtype=_BF16):
+        inputs = [t.view_as(t) if need else t for t, need in zip(inputs, needs)]
         outs = fn(*inputs)
+    wanted = [t for t, need in zip(inputs, needs) if need]
     pairs = [(o, g) for o, g in zip(outs, grads) if g is not None]
     found = iter(torch.autograd.grad([o for o, _ in pairs], wanted, [g for _, g in pairs], create_graph=True,
                                      allow_unused=True))

@@ -274,3 +274,41 @@ def test_hidden_states_of_another_shape_or_device_are_refused(at, fn):
     ids = torch.randint(0, 1000, (2, 40), generator=_gen(4), device=DEV)
     with pytest.raises((ValueError, RuntimeError)):
         _grads(model, ids, ids)
+
+
+def _as_modules(model):
+    """Hooks that send the whole pass through the modules."""
+    return [m.register_forward_hook(lambda *a: None) for m in (model.norm, *(layer.mlp for layer in model.layers))]
+
+
+def _embedding_penalty(model, ids):
+    """Recorded gradients of the loss, and a gradient of one of them that passes through no recurrent core."""
+    loss, grads = _grads(model, ids, ids, create_graph=True)
+    names = [n for n, _ in model.named_parameters()]
+    k = names.index("norm.weight")
+    second = torch.autograd.grad(grads[k].square().sum(), [model.norm.weight])
+    return [g.detach() for g in grads], second[0]
+
+
+@pytest.mark.parametrize("share", ["nothing", "head and embedding", "one layer twice", "both gates"])
+def test_recorded_gradients_are_those_of_the_modules(share):
+    """create_graph=True on two layers: the nodes replay their operations, each parameter's uses counted once."""
+    model = _model()
+    if share == "head and embedding":
+        model.lm_head.weight = model.embed_tokens.weight
+    elif share == "one layer twice":
+        model.layers[1] = model.layers[0]
+    elif share == "both gates":
+        for layer in model.layers:
+            layer.recc.rg_lru_a_gate.w = layer.recc.rg_lru_input_gate.w
+    ids = torch.randint(0, 1000, (2, 40), generator=_gen(5), device=DEV)
+    _, unrecorded = _grads(model, ids, ids)
+    got, got_second = _embedding_penalty(model, ids)
+    hooks = _as_modules(model)
+    want, want_second = _embedding_penalty(model, ids)
+    for h in hooks:
+        h.remove()
+    for g, u, w, (name, _) in zip(got, unrecorded, want, model.named_parameters()):
+        assert float((g - w).norm()) <= 2e-2 * float(w.norm()), name
+        assert float((g - u).norm()) <= 2e-2 * float(u.norm()), name
+    assert float((got_second - want_second).norm()) <= 2e-2 * float(want_second.norm())

@@ -570,3 +570,46 @@ def test_training_nodes_take_only_hidden_states_their_kernels_can_read():
     assert not _node_input(torch.zeros(3, 2, 8).transpose(0, 1), shape, cpu)
     assert not _node_input(torch.zeros(49)[1:].view(shape), shape, cpu)          # not on a 16-byte boundary
     assert not _node_input(torch.nn.Parameter(good), shape, cpu)
+
+
+class _Product(torch.autograd.Function):
+    """tanh(x w^T) v^T with the same replay in a recorded backward as the training nodes have."""
+
+    @staticmethod
+    def plain(x, w, v):
+        return (torch.tanh(x @ w.t()) @ v.t(),)
+
+    @staticmethod
+    def forward(ctx, x, w, v):
+        ctx.save_for_backward(x, w, v)
+        return _Product.plain(x, w, v)[0]
+
+    @staticmethod
+    def backward(ctx, g):
+        from hawk_pytorch_amd import train_fused
+
+        if torch.is_grad_enabled():
+            return train_fused._replayed(_Product.plain, ctx.saved_tensors, (g,), ctx.needs_input_grad)
+        with torch.enable_grad():
+            leaves = [t.detach().requires_grad_() for t in ctx.saved_tensors]
+            return torch.autograd.grad(_Product.plain(*leaves)[0], leaves, g)
+
+
+@pytest.mark.parametrize("uses", ["one layer twice", "tied ends", "one weight in both places", "nothing shared"])
+def test_recorded_backward_counts_a_shared_parameter_once_per_use(uses):
+    """First and second derivatives of a recorded backward, against the same operations without nodes."""
+    gen = torch.Generator().manual_seed(3)
+    x0, w1, v1, w2, v2 = (torch.randn(4, 4, generator=gen, dtype=torch.float64) for _ in range(5))
+    params = [t.requires_grad_() for t in (w1, v1, w2, v2)]
+    a, b, c, d = {"one layer twice": (w1, v1, w1, v1), "tied ends": (w1, v1, w2, w1),
+                  "one weight in both places": (w1, w1, w2, w2), "nothing shared": (w1, v1, w2, v2)}[uses]
+
+    def derivatives(layer):
+        loss = layer(layer(x0, a, b), c, d).square().sum()
+        used = [p for p in params if any(p is t for t in (a, b, c, d))]
+        first = torch.autograd.grad(loss, used, create_graph=True)
+        second = torch.autograd.grad(sum(g.square().sum() for g in first), used)
+        return [*first, *second]
+
+    for got, want in zip(derivatives(_Product.apply), derivatives(lambda *t: _Product.plain(*t)[0])):
+        assert torch.allclose(got, want, rtol=1e-10, atol=1e-10)
