@@ -362,7 +362,9 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(
     const long long label = label_of(labels, row, T, V, counted);
     const bf16_t* p = logits + (size_t)row * V;
     bf16_t* o = dlogits + (size_t)row * V;
-    const float g = counted ? dloss[0] / mean[1] : 0.0f;
+    // a label outside the vocabulary has no loss (NaN, as the forward says) and so no gradient either
+    const bool known = label >= 0 && label < V;
+    const float g = !counted ? 0.0f : known ? dloss[0] / mean[1] : __builtin_nanf("");
     const float lse = lse_all[row];
     for (int c = 8 * (int)threadIdx.x; c < V; c += 8 * kCeThreads) {
         u32x4 r = {0u, 0u, 0u, 0u};

@@ -114,6 +114,23 @@ def test_cross_entropy_of_infinite_logits_and_uncounted_rows():
     assert bool(torch.isnan(train_fused.loss(hidden, None, 1e-6, norm, head, labels)))
 
 
+@pytest.mark.parametrize("label", [32, 33, -1, -99, 1 << 40])
+def test_labels_outside_the_vocabulary_give_no_loss_and_no_gradient(label):
+    """The gradients do not look healthy beside a loss that is NaN."""
+    gen = _gen(7)
+    V, H = 32, 8
+    hidden, head = _randn(gen, 2, 4, H).requires_grad_(), _randn(gen, V, H).requires_grad_()
+    labels = torch.randint(0, V, (2, 4), generator=gen, device=DEV)
+    labels[1, 2] = label
+    loss = train_fused.loss(hidden, None, 1e-6, torch.ones(H, device=DEV), head, labels)
+    d_hidden, d_head = torch.autograd.grad(loss, [hidden, head])
+    assert bool(torch.isnan(loss)) and bool(torch.isnan(d_head).all()) and bool(torch.isnan(d_hidden[1, 1]).all())
+    labels[1, 2] = -100                                  # a row that is left out gives none
+    loss = train_fused.loss(hidden, None, 1e-6, torch.ones(H, device=DEV), head, labels)
+    d_hidden, d_head = torch.autograd.grad(loss, [hidden, head])
+    assert bool(torch.isfinite(d_head).all()) and float(d_hidden[1, 1].abs().max()) == 0
+
+
 @pytest.mark.parametrize("rows,V,D", [(1, 5, 8), (130, 7, 264), (2048, 50, 512), (8192, 3, 1032)])
 def test_embedding_gradient(rows, V, D):
     gen = _gen(rows)
