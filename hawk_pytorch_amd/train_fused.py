@@ -115,6 +115,21 @@ def _replayed(fn, inputs, grads, needs):
     return tuple(next(found) if need else None for need in needs)
 
 
+class _Kept:
+    """Parameters that only a recorded backward needs again: a plain one reads the bf16 copies, as the separate
+    operations' does, so the parameters may change in place before it.  (Saved tensors would refuse that, and
+    hooks that pack saved tensors would be handed the weights twice.)"""
+
+    def __init__(self, *tensors: torch.Tensor):
+        self.tensors, self.versions = tensors, [t._version for t in tensors]
+
+    def unchanged(self):
+        if any(t._version != v for t, v in zip(self.tensors, self.versions)):
+            raise RuntimeError("a parameter was modified by an inplace operation after the forward pass: a backward "
+                               "pass with create_graph=True needs it as it was")
+        return self.tensors
+
+
 def _dense(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return _lib.dense16(t if t.dtype == dtype else t.to(dtype))
 
@@ -154,23 +169,21 @@ class _Layer(Function):
         out = torch.mm(act, w_dn16.t())
         if grad:
             ctx.eps = (eps1, eps2)
-            ctx.save_for_backward(hidden, delta, n1, n2, w_in, w_out, w_gu, w_dn, cw, cb, wi, bi, wa, ba, lam,
-                                  w_in16, w_out16, w_gu16, w_dn16, wi16, wa16, total1, x1, rstd1, xy, u, xg, ag, h,
-                                  gated, total2, x2, rstd2, gu, act)
+            ctx.kept = _Kept(w_in, w_out, w_gu, w_dn, cb, wi, bi, wa, ba)
+            ctx.save_for_backward(hidden, delta, n1, n2, cw, lam, w_in16, w_out16, w_gu16, w_dn16, wi16, wa16, total1,
+                                  x1, rstd1, xy, u, xg, ag, h, gated, total2, x2, rstd2, gu, act)
         return total2.view(B, T, H), out.view(B, T, H)
 
     @staticmethod
     def backward(ctx, d_total, d_out):  # type: ignore[override]
-        saved = ctx.saved_tensors
-        inputs = saved[:15]
+        (hidden, delta, n1, n2, cw, lam, w_in16, w_out16, w_gu16, w_dn16, wi16, wa16, total1, x1, rstd1, xy, u, xg, ag,
+         h, gated, total2, x2, rstd2, gu, act) = ctx.saved_tensors
         if torch.is_grad_enabled():
+            w_in, w_out, w_gu, w_dn, cb, wi, bi, wa, ba = ctx.kept.unchanged()
+            inputs = (hidden, delta, n1, n2, w_in, w_out, w_gu, w_dn, cw, cb, wi, bi, wa, ba, lam)
             grads = _replayed(lambda *a: _Layer.plain(*ctx.eps, *a), inputs, (d_total, d_out),
                               ctx.needs_input_grad[3:])
             return (None, None, None) + grads
-        hidden, delta, n1, n2 = inputs[:4]
-        cw, wi, bi, lam = inputs[8], inputs[10], inputs[11], inputs[14]
-        (w_in16, w_out16, w_gu16, w_dn16, wi16, wa16, total1, x1, rstd1, xy, u, xg, ag, h, gated, total2, x2, rstd2,
-         gu, act) = saved[15:]
         B, T, H = hidden.shape
         rows, inter = act.shape
         R = gated.shape[-1]
@@ -195,8 +208,9 @@ class _Layer(Function):
         d_hidden, d_delta, d_n1 = _add_norm_backward(d_x1, total1, rstd1, n1, d_total, delta is not None)
         d_in_w, d_out_w, d_gu_w, d_dn = _all_fp32([d_in_w, d_out_w, d_gu_w, d_dn])
         shape = (B, T, H)
+        blocks = wi16.shape[:2]
         grads = (d_hidden.view(shape), None if d_delta is None else d_delta.view(shape), d_n1, d_n2, d_in_w, d_out_w,
-                 d_gu_w, d_dn, dcw, dcb, dwi, dbi.view(bi.shape), dwa, dba.view(bi.shape), dlam)
+                 d_gu_w, d_dn, dcw, dcb, dwi, dbi.view(blocks), dwa, dba.view(blocks), dlam)
         return (None, None, None) + tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad[3:]))
 
 
@@ -224,18 +238,22 @@ class _Loss(Function):
                    mean.data_ptr(), B, T, V, _lib.stream_ptr(dev))
         if any(ctx.needs_input_grad):
             ctx.eps = eps
-            ctx.save_for_backward(labels, hidden, delta, norm, head, head16, total, x, rstd, logits, lse, mean)
+            ctx.kept = _Kept(head)
+            # (the labels of several sequences, cut by a position each, were a copy; they may be changed as well)
+            ctx.save_for_backward(labels if B == 1 else labels.clone(), hidden, delta, norm, head16, total, x, rstd,
+                                  logits, lse, mean)
         return mean[0].clone()
 
     @staticmethod
     def backward(ctx, d_loss):  # type: ignore[override]
-        labels, hidden, delta, norm, head, head16, total, x, rstd, logits, lse, mean = ctx.saved_tensors
+        labels, hidden, delta, norm, head16, total, x, rstd, logits, lse, mean = ctx.saved_tensors
         if torch.is_grad_enabled():
+            head, = ctx.kept.unchanged()
             grads = _replayed(lambda *a: _Loss.plain(ctx.eps, labels, *a), (hidden, delta, norm, head), (d_loss,),
                               ctx.needs_input_grad[2:])
             return (None, None) + grads
         B, T, H = hidden.shape
-        V, dev = head.shape[0], hidden.device
+        V, dev = head16.shape[0], hidden.device
         d_loss = d_loss.to(_F32)
         d_logits = torch.empty_like(logits)
         with _lib.on_device(dev):

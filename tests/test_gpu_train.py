@@ -329,3 +329,37 @@ def test_recorded_gradients_are_those_of_the_modules(share):
         assert float((g - w).norm()) <= 2e-2 * float(w.norm()), name
         assert float((g - u).norm()) <= 2e-2 * float(u.norm()), name
     assert float((got_second - want_second).norm()) <= 2e-2 * float(want_second.norm())
+
+
+@pytest.mark.parametrize("name", ["lm_head.weight", "layers.0.recc.input_xy.weight", "layers.1.recc.resid_proj.weight",
+                                  "layers.0.mlp.gate_up_proj.weight", "layers.1.mlp.resid_proj.weight",
+                                  "layers.0.recc.conv1d.b", "layers.1.recc.rg_lru_a_gate.b", "labels"])
+def test_what_may_change_between_forward_and_backward(name):
+    """The separate operations keep bf16 copies of these (nothing of the biases): the backward does not see a
+    change.  A recorded one would, and says so."""
+    model = _model()
+    ids = torch.randint(0, 1000, (2, 40), generator=_gen(8), device=DEV)
+    labels = ids.clone()
+    _, want = _grads(model, ids, labels)
+
+    def changed(**kw):
+        model.zero_grad(set_to_none=True)
+        with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+            loss = model(ids, labels)
+        t = labels if name == "labels" else model.get_parameter(name).detach()
+        before = t.clone()
+        t.copy_(t.roll(1, 0) if name == "labels" else t * 2 + 1)
+        try:
+            return torch.autograd.grad(loss, list(model.parameters()), **kw)
+        finally:
+            t.copy_(before)
+
+    assert all(torch.equal(g, w) for g, w in zip(changed(), want))
+    hooks = _as_modules(model)
+    through_modules = changed()
+    for h in hooks:
+        h.remove()
+    assert all(float((g - w).norm()) <= 2e-2 * float(w.norm()) for g, w in zip(through_modules, want))
+    if name != "labels":
+        with pytest.raises(RuntimeError, match="inplace"):
+            changed(create_graph=True)
