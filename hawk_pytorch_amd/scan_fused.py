@@ -389,12 +389,13 @@ class GatedDiagonalRecurrence(Function):
     autograd mirrors).  Dtype rules are DiagonalRecurrence's; y and out have h's dtype.
     The state sequence h is written only when a gradient will be asked for (``recorded``: whether
     gradients are enabled at the call; inside a Function's forward they never are, and its
-    ``needs_input_grad`` speaks of the inputs alone); h_last (what the decode cache keeps,
+    ``needs_input_grad`` speaks of the inputs alone; a caller that leaves it out gets h written
+    wherever an input requires a gradient); h_last (what the decode cache keeps,
     hawk/hawk.py:190) is not differentiable.
     """
 
     @staticmethod
-    def forward(ctx, x, x_rg_lru, a_rg_lru, a_param, y, want_last, recorded):
+    def forward(ctx, x, x_rg_lru, a_rg_lru, a_param, y, want_last, recorded=True):
         in_dtype = _common_input_dtype(x, x_rg_lru, a_rg_lru)
         xc, xgc, agc = (t if t.dtype == in_dtype else t.to(in_dtype) for t in (x, x_rg_lru, a_rg_lru))
         autocast = torch.is_autocast_enabled("cuda")
@@ -448,7 +449,7 @@ def fused_linear_scan_gated(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state
 # ---------------------------------------------------------------------------------------
 class RecurrentCore(Function):
     @staticmethod
-    def forward(ctx, u, w_i, b_i, w_a, b_a, a_param, y, want_last, recorded):
+    def forward(ctx, u, w_i, b_i, w_a, b_a, a_param, y, want_last, recorded=True):
         from .external import gate_proj_fwd, kernel_weights  # deferred: external imports nothing from here
 
         assert u.dtype == torch.bfloat16, "the fused core runs on bf16 activations"
@@ -650,7 +651,7 @@ def _block_core(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h: bool, w
 
 class BlockCore(Function):
     @staticmethod
-    def forward(ctx, xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_last, recorded):
+    def forward(ctx, xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_last, recorded=True):
         ctx.dtypes = tuple(t.dtype for t in (conv_w, conv_b, w_i, b_i, w_a, b_a, a_param))
         want_h = recorded and any(ctx.needs_input_grad[:8])
         out, h_last, saved = _block_core(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, a_param, want_h, bool(want_last))

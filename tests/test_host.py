@@ -613,3 +613,35 @@ def test_recorded_backward_counts_a_shared_parameter_once_per_use(uses):
 
     for got, want in zip(derivatives(_Product.apply), derivatives(lambda *t: _Product.plain(*t)[0])):
         assert torch.allclose(got, want, rtol=1e-10, atol=1e-10)
+
+
+@pytest.mark.parametrize("recorded", [(), (True,)], ids=["left out", "given"])
+def test_autograd_nodes_take_the_arguments_they_always_took(recorded, monkeypatch):
+    """GatedDiagonalRecurrence.apply and the two cores' without the trailing ``recorded``: the same results
+    and gradients, with the kernels replaced by shapes."""
+    from hawk_pytorch_amd import external, scan_fused
+
+    B, T, D, bf = 2, 5, 64, torch.bfloat16
+
+    def scan(x, *rest):
+        return x * 2, x * 3, x[:, -1:] * 3
+
+    monkeypatch.setattr(scan_fused, "_scan_gated_fwd", lambda x, xg, ag, lam, y, bf16, want_h, want_last: scan(x))
+    monkeypatch.setattr(scan_fused, "_scan_gated_bwd", lambda x, xg, ag, lam, y, h, go: (go, go, go, lam, go))
+    monkeypatch.setattr(external, "gate_proj_fwd", lambda u, *rest: (u, u))
+    monkeypatch.setattr(external, "gate_proj_bwd", lambda u, dxg, dag, w_i, w_a, add: (add, w_i, w_i[..., 0], w_a, w_a[..., 0]))
+    monkeypatch.setattr(scan_fused, "block_core_layout_ok", lambda xy: True)
+    monkeypatch.setattr(scan_fused, "block_core_forward", lambda xy, *rest: (
+        xy[..., :D] * 2, *(xy[..., :D] * 1 for _ in range(4)), xy[:, -1:, :D] * 1))
+    monkeypatch.setattr(scan_fused, "block_core_backward", lambda xy, u, xg, ag, h, cw, w_i, w_a, lam, go: (
+        xy, cw, lam, w_i, w_i[..., 0], w_a, w_a[..., 0], lam))
+    x, w, b = (torch.ones(s, dtype=bf).requires_grad_() for s in ((B, T, D), (1, D, D), (1, D)))
+    xy, cw, lam = (torch.ones(s, dtype=d).requires_grad_() for s, d in (((B, T, 2 * D), bf), ((4, D), torch.float32),
+                                                                        ((D,), torch.float32)))
+    for node, args in ((hk.GatedDiagonalRecurrence, (x, x, x, lam, x, True)),
+                       (scan_fused.RecurrentCore, (x, w, b, w, b, lam, x, True)),
+                       (scan_fused.BlockCore, (xy, cw, lam, w, b, w, b, lam, True))):
+        out, last = node.apply(*args, *recorded)
+        assert out.shape == (B, T, D) and last.shape == (B, 1, D) and out.requires_grad and not last.requires_grad
+        grads = torch.autograd.grad(out.sum(), [a for a in dict.fromkeys(args) if isinstance(a, torch.Tensor)])
+        assert all(g is not None for g in grads)
