@@ -645,3 +645,18 @@ def test_autograd_nodes_take_the_arguments_they_always_took(recorded, monkeypatc
         assert out.shape == (B, T, D) and last.shape == (B, 1, D) and out.requires_grad and not last.requires_grad
         grads = torch.autograd.grad(out.sum(), [a for a in dict.fromkeys(args) if isinstance(a, torch.Tensor)])
         assert all(g is not None for g in grads)
+
+
+def test_weight_gradient_offsets_fit_32_bits():
+    """A step reads 64 rows whatever their number; the byte offset of row 63 has to fit 32 bits for the range
+    check to see that it lies past the end."""
+    lib = _lib.load()
+    wide = 1 << 25
+    for n in (wide, wide + 8, 1 << 26):
+        assert not lib.hawk_weight_grad_supported(1, n, 8) and not lib.hawk_weight_grad_supported(1, 8, n)
+        assert lib.hawk_weight_grad_workspace_bytes(1, n, 8) == 0
+        assert lib.hawk_weight_grad(16, 16, 16, 1, n, 8, None, 0, None) == _lib.HAWK_ERR_BAD_SHAPE
+    assert lib.hawk_weight_grad_supported(1, wide - 8, 8) and lib.hawk_weight_grad_supported(1, 8, wide - 8)
+    for rows, n in ((1, wide - 8), (31, wide - 8), (32, wide - 8), (64, (1 << 24) - 8), (65, (1 << 24) - 8), (1 << 26, 8)):
+        if lib.hawk_weight_grad_supported(rows, n, 8):
+            assert ((rows + 63) // 64 * 64 - 1) * 2 * n + 256 < 1 << 32
