@@ -14,6 +14,7 @@ import os
 import threading
 
 import torch
+from torch.utils._device import DeviceContext
 
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 # HAWK_HIP_LIB selects another build of the library (e.g. one compiled with other tile shapes)
@@ -217,10 +218,17 @@ def stream_ptr(dev: torch.device) -> int:
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
+def _function_mode_active() -> bool:
+    """Whether a function mode is on that could see these calls.  A DeviceContext (``torch.set_default_device``,
+    ``with torch.device(...)``) only fills in the device of factory calls that name none, and here all name it."""
+    return any(type(torch._C._get_function_stack_at(k)) is not DeviceContext
+               for k in range(torch._C._len_torch_function_stack()))
+
+
 def transforms_active() -> bool:
     """Whether anything watches or rewrites operator calls: dispatch and function modes, functorch's
     transforms (vmap, grad, jvp), forward-mode differentiation."""
-    return (torch._C._len_torch_dispatch_stack() != 0 or torch._C._len_torch_function_stack() != 0
+    return (torch._C._len_torch_dispatch_stack() != 0 or _function_mode_active()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0)
 

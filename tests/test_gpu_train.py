@@ -363,3 +363,23 @@ def test_what_may_change_between_forward_and_backward(name):
     if name != "labels":
         with pytest.raises(RuntimeError, match="inplace"):
             changed(create_graph=True)
+
+
+@pytest.mark.parametrize("how", ["default device", "context"])
+def test_a_default_device_leaves_the_nodes_on(how, monkeypatch):
+    model = _model()
+    ids = torch.randint(0, 1000, (1, 40), generator=_gen(9), device=DEV)
+    want_loss, want = _grads(model, ids, ids)
+    nodes, real = [], train_fused.layer
+    monkeypatch.setattr(train_fused, "layer", lambda *a: (nodes.append(1), real(*a))[1])
+    if how == "context":
+        with torch.device("cuda"):
+            loss, grads = _grads(model, ids, ids)
+    else:
+        torch.set_default_device("cuda")
+        try:
+            loss, grads = _grads(model, ids, ids)
+        finally:
+            torch.set_default_device(None)
+    assert len(nodes) == 2 and torch.equal(loss, want_loss)
+    assert all(torch.equal(g, w) for g, w in zip(grads, want))

@@ -660,3 +660,53 @@ def test_weight_gradient_offsets_fit_32_bits():
     for rows, n in ((1, wide - 8), (31, wide - 8), (32, wide - 8), (64, (1 << 24) - 8), (65, (1 << 24) - 8), (1 << 26, 8)):
         if lib.hawk_weight_grad_supported(rows, n, 8):
             assert ((rows + 63) // 64 * 64 - 1) * 2 * n + 256 < 1 << 32
+
+
+def test_a_default_device_does_not_count_as_watching():
+    """Modes that see or rewrite operator calls send them through the torch.library ops; a default device
+    does neither, whichever way it is set, and hides no mode that does."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Watching(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatching(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert not _lib.transforms_active()
+    with torch.device("cpu"):
+        assert not _lib.transforms_active()
+        with torch.device("meta"):
+            assert not _lib.transforms_active()
+        with Watching():
+            assert _lib.transforms_active()
+            with torch.device("cpu"):
+                assert _lib.transforms_active()
+        with Dispatching():
+            assert _lib.transforms_active()
+    torch.set_default_device("cpu")
+    try:
+        assert not _lib.transforms_active()
+        with Watching():
+            assert _lib.transforms_active()
+    finally:
+        torch.set_default_device(None)
+    with Watching():
+        assert _lib.transforms_active()
+
+
+def test_every_allocation_names_its_device():
+    """What the rule above rests on: no factory call of the package leaves its device to a default (the
+    constructors of modules do, on purpose)."""
+    import ast
+
+    package = os.path.join(ROOT, "hawk_pytorch_amd")
+    for name in ("_lib.py", "external.py", "scan_fused.py", "train_fused.py", "hawk.py", "cache.py"):
+        calls = [n for n in ast.walk(ast.parse(open(os.path.join(package, name)).read())) if isinstance(n, ast.Call)]
+        parameters = {id(a) for c in calls if ast.unparse(c.func) == "nn.Parameter" for a in c.args}
+        for c in calls:
+            if re.fullmatch(r"torch\.(empty|zeros|ones|full|tensor|arange)", ast.unparse(c.func)) and id(c) not in parameters:
+                assert any(k.arg in ("device", None) for k in c.keywords), (name, c.lineno)   # (None: **kwargs)
