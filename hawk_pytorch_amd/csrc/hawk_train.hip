@@ -380,61 +380,93 @@ __global__ __launch_bounds__(kCeThreads) void cross_entropy_bwd_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Embedding gradient: dweight (zeroed by the caller) [V, D], row id = sum of dout's rows whose token is
-// id, in their order.  The workgroup of a token's first occurrence lists all of them (one wave, 64
-// positions per ballot) and adds the rows; the eight waves take an eighth of the list each, so that
-// one frequent token (padding) is not one wave's work.  Looking through all positions costs
-// every workgroup rows / 64 ballots, which is why the number of rows is limited.  2048 tokens of 512
-// channels: 23 us (the library's kernel 126).
+// Embedding gradient: dweight (zeroed by the caller) [V, D], row id = sum of dout's rows whose token is id.
+// One workgroup per position looks through all of them, an eighth per wave and 64 per ballot, and so knows
+// every position of its token and which of them it is itself.  The workgroups of a token's n positions take
+// its columns in turns, 256 at a time, so that the rows of a frequent token (padding) pass through as many
+// compute units as there are columns for: one takes in about 45 bytes per ns.  Of a list of up to eight
+// rows a wave adds all; of a longer one each wave adds an eighth, eight rows in flight, and the waves' sums
+// are added in order (a sum's order depends on the positions alone).  Looking through the positions is rows^2
+// in all and what it costs where tokens repeat little; with the zeros before it, random tokens of 32000 /
+// one token throughout, against the library's gradient: 2048 rows of 512 take 22 / 33 us (136 / 208), of 4096
+// 102 / 117 (254 / 295); 8192 rows of 512 94 / 102 (100 / 297), of 4096 205 / 237 (402 / 461).  Beyond 8192
+// rows the library is as fast.
 // ---------------------------------------------------------------------------------------
-constexpr int kEmbedWaves = 8;
+constexpr int kEmbedWaves = 8, kEmbedCols = 4 * kWave, kEmbedInFlight = 8;
 
 __global__ __launch_bounds__(kEmbedWaves* kWave) void embedding_bwd_kernel(const long long* __restrict__ ids,
                                                                            const float* __restrict__ dout,
                                                                            float* __restrict__ dweight, int rows,
                                                                            int V, int D) {
-    __shared__ uint16_t s_list[kEmbeddingMaxRows];
-    __shared__ int s_count;
-    __shared__ float s_sum[kEmbedWaves][8 * kWave];
+    __shared__ uint16_t s_list[kEmbeddingMaxRows];        // wave w's hits from position w * share on
+    __shared__ int s_count[kEmbedWaves], s_front[kEmbedWaves];
+    __shared__ __align__(16) float s_sum[kEmbedWaves][kEmbedCols];
     const int self = (int)blockIdx.x;
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const long long id = ids[self];
     if (id < 0 || id >= V) return;     // (uniform)
-    if (wv == 0) {
+    const int share = ((rows + kEmbedWaves - 1) / kEmbedWaves + kWave - 1) / kWave * kWave;
+    {
         int count = 0;
-        bool first = true;
-        for (int j0 = 0; j0 < rows && first; j0 += kWave) {
+        int in_front = 0;                     // of the token's positions, those in front of this workgroup's
+        const int end = min((wv + 1) * share, rows);
+#pragma unroll 4
+        for (int j0 = wv * share; j0 < end; j0 += kWave) {
             const int j = j0 + lane;
-            const unsigned long long hits = __ballot(j < rows && ids[j < rows ? j : 0] == id);
-            if (hits != 0ull && count == 0) first = j0 + __builtin_ctzll(hits) == self;
-            if (!first) break;
+            const unsigned long long hits = __ballot(j < end && ids[j < end ? j : 0] == id);
+            const int ahead = self - j0;
+            in_front += __builtin_popcountll(ahead >= kWave ? hits : ahead <= 0 ? 0ull : hits & ((1ull << ahead) - 1ull));
             const int before = __builtin_popcountll(hits & ((1ull << lane) - 1ull));
-            if ((hits >> lane) & 1ull) s_list[count + before] = (uint16_t)j;
+            if ((hits >> lane) & 1ull) s_list[wv * share + count + before] = (uint16_t)j;
             count += __builtin_popcountll(hits);
         }
-        if (lane == 0) s_count = first ? count : 0;
+        if (lane == 0) { s_count[wv] = count; s_front[wv] = in_front; }
     }
     __syncthreads();
-    const int count = s_count;
-    if (count == 0) return;            // (uniform)
-    const int from = count * wv / kEmbedWaves, to = count * (wv + 1) / kEmbedWaves;
-    for (int c0 = 0; c0 < D; c0 += 8 * kWave) {
-        const int c = c0 + 8 * lane;
-        float sum[8];
+    int total = 0, rank = 0;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) sum[k] = 0.0f;
-        if (c < D) {
-            for (int n = from; n < to; ++n) {
-                float v[8];
-                load8(dout + (size_t)s_list[n] * D + c, v);
+    for (int k = 0; k < kEmbedWaves; ++k) { total += s_count[k]; rank += s_front[k]; }
+    const int chunks = (D + kEmbedCols - 1) / kEmbedCols;
+    // the sum of the list's entries [from, to) at columns c..c+3
+    auto add_rows = [&](int from, int to, int c) {
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        int base = 0;              // entries of the waves in front
+        for (int k = 0; k < kEmbedWaves; ++k) {
+            const int at = k * share - base, hi = min(to, base + s_count[k]);
+            int n = max(from, base);
+            for (; n + kEmbedInFlight <= hi; n += kEmbedInFlight) {
+                f32x4 v[kEmbedInFlight];
 #pragma unroll
-                for (int k = 0; k < 8; ++k) sum[k] += v[k];
+                for (int q = 0; q < kEmbedInFlight; ++q)
+                    v[q] = *reinterpret_cast<const f32x4*>(dout + (size_t)s_list[at + n + q] * D + c);
+#pragma unroll
+                for (int q = 0; q < kEmbedInFlight; ++q) sum += v[q];
             }
+            for (; n < hi; ++n) sum += *reinterpret_cast<const f32x4*>(dout + (size_t)s_list[at + n] * D + c);
+            base += s_count[k];
         }
-        store8(&s_sum[wv][8 * lane], sum);
+        return sum;
+    };
+    if (total <= kEmbedWaves) {        // (uniform)
+        for (long long k = wv; rank + k * total < chunks; k += kEmbedWaves) {
+            const int c = (int)(rank + k * total) * kEmbedCols + 4 * lane;
+            if (c >= D) continue;
+            const f32x4 sum = add_rows(0, total, c);
+            float* o = dweight + (size_t)id * D + c;     // (on any 4-byte boundary)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) o[q] = sum[q];
+        }
+        return;
+    }
+    const int from = total * wv / kEmbedWaves, to = total * (wv + 1) / kEmbedWaves;
+    for (int chunk = rank; chunk < chunks; chunk += total) {
+        const int c0 = chunk * kEmbedCols, c = c0 + 4 * lane;
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (c < D) sum = add_rows(from, to, c);
+        *reinterpret_cast<f32x4*>(&s_sum[wv][4 * lane]) = sum;
         __syncthreads();
-        const int oc = threadIdx.x;    // 8 * kWave columns, one per thread
-        if (c0 + oc < D) {
+        const int oc = threadIdx.x;    // a column per thread of the first four waves
+        if (oc < kEmbedCols && c0 + oc < D) {
             float v = 0.0f;
 #pragma unroll
             for (int k = 0; k < kEmbedWaves; ++k) v += s_sum[k][oc];

@@ -23,7 +23,9 @@ from .external import kernel_weights
 from .scan_fused import BlockCore, block_core_backward, block_core_forward
 
 _BF16, _F32 = torch.bfloat16, torch.float32
-EMBEDDING_MAX_ROWS = 8192   # hawk_embedding_bwd's limit; more tokens take the library's gradient
+# hawk_embedding_bwd's limit, and where the library's gradient, which sorts, has caught up: 94 against 100 us for
+# 8192 random tokens of 512 channels (39 against 77 for 4096)
+EMBEDDING_MAX_ROWS = 8192
 
 
 def _check(name: str, *args) -> None:
@@ -267,7 +269,7 @@ class _Loss(Function):
 
 
 class _Embedding(Function):
-    """weight[ids]; the gradient adds a token's rows in their order."""
+    """weight[ids]; the gradient adds a token's rows in an order that depends on its positions alone."""
 
     @staticmethod
     def forward(ctx, ids, weight):

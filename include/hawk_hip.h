@@ -329,8 +329,10 @@ int hawk_cross_entropy_fwd(const void* logits, const long long* labels, float* l
                            int B, int T, int V, void* stream);
 int hawk_cross_entropy_bwd(const void* logits, const long long* labels, const float* lse, const float* mean,
                            const float* dloss, void* dlogits, int B, int T, int V, void* stream);
-/* dweight [V, D] fp32, zeroed by the caller: row id += the rows of dout [rows, D] fp32 whose token is id,
- * in their order.  rows at most 8192, D a multiple of 8; tokens outside [0, V) add nothing. */
+/* dweight [V, D] fp32, zeroed by the caller: row id = the sum of the rows of dout [rows, D] fp32 whose token is
+ * id (written, not added to; rows of tokens that do not occur are left alone).  Up to 8 of them are added in
+ * their order; more in eight runs of consecutive ones, whose sums are then added in order.  rows at most 8192,
+ * D a multiple of 8; tokens outside [0, V) add nothing. */
 int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, int rows, int V, int D,
                        void* stream);
 

@@ -145,6 +145,33 @@ def test_embedding_gradient(rows, V, D):
     _close(got, want, rows * EPS32 * scale)
 
 
+# positions: ends of a ballot and of a wave's share, the most the kernel takes; columns: a lane, either side of a
+# workgroup's 256, more of them than waves or than a token's workgroups
+@pytest.mark.parametrize("rows,D", [(63, 248), (64, 256), (65, 264), (511, 8), (513, 520), (4097, 264), (8191, 256),
+                                    (100, 16648)])
+@pytest.mark.parametrize("ids", ["distinct", "equal", "padded", "few", "outside"])
+def test_embedding_gradient_over_the_ways_tokens_repeat(rows, D, ids):
+    from hawk_pytorch_amd import _lib
+
+    gen = _gen(rows + D)
+    V = rows
+    t = dict(distinct=torch.randperm(V, generator=gen, device=DEV), equal=torch.full((rows,), V - 1, device=DEV),
+             padded=torch.randperm(V, generator=gen, device=DEV), few=torch.randint(0, 9, (rows,), generator=gen, device=DEV),
+             outside=torch.randint(-2, V + 2, (rows,), generator=gen, device=DEV))[ids]
+    if ids == "padded":
+        t[rows // 3:] = 0
+    d = _randn(gen, rows, D)
+    guard = 1024
+    whole = torch.zeros(1 + V * D + guard, device=DEV)
+    got = whole[1:1 + V * D].view(V, D)      # (no more than a 4-byte boundary is asked of it)
+    train_fused._check("hawk_embedding_bwd", t.data_ptr(), d.data_ptr(), got.data_ptr(), rows, V, D, _lib.stream_ptr(DEV))
+    known = (t >= 0) & (t < V)
+    want = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, t[known], d[known].double())
+    scale = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, t[known], d[known].double().abs())
+    _close(got, want, rows * EPS32 * scale)
+    assert float(whole[1 + V * D:].abs().max()) == 0 and float(whole[0]) == 0
+
+
 def _model(vocab=1000, D=256, inter=520, layers=2, nb=4, **kw):
     torch.manual_seed(6)
     model = hk.HawkModel(hk.HawkConfig(vocab_size=vocab, hidden_size=D, intermediate_size=inter, num_hidden_layers=layers,
