@@ -498,10 +498,13 @@ struct Cut {
     int mt, nt, depth, splits;
 };
 // Workgroups a product that is split over K is cut into: one per compute unit.  Measured on a layer
-// of 2560 x 7680 (four products, two norms): 240 gives 49 / 53 / 63 / 82 / 104 us at 1 / 32 / 64 / 128 /
-// 256 rows, 320 gives 52 / 59 / 71 / 95 / 121 (the partial sums of more splits cost more than the
-// second workgroup on a compute unit brings), 160 gives 49 / 55 / 67 / 84 / 114.
-constexpr int kSplitWorkgroups = 240;
+// of 2560 x 7680 (four products, two norms): 240 to 266 (the same cuts there) give 49 / 53 / 63 / 82 / 104 us
+// at 1 / 32 / 64 / 128 / 256 rows, 320 gives 52 / 59 / 71 / 95 / 121 (the partial sums of more splits cost more
+// than the second workgroup on a compute unit brings), 160 gives 49 / 55 / 67 / 84 / 114.  With 240 the 128
+// tiles of 4096 columns at 129 rows and more, and of 8192 at 33 to 128, were not split and left half of the
+// chip idle: steps of two and four such layers took 999 and 1094 us at 64 and 256 rows, in two splits 887 and
+// 908.  From 129 tiles on one split stays: 160 tiles over K = 2560 in two take 2 % more of a layer's time.
+constexpr int kSplitWorkgroups = 256;
 // Tiles of 128 x 128 from this many of them on; with fewer, part of the chip would be idle.
 constexpr int kMinWideTiles = 200;
 

@@ -50,7 +50,9 @@ def test_linear_matches_64_bit_sums(M, N, K):
 
 @pytest.mark.parametrize("M,H,R,inter,n_next", [(1, 128, 128, 128, 8), (3, 512, 256, 640, 1032), (33, 256, 512, 768, 512),
                                                 (64, 384, 640, 1152, 64), (130, 1024, 1024, 3072, 2048),
-                                                (256, 2560, 2560, 7680, 5120), (5, 8192, 128, 256, 72)])
+                                                (256, 2560, 2560, 7680, 5120), (5, 8192, 128, 256, 72),
+                                                # 128 tiles, two splits of each
+                                                (200, 4096, 512, 640, 72), (64, 8192, 512, 1024, 72)])
 def test_layer_tail_matches_the_separate_operations(M, H, R, inter, n_next):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(H + M)

@@ -710,3 +710,12 @@ def test_every_allocation_names_its_device():
         for c in calls:
             if re.fullmatch(r"torch\.(empty|zeros|ones|full|tensor|arange)", ast.unparse(c.func)) and id(c) not in parameters:
                 assert any(k.arg in ("device", None) for k in c.keywords), (name, c.lineno)   # (None: **kwargs)
+
+
+@pytest.mark.parametrize("M,N,splits", [(256, 2560, 3), (1, 2560, 6), (129, 4096, 2), (256, 4096, 2), (64, 8192, 2),
+                                        (128, 8192, 2), (256, 4160, 1), (256, 8192, 1), (1, 512, 8)])
+def test_decode_products_are_split_over_the_compute_units(M, N, splits):
+    """Tiles of 64 columns (and 32, 64 or 128 rows) in as many splits as give one workgroup per compute unit:
+    128 tiles are split in two rather than left on half of the chip."""
+    need = _lib.load().hawk_decode_linear_workspace_bytes(M, N, 8192)
+    assert need == (splits * M * N * 4 if splits > 1 else 0)
