@@ -347,8 +347,21 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
 # The dense part of a decode step: the layers' projections, norms, residual adds and gated GELU for
 # up to 256 rows (hawk/hawk.py:53-58, :70-86, :163-166, :198-203, :222-243, :284-303 upstream).
 # ---------------------------------------------------------------------------------------
+# Layers wider than DECODE_LAYERS_MAX_WIDTH go through the modules for more than DECODE_LAYERS_NARROW_ROWS rows.
+# A second row tile of 128, mostly padding at first, then comes with products of more than 128 tiles, which are not
+# split over K and leave compute units with one workgroup beside others with two.  Steps of 3 layers (MLP three
+# times as wide) at 129 / 144 / 240 / 256 rows, kernels against modules in us: width 4608 922 / 924 / 1031 / 1057
+# against 743 / 770 / 941 / 1139, 5120 1022 / 1028 / 1161 / 1197 against 826 / 946 / 1059 / 1279; at 128 rows 625
+# against 786 and 707 against 890.  At width 4096 the kernels are ahead at every number of rows (4 layers, 129
+# rows: 827 against 848).
+DECODE_LAYERS_NARROW_ROWS = 128
+DECODE_LAYERS_MAX_WIDTH = 4096
+
+
 def decode_layers_supported(M: int, H: int, R: int, inter: int, vocab: int) -> bool:
     lib = _lib.load()
+    if M > DECODE_LAYERS_NARROW_ROWS and H > DECODE_LAYERS_MAX_WIDTH:
+        return False
     return bool(lib.hawk_decode_layer_supported(M, H, R, inter) and lib.hawk_decode_linear_supported(M, 2 * R, H)
                 and lib.hawk_decode_linear_supported(M, vocab, H))
 

@@ -356,7 +356,8 @@ class HawkModel(nn.Module):
     def _decode_step(self, input_ids, layer_past) -> Optional[torch.Tensor]:
         """Logits of one token per sequence on warm caches through the decode kernels, or None where
         they do not apply (nothing has been touched then): bf16 weights in the modules that the
-        constructor made, up to 256 rows, no gradients, nothing that records or rewrites operator calls."""
+        constructor made, up to 256 rows (128 of wide layers), no gradients, nothing that records or
+        rewrites operator calls."""
         cfg = self.config
         if (torch.is_grad_enabled() or not isinstance(input_ids, torch.Tensor) or input_ids.ndim != 2
                 or input_ids.shape[1] != 1 or not input_ids.is_cuda or not (cfg.fused_gates and cfg.fused_epilogue)

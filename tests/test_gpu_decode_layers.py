@@ -155,3 +155,16 @@ def test_model_step_falls_back_where_the_kernels_do_not_apply(monkeypatch):
     biased.lm_head = torch.nn.Linear(256, 520, bias=True).cuda().bfloat16()
     step(biased)
     step(_model().float())
+
+
+def test_wide_layers_of_many_rows_step_through_the_modules(monkeypatch):
+    starts, real = [], external.DecodeLayers.__init__
+    monkeypatch.setattr(external.DecodeLayers, "__init__", lambda self, *a: (starts.append(1), real(self, *a))[1])
+    model = _model(hidden_size=4224, intermediate_size=256, num_hidden_layers=1)
+    for B, kernels in ((128, 1), (129, 0)):
+        starts.clear()
+        ids = torch.randint(1, 520, (B, 3), device="cuda")
+        with torch.no_grad():
+            _, caches = model(ids[:, :2], layer_past=model.new_cache(B))
+            assert model(ids[:, 2:], layer_past=caches)[0].shape == (B, 1, 520)
+        assert len(starts) == kernels

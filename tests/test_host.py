@@ -719,3 +719,11 @@ def test_decode_products_are_split_over_the_compute_units(M, N, splits):
     128 tiles are split in two rather than left on half of the chip."""
     need = _lib.load().hawk_decode_linear_workspace_bytes(M, N, 8192)
     assert need == (splits * M * N * 4 if splits > 1 else 0)
+
+
+@pytest.mark.parametrize("M,H,served", [(128, 4608, True), (129, 4608, False), (256, 4608, False), (256, 4096, True),
+                                        (129, 8192, False), (1, 8192, True), (257, 2560, False), (1, 8320, False)])
+def test_wide_layers_of_many_rows_decode_through_the_modules(M, H, served):
+    from hawk_pytorch_amd import external
+
+    assert external.decode_layers_supported(M, H, H, 2 * H, 32000) is served
