@@ -256,6 +256,13 @@ def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.devi
     return _dense_param(module, "weight", shape, dtype, dev)
 
 
+def _norm_weight(module: Optional[nn.Module], H: int, dev: torch.device,
+                 dtype: torch.dtype = torch.bfloat16) -> Optional[torch.Tensor]:
+    """The weight of a plain norm whose epsilon is a number (the library's norm also takes None)."""
+    w = _dense_weight(module, RMSNorm, (H,), dev, dtype)
+    return w if w is not None and type(module.eps) in (int, float) else None
+
+
 def _node_input(hidden: torch.Tensor, shape, dev: torch.device) -> bool:
     """Whether a training node can read a hidden state that a module returned: the kernels take its
     pointer, and the labels are read by its rows, so nothing about it can be taken for granted."""
@@ -287,7 +294,7 @@ class RNNLayer(nn.Module):
         recc, mlp, n1, n2 = m.get("recc"), m.get("mlp"), m.get("input_norm"), m.get("post_recurrent_norm")
         if not (_plain(self, RNNLayer) and _plain(recc, Hawk) and _plain(mlp, MLP) and recc.use_cache):
             return None
-        ws = (_dense_weight(n1, RMSNorm, (H,), dev), _dense_weight(n2, RMSNorm, (H,), dev),
+        ws = (_norm_weight(n1, H, dev), _norm_weight(n2, H, dev),
               _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev),
               _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev),
               _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev),
@@ -309,7 +316,7 @@ class RNNLayer(nn.Module):
             return None
         H, R, inter, nb = cfg.hidden_size, cfg.recurrent_size, cfg.intermediate_size, cfg.num_blocks
         f32, bw = torch.float32, R // nb
-        ws = (_dense_weight(n1, RMSNorm, (H,), dev, f32), _dense_weight(n2, RMSNorm, (H,), dev, f32),
+        ws = (_norm_weight(n1, H, dev, f32), _norm_weight(n2, H, dev, f32),
               _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev, f32),
               _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev, f32),
               _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev, f32),
@@ -371,7 +378,7 @@ class HawkModel(nn.Module):
         if M < 1 or not decode_layers_supported(M, H, R, inter, cfg.vocab_size):
             return None
         embed = self.embed_tokens.weight
-        norm = _dense_weight(self.norm, RMSNorm, (H,), dev)
+        norm = _norm_weight(self.norm, H, dev)
         head = _dense_weight(self.lm_head, nn.Linear, (cfg.vocab_size, H), dev)
         weights = [layer.decode_weights(H, R, inter, dev) if type(layer) is RNNLayer else None
                    for layer in self.layers]
@@ -406,8 +413,7 @@ class HawkModel(nn.Module):
         H, V, dev, f32 = cfg.hidden_size, cfg.vocab_size, input_ids.device, torch.float32
         rows, emb = input_ids.numel(), self.embed_tokens
         grad = torch.is_grad_enabled()
-        norm, head = _dense_weight(self.norm, RMSNorm, (H,), dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H),
-                                                                                     dev, f32)
+        norm, head = _norm_weight(self.norm, H, dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H), dev, f32)
         if (H % 8 != 0 or H > 4096 or V % 8 != 0 or norm is None or head is None or rows * V >= 1 << 40
                 or (grad and not (norm.requires_grad and head.requires_grad))):
             return None

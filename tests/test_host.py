@@ -727,3 +727,26 @@ def test_wide_layers_of_many_rows_decode_through_the_modules(M, H, served):
     from hawk_pytorch_amd import external
 
     assert external.decode_layers_supported(M, H, H, 2 * H, 32000) is served
+
+
+def _layer_on_cpu():
+    """(layer, what the decode kernels are given of it, what the training nodes are) on the CPU."""
+    from hawk_pytorch_amd.hawk import RNNLayer
+
+    cfg = hk.HawkConfig(vocab_size=64, hidden_size=64, intermediate_size=96, num_hidden_layers=1, recurrent_size=64,
+                        num_blocks=1)
+    cpu = torch.device("cpu")
+    server, trained = RNNLayer(cfg, use_cache=True).bfloat16(), RNNLayer(cfg)
+    return ((server, lambda: server.decode_weights(64, 64, 96, cpu)), (trained, lambda: trained.train_weights(cfg, cpu)))
+
+
+@pytest.mark.parametrize("eps", [None, torch.tensor(1e-6)], ids=["None", "a tensor"])
+def test_norms_whose_epsilon_is_no_number_stay_modules(eps):
+    for layer, weights in _layer_on_cpu():
+        for norm in (layer.input_norm, layer.post_recurrent_norm):
+            assert weights() is not None
+            before, norm.eps = norm.eps, eps
+            assert weights() is None
+            norm.eps = before
+        layer.input_norm.eps = 1      # a number, if an odd one
+        assert weights() is not None
