@@ -17,6 +17,8 @@ inline hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
 constexpr int kMaxGridY = 65535;
 constexpr long long kMaxTiles = 0x7fffffffLL;
+// rows of a launch of one 512-thread workgroup each: HIP counts a grid's threads in 32 bits
+constexpr long long kMaxWorkgroups512 = (1LL << 23) - 1;
 constexpr long long kMaxRowStride = 1LL << 24;  // elements; keeps 16 rows of any dtype within 32-bit byte offsets
 
 int check_scan_shape(int B, int T, int D) {
@@ -361,7 +363,8 @@ int hawk_gelu_mul_bwd(const void* gate_up, const void* dact, void* d_gate_up, in
 int hawk_cross_entropy_fwd(const void* logits, const long long* labels, float* lse, float* loss, float* mean, int B,
                            int T, int V, void* stream) {
     if (!logits || !labels || !lse || !loss || !mean) return HAWK_ERR_NULL_POINTER;
-    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxWorkgroups512)
+        return HAWK_ERR_BAD_SHAPE;
     if (!aligned16(logits)) return HAWK_ERR_ALIGNMENT;
     return hawk::cross_entropy_fwd(logits, labels, lse, loss, mean, B * T, T, V, as_stream(stream));
 }
@@ -369,7 +372,8 @@ int hawk_cross_entropy_fwd(const void* logits, const long long* labels, float* l
 int hawk_cross_entropy_bwd(const void* logits, const long long* labels, const float* lse, const float* mean,
                            const float* dloss, void* dlogits, int B, int T, int V, void* stream) {
     if (!logits || !labels || !lse || !mean || !dloss || !dlogits) return HAWK_ERR_NULL_POINTER;
-    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxTiles) return HAWK_ERR_BAD_SHAPE;
+    if (B < 1 || T < 1 || V < 8 || V % 8 != 0 || V > (1 << 30) || (long long)B * T > kMaxWorkgroups512)
+        return HAWK_ERR_BAD_SHAPE;
     if (!aligned16(logits) || !aligned16(dlogits)) return HAWK_ERR_ALIGNMENT;
     return hawk::cross_entropy_bwd(logits, labels, lse, mean, dloss, dlogits, B * T, T, V, as_stream(stream));
 }

@@ -419,6 +419,7 @@ class HawkModel(nn.Module):
         grad = torch.is_grad_enabled()
         norm, head = _norm_weight(self.norm, H, dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H), dev, f32)
         if (H % 8 != 0 or H > 4096 or V % 8 != 0 or norm is None or head is None or rows * V >= 1 << 40
+                or rows > train_fused.LOSS_MAX_ROWS
                 or (grad and not (norm.requires_grad and head.requires_grad))):
             return None
         table = _dense_param(emb, "weight", (V, H), f32, dev) if _plain(emb, nn.Embedding) else None

@@ -26,6 +26,7 @@ _BF16, _F32 = torch.bfloat16, torch.float32
 # hawk_embedding_bwd's limit, and where the library's gradient, which sorts, has caught up: 94 against 100 us for
 # 8192 random tokens of 512 channels (39 against 77 for 4096)
 EMBEDDING_MAX_ROWS = 8192
+LOSS_MAX_ROWS = (1 << 23) - 1   # hawk_cross_entropy_fwd's: a workgroup of 512 threads per row
 
 
 def _check(name: str, *args) -> None:

@@ -768,3 +768,17 @@ def test_a_forward_put_into_a_class_is_not_passed_by(monkeypatch):
     assert hawk._plain(embed, torch.nn.Embedding)
     monkeypatch.setattr(torch.nn.Embedding, "forward", lambda self, ids: None)
     assert not hawk._plain(embed, torch.nn.Embedding)
+
+
+def test_cross_entropy_rows_fit_a_grid():
+    """A grid's threads are counted in 32 bits, 512 of them per row; more rows are refused before a launch (and
+    the model takes such a loss through torch)."""
+    from hawk_pytorch_amd import train_fused
+
+    lib, most = _lib.load(), train_fused.LOSS_MAX_ROWS
+    assert most * 512 < 1 << 32 <= (most + 1) * 512
+    # with pointers off a 16-byte boundary, which are looked at after the shape
+    for B, T, want in ((1, most, _lib.HAWK_ERR_ALIGNMENT), (1, most + 1, _lib.HAWK_ERR_BAD_SHAPE),
+                       (1 << 12, 1 << 12, _lib.HAWK_ERR_BAD_SHAPE), (most, 1, _lib.HAWK_ERR_ALIGNMENT)):
+        assert lib.hawk_cross_entropy_fwd(8, 8, 8, 8, 8, B, T, 8, None) == want
+        assert lib.hawk_cross_entropy_bwd(8, 8, 8, 8, 8, 8, B, T, 8, None) == want
