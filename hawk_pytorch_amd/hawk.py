@@ -418,8 +418,7 @@ class HawkModel(nn.Module):
         rows, emb = input_ids.numel(), self.embed_tokens
         grad = torch.is_grad_enabled()
         norm, head = _norm_weight(self.norm, H, dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H), dev, f32)
-        if (H % 8 != 0 or H > 4096 or V % 8 != 0 or norm is None or head is None or rows * V >= 1 << 40
-                or rows > train_fused.LOSS_MAX_ROWS
+        if (norm is None or head is None or not train_fused.loss_supported(rows, H, V)
                 or (grad and not (norm.requires_grad and head.requires_grad))):
             return None
         table = _dense_param(emb, "weight", (V, H), f32, dev) if _plain(emb, nn.Embedding) else None
@@ -428,10 +427,9 @@ class HawkModel(nn.Module):
             hidden = train_fused.embedding(input_ids, table)
         else:
             hidden = emb(input_ids)
-        kernels = (cfg.fused_gates and cfg.fused_epilogue and cfg.fused_block_core and cfg.intermediate_size % 8 == 0
-                   and cfg.recurrent_size % cfg.num_blocks == 0 and 1 <= cfg.conv_width <= 8
-                   and cfg.recurrent_size // cfg.num_blocks in (32, 64, 128, 256)
-                   and rows * max(cfg.intermediate_size, cfg.recurrent_size) < 1 << 31)
+        kernels = (cfg.fused_gates and cfg.fused_epilogue and cfg.fused_block_core
+                   and train_fused.layer_supported(rows, H, cfg.recurrent_size, cfg.intermediate_size, cfg.num_blocks,
+                                                   cfg.conv_width))
         delta = None
         shape = (*input_ids.shape, H)
         for layer in self.layers:

@@ -292,6 +292,19 @@ class _Embedding(Function):
         return None, dweight
 
 
+def loss_supported(rows: int, H: int, V: int) -> bool:
+    """Whether the head's kernels serve these sizes: the norm's limits are the library's to say."""
+    return (V % 8 == 0 and rows <= LOSS_MAX_ROWS and rows * V < 1 << 40
+            and _lib.load().hawk_add_norm_bwd_workspace_bytes(rows, H) > 0)
+
+
+def layer_supported(rows: int, H: int, R: int, inter: int, num_blocks: int, conv_width: int) -> bool:
+    """The same for a layer's: its norms, its gated GELU and the recurrent core of R channels."""
+    lib = _lib.load()
+    return (inter % 8 == 0 and rows * max(inter, R) < 1 << 31 and lib.hawk_add_norm_bwd_workspace_bytes(rows, H) > 0
+            and bool(lib.hawk_decode_core_supported(R, num_blocks, conv_width)))
+
+
 def embedding(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return _Embedding.apply(ids, weight)
 

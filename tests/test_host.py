@@ -782,3 +782,17 @@ def test_cross_entropy_rows_fit_a_grid():
                        (1 << 12, 1 << 12, _lib.HAWK_ERR_BAD_SHAPE), (most, 1, _lib.HAWK_ERR_ALIGNMENT)):
         assert lib.hawk_cross_entropy_fwd(8, 8, 8, 8, 8, B, T, 8, None) == want
         assert lib.hawk_cross_entropy_bwd(8, 8, 8, 8, 8, 8, B, T, 8, None) == want
+
+
+def test_sizes_the_training_nodes_serve():
+    from hawk_pytorch_amd import train_fused
+
+    assert train_fused.loss_supported(1, 8, 8) and train_fused.loss_supported(5, 4096, 32000)
+    for rows, H, V in ((1, 12, 8), (1, 4104, 8), (1, 8, 12), (1 << 23, 8, 8), (1 << 22, 8, 1 << 18)):
+        assert not train_fused.loss_supported(rows, H, V)
+    assert train_fused.layer_supported(7, 512, 512, 1024, 16, 4)
+    for change in (dict(H=516), dict(H=4104), dict(inter=1020), dict(num_blocks=3), dict(num_blocks=32), dict(num_blocks=1),
+                   dict(conv_width=9), dict(conv_width=0), dict(rows=1 << 22)):
+        sizes = dict(rows=7, H=512, R=512, inter=1024, num_blocks=16, conv_width=4)
+        sizes.update(change)
+        assert not train_fused.layer_supported(**sizes), change
