@@ -562,17 +562,16 @@ bool decode_linear_supported(int M, int N, int K) {
 }
 bool decode_norm_supported(int D) { return D >= 8 && D % 8 == 0 && D <= 8 * kNormMaxThreads; }
 
-// The workspace of a layer: normed rows, the MLP's product, partial sums.
-size_t decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next) {
-    const size_t a = (size_t)cut_for(M, H, R, false, true).splits * H, b = (size_t)cut_for(M, H, I, false, true).splits * H;
-    const size_t c = (size_t)cut_for(M, n_next, H, false, true).splits * n_next;
-    const size_t most = a > b ? (a > c ? a : c) : (b > c ? b : c);
-    return align256((size_t)M * H * 2) + align256((size_t)M * I * 2) + align256(most * M * sizeof(float));
-}
-
 size_t decode_linear_workspace_bytes(int M, int N, int K) {
     const Cut c = cut_for(M, N, K, false, true);
     return c.splits > 1 ? (size_t)c.splits * M * N * sizeof(float) : 0;
+}
+
+// The workspace of a layer: normed rows, the MLP's product, partial sums.
+size_t decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next) {
+    const size_t a = (size_t)cut_for(M, H, R, false, true).splits * H, b = (size_t)cut_for(M, H, I, false, true).splits * H;
+    const size_t sums = (a > b ? a : b) * M * sizeof(float), next = decode_linear_workspace_bytes(M, n_next, H);
+    return align256((size_t)M * H * 2) + align256((size_t)M * I * 2) + align256(sums > next ? sums : next);
 }
 
 int decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* ws, hipStream_t st) {

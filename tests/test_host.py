@@ -796,3 +796,13 @@ def test_sizes_the_training_nodes_serve():
         sizes = dict(rows=7, H=512, R=512, inter=1024, num_blocks=16, conv_width=4)
         sizes.update(change)
         assert not train_fused.layer_supported(**sizes), change
+
+
+def test_decode_workspace_holds_no_sums_of_a_head_that_is_not_split():
+    lib = _lib.load()
+    small, large = (lib.hawk_decode_layer_workspace_bytes(256, 2560, 2560, 7680, n) for n in (8192, 256000))
+    assert lib.hawk_decode_linear_workspace_bytes(256, 256000, 2560) == 0 and large <= small
+    for M, H, R, inter, n in ((256, 2560, 2560, 7680, 256000), (1, 512, 512, 1024, 1024), (70, 512, 2560, 256, 2048)):
+        sums = max(lib.hawk_decode_linear_workspace_bytes(M, N, K) or M * N * 4 for N, K in ((H, R), (H, inter)))
+        need = M * (H + inter) * 2 + max(sums, lib.hawk_decode_linear_workspace_bytes(M, n, H))
+        assert need <= lib.hawk_decode_layer_workspace_bytes(M, H, R, inter, n) < need + 1024
