@@ -52,7 +52,10 @@ def test_linear_matches_64_bit_sums(M, N, K):
                                                 (64, 384, 640, 1152, 64), (130, 1024, 1024, 3072, 2048),
                                                 (256, 2560, 2560, 7680, 5120), (5, 8192, 128, 256, 72),
                                                 # 128 tiles, two splits of each
-                                                (200, 4096, 512, 640, 72), (64, 8192, 512, 1024, 72)])
+                                                (200, 4096, 512, 640, 72), (64, 8192, 512, 1024, 72),
+                                                # gated GELU in 128-wide tiles of ragged rows (its columns, a
+                                                # multiple of 128, are whole tiles), loads 4 and 2 steps ahead
+                                                (200, 256, 256, 13056, 64), (131, 384, 384, 12928, 72)])
 def test_layer_tail_matches_the_separate_operations(M, H, R, inter, n_next):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(H + M)
@@ -65,11 +68,19 @@ def test_layer_tail_matches_the_separate_operations(M, H, R, inter, n_next):
     want_h = want_h + _exact_linear(F.gelu(gate) * up, w_down)
     want = _exact_linear(F.rms_norm(want_h, (H,), n2, 1e-6), w_next)
     run = external.DecodeLayers(hidden, R, inter, n_next)
+    need, guard = run.ws.numel(), 4096
+    guarded = torch.full((need + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    run.ws = guarded[:need]
     got = run.tail(gated, w_out, n1, 1e-6, w_gu, w_down, n2, 1e-6, w_next)
     for a, b in ((hidden, want_h), (got, want)):
         # rounded at the same places: what is left are values that an fp32 sum in another order rounds to
         # the neighbouring bf16, at most four of them on the way, each off by 2^-8 of itself at most
-        assert float((a.double() - b.double()).norm() / b.double().norm()) < 2.0 ** -7
+        error, size = (a.double() - b.double()).abs(), b.double()
+        assert float(error.norm() / size.norm()) < 2.0 ** -7
+        # an element by itself: four such values of its own, or of the sums it is made of, whose size is the
+        # tensor's; one that a tile's edge lost or doubled is off by about that size
+        assert bool((error <= 2.0 ** -6 * (size.abs() + size.square().mean().sqrt())).all())
+    assert bool((guarded[need:] == 0xA5).all())
     again = external.DecodeLayers(hidden.clone(), R, inter, n_next).first(n2, 1e-6, w_next)
     assert torch.equal(again, got)     # the same norm and projection, on the hidden state as it was left
 
@@ -155,6 +166,8 @@ def test_model_step_falls_back_where_the_kernels_do_not_apply(monkeypatch):
     biased.lm_head = torch.nn.Linear(256, 520, bias=True).cuda().bfloat16()
     step(biased)
     step(_model().float())
+    with torch.autocast("cuda", torch.float16):
+        step(model)
 
 
 def test_wide_layers_of_many_rows_step_through_the_modules(monkeypatch):
