@@ -218,17 +218,18 @@ def stream_ptr(dev: torch.device) -> int:
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
-def _function_mode_active() -> bool:
-    """Whether a function mode is on that could see these calls.  A DeviceContext (``torch.set_default_device``,
-    ``with torch.device(...)``) only fills in the device of factory calls that name none, and here all name it."""
-    return any(type(torch._C._get_function_stack_at(k)) is not DeviceContext
-               for k in range(torch._C._len_torch_function_stack()))
+def _watching_function_modes(n: int) -> bool:
+    """Whether one of the n function modes that are on could see these calls.  A DeviceContext
+    (``torch.set_default_device``, ``with torch.device(...)``) only fills in the device of factory calls that
+    name none, and here all name it."""
+    return any(type(torch._C._get_function_stack_at(k)) is not DeviceContext for k in range(n))
 
 
 def transforms_active() -> bool:
     """Whether anything watches or rewrites operator calls: dispatch and function modes, functorch's
     transforms (vmap, grad, jvp), forward-mode differentiation."""
-    return (torch._C._len_torch_dispatch_stack() != 0 or _function_mode_active()
+    modes = torch._C._len_torch_function_stack()
+    return (torch._C._len_torch_dispatch_stack() != 0 or (modes != 0 and _watching_function_modes(modes))
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch.autograd.forward_ad._current_level >= 0)
 

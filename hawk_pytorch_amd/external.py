@@ -305,10 +305,14 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
         if index < 0 or t.get_device() != index:
             _lib.require_cuda(conv_state, x_new, conv_w, w_i, w_a, a_param, recc_state, y)   # says which
 
+    dense = (B, 1, D)
+
     def rows(t):
         """[B, D] rows with unit column stride and the distance between them, copying only if it must."""
-        if t.dtype == torch.bfloat16 and t.shape == (B, 1, D) and t.stride(2) == 1 and t.stride(0) >= D:
-            return t, (t.stride(0) if B > 1 else D)
+        if t.dtype == torch.bfloat16 and t.shape == dense:
+            ld, _, unit = t.stride()
+            if unit == 1 and ld >= D:
+                return t, (ld if B > 1 else D)
         # any other shape of B * D elements is folded into rows; one of more or fewer raises here
         t2 = t.reshape(B, D) if t.dtype == torch.bfloat16 else t.reshape(B, D).to(torch.bfloat16)
         if t2.stride(1) != 1 or (B > 1 and t2.stride(0) < D):
@@ -319,7 +323,9 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     if ldx % 8 != 0 or xn.data_ptr() % 16 != 0:
         xn, ldx = _lib.dense16(xn.contiguous()), D
     y2, ldy = rows(y)
-    b_i, b_a = (t if t.numel() == D else t.reshape(D) for t in (input_gate.b, a_gate.b))   # (raises for another size)
+    b_i, b_a = input_gate.b, a_gate.b
+    if b_i.numel() != D or b_a.numel() != D:
+        b_i, b_a = b_i.reshape(D), b_a.reshape(D)   # raises for the one of another size
     w32, b32, b_i, b_a, lam = (
         t if t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
         else _lib.dense16(t.detach().float()) for t in (conv_w, conv.b, b_i, b_a, a_param))

@@ -232,10 +232,10 @@ class Hawk(nn.Module):
 
 
 def _plain(module: Optional[nn.Module], cls: type) -> bool:
-    """Exactly this class, and a call of it runs the forward that the class was written with and nothing else."""
-    return (type(module) is cls and cls.forward is _FORWARDS[cls] and "forward" not in module.__dict__
-            and not module._forward_hooks and not module._forward_pre_hooks and not module._backward_hooks
-            and not module._backward_pre_hooks and module._compiled_call_impl is None)
+    """Exactly this class, and a call of it runs this class's forward and nothing else."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks
+            and module._compiled_call_impl is None)
 
 
 def _dense_param(module: Optional[nn.Module], name: str, shape, dtype: torch.dtype,
@@ -330,8 +330,16 @@ class RNNLayer(nn.Module):
         return n1.eps, n2.eps, ws
 
 
-# what _plain compares with: a program may also put another forward into a class
-_FORWARDS = {cls: cls.forward for cls in (RNNLayer, Hawk, MLP, RMSNorm, Conv1D, BlockDiagonalLinear, nn.Linear, nn.Embedding)}
+_FORWARDS = [(cls, cls.forward) for cls in (RNNLayer, Hawk, MLP, RMSNorm, Conv1D, BlockDiagonalLinear, nn.Linear,
+                                            nn.Embedding)]
+
+
+def _classes_as_written() -> bool:
+    """A program may also put another forward into a class: looked at once per pass, for all modules of it."""
+    for cls, forward in _FORWARDS:
+        if cls.forward is not forward:
+            return False
+    return True
 
 
 class HawkModel(nn.Module):
@@ -374,6 +382,7 @@ class HawkModel(nn.Module):
                 or input_ids.shape[1] != 1 or not input_ids.is_cuda or not (cfg.fused_gates and cfg.fused_epilogue)
                 or any(p is None or p.current_cache_size <= 0 for p in layer_past)
                 or not _lib.launches_directly(input_ids) or nn.modules.module._has_any_global_hook()
+                or not _classes_as_written()
                 or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16)
                 or not _plain(self.embed_tokens, nn.Embedding)):
             return None
@@ -412,7 +421,8 @@ class HawkModel(nn.Module):
                 or input_ids.dtype != torch.int64 or labels.dtype != torch.int64 or input_ids.numel() == 0
                 or not input_ids.is_contiguous() or not labels.is_contiguous()
                 or not torch.is_autocast_enabled("cuda") or torch.get_autocast_dtype("cuda") != torch.bfloat16
-                or not _lib.launches_directly(input_ids, labels) or nn.modules.module._has_any_global_hook()):
+                or not _lib.launches_directly(input_ids, labels) or nn.modules.module._has_any_global_hook()
+                or not _classes_as_written()):
             return None
         H, V, dev, f32 = cfg.hidden_size, cfg.vocab_size, input_ids.device, torch.float32
         rows, emb = input_ids.numel(), self.embed_tokens

@@ -410,3 +410,13 @@ def test_a_default_device_leaves_the_nodes_on(how, monkeypatch):
             torch.set_default_device(None)
     assert len(nodes) == 2 and torch.equal(loss, want_loss)
     assert all(torch.equal(g, w) for g, w in zip(grads, want))
+
+
+@pytest.mark.parametrize("cls", [hk.MLP, hk.RMSNorm, torch.nn.Linear])
+def test_a_forward_put_into_a_class_runs(cls, monkeypatch):
+    model = _model()
+    ids = torch.randint(0, 1000, (1, 40), generator=_gen(2), device=DEV)
+    calls, real = [], cls.forward
+    monkeypatch.setattr(cls, "forward", lambda self, x: (calls.append(1), real(self, x))[1])
+    _grads(model, ids, ids)
+    assert len(calls) == {hk.MLP: 2, hk.RMSNorm: 5, torch.nn.Linear: 9}[cls]
