@@ -516,6 +516,8 @@ Cut cut_for(int M, int N, int K, bool gelu, bool may_split) {
     c.splits = 1;
     const int mtiles = ceil_div(M, c.mt), cols = gelu ? 2 * N : N;
     if (c.mt == 128) {
+        // (split products keep 64 columns: of 128-wide ones 256 x 5120 x 2560 in three splits was measured, 19.1 us
+        // and 5.0 for the sums against 24, and no other)
         if (!may_split && ceil_div(cols, 128) * mtiles >= kMinWideTiles) c.nt = 128;
         else c.depth = 2;
     }

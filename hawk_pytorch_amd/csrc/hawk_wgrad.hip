@@ -9,8 +9,10 @@
 // (1024 x 512: 32 of them), so the rows are split over workgroups, and a second kernel adds the fp32 partial
 // results in a fixed order.  What that spares next to the library's product is the conversion to fp32, and the
 // chip is not left idle by few tiles: 2048 rows, 512 x 512 13.9 us (library and conversion 17.8), 4593
-// rows, 2048 x 1024 43.3 (50.0), 1024 x 1024 27.8 (38.5).  From 128 tiles on the library is as fast or faster
-// (8192 rows, 2560 x 2560: 148 against 123); callers go there.
+// rows, 2048 x 1024 43.3 (50.0), 1024 x 1024 27.8 (38.5).  Between 512 and 4096 rows, where a few steps are split
+// and the sums cost a launch, results of more than 32 tiles take up to a fifth longer than the library's (1024
+// rows, 2048 x 1024: 21.2 against 17.4).  From 128 tiles on the library is as fast or faster (8192 rows, 2560 x
+// 2560: 148 against 123); callers go there.
 #include "hawk_scan.h"
 
 #include <stdint.h>

@@ -321,7 +321,7 @@ int hawk_add_norm_bwd(const void* dout, const float* sum, const float* rstd, con
  * a multiple of 8. */
 int hawk_gelu_mul_fwd(const void* gate_up, void* act, int rows, int I, void* stream);
 int hawk_gelu_mul_bwd(const void* gate_up, const void* dact, void* d_gate_up, int rows, int I, void* stream);
-/* Mean next-token cross entropy of bf16 logits [B * T, V] (V a multiple of 8): row (b, t) against
+/* Mean next-token cross entropy of bf16 logits [B * T, V] (V a multiple of 8, B * T < 2^23): row (b, t) against
  * labels[b, t + 1] (int64, [B, T]); the last row of a sequence and rows with label -100 do not count; a
  * label outside [0, V) makes the loss and its row of the gradient NaN.  lse, loss: [B * T] fp32 scratch
  * (lse is read by the backward); mean: [2] fp32, the mean loss and the number of counted rows. */
