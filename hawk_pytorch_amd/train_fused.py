@@ -235,7 +235,7 @@ class _Loss(Function):
         return (F.cross_entropy(logits.reshape(-1, logits.shape[-1]).float(), labels[:, 1:].reshape(-1)),)
 
     @staticmethod
-    def forward(ctx, eps, labels, hidden, delta, norm, head):
+    def forward(ctx, recorded, eps, labels, hidden, delta, norm, head):
         B, T, H = hidden.shape
         rows, V, dev = B * T, head.shape[0], hidden.device
         head16, = _cast([head], _BF16)
@@ -247,7 +247,7 @@ class _Loss(Function):
         with _lib.on_device(dev):
             _check("hawk_cross_entropy_fwd", logits.data_ptr(), labels.data_ptr(), lse.data_ptr(), each.data_ptr(),
                    mean.data_ptr(), B, T, V, _lib.stream_ptr(dev))
-        if any(ctx.needs_input_grad):
+        if recorded and any(ctx.needs_input_grad):
             ctx.eps = eps
             ctx.kept = _Kept(head)
             # (the labels of several sequences, cut by a position each, were a copy; they may be changed as well)
@@ -261,8 +261,8 @@ class _Loss(Function):
         if torch.is_grad_enabled():
             head, = ctx.kept.unchanged()
             grads = _replayed(lambda *a: _Loss.plain(ctx.eps, labels, *a), (hidden, delta, norm, head), (d_loss,),
-                              ctx.needs_input_grad[2:])
-            return (None, None) + grads
+                              ctx.needs_input_grad[3:])
+            return (None, None, None) + grads
         B, T, H = hidden.shape
         V, dev = head16.shape[0], hidden.device
         d_loss = d_loss.to(_F32)
@@ -274,7 +274,7 @@ class _Loss(Function):
         d_head, = _cast([torch.mm(d_logits.t(), x)], _F32)
         d_hidden, d_delta, d_norm = _add_norm_backward(d_x, total, rstd, norm, None, delta is not None)
         grads = (d_hidden.view(hidden.shape), None if d_delta is None else d_delta.view(hidden.shape), d_norm, d_head)
-        return (None, None) + tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad[2:]))
+        return (None, None, None) + tuple(g if need else None for g, need in zip(grads, ctx.needs_input_grad[3:]))
 
 
 class _Embedding(Function):
@@ -322,4 +322,4 @@ def layer(hidden, delta: Optional[torch.Tensor], eps1: float, eps2: float, param
 
 
 def loss(hidden, delta, eps: float, norm, head, labels) -> torch.Tensor:
-    return _Loss.apply(eps, labels, hidden, delta, norm, head)
+    return _Loss.apply(torch.is_grad_enabled(), eps, labels, hidden, delta, norm, head)

@@ -337,8 +337,8 @@ int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, 
                        void* stream);
 
 /* dw [N, K] fp32 = dy^T x for dy [rows, N] and x [rows, K] bf16: the weight gradient of a linear layer, summed
- * in fp32 in a fixed order.  Dense and 16-byte aligned, N and K multiples of 8, rows * N and rows * K below
- * 2^30.  The workspace (NULL where the query says 0) takes partial results. */
+ * in fp32 in a fixed order.  Dense and 16-byte aligned, N and K multiples of 8 below 2^25, rows * N and
+ * rows * K below 2^30.  The workspace (NULL where the query says 0) takes partial results. */
 int hawk_weight_grad_supported(int rows, int N, int K);
 size_t hawk_weight_grad_workspace_bytes(int rows, int N, int K);
 int hawk_weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K,

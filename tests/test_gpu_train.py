@@ -420,3 +420,16 @@ def test_a_forward_put_into_a_class_runs(cls, monkeypatch):
     monkeypatch.setattr(cls, "forward", lambda self, x: (calls.append(1), real(self, x))[1])
     _grads(model, ids, ids)
     assert len(calls) == {hk.MLP: 2, hk.RMSNorm: 5, torch.nn.Linear: 9}[cls]
+
+
+@pytest.mark.parametrize("made", ["outside", "inside"])
+def test_loss_in_inference_mode(made):
+    """An evaluation under inference_mode, with parameters made in front of it or in it (those have no version)."""
+    model = _model()
+    ids = torch.randint(0, 1000, (2, 40), generator=_gen(3), device=DEV)
+    want, _ = _grads(model, ids, ids)
+    with torch.inference_mode():
+        if made == "inside":
+            model = _model()
+        with torch.autocast(device_type="cuda", dtype=torch.bfloat16):
+            assert torch.equal(model(ids, ids), want)
