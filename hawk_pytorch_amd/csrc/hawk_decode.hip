@@ -24,13 +24,10 @@
 
 #include <stdint.h>
 
-#include "hawk_device.h"
+#include "hawk_tile.h"
 
 namespace hawk {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * kWave;
@@ -40,18 +37,11 @@ constexpr int kRowBytes = kKT * 2;
 
 enum Epilogue { kStoreBf16 = 0, kStorePartial = 1, kStoreGelu = 2 };
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 // 16-byte piece `c` of row `r` of a staged tile.  The pieces of a row are permuted by the row's
 // number, so that the 8 rows one LDS cycle reads the same piece of cover all banks.
 __device__ __forceinline__ int piece_offset(int r, int c) { return r * kRowBytes + ((c ^ (r & 7)) << 4); }
-
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
 
 // One thread's share of a finished row: 8 adjacent columns a, c, or 4 gate columns a and the up
 // columns c beside them.

@@ -17,13 +17,10 @@
 
 #include <stdint.h>
 
-#include "hawk_device.h"
+#include "hawk_tile.h"
 
 namespace hawk {
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 4 * kWave;
 constexpr int kTile = 128, kKT = 64;
@@ -31,18 +28,11 @@ constexpr int kRowBytes = kKT * 2;
 constexpr int kOperand = kTile * kRowBytes;      // bytes of one operand's tile
 constexpr int kMaxSplits = 8;
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // 16-byte piece c (8 values along the sum) of row r.  The permutation differs between the 8 rows that one
 // LDS cycle reads and between rows 8 apart, which a transposed operand's lanes write together.
 __device__ __forceinline__ int piece_offset(int r, int c) {
     return r * kRowBytes + ((c ^ ((r ^ (r >> 3)) & 7)) << 4);
-}
-
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
 }
 
 // out [M, N] (or [splits, M, N]) = a^T b for a [K, M] and b [K, N].
