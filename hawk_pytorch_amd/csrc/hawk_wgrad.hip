@@ -201,7 +201,8 @@ bool weight_grad_supported(int rows, int N, int K) {
     // byte offsets within an operand stay below 2^31, and those of the rows that fill the last step (range
     // checked, so never read) below 2^32: past that they would come out as other rows'
     return rows >= 1 && N >= 8 && N % 8 == 0 && K >= 8 && K % 8 == 0 && N < (1 << 25) && K < (1 << 25) &&
-           (long long)rows * N < (1ll << 30) && (long long)rows * K < (1ll << 30) && (long long)ceil_div(N, kTile) * ceil_div(K, kTile) < (1 << 20);
+           (long long)rows * N < (1ll << 30) && (long long)rows * K < (1ll << 30) &&
+           (long long)ceil_div(N, kTile) * ceil_div(K, kTile) < (1 << 20);
 }
 size_t weight_grad_workspace_bytes(int rows, int N, int K) {
     const int s = splits_for(N, K, rows);
