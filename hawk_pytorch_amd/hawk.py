@@ -256,11 +256,7 @@ def _dense_weight(module: Optional[nn.Module], cls: type, shape, dev: torch.devi
     return _dense_param(module, "weight", shape, dtype, dev)
 
 
-def _norm_weight(module: Optional[nn.Module], H: int, dev: torch.device,
-                 dtype: torch.dtype = torch.bfloat16) -> Optional[torch.Tensor]:
-    """The weight of a plain norm whose epsilon is a number (the library's norm also takes None)."""
-    w = _dense_weight(module, RMSNorm, (H,), dev, dtype)
-    return w if w is not None and type(module.eps) in (int, float) else None
+_NUMBERS = (int, float)   # of a norm's epsilon; the library's norm takes None as well, and then it runs
 
 
 def _node_input(hidden: torch.Tensor, shape, dev: torch.device) -> bool:
@@ -294,12 +290,12 @@ class RNNLayer(nn.Module):
         recc, mlp, n1, n2 = m.get("recc"), m.get("mlp"), m.get("input_norm"), m.get("post_recurrent_norm")
         if not (_plain(self, RNNLayer) and _plain(recc, Hawk) and _plain(mlp, MLP) and recc.use_cache):
             return None
-        ws = (_norm_weight(n1, H, dev), _norm_weight(n2, H, dev),
+        ws = (_dense_weight(n1, RMSNorm, (H,), dev), _dense_weight(n2, RMSNorm, (H,), dev),
               _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev),
               _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev),
               _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev),
               _dense_weight(mlp._modules.get("resid_proj"), nn.Linear, (H, inter), dev))
-        if any(w is None for w in ws):
+        if any(w is None for w in ws) or type(n1.eps) not in _NUMBERS or type(n2.eps) not in _NUMBERS:
             return None
         return ws[0], n1.eps, ws[2], ws[3], ws[1], n2.eps, ws[4], ws[5]
 
@@ -316,7 +312,7 @@ class RNNLayer(nn.Module):
             return None
         H, R, inter, nb = cfg.hidden_size, cfg.recurrent_size, cfg.intermediate_size, cfg.num_blocks
         f32, bw = torch.float32, R // nb
-        ws = (_norm_weight(n1, H, dev, f32), _norm_weight(n2, H, dev, f32),
+        ws = (_dense_weight(n1, RMSNorm, (H,), dev, f32), _dense_weight(n2, RMSNorm, (H,), dev, f32),
               _dense_weight(recc._modules.get("input_xy"), nn.Linear, (2 * R, H), dev, f32),
               _dense_weight(recc._modules.get("resid_proj"), nn.Linear, (H, R), dev, f32),
               _dense_weight(mlp._modules.get("gate_up_proj"), nn.Linear, (2 * inter, H), dev, f32),
@@ -325,7 +321,7 @@ class RNNLayer(nn.Module):
               _dense_param(gi, "w", (nb, bw, bw), f32, dev), _dense_param(gi, "b", (nb, bw), f32, dev),
               _dense_param(ga, "w", (nb, bw, bw), f32, dev), _dense_param(ga, "b", (nb, bw), f32, dev),
               _dense_param(recc, "rg_lru_a_param", (R,), f32, dev))
-        if any(w is None for w in ws):
+        if any(w is None for w in ws) or type(n1.eps) not in _NUMBERS or type(n2.eps) not in _NUMBERS:
             return None
         return n1.eps, n2.eps, ws
 
@@ -391,11 +387,12 @@ class HawkModel(nn.Module):
         if M < 1 or not decode_layers_supported(M, H, R, inter, cfg.vocab_size):
             return None
         embed = self.embed_tokens.weight
-        norm = _norm_weight(self.norm, H, dev)
+        norm = _dense_weight(self.norm, RMSNorm, (H,), dev)
         head = _dense_weight(self.lm_head, nn.Linear, (cfg.vocab_size, H), dev)
         weights = [layer.decode_weights(H, R, inter, dev) if type(layer) is RNNLayer else None
                    for layer in self.layers]
-        if (norm is None or head is None or not weights or any(w is None for w in weights)
+        if (norm is None or type(self.norm.eps) not in _NUMBERS or head is None or not weights
+                or any(w is None for w in weights)
                 or embed.dtype != torch.bfloat16 or embed.device != dev or embed.shape[1] != H):
             return None
 
@@ -427,8 +424,10 @@ class HawkModel(nn.Module):
         H, V, dev, f32 = cfg.hidden_size, cfg.vocab_size, input_ids.device, torch.float32
         rows, emb = input_ids.numel(), self.embed_tokens
         grad = torch.is_grad_enabled()
-        norm, head = _norm_weight(self.norm, H, dev, f32), _dense_weight(self.lm_head, nn.Linear, (V, H), dev, f32)
-        if (norm is None or head is None or not train_fused.loss_supported(rows, H, V)
+        norm = _dense_weight(self.norm, RMSNorm, (H,), dev, f32)
+        head = _dense_weight(self.lm_head, nn.Linear, (V, H), dev, f32)
+        if (norm is None or head is None or type(self.norm.eps) not in _NUMBERS
+                or not train_fused.loss_supported(rows, H, V)
                 or (grad and not (norm.requires_grad and head.requires_grad))):
             return None
         table = _dense_param(emb, "weight", (V, H), f32, dev) if _plain(emb, nn.Embedding) else None

@@ -84,10 +84,10 @@ def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     ahead up to 512 rows and from 4096 on, and behind between them where the result has more than 32 tiles
     (2048 x 1024: 512 rows 12.2 against 14.7 us, 1024 rows 21.2 against 17.4, 2048 rows 27.3 against 24.2, 4096
     rows 39.7 against 39.7; two columns of 64 tiles, 8192 x 256, are behind at most sizes: 20.0 against 16.6 at 512
-    rows, 90.7 against 96.2 at 8192, 325 against 243 at 32768).  But its call costs the host less, and such passes wait for the host: with the
-    library's products throughout, passes of 4 layers of 256 to 1280 channels take 0.4 to 18 % longer at 128 to
-    8192 tokens (1024 channels: 3190 against 3061 us at 1024 tokens, 3235 against 3221 at 2048; of 45 sizes one
-    was 1.5 % shorter, 1280 channels at 128 tokens, where both routes vary by more)."""
+    rows, 90.7 against 96.2 at 8192, 325 against 243 at 32768).  But its call costs the host less, and such passes
+    wait for the host: with the library's products throughout, passes of 4 layers of 256 to 1280 channels take 0.4
+    to 18 % longer at 128 to 8192 tokens (1024 channels: 3190 against 3061 us at 1024 tokens, 3235 against 3221 at
+    2048; of 45 sizes one was 1.5 % shorter, 1280 channels at 128 tokens, where both routes vary by more)."""
     n, N = dy.shape
     K = x.shape[1]
     lib = _lib.load()

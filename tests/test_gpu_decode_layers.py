@@ -181,3 +181,15 @@ def test_wide_layers_of_many_rows_step_through_the_modules(monkeypatch):
             _, caches = model(ids[:, :2], layer_past=model.new_cache(B))
             assert model(ids[:, 2:], layer_past=caches)[0].shape == (B, 1, 520)
         assert len(starts) == kernels
+
+
+def test_model_step_with_a_norm_without_epsilon():
+    """eps=None is the library norm's own default; such a model steps through the modules."""
+    model = _model()
+    ids = torch.randint(1, 520, (2, 3), device="cuda")
+    for norm in (model.norm, model.layers[1].input_norm):
+        before, norm.eps = norm.eps, None
+        with torch.no_grad():
+            _, caches = model(ids[:, :2], layer_past=model.new_cache(2))
+            assert bool(torch.isfinite(model(ids[:, 2:], layer_past=caches)[0]).all())
+        norm.eps = before
