@@ -16,8 +16,8 @@
 //   * projections with few columns also split K over workgroups and leave fp32 partial sums, which
 //     the kernel that follows (residual add + norm) adds up in a fixed order on its way.
 // A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 49 / 53 / 63 /
-// 82 / 104 us at 1 / 32 / 64 / 128 / 256 rows with cold weights (157 MB); the library's four products alone
-// took 121 us at 256 rows, with the norms, additions, GELU and product around them 149.
+// 79 / 86 / 101 us at 1 / 32 / 64 / 128 / 129 / 256 rows with cold weights (157 MB); the library's four products
+// alone took 121 us at 256 rows, with the norms, additions, GELU and product around them 149.
 // All sums are fp32, in an order that depends on the shape alone, and values are rounded to bf16 where
 // the separate operations round them, so both routes differ by the order of the sums only.
 #include "hawk_scan.h"
@@ -216,33 +216,51 @@ __global__ __launch_bounds__(kThreads, 3) void decode_gemm_kernel(
     }
 }
 
-// The same products for more than 64 rows, in tiles of 128 rows x NT columns.  Here the bytes that
-// pass from the L2s into the compute units set the pace, not HBM: one compute unit takes in about
-// 23 bytes per clock (counters: 77 cache lines in flight at 430 clocks each, the L1 stalled on
-// pending misses for half of the time, LDS and matrix cores below 40 %), so the tile is as square as
-// the number of workgroups allows: 256 rows x 15360 columns x 2560 take 43 us in tiles of 128 x 64, 39 in
-// tiles of 256 x 64 and 36.5 in tiles of 128 x 128.  (Eight waves instead of four and loads four
-// steps ahead instead of two changed nothing; neither did starting at different places of K.)  The waves split the tile 2 x 2; what that reads from LDS more than
-// once stays below what arrives from the L1.
-template <int NT>
+// The same products for more than 64 rows, in tiles of 128 rows x NT columns.  What sets the pace is how much a
+// compute unit can have in flight: loads return in order and no more than about 32 KB of them are outstanding (more
+// in the queue changes nothing: a stream from HBM into one compute unit of 64 stays at 47 bytes per ns, from L2 at
+// 123), and since a quarter to a half of a tile's bytes are weights that HBM takes 0.7 us to deliver, all of them
+// arrive at that pace.  So the tile is as square as the number of workgroups allows, and tiles go from memory into
+// LDS without passing through registers, a few steps ahead, one barrier a step.  Eight waves split the tile
+// (2 x 4, or 4 x 2 of 64 columns); each sums all of a workgroup's K in order.  256 x 15360 x 2560 takes 34.7 us (36.6 through registers with four
+// waves; 35 without any products, 24 with the weights alone), 256 x 5120 x 2560 17.7 (20.4), 129 x 15360 x 2560 29.3
+// (32.7), 65 x 32000 x 512 10.0 (12.2); where each workgroup starts along K makes no difference.
+//
+// STAGES tiles of a step are held: four where no compute unit has a second workgroup; where there are more workgroups
+// than compute units two share one, and the tiles held are what both have room for, three of 64 columns or two of
+// 128 (256 x 32000 x 512 in us: 17.6 with four, 15.7 with two; with no second workgroup, 256 x 15360 x 2560, 35.5
+// with four, 35.7 with three, 45.5 with two).
+template <int NT, int STAGES>
 struct WideLds {
+    static constexpr int kGroups = (128 + NT) / 8;             // wave loads of 8 rows x 128 bytes per step
     static constexpr int kStage = (128 + NT) * kRowBytes;
-    static constexpr int kBytes = 2 * kStage > 128 * NT * 4 ? 2 * kStage : 128 * NT * 4;
+    static constexpr int kSums = 128 * NT * 4;                 // the tile on its way out
+    static constexpr int kBytes = STAGES * kStage > kSums ? STAGES * kStage : kSums;
 };
+constexpr int kWideWaves = 8;
+constexpr int kWideThreads = kWideWaves * kWave;
 
-template <int NT, int DEPTH, int EPI>
-__global__ __launch_bounds__(kThreads, NT >= 128 ? 1 : 2) void decode_gemm_wide_kernel(
+// Until at most N of this wave's loads are in flight (they arrive in order).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+template <int NT, int STAGES, int EPI>
+__global__ __launch_bounds__(kWideThreads, STAGES == 4 ? 2 : 4) void decode_gemm_wide_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
     int ntiles, int mtiles, int splits) {
     constexpr int MT = 128;
-    constexpr int XP = MT / 32, WP = NT / 32, NB = NT / 64;
+    constexpr int WN = NT / 32, WM = kWideWaves / WN, MB = MT / WM / 32;    // waves side by side, and blocks of 32 rows of one
     constexpr int NC = EPI == kStoreGelu ? NT / 2 : NT;       // output columns of a tile
-    __shared__ __align__(16) unsigned char smem[WideLds<NT>::kBytes];
+    using Lds = WideLds<NT, STAGES>;
+    constexpr int S = STAGES, L = Lds::kGroups / kWideWaves;
+    __shared__ __align__(16) unsigned char smem[Lds::kBytes];
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int wm = wv & 1, wn = wv >> 1;
+    const int wm = wv % WM, wn = wv / WM;
 
     // row tiles of one weight tile 8 workgroups apart, as above
     const int b = (int)blockIdx.x;
@@ -253,110 +271,107 @@ __global__ __launch_bounds__(kThreads, NT >= 128 ? 1 : 2) void decode_gemm_wide_
     const int nt = item - split * ntiles;
     const int m0 = in_group / 8 * MT, n0 = nt * NC;
 
-    const int turns = K / (DEPTH * kKT);
-    const int turn0 = (int)((long long)turns * split / splits);
-    const int turn1 = (int)((long long)turns * (split + 1) / splits);
-    const int steps = (turn1 - turn0) * DEPTH;
-    const uint32_t k_bytes0 = (uint32_t)turn0 * DEPTH * kRowBytes;
+    const int pairs = K / (2 * kKT);          // this split's share of K, in pairs of steps
+    const int step0 = 2 * (int)((long long)pairs * split / splits);
+    const int steps = 2 * (int)((long long)pairs * (split + 1) / splits) - step0;
     const uint32_t row_bytes = (uint32_t)K * 2u;
+    const uint32_t k_bytes0 = (uint32_t)step0 * kRowBytes;
 
-    // rows past M and weight rows past N read as zeros
+    // A load brings 8 rows of 128 bytes, lane by lane one behind the other; the permutation of a row's pieces is
+    // in the address a lane reads from.  Rows past the last repeat it: their results are not stored.
     const rsrc_t bx = make_rsrc(x + (size_t)m0 * K, (uint32_t)min(MT, M - m0) * row_bytes);
-    const uint32_t w_bytes = (uint32_t)min(NC, N - n0) * row_bytes;
-    const rsrc_t bw = make_rsrc(w + (size_t)n0 * K, w_bytes);
-    const rsrc_t bup = make_rsrc(EPI == kStoreGelu ? w + (size_t)(N + n0) * K : w, w_bytes);
-
-    const int lr = tid / 8, lc = tid & 7;
-    const uint32_t lane_bytes = (uint32_t)lr * row_bytes + (uint32_t)lc * 16u;
-    const int piece = piece_offset(lr, lc);
-
-    u32x4 rx[DEPTH][XP], rw[DEPTH][WP];
-    auto load = [&](int slot, int step) {
-        const uint32_t k = k_bytes0 + (uint32_t)min(step, steps - 1) * kRowBytes;
+    const int ncols = min(NC, N - n0);
+    const rsrc_t bw = make_rsrc(w + (size_t)n0 * K, (uint32_t)ncols * row_bytes);
+    const rsrc_t bup = make_rsrc(EPI == kStoreGelu ? w + (size_t)(N + n0) * K : w, (uint32_t)ncols * row_bytes);
+    const uint32_t piece = (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+    uint32_t at[L];
 #pragma unroll
-        for (int p = 0; p < XP; ++p) {
-            rx[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                        bx, lane_bytes + p * 32u * row_bytes + k, 0, kAuxDefault));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int p = 0; p < WP; ++p) {
-            const bool up = EPI == kStoreGelu && p >= WP / 2;
-            const uint32_t off = lane_bytes + (uint32_t)(up ? p - WP / 2 : p) * 32u * row_bytes + k;
-            rw[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(up ? bup : bw, off, 0,
-                                                                                          kAuxDefault));
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    auto stage = [&](int slot, int buf) {
-        unsigned char* s = smem + buf * WideLds<NT>::kStage + piece;
-#pragma unroll
-        for (int p = 0; p < XP; ++p) *reinterpret_cast<u32x4*>(s + p * 32 * kRowBytes) = rx[slot][p];
-#pragma unroll
-        for (int p = 0; p < WP; ++p) *reinterpret_cast<u32x4*>(s + (MT + p * 32) * kRowBytes) = rw[slot][p];
-    };
-
-    f32x16 acc[2][NB];
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.0f;
-
-    const int xrow = wm * 64 + (lane & 31), wrow = MT + wn * (NT / 2) + (lane & 31);
-#pragma unroll
-    for (int d = 0; d < DEPTH; ++d) load(d, d);
-    stage(0, 0);
-    load(0, DEPTH);
-    lds_barrier();
-    for (int t = 0; t < steps; t += DEPTH) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            const unsigned char* s = smem + (d & 1) * WideLds<NT>::kStage;
-            stage((d + 1) % DEPTH, (d + 1) & 1);
-            load((d + 1) % DEPTH, t + d + 1 + DEPTH);
-#pragma unroll
-            for (int ks = 0; ks < kKT / 16; ++ks) {
-                bf16x8 fx[2], fw[NB];
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-                    fx[mb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(xrow + 32 * mb, 2 * ks + (lane >> 5)));
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-                    fw[nb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(wrow + 32 * nb, 2 * ks + (lane >> 5)));
-#pragma unroll
-                for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[nb], fx[mb], acc[mb][nb], 0, 0, 0);
-            }
-            lds_barrier();
-        }
+    for (int l = 0; l < L; ++l) {
+        const int g = wv + l * kWideWaves;                    // groups 0..15 are rows of x
+        int row = (l < 2 ? g : g - 16) * 8 + (lane >> 3);
+        if (EPI == kStoreGelu && row >= NC && l >= 2) row -= NC;
+        row = min(row, (l < 2 ? min(MT, M - m0) : ncols) - 1);
+        at[l] = (uint32_t)row * row_bytes + piece;
     }
+    auto load = [&](int slot, int step) {
+        const uint32_t k = k_bytes0 + (uint32_t)step * kRowBytes;
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            const int g = wv + l * kWideWaves;
+            const bool up = EPI == kStoreGelu && l >= 2 && (g - 16) * 8 >= NC;
+            load_to_lds(l < 2 ? bx : (up ? bup : bw), smem + slot * Lds::kStage + g * 1024, at[l], k);
+        }
+    };
+
+    f32x16 acc[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mb][i] = 0.0f;
+
+    const int xrow = wm * (MT / WM) + (lane & 31), wrow = MT + wn * 32 + (lane & 31);
+    auto multiply = [&](int slot) {
+        const unsigned char* s = smem + slot * Lds::kStage;
+        bf16x8 fx[kKT / 16][MB], fw[kKT / 16];
+#pragma unroll
+        for (int ks = 0; ks < kKT / 16; ++ks) {
+            const int c = 2 * ks + (lane >> 5);
+            fw[ks] = *reinterpret_cast<const bf16x8*>(s + piece_offset(wrow, c));
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                fx[ks][mb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(xrow + 32 * mb, c));
+        }
+#pragma unroll
+        for (int ks = 0; ks < kKT / 16; ++ks)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+                acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[ks], fx[ks][mb], acc[mb], 0, 0, 0);
+    };
+
+    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
+    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
+#pragma unroll
+    for (int d = 0; d < S - 1; ++d)
+        if (d < steps) load(d, d);
+    int i = 0, slot = 0;
+    for (; i + S - 1 < steps; ++i) {
+        wait_loads<(S - 2) * L>();
+        lds_barrier();
+        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    for (; i < steps; ++i) {
+        switch (steps - 1 - i) {
+            case 0: wait_loads<0>(); break;
+            case 1: wait_loads<L>(); break;
+            default: wait_loads<2 * L>(); break;       // (no more than S - 2 = 2)
+        }
+        lds_barrier();
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    lds_barrier();
 
     // the tile through LDS, [128 rows][NT / 4 pieces of 4 columns] with the pieces permuted by the row,
     // so that it leaves in whole rows
     constexpr int PR = NT / 4;
 #pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int r = wm * 64 + mb * 32 + (lane & 31);
-                const int c = (wn * (NT / 2) + nb * 32) / 4 + 2 * g + (lane >> 5);
-                const f32x4 v = {acc[mb][nb][4 * g], acc[mb][nb][4 * g + 1], acc[mb][nb][4 * g + 2],
-                                 acc[mb][nb][4 * g + 3]};
-                *reinterpret_cast<f32x4*>(smem + (r * PR + (c ^ (r & 7))) * 16) = v;
-            }
+        for (int g = 0; g < 4; ++g) {
+            const int r = wm * (MT / WM) + mb * 32 + (lane & 31);
+            const int c = wn * 8 + 2 * g + (lane >> 5);
+            const f32x4 v = {acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
+            *reinterpret_cast<f32x4*>(smem + (r * PR + (c ^ (r & 7))) * 16) = v;
+        }
     lds_barrier();
     constexpr int CPT = EPI == kStoreGelu ? 4 : 8;            // output columns per thread
     constexpr int TPR = NC / CPT;                             // threads per row
     const int ec = tid % TPR;
     const int n = n0 + CPT * ec;
 #pragma unroll
-    for (int r = tid / TPR; r < MT; r += kThreads / TPR) {
+    for (int r = tid / TPR; r < MT; r += kWideThreads / TPR) {
         const int m = m0 + r;
         const int pa = EPI == kStoreGelu ? ec : 2 * ec, pc = EPI == kStoreGelu ? PR / 2 + ec : 2 * ec + 1;
         const f32x4 a = *reinterpret_cast<const f32x4*>(smem + (r * PR + (pa ^ (r & 7))) * 16);
@@ -494,7 +509,8 @@ struct Cut {
 // tiles of 4096 columns at 129 rows and more, and of 8192 at 33 to 128, were not split and left half of the
 // chip idle: steps of two and four such layers took 999 and 1094 us at 64 and 256 rows, in two splits 887 and
 // 908.  From 129 tiles on one split stays: 160 tiles over K = 2560 in two take 2 % more of a layer's time.
-constexpr int kSplitWorkgroups = 256;
+constexpr int kComputeUnits = 256;
+constexpr int kSplitWorkgroups = kComputeUnits;
 // Tiles of 128 x 128 from this many of them on; with fewer, part of the chip would be idle.
 constexpr int kMinWideTiles = 200;
 
@@ -506,8 +522,9 @@ Cut cut_for(int M, int N, int K, bool gelu, bool may_split) {
     c.splits = 1;
     const int mtiles = ceil_div(M, c.mt), cols = gelu ? 2 * N : N;
     if (c.mt == 128) {
-        // (split products keep 64 columns: of 128-wide ones 256 x 5120 x 2560 in three splits was measured, 19.1 us
-        // and 5.0 for the sums against 24, and no other)
+        // (split products keep 64 columns: in 128-wide tiles and as many workgroups 256 x 2560 x 7680 takes 22.0 us
+        // instead of 24.5, which twice the partial sums cost the norm behind it, 256 x 2560 x 2560 11.8 instead of
+        // 11.1, 256 x 5120 x 2560 15.7 and a launch for its sums instead of 17.4)
         if (!may_split && ceil_div(cols, 128) * mtiles >= kMinWideTiles) c.nt = 128;
         else c.depth = 2;
     }
@@ -527,20 +544,20 @@ int gemm(const void* x, const void* w, void* out, int M, int N, int K, const Cut
     const dim3 grid((unsigned)(ceil_div(ntiles * c.splits, 8) * 8 * mtiles));
     const bf16_t* xp = static_cast<const bf16_t*>(x);
     const bf16_t* wp = static_cast<const bf16_t*>(w);
-#define HAWK_GEMM(KERNEL, TILE, DEPTH)                                                                                      \
-    hipLaunchKernelGGL((KERNEL<TILE, DEPTH, EPI>), grid, dim3(kThreads), 0, st, xp, wp, out, M, N, K, ntiles, mtiles, \
-                       c.splits)
+#define HAWK_GEMM(THREADS, ...)                                                                                \
+    hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(THREADS), 0, st, xp, wp, out, M, N, K, ntiles, mtiles, c.splits)
     if (c.mt == 32) {
-        if (c.depth == 4) HAWK_GEMM(decode_gemm_kernel, 32, 4);
-        else HAWK_GEMM(decode_gemm_kernel, 32, 2);
+        if (c.depth == 4) HAWK_GEMM(kThreads, decode_gemm_kernel<32, 4, EPI>);
+        else HAWK_GEMM(kThreads, decode_gemm_kernel<32, 2, EPI>);
     } else if (c.mt == 64) {
-        if (c.depth == 4) HAWK_GEMM(decode_gemm_kernel, 64, 4);
-        else HAWK_GEMM(decode_gemm_kernel, 64, 2);
+        if (c.depth == 4) HAWK_GEMM(kThreads, decode_gemm_kernel<64, 4, EPI>);
+        else HAWK_GEMM(kThreads, decode_gemm_kernel<64, 2, EPI>);
     } else if (c.nt == 64) {
-        HAWK_GEMM(decode_gemm_wide_kernel, 64, 2);
+        if (ntiles * c.splits * mtiles <= kComputeUnits) HAWK_GEMM(kWideThreads, decode_gemm_wide_kernel<64, 4, EPI>);
+        else HAWK_GEMM(kWideThreads, decode_gemm_wide_kernel<64, 3, EPI>);
     } else {
-        if (c.depth == 4) HAWK_GEMM(decode_gemm_wide_kernel, 128, 4);
-        else HAWK_GEMM(decode_gemm_wide_kernel, 128, 2);
+        if (ntiles * c.splits * mtiles <= kComputeUnits) HAWK_GEMM(kWideThreads, decode_gemm_wide_kernel<128, 4, EPI>);
+        else HAWK_GEMM(kWideThreads, decode_gemm_wide_kernel<128, 2, EPI>);
     }
 #undef HAWK_GEMM
     return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;

@@ -17,4 +17,12 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// 16 bytes per lane from memory into LDS, without registers: lane l's bytes land at lds + 16 l (lds the same in
+// every lane of the wave).  Every address has to be in the resource's range.
+__device__ __forceinline__ void load_to_lds(rsrc_t r, unsigned char* lds, uint32_t lane_bytes, uint32_t bytes) {
+#if __HIP_DEVICE_COMPILE__    // (the host pass has no such builtin)
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, lane_bytes, bytes, 0, 0);
+#endif
+}
+
 }  // namespace hawk

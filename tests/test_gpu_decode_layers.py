@@ -27,7 +27,9 @@ def _exact_linear(x, w):
 # enough for 128-wide tiles (26000 x 1 row tile); K: one turn of each loop, odd turns, split over K
 @pytest.mark.parametrize("M,N,K", [(1, 8, 128), (1, 1024, 512), (2, 72, 384), (32, 200, 2560), (33, 64, 256),
                                    (64, 136, 640), (65, 328, 640), (128, 520, 256), (129, 5120, 2560), (256, 8, 128),
-                                   (255, 264, 7680), (70, 26000, 256), (200, 13064, 384)])
+                                   (255, 264, 7680), (70, 26000, 256), (200, 13064, 384),
+                                   # more workgroups than compute units, tiles of 128 and of 64 columns, and one pair of steps
+                                   (200, 17000, 256), (129, 9000, 640), (150, 9000, 128)])
 def test_linear_matches_64_bit_sums(M, N, K):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(M + N + K)
