@@ -8,6 +8,8 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import importlib.machinery
+import importlib.util
 import itertools
 import math
 import os
@@ -19,6 +21,7 @@ from torch.utils._device import DeviceContext
 _CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 # HAWK_HIP_LIB selects another build of the library (e.g. one compiled with other tile shapes)
 LIB_PATH = os.environ.get("HAWK_HIP_LIB") or os.path.join(_CSRC, "libhawk_hip.so")
+NATIVE_PATH = os.path.join(_CSRC, "_hawk_torch.so")
 
 HAWK_OK = 0
 HAWK_ERR_NULL_POINTER = 1
@@ -169,6 +172,59 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+_native = None
+
+
+def native():
+    """The host side of eager calls in native code (csrc/hawk_torch.cpp): allocation, launches and autograd nodes on
+    torch tensors, over the library that load() found.  Built first only if it is not there."""
+    global _native
+    if _native is not None:
+        return _native
+    lib = load()
+    with _lock:
+        if _native is not None:
+            return _native
+        if not os.path.exists(NATIVE_PATH):
+            from .csrc.build import build_native
+
+            build_native()
+        loader = importlib.machinery.ExtensionFileLoader("_hawk_torch", NATIVE_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_hawk_torch", loader))
+        loader.exec_module(module)
+        module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in module.functions()},
+                    _native_callables())
+        _native = module
+        return module
+
+
+def _native_callables() -> dict:
+    """What native code calls back: errors, buffers that Python keeps, and the backward passes it leaves to Python."""
+    from . import external, scan_fused
+
+    def device(index):
+        return torch.device("cuda", index)
+
+    return {
+        "check": check,
+        "activation_empty": lambda shape, bf16, index: activation_empty(
+            shape, torch.bfloat16 if bf16 else torch.float32, device(index)),
+        "scan_workspace": lambda index, nbytes: scan_workspace(device(index), nbytes),
+        "decode_workspace": lambda index, nbytes: decode_workspace(device(index), nbytes),
+        "gate_workspace": lambda index, nbytes: external._gate_workspace(device(index), nbytes),
+        "scan_backward": scan_fused.scan_backward,
+        "gated_backward": scan_fused.gated_backward,
+        "core_backward": scan_fused.core_backward,
+        "conv_backward": external.conv_backward,
+    }
+
+
+def forget_native(which: str) -> None:
+    """A workspace that native code may have seen is replaced or dropped."""
+    if _native is not None:
+        _native.forget(which)
+
+
 def status_string(status: int) -> str:
     return load().hawk_status_string(status).decode()
 
@@ -234,15 +290,26 @@ def transforms_active() -> bool:
             or torch.autograd.forward_ad._current_level >= 0)
 
 
+def eager() -> bool:
+    """Whether this call runs as written: nothing traces, watches or rewrites it."""
+    return (not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and not transforms_active())
+
+
+def plain_cuda(*tensors) -> bool:
+    for t in tensors:
+        if type(t) not in _PLAIN_TENSORS or not t.is_cuda:
+            return False
+    return True
+
+
 def launches_directly(*tensors) -> bool:
     """Whether a kernel can be launched on these tensors without going through its
     ``torch.library`` op.  The op exists for tracing (``torch.compile``, fake tensors, dispatch
     modes) and for the error that differentiating through it raises; its wrapper costs about 25 us
     of host time per call, as much as a small scan takes on the GPU.  Plain CUDA tensors outside
     any of that need none of it: same launch function, same results."""
-    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:
-        return False
-    if transforms_active():
+    if not eager():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:
@@ -351,6 +418,7 @@ def scan_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
         if ws is None or ws.numel() < nbytes:
             ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
             _workspaces[key] = ws
+            forget_native("scan_workspace")
     return ws
 
 
@@ -386,6 +454,7 @@ def decode_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
         if ws is None or ws.numel() < nbytes:
             ws = torch.zeros(max(nbytes, 4096), dtype=torch.uint8, device=dev)
             _decode_workspaces[key] = ws
+            forget_native("decode_workspace")
     return ws
 
 
@@ -396,6 +465,8 @@ def release_workspaces() -> None:
         _captured.clear()
         _decode_workspaces.clear()
         _decode_captured.clear()
+        forget_native("scan_workspace")
+        forget_native("decode_workspace")
 
 
 def _flag_of(ws: torch.Tensor, dev: torch.device) -> int:

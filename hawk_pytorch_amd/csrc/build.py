@@ -1,4 +1,5 @@
-"""Builds libhawk_hip.so (the C-ABI HIP library) in-tree with hipcc for gfx950.
+"""Builds libhawk_hip.so (the C-ABI HIP library) in-tree with hipcc for gfx950, and _hawk_torch.so (the host side of
+eager calls, no device code) with g++ against the installed torch.
 
 Usage:  python -m hawk_pytorch_amd.csrc.build [--force]
 """
@@ -14,6 +15,8 @@ from concurrent.futures import ThreadPoolExecutor
 CSRC = os.path.dirname(os.path.abspath(__file__))
 LIB_NAME = "libhawk_hip.so"
 LIB_PATH = os.path.join(CSRC, LIB_NAME)
+NATIVE_NAME = "_hawk_torch.so"
+NATIVE_PATH = os.path.join(CSRC, NATIVE_NAME)
 SOURCES = ["hawk_scan.hip", "hawk_conv.hip", "hawk_step.hip", "hawk_gates.hip", "hawk_block.hip", "hawk_decode.hip", "hawk_train.hip", "hawk_wgrad.hip", "hawk_probe.hip", "hawk_capi.hip"]
 HEADERS = ["hawk_scan.h", "hawk_device.h", "hawk_reduce.h", "hawk_tile.h", os.path.join("..", "..", "include", "hawk_hip.h")]
 
@@ -43,8 +46,33 @@ def _run(cmd):
     return proc
 
 
+def build_native(force: bool = True, verbose: bool = False) -> str:
+    """Compile the torch extension module.  Returns its path."""
+    import sysconfig
+
+    import torch
+
+    source, header = os.path.join(CSRC, "hawk_torch.cpp"), os.path.join(CSRC, "..", "..", "include", "hawk_hip.h")
+    if not force and os.path.exists(NATIVE_PATH) and os.path.getmtime(NATIVE_PATH) >= max(map(os.path.getmtime, (source, header))):
+        return NATIVE_PATH
+    if verbose:
+        print("g++ hawk_torch.cpp", flush=True)
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    tmp = NATIVE_PATH + ".%d.tmp" % os.getpid()
+    _run([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
+          "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch.compiled_with_cxx11_abi(),
+          "-isystem", os.path.join(root, "include"),
+          "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+          "-isystem", sysconfig.get_paths()["include"], "-isystem", os.path.join(rocm, "include"), source, "-o", tmp,
+          "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"])
+    os.replace(tmp, NATIVE_PATH)
+    return NATIVE_PATH
+
+
 def build(force: bool = True, verbose: bool = False) -> str:
-    """Compile every translation unit and link the shared library.  Returns its path."""
+    """Compile every translation unit and link the shared library, and the torch extension beside it.  Returns the
+    library's path."""
     hipcc = _hipcc()
     objdir = os.path.join(CSRC, "build")
     os.makedirs(objdir, exist_ok=True)
@@ -64,8 +92,10 @@ def build(force: bool = True, verbose: bool = False) -> str:
             _run([hipcc, *HIPCC_FLAGS, "-c", src_path, "-o", obj])
         return obj
 
-    with ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:
+    with ThreadPoolExecutor(max_workers=len(SOURCES) + 1) as pool:
+        native = pool.submit(build_native, force, verbose)
         objs = list(pool.map(compile_one, SOURCES))
+        native.result()
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs])
     return LIB_PATH
 

@@ -25,43 +25,15 @@ MAX_TEMPORAL_WIDTH = 8
 # conv1d custom ops
 # ---------------------------------------------------------------------------------------
 def _launch_conv_fwd(x, w, b, state, out_dtype) -> torch.Tensor:
-    tensors = [x, w, b] + ([state] if state is not None else [])
-    dev = _lib.require_cuda(*tensors)
-    x, w, b = _lib.dense16(x), _lib.dense16(w), _lib.dense16(b)
-    if state is not None:
-        state = _lib.dense16(state)
-    B, T, D = x.shape
-    W = w.shape[0]
-    y = _lib.activation_empty((B, T, D), out_dtype, dev)
-    lib = _lib.load()
-    with _lib.on_device(dev):
-        status = lib.hawk_conv1d_fwd(
-            x.data_ptr(), w.data_ptr(), b.data_ptr(), _lib.ptr(state), y.data_ptr(),
-            B, T, D, W, _lib.dtype_code(x.dtype), _lib.dtype_code(out_dtype), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_conv1d_fwd", status)
-    return y
+    _lib.require_cuda(x, w, b, *(() if state is None else (state,)))
+    _lib.dtype_code(x.dtype)
+    return _lib.native().conv_fwd(x, w, b, state, out_dtype == torch.float32)
 
 
 def _launch_conv_bwd(grad_y, x, w):
-    dev = _lib.require_cuda(grad_y, x, w)
-    grad_y, x, w = _lib.dense16(grad_y), _lib.dense16(x), _lib.dense16(w)
-    B, T, D = x.shape
-    W = w.shape[0]
-    dx = _lib.activation_empty(x.shape, x.dtype, dev)
-    dw = torch.empty((W, D), dtype=torch.float32, device=dev)
-    db = torch.empty((D,), dtype=torch.float32, device=dev)
-    lib = _lib.load()
-    nbytes = lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-    with _lib.on_device(dev):
-        status = lib.hawk_conv1d_bwd(
-            grad_y.data_ptr(), x.data_ptr(), w.data_ptr(), dx.data_ptr(), dw.data_ptr(), db.data_ptr(),
-            B, T, D, W, _lib.dtype_code(x.dtype), _lib.dtype_code(grad_y.dtype),
-            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_conv1d_bwd", status)
-    return dx, dw, db
+    _lib.require_cuda(grad_y, x, w)
+    _lib.dtype_code(x.dtype), _lib.dtype_code(grad_y.dtype)
+    return _lib.native().conv_bwd(grad_y, x, w)
 
 
 @torch.library.custom_op("hawk_amd::conv1d_fwd", mutates_args=(), device_types="cuda")
@@ -117,12 +89,15 @@ class _TemporalConv(Function):
 
     @staticmethod
     def backward(ctx, grad_y):  # type: ignore[override]
-        xc, w = ctx.saved_tensors
-        if grad_y.dtype not in (torch.bfloat16, torch.float32):
-            grad_y = grad_y.float()
-        gy = grad_y if grad_y.is_contiguous() else grad_y.contiguous()
-        dx, dw, db = _conv1d_bwd(gy, xc, w)
-        return dx, dw, db, None
+        return *conv_backward(grad_y, *ctx.saved_tensors), None
+
+
+def conv_backward(grad_y, x, w):
+    """(dx, dw, db) of the conv with zero history."""
+    if grad_y.dtype not in (torch.bfloat16, torch.float32):
+        grad_y = grad_y.float()
+    gy = grad_y if grad_y.is_contiguous() else grad_y.contiguous()
+    return _conv1d_bwd(gy, x, w)
 
 
 def temporal_conv1d(x, w, b, out_dtype: Optional[torch.dtype] = None, state=None):
@@ -146,6 +121,10 @@ def temporal_conv1d(x, w, b, out_dtype: Optional[torch.dtype] = None, state=None
         assert state.shape == (x.shape[0], W - 1, D)
         xc = x if x.is_contiguous() else x.contiguous()
         return _conv1d_fwd(xc, w32, b32, state.to(x.dtype), out_dtype == torch.float32)
+    if _lib.plain_cuda(x) and _lib.eager():
+        y = _lib.native().conv_node(x, w32, b32, out_dtype == torch.float32)
+        if y is not None:
+            return y
     return _TemporalConv.apply(x, w32, b32, out_dtype == torch.float32)
 
 
@@ -291,6 +270,11 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     hawk/cache.py:29-43.  ``x_new`` and ``y`` may be the two halves of the input projection,
     passed in place.
     """
+    if _lib.plain_cuda(x_new) and not torch.compiler.is_compiling():
+        out = _lib.native().decode_core(x_new, y, conv_state, recc_state, conv.w, conv.b, input_gate.w, input_gate.b,
+                                        a_gate.w, a_gate.b, a_param)
+        if out is not None:    # (None: an operand that has to be converted or copied first, or is refused)
+            return out
     W, D = conv.w.shape
     shape = x_new.shape
     B = x_new.numel() // D
@@ -380,33 +364,20 @@ class DecodeLayers:
         self.hidden = hidden
         self.M, self.H = hidden.shape
         self.R, self.inter = R, inter
-        dev = self.dev = hidden.device
-        self.lib = _lib.load()
-        nbytes = max(self.lib.hawk_decode_layer_workspace_bytes(self.M, self.H, R, inter, n) for n in (2 * R, vocab))
+        lib = _lib.load()
+        nbytes = max(lib.hawk_decode_layer_workspace_bytes(self.M, self.H, R, inter, n) for n in (2 * R, vocab))
         # one allocation per step, not a buffer kept per stream: a layer is several launches that hand
         # values on in it, and two threads may issue steps to one stream
-        self.ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
-        self.stream = _lib.stream_ptr(dev)
+        self.ws = torch.empty(nbytes, dtype=torch.uint8, device=hidden.device)
 
     def first(self, norm_w: torch.Tensor, eps: float, w: torch.Tensor) -> torch.Tensor:
         """rmsnorm(hidden) w^T"""
-        out = torch.empty((self.M, w.shape[0]), dtype=torch.bfloat16, device=self.dev)
-        with _lib.on_device(self.dev):
-            _lib.check("hawk_decode_norm_linear", self.lib.hawk_decode_norm_linear(
-                self.hidden.data_ptr(), norm_w.data_ptr(), eps, w.data_ptr(), out.data_ptr(), self.M, w.shape[0],
-                self.H, self.ws.data_ptr(), self.ws.numel(), self.stream))
-        return out
+        return _lib.native().decode_first(self.hidden, norm_w, eps, w, self.ws)
 
     def tail(self, gated, w_resid, norm_w, eps, w_gate_up, w_down, next_norm_w, next_eps, w_next) -> torch.Tensor:
         """What follows a layer's recurrent core, up to the next layer's input projection (or the head)."""
-        out = torch.empty((self.M, w_next.shape[0]), dtype=torch.bfloat16, device=self.dev)
-        with _lib.on_device(self.dev):
-            _lib.check("hawk_decode_layer_tail", self.lib.hawk_decode_layer_tail(
-                gated.data_ptr(), w_resid.data_ptr(), self.hidden.data_ptr(), norm_w.data_ptr(), eps,
-                w_gate_up.data_ptr(), w_down.data_ptr(), next_norm_w.data_ptr(), next_eps, w_next.data_ptr(),
-                out.data_ptr(), self.M, self.H, self.R, self.inter, w_next.shape[0], self.ws.data_ptr(),
-                self.ws.numel(), self.stream))
-        return out
+        return _lib.native().decode_tail(self.hidden, gated, w_resid, norm_w, eps, w_gate_up, w_down, next_norm_w,
+                                         next_eps, w_next, self.ws, self.R, self.inter)
 
 
 # ---------------------------------------------------------------------------------------
@@ -479,6 +450,7 @@ def _gate_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             _gate_ws[key] = ws
+            _lib.forget_native("gate_workspace")
     return ws
 
 
@@ -591,13 +563,7 @@ def kernel_weights(w_i: torch.Tensor, w_a: torch.Tensor, rows: int):
         nb, bw, _ = w_i.shape
         if w_i.is_cuda and w_a.dtype == torch.float32 and w_a.shape == w_i.shape and bw % 4 == 0:
             # both gates in one launch
-            wi, wa = _lib.dense16(w_i.detach()), _lib.dense16(w_a.detach())
-            both = torch.empty((2, nb, bw, bw), dtype=torch.bfloat16, device=w_i.device)
-            with _lib.on_device(w_i.device):
-                _lib.check("hawk_gate_weights_to_bf16", _lib.load().hawk_gate_weights_to_bf16(
-                    wi.data_ptr(), wa.data_ptr(), both[0].data_ptr(), both[1].data_ptr(), nb, bw,
-                    _lib.stream_ptr(w_i.device)))
-            return both[0], both[1]
+            return _lib.native().gate_weights_to_bf16(w_i.detach(), w_a.detach())
         return w_i.detach().to(torch.bfloat16), w_a.detach().to(torch.bfloat16)
     return w_i, w_a
 

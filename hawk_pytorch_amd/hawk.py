@@ -242,6 +242,9 @@ def _dense_param(module: Optional[nn.Module], name: str, shape, dtype: torch.dty
                  dev: torch.device) -> Optional[torch.Tensor]:
     """A module's parameter if a kernel can read it as it is: of this type and shape, dense, aligned."""
     w = module._parameters.get(name)
+    if dev.type == "cuda":
+        return w if type(w) is nn.Parameter and _lib.native().dense_parameter(w, shape, dtype == torch.bfloat16,
+                                                                             dev.index) else None
     if (type(w) is not nn.Parameter or w.dtype != dtype or w.shape != shape or w.device != dev
             or not w.is_contiguous() or w.data_ptr() % 16 != 0):
         return None

@@ -45,45 +45,15 @@ def _prepare(*tensors: torch.Tensor):
 
 
 def _launch_scan_fwd(x, x_rg_lru, a_rg_lru, a_param, h_bf16: bool) -> torch.Tensor:
-    dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param)
-    x, x_rg_lru, a_rg_lru, a_param = (_lib.dense16(t) for t in (x, x_rg_lru, a_rg_lru, a_param))
-    b, sq, d = x.shape
-    in_code = _lib.dtype_code(x.dtype)
-    out_dtype = torch.bfloat16 if h_bf16 else x.dtype
-    lib = _lib.load()
-    h = _lib.activation_empty((b, sq, d), out_dtype, dev)
-    nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
-    ws = _lib.scan_workspace(dev, nbytes)
-    with _lib.on_device(dev):
-        status = lib.hawk_rglru_scan_fwd_mixed(
-            x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), h.data_ptr(),
-            b, sq, d, in_code, _lib.dtype_code(out_dtype), ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_rglru_scan_fwd_mixed", status)
-    return h
+    _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param)
+    _lib.dtype_code(x.dtype)
+    return _lib.native().scan_fwd(x, x_rg_lru, a_rg_lru, a_param, h_bf16)
 
 
 def _launch_scan_bwd(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out):
-    dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
-    x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out = (
-        _lib.dense16(t) for t in (x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
-    )
-    b, sq, d = x.shape
-    in_code = _lib.dtype_code(x.dtype)
-    lib = _lib.load()
-    dx, dxg, dag = (_lib.activation_empty(x.shape, x.dtype, dev) for _ in range(3))
-    dlam = torch.empty(d, dtype=torch.float32, device=dev)
-    nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
-    ws = _lib.scan_workspace(dev, nbytes)
-    with _lib.on_device(dev):
-        status = lib.hawk_rglru_scan_bwd_mixed(
-            x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(),
-            h_saved.data_ptr(), grad_out.data_ptr(), dx.data_ptr(), dxg.data_ptr(), dag.data_ptr(),
-            dlam.data_ptr(), b, sq, d, in_code, _lib.dtype_code(h_saved.dtype),
-            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_rglru_scan_bwd_mixed", status)
-    return dx, dxg, dag, dlam
+    _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
+    _lib.dtype_code(x.dtype), _lib.dtype_code(h_saved.dtype)
+    return _lib.native().scan_bwd(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
 
 
 # ---------------------------------------------------------------------------------------
@@ -234,14 +204,25 @@ class DiagonalRecurrence(Function):
 
     @staticmethod
     def backward(ctx, grad_output):  # type: ignore[override]
-        (x, x_rg_lru, a_rg_lru, a_param, h_saved) = ctx.saved_tensors
-        x_grad, x_rg_lru_grad, a_rg_lru_grad, a_param_grad = sequential_scan_backward(
-            x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_output
-        )
-        return x_grad, x_rg_lru_grad, a_rg_lru_grad, a_param_grad.to(a_param.dtype)
+        return scan_backward(*ctx.saved_tensors, grad_output)
 
 
-fused_linear_scan = DiagonalRecurrence.apply
+def scan_backward(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_output):
+    """The four gradients of a scan's inputs, Lambda's in its own dtype."""
+    x_grad, x_rg_lru_grad, a_rg_lru_grad, a_param_grad = sequential_scan_backward(
+        x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_output
+    )
+    return x_grad, x_rg_lru_grad, a_rg_lru_grad, a_param_grad.to(a_param.dtype)
+
+
+def fused_linear_scan(x, x_rg_lru, a_rg_lru, a_param) -> torch.Tensor:
+    """``DiagonalRecurrence.apply``; an eager call on dense bf16 or fp32 tensors with Lambda in fp32 makes the same
+    node in native code, whose backward pass does without the interpreter."""
+    if _lib.plain_cuda(x) and _lib.eager():
+        h = _lib.native().scan_node(x, x_rg_lru, a_rg_lru, a_param)
+        if h is not None:
+            return h
+    return DiagonalRecurrence.apply(x, x_rg_lru, a_rg_lru, a_param)
 
 
 # ---------------------------------------------------------------------------------------
@@ -267,61 +248,15 @@ def _row_stride(t: torch.Tensor):
 
 
 def _launch_scan_gated_fwd(x, x_rg_lru, a_rg_lru, a_param, y, h_bf16: bool, want_h: bool, want_last: bool):
-    dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, y)
-    x, x_rg_lru, a_rg_lru, a_param = (_lib.dense16(t) for t in (x, x_rg_lru, a_rg_lru, a_param))
-    b, sq, d = x.shape
-    in_code = _lib.dtype_code(x.dtype)
-    out_dtype = torch.bfloat16 if h_bf16 else x.dtype
-    if y.dtype != out_dtype:
-        y = y.to(out_dtype)
-    ldy = _row_stride(y)
-    if ldy is None:
-        y = _lib.dense16(y)
-        ldy = d
-    lib = _lib.load()
-    out = _lib.activation_empty((b, sq, d), out_dtype, dev)
-    h = _lib.activation_empty((b, sq, d) if want_h else (0,), out_dtype, dev)
-    h_last = torch.empty((b, 1, d) if want_last else (0,), dtype=out_dtype, device=dev)
-    nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
-    ws = _lib.scan_workspace(dev, nbytes)
-    with _lib.on_device(dev):
-        status = lib.hawk_rglru_scan_gated_fwd(
-            x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), y.data_ptr(), ldy,
-            h.data_ptr() if want_h else None, out.data_ptr(), h_last.data_ptr() if want_last else None,
-            b, sq, d, in_code, _lib.dtype_code(out_dtype), ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_rglru_scan_gated_fwd", status)
-    return out, h, h_last
+    _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, y)
+    _lib.dtype_code(x.dtype)
+    return _lib.native().gated_fwd(x, x_rg_lru, a_rg_lru, a_param, y, h_bf16, want_h, want_last)
 
 
 def _launch_scan_gated_bwd(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out):
-    dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out)
-    x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out = (
-        _lib.dense16(t) for t in (x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
-    )
-    b, sq, d = x.shape
-    in_code = _lib.dtype_code(x.dtype)
-    if y.dtype != h_saved.dtype:
-        y = y.to(h_saved.dtype)
-    ldy = _row_stride(y)
-    if ldy is None:
-        y = _lib.dense16(y)
-        ldy = d
-    lib = _lib.load()
-    dx, dxg, dag = (_lib.activation_empty(x.shape, x.dtype, dev) for _ in range(3))
-    dy = _lib.activation_empty((b, sq, d), h_saved.dtype, dev)
-    dlam = torch.empty(d, dtype=torch.float32, device=dev)
-    nbytes = lib.hawk_scan_workspace_bytes(b, sq, d, in_code)
-    ws = _lib.scan_workspace(dev, nbytes)
-    with _lib.on_device(dev):
-        status = lib.hawk_rglru_scan_gated_bwd(
-            x.data_ptr(), x_rg_lru.data_ptr(), a_rg_lru.data_ptr(), a_param.data_ptr(), y.data_ptr(), ldy,
-            h_saved.data_ptr(), grad_out.data_ptr(), dx.data_ptr(), dxg.data_ptr(), dag.data_ptr(),
-            dy.data_ptr(), d, dlam.data_ptr(), b, sq, d, in_code, _lib.dtype_code(h_saved.dtype),
-            ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev),
-        )
-    _lib.check("hawk_rglru_scan_gated_bwd", status)
-    return dx, dxg, dag, dlam, dy
+    _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out)
+    _lib.dtype_code(x.dtype), _lib.dtype_code(h_saved.dtype)
+    return _lib.native().gated_bwd(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out)
 
 
 @torch.library.custom_op("hawk_amd::rglru_scan_gated_fwd", mutates_args=(), device_types="cuda")
@@ -416,17 +351,22 @@ class GatedDiagonalRecurrence(Function):
 
     @staticmethod
     def backward(ctx, grad_out, _grad_last):  # type: ignore[override]
-        (x, x_rg_lru, a_rg_lru, a_param, y, h_saved) = ctx.saved_tensors
-        if not grad_out.is_contiguous():
-            grad_out = grad_out.contiguous()
-        if grad_out.dtype != h_saved.dtype:
-            grad_out = grad_out.to(h_saved.dtype)
-        dx, dxg, dag, dlam, dy = _scan_gated_bwd(
-            x, x_rg_lru, a_rg_lru, a_param.float().contiguous(), y, h_saved, grad_out
-        )
+        dx, dxg, dag, dlam, dy = gated_backward(*ctx.saved_tensors, grad_out)
         if dy.dtype != ctx.y_dtype:
             dy = dy.to(ctx.y_dtype)
-        return dx, dxg, dag, dlam.to(a_param.dtype), dy, None, None
+        return dx, dxg, dag, dlam, dy, None, None
+
+
+def gated_backward(x, x_rg_lru, a_rg_lru, a_param, y, h_saved, grad_out):
+    """Gradients of the gated scan's inputs, Lambda's in its own dtype, y's in the state's."""
+    if not grad_out.is_contiguous():
+        grad_out = grad_out.contiguous()
+    if grad_out.dtype != h_saved.dtype:
+        grad_out = grad_out.to(h_saved.dtype)
+    dx, dxg, dag, dlam, dy = _scan_gated_bwd(
+        x, x_rg_lru, a_rg_lru, a_param.float().contiguous(), y, h_saved, grad_out
+    )
+    return dx, dxg, dag, dlam.to(a_param.dtype), dy
 
 
 def fused_linear_scan_gated(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state: bool = False):
@@ -435,8 +375,13 @@ def fused_linear_scan_gated(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state
     With ``return_last_state`` also returns h[:, -1:, :] (shape [B, 1, D]), the recurrent
     state a decode cache keeps after prefill.
     """
-    out, h_last = GatedDiagonalRecurrence.apply(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state,
-                                                torch.is_grad_enabled())
+    made = None
+    if _lib.plain_cuda(x) and _lib.eager():
+        made = _lib.native().gated_node(x, x_rg_lru, a_rg_lru, a_param, y, bool(return_last_state))
+    if made is None:
+        made = GatedDiagonalRecurrence.apply(x, x_rg_lru, a_rg_lru, a_param, y, return_last_state,
+                                             torch.is_grad_enabled())
+    out, h_last = made
     return (out, h_last) if return_last_state else out
 
 
@@ -498,9 +443,6 @@ def recurrent_core(u, input_gate, a_gate, a_param, y, return_last_state: bool = 
 # xy side by side into one tensor, where autograd would concatenate two.  One custom op per
 # direction, so the host issues two calls per layer.
 # ---------------------------------------------------------------------------------------
-_FUSED_CONV_MIN_T = 32   # hawk_conv_gate_proj_fwd needs T >= 32 and a temporal width of 4
-
-
 def block_core_layout_ok(xy: torch.Tensor) -> bool:
     """xy [B,T,2D] bf16 on the GPU with unit channel stride and evenly spaced rows a multiple of
     8 elements apart: what the kernels read in place.  (Plain Python on shapes and strides, so a
@@ -512,80 +454,13 @@ def block_core_layout_ok(xy: torch.Tensor) -> bool:
 
 
 def _launch_block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, want_h: bool, want_last: bool):
-    dev = _lib.require_cuda(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam)
-    if xy.data_ptr() % 16 != 0:
-        xy = xy.clone(memory_format=torch.contiguous_format)
-    B, T, D2 = xy.shape
-    D = D2 // 2
-    ld = _row_stride(xy)
-    W = conv_w.shape[0]
-    nb = w_i.shape[0]
-    conv_w, conv_b, w_i, w_a, b_i, b_a, lam = (_lib.dense16(t) for t in (conv_w, conv_b, w_i, w_a, b_i, b_a, lam))
-    bf, code = torch.bfloat16, _lib.HAWK_DTYPE_BF16
-    u, xg, ag, out = (_lib.activation_empty((B, T, D), bf, dev) for _ in range(4))
-    h = _lib.activation_empty((B, T, D) if want_h else (0,), bf, dev)
-    h_last = torch.empty((B, 1, D) if want_last else (0,), dtype=bf, device=dev)
-    lib = _lib.load()
-    ws = _lib.scan_workspace(dev, lib.hawk_scan_workspace_bytes(B, T, D, code))
-    y_ptr = xy.data_ptr() + D * xy.element_size()
-    with _lib.on_device(dev):
-        st = _lib.stream_ptr(dev)
-        if W == 4 and T >= _FUSED_CONV_MIN_T:
-            # conv + both projections, then the gated scan: one host call
-            _lib.check("hawk_block_core_fwd", lib.hawk_block_core_fwd(
-                xy.data_ptr(), ld, conv_w.data_ptr(), conv_b.data_ptr(), w_i.data_ptr(), b_i.data_ptr(),
-                w_a.data_ptr(), b_a.data_ptr(), _lib.dtype_code(w_i.dtype), None, lam.data_ptr(), u.data_ptr(),
-                xg.data_ptr(), ag.data_ptr(), h.data_ptr() if want_h else None, out.data_ptr(),
-                h_last.data_ptr() if want_last else None, B, T, D, nb, W, ws.data_ptr(), ws.numel(), st))
-        else:
-            _lib.check("hawk_conv1d_fwd_strided", lib.hawk_conv1d_fwd_strided(
-                xy.data_ptr(), ld, conv_w.data_ptr(), conv_b.data_ptr(), None, u.data_ptr(), D, B, T, D, W, code,
-                code, st))
-            _lib.check("hawk_gate_proj_fwd", lib.hawk_gate_proj_fwd(
-                u.data_ptr(), w_i.data_ptr(), b_i.data_ptr(), w_a.data_ptr(), b_a.data_ptr(), xg.data_ptr(),
-                ag.data_ptr(), B * T, D, nb, code, _lib.dtype_code(w_i.dtype), code, st))
-            _lib.check("hawk_rglru_scan_gated_fwd", lib.hawk_rglru_scan_gated_fwd(
-                u.data_ptr(), xg.data_ptr(), ag.data_ptr(), lam.data_ptr(), y_ptr, ld,
-                h.data_ptr() if want_h else None, out.data_ptr(), h_last.data_ptr() if want_last else None,
-                B, T, D, code, code, ws.data_ptr(), ws.numel(), st))
-    return out, u, xg, ag, h, h_last
+    _lib.require_cuda(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam)
+    return _lib.native().core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, want_h, want_last)
 
 
 def _launch_block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out):
-    from .external import _gate_workspace  # deferred: external imports nothing from here
-
-    dev = _lib.require_cuda(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out)
-    if xy.data_ptr() % 16 != 0:
-        xy = xy.clone(memory_format=torch.contiguous_format)
-    B, T, D2 = xy.shape
-    D = D2 // 2
-    ld = _row_stride(xy)
-    W = conv_w.shape[0]
-    nb, bw, _ = w_i.shape
-    M = B * T
-    conv_w, w_i, w_a, lam, grad_out = (_lib.dense16(t) for t in (conv_w, w_i, w_a, lam, grad_out))
-    bf, code, f32 = torch.bfloat16, _lib.HAWK_DTYPE_BF16, torch.float32
-    lib = _lib.load()
-    d_xy = _lib.activation_empty((B, T, D2), bf, dev)
-    du, dxg, dag = (_lib.activation_empty((B, T, D), bf, dev) for _ in range(3))
-    dlam = torch.empty(D, dtype=f32, device=dev)
-    dw_i, dw_a = (torch.empty((nb, bw, bw), dtype=f32, device=dev) for _ in range(2))
-    db_i, db_a, dcb = (torch.empty(D, dtype=f32, device=dev) for _ in range(3))
-    dcw = torch.empty((W, D), dtype=f32, device=dev)
-    ws = _lib.scan_workspace(dev, lib.hawk_scan_workspace_bytes(B, T, D, code))
-    gws = _gate_workspace(dev, lib.hawk_gate_proj_bwd_weights_workspace_bytes(M, D, nb))
-    cws = torch.empty(lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W), dtype=torch.uint8, device=dev)
-    with _lib.on_device(dev):
-        # scan (with the output gate) -> projections' input gradient onto the scan's, in place ->
-        # conv -> projections' weight gradients, and one launch for the three closing reductions
-        _lib.check("hawk_block_core_bwd", lib.hawk_block_core_bwd(
-            xy.data_ptr(), ld, u.data_ptr(), xg.data_ptr(), ag.data_ptr(), h.data_ptr(), conv_w.data_ptr(),
-            w_i.data_ptr(), w_a.data_ptr(), _lib.dtype_code(w_i.dtype), lam.data_ptr(), grad_out.data_ptr(),
-            d_xy.data_ptr(), D2, du.data_ptr(), dxg.data_ptr(), dag.data_ptr(), dcw.data_ptr(), dcb.data_ptr(),
-            dw_i.data_ptr(), db_i.data_ptr(), dw_a.data_ptr(), db_a.data_ptr(), dlam.data_ptr(), B, T, D, nb, W,
-            ws.data_ptr(), ws.numel(), gws.data_ptr(), gws.numel(), cws.data_ptr(), cws.numel(),
-            _lib.stream_ptr(dev)))
-    return d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam
+    _lib.require_cuda(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out)
+    return _lib.native().core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out)
 
 
 @torch.library.custom_op("hawk_amd::block_core_fwd", mutates_args=(), device_types="cuda")
@@ -662,14 +537,17 @@ class BlockCore(Function):
 
     @staticmethod
     def backward(ctx, grad_out, _grad_last):  # type: ignore[override]
-        xy, u, xg, ag, h, cw, w_i, w_a, lam = ctx.saved_tensors
-        go = grad_out if grad_out.dtype == torch.bfloat16 else grad_out.to(torch.bfloat16)
-        go = go if go.is_contiguous() else go.contiguous()
-        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = block_core_backward(xy, u, xg, ag, h, cw, w_i, w_a, lam, go)
-        nb, bw, _ = w_i.shape
+        d_xy, dcw, dcb, dw_i, db_i, dw_a, db_a, dlam = core_backward(*ctx.saved_tensors, grad_out)
+        nb, bw, _ = dw_i.shape
         t = ctx.dtypes
         return (d_xy, dcw.to(t[0]), dcb.to(t[1]), dw_i.to(t[2]), db_i.reshape(nb, bw).to(t[3]), dw_a.to(t[4]),
                 db_a.reshape(nb, bw).to(t[5]), dlam.to(t[6]), None, None)
+
+
+def core_backward(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out):
+    go = grad_out if grad_out.dtype == torch.bfloat16 else grad_out.to(torch.bfloat16)
+    go = go if go.is_contiguous() else go.contiguous()
+    return block_core_backward(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, go)
 
 
 def recurrent_block_core(xy, conv, input_gate, a_gate, a_param, return_last_state: bool = False):
@@ -677,10 +555,16 @@ def recurrent_block_core(xy, conv, input_gate, a_gate, a_param, return_last_stat
     ``x, y = xy.chunk(2, -1)``, for a bf16 ``xy`` that ``block_core_layout_ok`` accepts and gate
     modules the fused projection kernels serve (``external.gate_projections_supported``)."""
     args = (xy, conv.w, conv.b, input_gate.w, input_gate.b, a_gate.w, a_gate.b, a_param)
-    if not torch.is_grad_enabled() and _lib.launches_directly(*args):
-        # a prompt on a server: nothing is recorded, so the scan leaves its states unwritten (a sixth of
-        # its bytes: 37.5 against 34.8 us at B=1, T=4096, D=2560) and no autograd node is made
-        out, h_last, _ = _block_core(*args, False, bool(return_last_state))
+    want_last = bool(return_last_state)
+    if _lib.eager() and _lib.plain_cuda(*args):
+        # the launches, and a node in native code around them if something asks for a gradient; if nothing does, as
+        # for a prompt on a server, the scan leaves its states unwritten (a sixth of its bytes: 37.5 against 34.8 us
+        # at B=1, T=4096, D=2560)
+        recorded = torch.is_grad_enabled() and any(t.requires_grad for t in args)
+        with torch.no_grad():
+            out, h_last, (_, u, xg, ag, h, cw, w_i, w_a, lam) = _block_core(*args, recorded, want_last)
+        if recorded:
+            out, h_last = _lib.native().core_node(args, (out, u, xg, ag, h, h_last), (cw, w_i, w_a, lam))
     else:
         out, h_last = BlockCore.apply(*args, return_last_state, torch.is_grad_enabled())
     return (out, h_last) if return_last_state else out
