@@ -102,6 +102,11 @@ SIGNATURES = {
     "hawk_weight_grad_supported": (_c_int, [_c_int] * 3),
     "hawk_weight_grad_workspace_bytes": (_c_size_t, [_c_int] * 3),
     "hawk_weight_grad": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),
+    "hawk_weight_grads_workspace_bytes": (_c_size_t, [_c_int] * 2 + [ctypes.POINTER(_c_int)] * 2),
+    "hawk_weight_grads": (
+        _c_int, [_c_int] + [ctypes.POINTER(_c_void_p)] * 3 + [_c_int] + [ctypes.POINTER(_c_int)] * 2
+        + [_c_void_p, _c_size_t, _c_void_p]
+    ),
     "hawk_decode_linear_supported": (_c_int, [_c_int] * 3),
     "hawk_decode_linear_workspace_bytes": (_c_size_t, [_c_int] * 3),
     "hawk_decode_linear": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),

@@ -388,17 +388,34 @@ int hawk_embedding_bwd(const long long* ids, const float* dout, float* dweight, 
 int hawk_weight_grad_supported(int rows, int N, int K) { return hawk::weight_grad_supported(rows, N, K) ? 1 : 0; }
 
 size_t hawk_weight_grad_workspace_bytes(int rows, int N, int K) {
-    return hawk::weight_grad_supported(rows, N, K) ? hawk::weight_grad_workspace_bytes(rows, N, K) : 0;
+    return hawk::weight_grad_supported(rows, N, K) ? hawk::weight_grads_workspace_bytes(1, rows, &N, &K) : 0;
 }
 
 int hawk_weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K, void* workspace_device,
                      size_t workspace_bytes, void* stream) {
-    if (!dy || !x || !dw) return HAWK_ERR_NULL_POINTER;
-    if (!hawk::weight_grad_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
-    if (!aligned16(dy) || !aligned16(x) || !aligned16(dw) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
-    const size_t need = hawk::weight_grad_workspace_bytes(rows, N, K);
+    return hawk_weight_grads(1, &dy, &x, &dw, rows, &N, &K, workspace_device, workspace_bytes, stream);
+}
+
+size_t hawk_weight_grads_workspace_bytes(int n, int rows, const int* N, const int* K) {
+    if (n < 1 || n > hawk::kWeightGradTasks || !N || !K) return 0;
+    for (int k = 0; k < n; ++k)
+        if (!hawk::weight_grad_supported(rows, N[k], K[k])) return 0;
+    return hawk::weight_grads_workspace_bytes(n, rows, N, K);
+}
+
+int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float* const* dw, int rows, const int* N,
+                      const int* K, void* workspace_device, size_t workspace_bytes, void* stream) {
+    if (n < 1 || n > hawk::kWeightGradTasks) return HAWK_ERR_BAD_SHAPE;
+    if (!dy || !x || !dw || !N || !K) return HAWK_ERR_NULL_POINTER;
+    for (int k = 0; k < n; ++k) {
+        if (!dy[k] || !x[k] || !dw[k]) return HAWK_ERR_NULL_POINTER;
+        if (!hawk::weight_grad_supported(rows, N[k], K[k])) return HAWK_ERR_BAD_SHAPE;
+        if (!aligned16(dy[k]) || !aligned16(x[k]) || !aligned16(dw[k])) return HAWK_ERR_ALIGNMENT;
+    }
+    if (!aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    const size_t need = hawk::weight_grads_workspace_bytes(n, rows, N, K);
     if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;
-    return hawk::weight_grad(dy, x, dw, rows, N, K, workspace_device, as_stream(stream));
+    return hawk::weight_grads(n, dy, x, dw, rows, N, K, workspace_device, as_stream(stream));
 }
 
 int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }

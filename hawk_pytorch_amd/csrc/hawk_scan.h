@@ -138,8 +138,10 @@ int embedding_bwd(const long long* ids, const float* dout, float* dweight, int r
 
 // hawk_wgrad.hip
 bool weight_grad_supported(int rows, int N, int K);
-size_t weight_grad_workspace_bytes(int rows, int N, int K);
-int weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K, void* ws, hipStream_t st);
+constexpr int kWeightGradTasks = 8;
+size_t weight_grads_workspace_bytes(int n, int rows, const int* N, const int* K);
+int weight_grads(int n, const void* const* dy, const void* const* x, float* const* dw, int rows, const int* N, const int* K,
+                 void* ws, hipStream_t st);
 
 // hawk_probe.hip
 bool stream_probe_shape_ok(size_t bytes, size_t row_pitch, int shape);

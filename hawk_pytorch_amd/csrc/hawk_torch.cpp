@@ -60,8 +60,8 @@ constexpr int64_t kStaggerMinBytes = 16 << 20;   // _lib.activation_empty places
     X(hawk_decode_core_workspace_bytes) X(hawk_decode_core_step_ws) X(hawk_decode_layer_tail)                         \
     X(hawk_decode_norm_linear) X(hawk_cast) X(hawk_add_norm_fwd) X(hawk_add_norm_bwd)                                 \
     X(hawk_add_norm_bwd_workspace_bytes) X(hawk_gelu_mul_fwd) X(hawk_gelu_mul_bwd) X(hawk_cross_entropy_fwd)          \
-    X(hawk_cross_entropy_bwd) X(hawk_embedding_bwd) X(hawk_weight_grad) X(hawk_weight_grad_supported)                 \
-    X(hawk_weight_grad_workspace_bytes)
+    X(hawk_cross_entropy_bwd) X(hawk_embedding_bwd) X(hawk_weight_grads) X(hawk_weight_grad_supported)                \
+    X(hawk_weight_grads_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     HAWK_FUNCTIONS(X)
@@ -660,22 +660,36 @@ std::tuple<Tensor, std::optional<Tensor>, Tensor> add_norm_bwd(const Tensor& dou
     return {d_sum, d_delta, d_weight};
 }
 
-// dy^T x of [n, N] and [n, K]: fp32 by the kernel that splits the rows, where the result is at most 128 of its tiles;
-// from there on the library's product is as fast or faster, in bf16.  By itself (against product and conversion) the
-// kernel is ahead up to 512 rows and from 4096 on, and behind between them where the result has more than 32 tiles
-// (2048 x 1024: 512 rows 12.2 against 14.7 us, 1024 rows 21.2 against 17.4, 2048 rows 27.3 against 24.2, 4096 rows
-// 39.7 against 39.7).
-Tensor weight_grad(const Tensor& dy, const Tensor& x) {
-    Call c(dy.device());
-    const int n = dy.size(0), N = dy.size(1), K = x.size(1);
-    if ((int64_t)((N + 127) / 128) * ((K + 127) / 128) > 128 || !lib.hawk_weight_grad_supported(n, N, K))
-        return at::mm(dy.t(), x);
-    Tensor dw = c.empty({N, K}, kF32);
-    const size_t bytes = lib.hawk_weight_grad_workspace_bytes(n, N, K);
+// dy^T x of [n, N] and [n, K] each: in fp32, those whose result is at most 128 of the kernel's tiles together in one
+// launch; from there on the library's product is as fast or faster, in bf16.  (Alone, against product and conversion, the
+// kernel is ahead up to 512 rows and from 4096 on, and behind between them where the result has more than 32 tiles:
+// 2048 x 1024 at 512 rows 12.2 against 14.7 us, 1024 rows 21.2 against 17.4, 2048 rows 27.3 against 24.2, 4096 rows
+// 39.7 against 39.7.)
+std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& products) {
+    Call c(products[0].first.device());
+    const int n = products[0].first.size(0);
+    std::vector<Tensor> out(products.size());
+    std::vector<const void*> dy, x;
+    std::vector<float*> dw;
+    std::vector<int> N, K;
+    for (size_t k = 0; k < products.size(); ++k) {
+        const auto& [g, in] = products[k];
+        const int rows = g.size(1), cols = in.size(1);
+        if ((int64_t)((rows + 127) / 128) * ((cols + 127) / 128) > 128 || !lib.hawk_weight_grad_supported(n, rows, cols)) {
+            out[k] = at::mm(g.t(), in);
+            continue;
+        }
+        out[k] = c.empty({rows, cols}, kF32);
+        dy.push_back(data(g)), x.push_back(data(in)), dw.push_back(data<float>(out[k])), N.push_back(rows), K.push_back(cols);
+    }
+    if (dy.empty()) return out;
+    const size_t bytes = lib.hawk_weight_grads_workspace_bytes(dy.size(), n, N.data(), K.data());
     const Tensor ws = c.empty({(int64_t)bytes}, at::kByte);
-    check("hawk_weight_grad", lib.hawk_weight_grad(data(dy), data(x), data<float>(dw), n, N, K, data_or_null(ws), bytes, c.st));
-    return dw;
+    check("hawk_weight_grads", lib.hawk_weight_grads(dy.size(), dy.data(), x.data(), dw.data(), n, N.data(), K.data(),
+                                                     data_or_null(ws), bytes, c.st));
+    return out;
 }
+Tensor weight_grad(const Tensor& dy, const Tensor& x) { return weight_grads({{dy, x}})[0]; }
 
 Tensor gelu_mul(const Tensor& gu, int rows, int inter) {
     Call c(gu.device());
@@ -719,31 +733,29 @@ std::vector<Tensor> layer_bwd(const std::vector<Tensor>& s, const Tensor& d_tota
     auto as = [&](const Tensor& t, at::ScalarType type) { return dense16(t.scalar_type() == type ? t : t.to(type)).view({rows, H}); };
     const Tensor d_total = as(d_total_, kF32), d_out = as(d_out_, kBF16);
     const Tensor d_act = at::mm(d_out, w_dn);
-    Tensor g_dn = weight_grad(d_out, act);
     const Tensor d_gu = c.empty(gu.sizes(), kBF16);
     check("hawk_gelu_mul_bwd", lib.hawk_gelu_mul_bwd(data(gu), data(d_act), data(d_gu), rows, inter, c.st));
     const Tensor d_x2 = at::mm(d_gu, w_gu);
-    Tensor g_gu = weight_grad(d_gu, x2);
     auto [d_total1, d_mixed, g_n2] = add_norm_bwd(d_x2, total2, rstd2, n2, d_total, true);
     const Tensor d_gated = at::mm(*d_mixed, w_out);
-    Tensor g_out = weight_grad(*d_mixed, gated.view({rows, R}));
     auto [d_xy_, dcw, dcb, dwi, dbi, dwa, dba, dlam] = core_bwd(xy, u, xg, ag, h, cw, wi, wa, lam, d_gated.view({B, T, R}));
     const Tensor d_xy = d_xy_.view({rows, 2 * R});
     const Tensor d_x1 = at::mm(d_xy, w_in);
-    Tensor g_in = weight_grad(d_xy, x1);
+    // (all four at the end: each alone is too few tiles for the chip)
+    std::vector<Tensor> g = weight_grads({{d_gu, x2}, {d_out, act}, {d_xy, x1}, {*d_mixed, gated.view({rows, R})}});
     auto [d_hidden, d_delta, g_n1] = add_norm_bwd(d_x1, total1, rstd1, n1, d_total1, want_delta);
     // gradients that the library's products left in bf16, converted by one launch
     std::vector<Tensor*> narrow;
     std::vector<Tensor> in;
-    for (Tensor* g : {&g_in, &g_out, &g_gu, &g_dn})
-        if (g->scalar_type() != kF32) narrow.push_back(g), in.push_back(*g);
+    for (Tensor& t : g)
+        if (t.scalar_type() != kF32) narrow.push_back(&t), in.push_back(t);
     if (!in.empty()) {
         const std::vector<Tensor> wide = cast_in(c, in, kF32);
         for (size_t k = 0; k < wide.size(); ++k) *narrow[k] = wide[k];
     }
     const int64_t nb = wi.size(0), bw = wi.size(1);
-    return {d_hidden.view({B, T, H}), d_delta.has_value() ? d_delta->view({B, T, H}) : Tensor(), g_n1, g_n2, g_in, g_out, g_gu,
-            g_dn, dcw, dcb, dwi, dbi.view({nb, bw}), dwa, dba.view({nb, bw}), dlam};
+    return {d_hidden.view({B, T, H}), d_delta.has_value() ? d_delta->view({B, T, H}) : Tensor(), g_n1, g_n2, g[2], g[3], g[0],
+            g[1], dcw, dcb, dwi, dbi.view({nb, bw}), dwa, dba.view({nb, bw}), dlam};
 }
 
 // Final norm, head and mean cross entropy: the loss and head16, total, x, rstd, logits, lse, mean.

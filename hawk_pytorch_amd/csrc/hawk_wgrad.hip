@@ -6,9 +6,11 @@
 //
 // A workgroup of four waves owns 128 x 128 results, two workgroups share a compute unit; waves 0 and 1 fetch
 // dy, waves 2 and 3 fetch x, two 64-row tiles ahead in registers.  A layer's weights are few tiles
-// (1024 x 512: 32 of them), so the rows are split over workgroups, and a second kernel adds the fp32 partial
-// results in a fixed order.  What that spares next to the library's product is the conversion to fp32, and the
-// chip is not left idle by few tiles: 2048 rows, 512 x 512 13.9 us (library and conversion 17.8), 4593
+// (1024 x 512: 32 of them), so a layer's four are one launch, the rows are split over workgroups where that still
+// leaves some of the chip idle, and a second kernel adds the fp32 partial results in a fixed order.  Four weights of a
+// layer of 512 channels over 2048 rows: 33.4 us in one launch, 67.8 in four (with their sums), 94.5 by the library.
+// What that spares next to the library's product is the conversion to fp32, and the chip is not left idle by few
+// tiles: 2048 rows, 512 x 512 13.9 us (library and conversion 17.8), 4593
 // rows, 2048 x 1024 43.3 (50.0), 1024 x 1024 27.8 (38.5).  Between 512 and 4096 rows, where a few steps are split
 // and the sums cost a launch, results of more than 32 tiles take up to a fifth longer than the library's (1024
 // rows, 2048 x 1024: 21.2 against 17.4).  From 128 tiles on the library is as fast or faster (8192 rows, 2560 x
@@ -35,22 +37,40 @@ __device__ __forceinline__ int piece_offset(int r, int c) {
     return r * kRowBytes + ((c ^ ((r ^ (r >> 3)) & 7)) << 4);
 }
 
-// out [M, N] (or [splits, M, N]) = a^T b for a [K, M] and b [K, N].
-__global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(const bf16_t* __restrict__ a,
-                                                                  const bf16_t* __restrict__ b,
-                                                                  float* __restrict__ out, int M, int N, int K,
-                                                                  int ntiles, int mtiles, int splits) {
+// One product of a launch: out [M, N] (or [splits, M, N]) = a^T b for a [K, M] and b [K, N].  Its workgroups start at
+// first; the launch's tasks share K and the number of splits.
+struct GradTask {
+    const bf16_t *a, *b;
+    float* out;
+    int M, N, ntiles, mtiles;
+    unsigned first;
+};
+struct GradTasks {
+    GradTask task[kWeightGradTasks];
+    int n, K, splits;
+};
+
+__global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(GradTasks tasks) {
     __shared__ __align__(16) unsigned char smem[4 * kOperand];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int wm = wv & 1, wn = wv >> 1;
 
+    int which = 0;
+    for (int k = 1; k < tasks.n; ++k)
+        if (blockIdx.x >= tasks.task[k].first) which = k;
+    const GradTask& task = tasks.task[which];
+    const bf16_t* const a = task.a;
+    const bf16_t* const b = task.b;
+    float* const out = task.out;
+    const int M = task.M, N = task.N, K = tasks.K, ntiles = task.ntiles, mtiles = task.mtiles, splits = tasks.splits;
+
     // row tiles of one column tile sit 8 workgroups apart: on one XCD, at about the same time
-    const int blk = (int)blockIdx.x;
+    const int blk = (int)(blockIdx.x - task.first);
     const int group = blk / (8 * mtiles), in_group = blk - group * 8 * mtiles;
     const int item = group * 8 + (in_group & 7);
-    if (item >= ntiles * splits) return;      // the grid is padded to whole groups of 8
+    if (item >= ntiles * splits) return;      // a task's workgroups are padded to whole groups of 8
     const int split = item / ntiles;
     const int m0 = in_group / 8 * kTile, n0 = (item - split * ntiles) * kTile;
     const int all = (K + kKT - 1) / kKT;
@@ -167,18 +187,33 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(const bf16_t* 
     }
 }
 
+// The partial results of a launch's tasks added up, 1024 values of one task per workgroup.
+struct SumTask {
+    const float* partial;
+    float* out;
+    size_t n;
+    unsigned first;
+};
+struct SumTasks {
+    SumTask task[kWeightGradTasks];
+    int n;
+};
+
 template <int S>
-__global__ __launch_bounds__(256) void weight_grad_sum_kernel(const float* __restrict__ partial,
-                                                              float* __restrict__ out, size_t n) {
-    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+__global__ __launch_bounds__(256) void weight_grad_sum_kernel(SumTasks tasks) {
+    int which = 0;
+    for (int k = 1; k < tasks.n; ++k)
+        if (blockIdx.x >= tasks.task[k].first) which = k;
+    const SumTask& task = tasks.task[which];
+    const size_t n = task.n, at = ((size_t)(blockIdx.x - task.first) * 256 + threadIdx.x) * 4;
     if (at >= n) return;
     f32x4 part[S];
 #pragma unroll
-    for (int s = 0; s < S; ++s) part[s] = *reinterpret_cast<const f32x4*>(partial + s * n + at);
+    for (int s = 0; s < S; ++s) part[s] = *reinterpret_cast<const f32x4*>(task.partial + s * n + at);
     f32x4 v = part[0];
 #pragma unroll
     for (int s = 1; s < S; ++s) v += part[s];
-    *reinterpret_cast<f32x4*>(out + at) = v;
+    *reinterpret_cast<f32x4*>(task.out + at) = v;
 }
 
 int launched() { return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH; }
@@ -186,13 +221,21 @@ int launched() { return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAU
 // Workgroups along the rows: one per compute unit in all, eight steps or more each.  With two per compute
 // unit the partial results cost more than it brings (2048 rows, 2048 x 1024: 29.6 against 26.2 us; 4593
 // rows, 1024 x 1024: 32.4 against 27.8), with half of one 28.6 and 34.2.
-constexpr int kWorkgroups = 256, kMinSteps = 8;
-int splits_for(int M, int N, int K) {
-    const int tiles = ceil_div(M, kTile) * ceil_div(N, kTile), steps = ceil_div(K, kKT);
-    int s = kWorkgroups / tiles;
+// Where every workgroup has 24 steps or more left, one split more than fills the chip once is faster: four weights of a
+// layer of 512 at 6144 rows 65.7 against 79.2 us, at 4000 49 against 55 (2048 rows, 16 steps: equal).
+constexpr int kWorkgroups = 256, kMinSteps = 8, kLongSteps = 24;
+int tiles_of(int M, int N) { return ceil_div(M, kTile) * ceil_div(N, kTile); }
+int splits_for(int tiles, int K) {
+    const int steps = ceil_div(K, kKT), more = ceil_div(kWorkgroups, tiles);
+    int s = steps / more >= kLongSteps ? more : kWorkgroups / tiles;
     if (s > steps / kMinSteps) s = steps / kMinSteps;
     if (s > kMaxSplits) s = kMaxSplits;
     return s < 1 ? 1 : s;
+}
+int splits_for(int n, int rows, const int* N, const int* K) {
+    int tiles = 0;
+    for (int k = 0; k < n; ++k) tiles += tiles_of(N[k], K[k]);
+    return splits_for(tiles, rows);
 }
 
 }  // namespace
@@ -204,24 +247,37 @@ bool weight_grad_supported(int rows, int N, int K) {
            (long long)rows * N < (1ll << 30) && (long long)rows * K < (1ll << 30) &&
            (long long)ceil_div(N, kTile) * ceil_div(K, kTile) < (1 << 20);
 }
-size_t weight_grad_workspace_bytes(int rows, int N, int K) {
-    const int s = splits_for(N, K, rows);
-    return s > 1 ? (size_t)s * N * K * sizeof(float) : 0;
+size_t weight_grads_workspace_bytes(int n, int rows, const int* N, const int* K) {
+    const int s = splits_for(n, rows, N, K);
+    size_t values = 0;
+    for (int k = 0; k < n; ++k) values += (size_t)N[k] * K[k];
+    return s > 1 ? (size_t)s * values * sizeof(float) : 0;
 }
-int weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K, void* ws, hipStream_t st) {
-    const int splits = splits_for(N, K, rows);
-    const int ntiles = ceil_div(K, kTile), mtiles = ceil_div(N, kTile);
-    float* out = splits > 1 ? static_cast<float*>(ws) : dw;
-    hipLaunchKernelGGL(weight_grad_kernel, dim3((unsigned)(ceil_div(ntiles * splits, 8) * 8 * mtiles)), dim3(kThreads),
-                       0, st, static_cast<const bf16_t*>(dy), static_cast<const bf16_t*>(x), out, N, K, rows, ntiles,
-                       mtiles, splits);
+int weight_grads(int n, const void* const* dy, const void* const* x, float* const* dw, int rows, const int* N, const int* K,
+                 void* ws, hipStream_t st) {
+    GradTasks tasks;
+    SumTasks sums;
+    tasks.n = sums.n = n;
+    tasks.K = rows;
+    const int splits = tasks.splits = splits_for(n, rows, N, K);
+    unsigned grid = 0, sum_grid = 0;
+    float* partial = static_cast<float*>(ws);
+    for (int k = 0; k < n; ++k) {
+        GradTask& t = tasks.task[k];
+        const size_t values = (size_t)N[k] * K[k];
+        t = {static_cast<const bf16_t*>(dy[k]), static_cast<const bf16_t*>(x[k]), splits > 1 ? partial : dw[k], N[k], K[k],
+             ceil_div(K[k], kTile), ceil_div(N[k], kTile), grid};
+        sums.task[k] = {partial, dw[k], values, sum_grid};
+        grid += (unsigned)(ceil_div(t.ntiles * splits, 8) * 8 * t.mtiles);
+        sum_grid += (unsigned)((values / 4 + 255) / 256);
+        if (splits > 1) partial += splits * values;
+    }
+    hipLaunchKernelGGL(weight_grad_kernel, dim3(grid), dim3(kThreads), 0, st, tasks);
     if (int rc = launched()) return rc;
-    const size_t n = (size_t)N * K;
-    const dim3 grid((unsigned)((n / 4 + 255) / 256));
     switch (splits) {
         case 1: return HAWK_OK;
 #define HAWK_SUM(S) \
-    case S: hipLaunchKernelGGL((weight_grad_sum_kernel<S>), grid, dim3(256), 0, st, out, dw, n); break;
+    case S: hipLaunchKernelGGL((weight_grad_sum_kernel<S>), dim3(sum_grid), dim3(256), 0, st, sums); break;
         HAWK_SUM(2) HAWK_SUM(3) HAWK_SUM(4) HAWK_SUM(5) HAWK_SUM(6) HAWK_SUM(7) HAWK_SUM(8)
 #undef HAWK_SUM
         default: return HAWK_ERR_BAD_SHAPE;

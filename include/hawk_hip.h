@@ -344,6 +344,13 @@ size_t hawk_weight_grad_workspace_bytes(int rows, int N, int K);
 int hawk_weight_grad(const void* dy, const void* x, float* dw, int rows, int N, int K,
                      void* workspace_device, size_t workspace_bytes, void* stream);
 
+/* Up to 8 such products of the same rows in one launch (and one that adds up partial results): dw[k] [N[k], K[k]].
+ * Tiles of several weights fill the chip together, where one weight's alone are too few. */
+size_t hawk_weight_grads_workspace_bytes(int n, int rows, const int* N, const int* K);
+int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float* const* dw, int rows,
+                      const int* N, const int* K, void* workspace_device, size_t workspace_bytes,
+                      void* stream);
+
 /* Dense projections of a decode step: out [M, N] = x [M, K] w^T for up to 256 rows, bf16 with
  * fp32 sums, w [N, K] as torch.nn.Linear keeps it (upstream: the Linear calls of
  * hawk/hawk.py:70-86, :163-203, :284-303 on one token per sequence).  K must be a multiple of

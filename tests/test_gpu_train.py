@@ -260,6 +260,31 @@ def test_weight_gradient(rows, N, K):
     assert torch.equal(train_fused._weight_grad(dy, x), got)
 
 
+@pytest.mark.parametrize("rows,sizes", [(70, [(8, 8), (136, 120), (128, 264)]), (520, [(256, 128), (8, 520), (264, 136), (128, 128)]),
+                                        (3100, [(512, 256), (256, 256), (1024, 256), (256, 512)]), (1, [(264, 8)] * 8)])
+def test_weight_gradients_of_one_launch(rows, sizes):
+    """Several products share a launch's workgroups: every one against 64 bits, one and several splits."""
+    import ctypes
+
+    from hawk_pytorch_amd import _lib
+
+    gen, lib, n = _gen(rows), _lib.load(), len(sizes)
+    dy, x = ([_randn(gen, rows, s[k], dtype=torch.bfloat16) for s in sizes] for k in (0, 1))
+    guard = 64
+    dw = [torch.full((N * K + guard,), float("nan"), device=DEV) for N, K in sizes]
+    Ns, Ks = ((ctypes.c_int * n)(*[s[k] for s in sizes]) for k in (0, 1))
+    nbytes = lib.hawk_weight_grads_workspace_bytes(n, rows, Ns, Ks)
+    ws = torch.full((nbytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])   # noqa: E731
+    train_fused._check("hawk_weight_grads", n, ptrs(dy), ptrs(x), ptrs(dw), rows, Ns, Ks, ws.data_ptr(), nbytes,
+                       _lib.stream_ptr(DEV))
+    for g, a, b, (N, K) in zip(dw, dy, x, sizes):
+        want = a.double().t() @ b.double()
+        _close(g[:N * K].view(N, K), want, (rows + 8) * EPS32 * (a.double().abs().t() @ b.double().abs()))
+        assert bool(g[N * K:].isnan().all())
+    assert bool((ws[nbytes:] == 0xA5).all())
+
+
 @pytest.mark.parametrize("where", ["layers.0", "layers.1.mlp", "layers.0.recc.input_xy", "norm", "lm_head", "embed_tokens"])
 def test_backward_hooks_of_modules_are_called(where):
     """Full backward hooks and backward pre-hooks, on every kind of module a node would stand for."""
