@@ -418,6 +418,21 @@ int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float*
     return hawk::weight_grads(n, dy, x, dw, rows, N, K, workspace_device, as_stream(stream));
 }
 
+int hawk_input_grad_supported(int rows, int N, int K) { return hawk::input_grad_supported(rows, N, K) ? 1 : 0; }
+
+size_t hawk_input_grad_workspace_bytes(int rows, int N, int K) {
+    return hawk::input_grad_supported(rows, N, K) ? hawk::input_grad_workspace_bytes(rows, N, K) : 0;
+}
+
+int hawk_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* workspace_device,
+                    size_t workspace_bytes, void* stream) {
+    if (!dy || !w || !dx) return HAWK_ERR_NULL_POINTER;
+    if (!hawk::input_grad_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(dy) || !aligned16(w) || !aligned16(dx) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    if (!workspace_device || workspace_bytes < hawk::input_grad_workspace_bytes(rows, N, K)) return HAWK_ERR_WORKSPACE;
+    return hawk::input_grad(dy, w, dx, rows, N, K, workspace_device, as_stream(stream));
+}
+
 int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }
 
 size_t hawk_decode_linear_workspace_bytes(int M, int N, int K) {

@@ -61,7 +61,7 @@ constexpr int64_t kStaggerMinBytes = 16 << 20;   // _lib.activation_empty places
     X(hawk_decode_norm_linear) X(hawk_cast) X(hawk_add_norm_fwd) X(hawk_add_norm_bwd)                                 \
     X(hawk_add_norm_bwd_workspace_bytes) X(hawk_gelu_mul_fwd) X(hawk_gelu_mul_bwd) X(hawk_cross_entropy_fwd)          \
     X(hawk_cross_entropy_bwd) X(hawk_embedding_bwd) X(hawk_weight_grads) X(hawk_weight_grad_supported)                \
-    X(hawk_weight_grads_workspace_bytes)
+    X(hawk_weight_grads_workspace_bytes) X(hawk_input_grad) X(hawk_input_grad_supported) X(hawk_input_grad_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     HAWK_FUNCTIONS(X)
@@ -660,11 +660,11 @@ std::tuple<Tensor, std::optional<Tensor>, Tensor> add_norm_bwd(const Tensor& dou
     return {d_sum, d_delta, d_weight};
 }
 
-// dy^T x of [n, N] and [n, K] each: in fp32, those whose result is at most 128 of the kernel's tiles together in one
-// launch; from there on the library's product is as fast or faster, in bf16.  (Alone, against product and conversion, the
-// kernel is ahead up to 512 rows and from 4096 on, and behind between them where the result has more than 32 tiles:
-// 2048 x 1024 at 512 rows 12.2 against 14.7 us, 1024 rows 21.2 against 17.4, 2048 rows 27.3 against 24.2, 4096 rows
-// 39.7 against 39.7.)
+// dy^T x of [n, N] and [n, K] each: in fp32 and together in one launch, but for large results over many rows, where the
+// library's product is faster, in bf16.  The line is at 256 tiles of 128 x 128 and 2048 rows: up to there the kernel was
+// ahead of the library's product and its conversion at every size measured (4096 x 1024 at 6144 rows 66.4 against
+// 70.6 us, 32000 x 512 at 1000 rows 52.0 against 63.5 and at 2048 90.2 against 89.4); beyond it is behind at most
+// (32000 x 512 at 4000 rows 169 against 149, 8192 x 2048 156 against 146, 2560 x 2560 at 6144 110 against 103).
 std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& products) {
     Call c(products[0].first.device());
     const int n = products[0].first.size(0);
@@ -675,7 +675,8 @@ std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& p
     for (size_t k = 0; k < products.size(); ++k) {
         const auto& [g, in] = products[k];
         const int rows = g.size(1), cols = in.size(1);
-        if ((int64_t)((rows + 127) / 128) * ((cols + 127) / 128) > 128 || !lib.hawk_weight_grad_supported(n, rows, cols)) {
+        const bool large = (int64_t)((rows + 127) / 128) * ((cols + 127) / 128) > 256 && n > 2048;
+        if (large || !lib.hawk_weight_grad_supported(n, rows, cols)) {
             out[k] = at::mm(g.t(), in);
             continue;
         }
@@ -690,6 +691,17 @@ std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& p
     return out;
 }
 Tensor weight_grad(const Tensor& dy, const Tensor& x) { return weight_grads({{dy, x}})[0]; }
+
+// dy w of [n, N] and [N, K] for a head: a long sum and few tiles of results.
+Tensor head_input_grad(const Tensor& dy, const Tensor& w) {
+    const int n = dy.size(0), N = w.size(0), K = w.size(1);
+    if (!lib.hawk_input_grad_supported(n, N, K)) return at::mm(dy, w);
+    Call c(dy.device());
+    Tensor dx = c.empty({n, K}, kBF16);
+    const Tensor ws = c.empty({(int64_t)lib.hawk_input_grad_workspace_bytes(n, N, K)}, at::kByte);
+    check("hawk_input_grad", lib.hawk_input_grad(data(dy), data(w), data(dx), n, N, K, data(ws), ws.numel(), c.st));
+    return dx;
+}
 
 Tensor gelu_mul(const Tensor& gu, int rows, int inter) {
     Call c(gu.device());
@@ -785,8 +797,9 @@ std::vector<Tensor> loss_bwd(const std::vector<Tensor>& s, const Tensor& labels,
     check("hawk_cross_entropy_bwd", lib.hawk_cross_entropy_bwd(
         data(logits), data<const long long>(labels), data<float>(s[6]), data<float>(s[7]), data<float>(d_loss),
         data(d_logits), shape[0], shape[1], s[1].size(0), c.st));
-    const Tensor d_x = at::mm(d_logits, s[1]);
-    const Tensor d_head = cast_in(c, {at::mm(d_logits.t(), s[3])}, kF32)[0];
+    const Tensor d_x = head_input_grad(d_logits, s[1]);
+    Tensor d_head = weight_grad(d_logits, s[3]);
+    if (d_head.scalar_type() != kF32) d_head = cast_in(c, {d_head}, kF32)[0];
     auto [d_hidden, d_delta, d_norm] = add_norm_bwd(d_x, s[2], s[4], s[0], std::nullopt, want_delta);
     return {d_hidden.view(shape), d_delta.has_value() ? d_delta->view(shape) : Tensor(), d_norm, d_head};
 }

@@ -1,44 +1,93 @@
-// Weight gradient of a linear layer in a training pass: dw [N, K] = dy^T x, fp32, for dy [n, N] and
-// x [n, K] in bf16 as they lie (the gradient of torch.nn.functional.linear in upstream's modules, which
-// autocast rounds to bf16 and casts back).  Both operands have the sum's index as their row, so 8 x 8 blocks
-// (8 rows of 16 bytes per lane) are turned in registers with 32 byte permutes on their way into LDS, where
-// a matrix operand's lane finds 8 consecutive values of the sum.
+// Products of a training pass whose sum is long for their result (upstream: the autograd of the Linear modules, which
+// autocast runs in bf16):
+//   * weight gradients dw [N, K] = dy^T x, fp32, for dy [n, N] and x [n, K] as they lie, up to eight in one launch;
+//   * the head's input gradient dx [n, K] = dy w, bf16, for w [N, K] with N a vocabulary.
+// Operands whose rows run along the sum are staged as they lie and turned by the transposing LDS reads; all go from
+// memory into LDS without passing through registers, one barrier a step of 64 values.  A workgroup of eight waves
+// (2 x 4, 64 x 32 results each) owns 128 x 128 results; where those are too few for the chip the sum is split over
+// workgroups, and a second kernel adds the fp32 partial results in a fixed order.
 //
-// A workgroup of four waves owns 128 x 128 results, two workgroups share a compute unit; waves 0 and 1 fetch
-// dy, waves 2 and 3 fetch x, two 64-row tiles ahead in registers.  A layer's weights are few tiles
-// (1024 x 512: 32 of them), so a layer's four are one launch, the rows are split over workgroups where that still
-// leaves some of the chip idle, and a second kernel adds the fp32 partial results in a fixed order.  Four weights of a
-// layer of 512 channels over 2048 rows: 33.4 us in one launch, 67.8 in four (with their sums), 94.5 by the library.
-// What that spares next to the library's product is the conversion to fp32, and the chip is not left idle by few
-// tiles: 2048 rows, 512 x 512 13.9 us (library and conversion 17.8), 4593
-// rows, 2048 x 1024 43.3 (50.0), 1024 x 1024 27.8 (38.5).  Between 512 and 4096 rows, where a few steps are split
-// and the sums cost a launch, results of more than 32 tiles take up to a fifth longer than the library's (1024
-// rows, 2048 x 1024: 21.2 against 17.4).  From 128 tiles on the library is as fast or faster (8192 rows, 2560 x
-// 2560: 148 against 123); callers go there.
+// What bounds a step is the 32 KiB that have to reach the compute unit (about 47 bytes per ns with HBM latency, 0.6 us),
+// so tiles that share an operand run beside each other on one XCD.  Four weights of a layer of 512 channels (MLP 1024)
+// over 2048 rows take 26.3 us together and 62.6 one by one; with operands turned in registers by byte permutes they took
+// 33.4 together, by the library, conversions included, 97.  dx of 2048 x 512 over 32000: 94 us (library 201, on 60
+// workgroups), 300 x 512 29 (99), 6144 x 512 291 (317).
 #include "hawk_scan.h"
 
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "hawk_tile.h"
 
 namespace hawk {
 namespace {
 
-constexpr int kThreads = 4 * kWave;
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * kWave;
 constexpr int kTile = 128, kKT = 64;
-constexpr int kRowBytes = kKT * 2;
-constexpr int kOperand = kTile * kRowBytes;      // bytes of one operand's tile
-constexpr int kMaxSplits = 8;
+constexpr int kOperand = kTile * kKT * 2;        // bytes of one operand's tile, and of a step's rows of it
+constexpr int kStage = 2 * kOperand;
+constexpr int kGroupsPerWave = kOperand / 1024 / kWaves;   // loads of 1 KiB per wave, operand and step
+constexpr int kMaxSplits = 8, kMaxInputSplits = 32;
+template <int STAGES>
+constexpr int kProductLds = STAGES * kStage > kTile * kTile * 4 ? STAGES * kStage : kTile * kTile * 4;
 
+// An operand whose rows run along the sum ([64 rows][128 columns], 256 bytes a row) is staged as it lies and read with
+// transposing LDS reads: 16 lanes read 4 rows of 16 columns (32 bytes each) and every lane gets the four values of
+// one column.  The 32-byte pieces of a row are permuted by its number, so that the rows an access covers (4 of them
+// and the 4 that lie 8 further on) fall on different banks.
+__device__ __forceinline__ int sum_row_swizzle(int row) { return (row & 3) | (((row >> 3) & 1) << 2); }
+// Two MFMA operands' worth (16 values of the sum each, 4 KiB apart) from one to three operands.  One block each, with its
+// wait: as a builtin the compiler has every such read wait for all loads into LDS that are in flight.
+__device__ __forceinline__ uint32_t lds_offset(const unsigned char* p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)const_cast<unsigned char*>(p);
+}
+#define HAWK_TR(OUT, AT, OFF) "ds_read_b64_tr_b16 %" #OUT ", %" #AT " offset:" #OFF "\n\t"
+template <int KS>
+__device__ __forceinline__ void read_transposed(uint32_t at, u32x2 (&v)[4]) {
+#if __HIP_DEVICE_COMPILE__
+    static_assert(KS == 0 || KS == 2, "half a step");
+    if constexpr (KS == 0)
+        asm volatile(HAWK_TR(0, 4, 0) HAWK_TR(1, 4, 1024) HAWK_TR(2, 4, 4096) HAWK_TR(3, 4, 5120) "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(at) : "memory");
+    else
+        asm volatile(HAWK_TR(0, 4, 8192) HAWK_TR(1, 4, 9216) HAWK_TR(2, 4, 12288) HAWK_TR(3, 4, 13312) "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(at) : "memory");
+#endif
+}
+template <int KS>
+__device__ __forceinline__ void read_transposed(uint32_t at0, uint32_t at1, uint32_t at2, u32x2 (&x)[4], u32x2 (&y)[4], u32x2 (&z)[4]) {
+#if __HIP_DEVICE_COMPILE__
+    if constexpr (KS == 0)
+        asm volatile(HAWK_TR(0, 12, 0) HAWK_TR(1, 12, 1024) HAWK_TR(4, 13, 0) HAWK_TR(5, 13, 1024) HAWK_TR(8, 14, 0)
+                         HAWK_TR(9, 14, 1024) HAWK_TR(2, 12, 4096) HAWK_TR(3, 12, 5120) HAWK_TR(6, 13, 4096)
+                             HAWK_TR(7, 13, 5120) HAWK_TR(10, 14, 4096) HAWK_TR(11, 14, 5120) "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(y[0]), "=&v"(y[1]), "=&v"(y[2]),
+                       "=&v"(y[3]), "=&v"(z[0]), "=&v"(z[1]), "=&v"(z[2]), "=&v"(z[3])
+                     : "v"(at0), "v"(at1), "v"(at2) : "memory");
+    else
+        asm volatile(HAWK_TR(0, 12, 8192) HAWK_TR(1, 12, 9216) HAWK_TR(4, 13, 8192) HAWK_TR(5, 13, 9216) HAWK_TR(8, 14, 8192)
+                         HAWK_TR(9, 14, 9216) HAWK_TR(2, 12, 12288) HAWK_TR(3, 12, 13312) HAWK_TR(6, 13, 12288)
+                             HAWK_TR(7, 13, 13312) HAWK_TR(10, 14, 12288) HAWK_TR(11, 14, 13312) "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(y[0]), "=&v"(y[1]), "=&v"(y[2]),
+                       "=&v"(y[3]), "=&v"(z[0]), "=&v"(z[1]), "=&v"(z[2]), "=&v"(z[3])
+                     : "v"(at0), "v"(at1), "v"(at2) : "memory");
+#endif
+}
+#undef HAWK_TR
+__device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}); }
+// One whose rows are the result's ([128 rows][64 values of the sum], 128 bytes a row): the 16-byte pieces of a row are
+// permuted by its number.
+__device__ __forceinline__ int piece_offset(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
 
-// 16-byte piece c (8 values along the sum) of row r.  The permutation differs between the 8 rows that one
-// LDS cycle reads and between rows 8 apart, which a transposed operand's lanes write together.
-__device__ __forceinline__ int piece_offset(int r, int c) {
-    return r * kRowBytes + ((c ^ ((r ^ (r >> 3)) & 7)) << 4);
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
-// One product of a launch: out [M, N] (or [splits, M, N]) = a^T b for a [K, M] and b [K, N].  Its workgroups start at
-// first; the launch's tasks share K and the number of splits.
+// One product of a launch: out [M, N] (or [splits, M, N]) = a^T b for a [K, M] and b [K, N], or a b for a [M, K].  Its
+// workgroups start at first; the launch's tasks share K and the number of splits.
 struct GradTask {
     const bf16_t *a, *b;
     float* out;
@@ -50,8 +99,11 @@ struct GradTasks {
     int n, K, splits;
 };
 
-__global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(GradTasks tasks) {
-    __shared__ __align__(16) unsigned char smem[4 * kOperand];
+// A_ROWS: a's rows are the result's ([M, K]; K a multiple of 64); else they run along the sum, as b's do.  Rows past
+// the end of the sum read as zeros (range check), rows and columns past the result repeat others and are not stored.
+template <bool A_ROWS, int STAGES>
+__global__ __launch_bounds__(kThreads, STAGES == 2 ? 4 : 2) void sum_product_kernel(GradTasks tasks) {
+    __shared__ __align__(16) unsigned char smem[kProductLds<STAGES>];
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -66,112 +118,131 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(GradTasks task
     float* const out = task.out;
     const int M = task.M, N = task.N, K = tasks.K, ntiles = task.ntiles, mtiles = task.mtiles, splits = tasks.splits;
 
-    // row tiles of one column tile sit 8 workgroups apart: on one XCD, at about the same time
+    // the tiles along the result's shorter side sit 8 workgroups apart: on one XCD, at about the same time, so that the
+    // longer side's operand comes to one L2
     const int blk = (int)(blockIdx.x - task.first);
-    const int group = blk / (8 * mtiles), in_group = blk - group * 8 * mtiles;
+    const bool rows_inside = mtiles < ntiles;
+    const int inner = min(mtiles, ntiles), outer = max(mtiles, ntiles);
+    const int group = blk / (8 * inner), in_group = blk - group * 8 * inner;
     const int item = group * 8 + (in_group & 7);
-    if (item >= ntiles * splits) return;      // a task's workgroups are padded to whole groups of 8
-    const int split = item / ntiles;
-    const int m0 = in_group / 8 * kTile, n0 = (item - split * ntiles) * kTile;
+    if (item >= outer * splits) return;       // a task's workgroups are padded to whole groups of 8
+    const int split = item / outer, ti = in_group / 8, to = item - split * outer;
+    const int m0 = (rows_inside ? ti : to) * kTile, n0 = (rows_inside ? to : ti) * kTile;
     const int all = (K + kKT - 1) / kKT;
     const int step0 = (int)((long long)all * split / splits), step1 = (int)((long long)all * (split + 1) / splits);
     const int steps = step1 - step0;
 
-    // lane -> (8 columns, 8 rows of a step): 8 loads of 16 bytes, one per row; rows past the last read as
-    // zeros (range check), columns past the last reach results that are not stored
-    const bool second = wv >= 2;
-    const int t = tid & 127;
-    const uint32_t ld = 2u * (uint32_t)(second ? N : M);
-    const size_t start = (size_t)(second ? n0 : m0) * 2u;
-    const rsrc_t src = make_rsrc(reinterpret_cast<const unsigned char*>(second ? b : a) + start,
-                                 (uint32_t)((size_t)K * ld - start));
-    const uint32_t base = (uint32_t)(t / 16) * 8u * ld + (uint32_t)(t & 15) * 16u;
-
-    u32x4 r[2][8];
+    constexpr int L = kGroupsPerWave, S = STAGES;
+    const uint32_t lda = 2u * (uint32_t)(A_ROWS ? K : M), ldb = 2u * (uint32_t)N;
+    const rsrc_t ra = make_rsrc(a, (uint32_t)((size_t)(A_ROWS ? M : K) * lda)), rb = make_rsrc(b, (uint32_t)((size_t)K * ldb));
+    // a load brings 1 KiB of an operand: 4 rows along the sum, or 8 rows of the result
+    auto sum_rows = [&](int l, uint32_t ld, int c0, int columns) {
+        const int row = 4 * (wv + l * kWaves) + (lane >> 4), p = lane & 15;
+        const int c = c0 + 8 * ((((p >> 1) ^ sum_row_swizzle(row)) << 1) | (p & 1));
+        return (uint32_t)row * ld + 2u * (uint32_t)(c < columns ? c : 0);
+    };
+    uint32_t at_a[L], at_b[L];
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+        if constexpr (A_ROWS) {
+            const int row = 8 * (wv + l * kWaves) + (lane >> 3);
+            at_a[l] = (uint32_t)min(m0 + row, M - 1) * lda + (uint32_t)(((lane & 7) ^ (lane >> 3)) << 4);
+        } else {
+            at_a[l] = sum_rows(l, lda, m0, M);
+        }
+        at_b[l] = sum_rows(l, ldb, n0, N);
+    }
     auto load = [&](int slot, int step) {
-        // (steps past the last repeat it; nothing reads them)
-        const uint32_t at = base + (uint32_t)(step0 + min(step, steps - 1)) * kKT * ld;
+        const uint32_t k = (uint32_t)(step0 + step) * kKT;
+        unsigned char* s = smem + slot * kStage + wv * 1024;
 #pragma unroll
-        for (int p = 0; p < 8; ++p) {
-            r[slot][p] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(src, at + p * ld, 0,
-                                                                                         kAuxDefault));
-            __builtin_amdgcn_sched_barrier(0);   // one order here and in front of the loop, or the waits merge
-        }
-    };
-    auto stage = [&](int slot, int buf) {
-        unsigned char* s = smem + buf * 2 * kOperand + (second ? kOperand : 0);
-        const int col = (t & 15) * 8, c = t / 16;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            u32x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[j] = __builtin_amdgcn_perm(r[slot][2 * j + 1][e / 2], r[slot][2 * j][e / 2],
-                                             e % 2 ? 0x07060302u : 0x05040100u);
-            *reinterpret_cast<u32x4*>(s + piece_offset(col + e, c)) = v;
+        for (int l = 0; l < L; ++l) {
+            load_to_lds(ra, s + l * kWaves * 1024, at_a[l] + k * (A_ROWS ? 2u : lda), 0);
+            load_to_lds(rb, s + kOperand + l * kWaves * 1024, at_b[l] + k * ldb, 0);
         }
     };
 
-    f32x16 acc[2][2];
+    f32x16 acc[2];
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) acc[mb][nb][i] = 0.0f;
+        for (int i = 0; i < 16; ++i) acc[mb][i] = 0.0f;
 
-    const int arow = wm * 64 + (lane & 31), brow = wn * 64 + (lane & 31);
-    auto multiply = [&](int buf) {
-        const unsigned char* s = smem + buf * 2 * kOperand;
+    // a lane's operand: column lane % 32, eight values of the sum from 8 (lane / 32) on; the transposing reads take the
+    // address of row (lane % 16) / 4, columns 4 (lane % 4) of 16
+    const int q = lane & 15, swz = (q >> 2) | ((lane >> 5) << 2);
+    auto transposed_at = [&](int c0) {
+        return (8 * (lane >> 5) + (q >> 2)) * 256 + ((((c0 >> 4) + ((lane >> 4) & 1)) ^ swz) << 5) + (q & 3) * 8;
+    };
+    const int b_at = kOperand + transposed_at(wn * 32);
+    int a_at[2];
 #pragma unroll
-        for (int ks = 0; ks < kKT / 16; ++ks) {
-            bf16x8 fa[2], fb[2];
+    for (int mb = 0; mb < 2; ++mb) a_at[mb] = A_ROWS ? wm * 64 + mb * 32 + (lane & 31) : transposed_at(wm * 64 + mb * 32);
+    auto half = [&](auto first, const unsigned char* s) {
+        constexpr int KS = decltype(first)::value;
+        u32x2 b4[4], a0[4], a1[4];
+        bf16x8 fa[2][2];
+        if constexpr (A_ROWS) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                fa[q] = *reinterpret_cast<const bf16x8*>(s + piece_offset(arow + 32 * q, 2 * ks + (lane >> 5)));
-                fb[q] = *reinterpret_cast<const bf16x8*>(s + kOperand + piece_offset(brow + 32 * q, 2 * ks + (lane >> 5)));
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int mb = 0; mb < 2; ++mb)
+                    fa[k][mb] = *reinterpret_cast<const bf16x8*>(s + piece_offset(a_at[mb], 2 * (KS + k) + (lane >> 5)));
+            read_transposed<KS>(lds_offset(s + b_at), b4);
+        } else {
+            read_transposed<KS>(lds_offset(s + b_at), lds_offset(s + a_at[0]), lds_offset(s + a_at[1]), b4, a0, a1);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                fa[k][0] = operand(a0[2 * k], a0[2 * k + 1]);
+                fa[k][1] = operand(a1[2 * k], a1[2 * k + 1]);
             }
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
 #pragma unroll
             for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-                for (int nb = 0; nb < 2; ++nb)
-                    acc[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[nb], fa[mb], acc[mb][nb], 0, 0, 0);
-        }
+                acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(operand(b4[2 * k], b4[2 * k + 1]), fa[k][mb], acc[mb], 0, 0, 0);
     };
-    load(0, 0);
-    load(1, 1);
-    stage(0, 0);
-    load(0, 2);
+    auto multiply = [&](int slot) {
+        const unsigned char* s = smem + slot * kStage;
+        half(std::integral_constant<int, 0>{}, s);
+        half(std::integral_constant<int, 2>{}, s);
+    };
+
+    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
+    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
+#pragma unroll
+    for (int d = 0; d < S - 1; ++d)
+        if (d < steps) load(d, d);
+    int i = 0, slot = 0;
+    for (; i + S - 1 < steps; ++i) {
+        wait_loads<(S - 2) * 2 * L>();
+        lds_barrier();
+        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    for (; i < steps; ++i) {
+        switch (steps - 1 - i) {
+            case 0: wait_loads<0>(); break;
+            case 1: wait_loads<2 * L>(); break;
+            default: wait_loads<4 * L>(); break;       // (no more than S - 2 = 2)
+        }
+        lds_barrier();
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
     lds_barrier();
-    int i = 0;
-    for (; i + 2 <= steps; i += 2) {
-        stage(1, 1);
-        load(1, i + 3);
-        multiply(0);
-        lds_barrier();
-        stage(0, 0);
-        load(0, i + 4);
-        multiply(1);
-        lds_barrier();
-    }
-    if (i < steps) {
-        multiply(0);
-        lds_barrier();
-    }
 
     // the tile through LDS, [128 rows][32 pieces of 4 columns], so that it leaves in whole rows
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int row = wm * 64 + mb * 32 + (lane & 31);
-                const int c = wn * 16 + nb * 8 + 2 * g + (lane >> 5);
-                const f32x4 v = {acc[mb][nb][4 * g], acc[mb][nb][4 * g + 1], acc[mb][nb][4 * g + 2],
-                                 acc[mb][nb][4 * g + 3]};
-                *reinterpret_cast<f32x4*>(smem + (row * 32 + (c ^ (row & 7))) * 16) = v;
-            }
+        for (int g = 0; g < 4; ++g) {
+            const int row = wm * 64 + mb * 32 + (lane & 31), c = wn * 8 + 2 * g + (lane >> 5);
+            const f32x4 v = {acc[mb][4 * g], acc[mb][4 * g + 1], acc[mb][4 * g + 2], acc[mb][4 * g + 3]};
+            *reinterpret_cast<f32x4*>(smem + (row * 32 + (c ^ (row & 7))) * 16) = v;
+        }
     lds_barrier();
     const int ec = tid & 15, n = n0 + 8 * ec;
 #pragma unroll
@@ -190,7 +261,7 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(GradTasks task
 // The partial results of a launch's tasks added up, 1024 values of one task per workgroup.
 struct SumTask {
     const float* partial;
-    float* out;
+    void* out;
     size_t n;
     unsigned first;
 };
@@ -199,8 +270,8 @@ struct SumTasks {
     int n;
 };
 
-template <int S>
-__global__ __launch_bounds__(256) void weight_grad_sum_kernel(SumTasks tasks) {
+template <int S, bool TO_BF16>
+__global__ __launch_bounds__(256) void sum_partial_kernel(SumTasks tasks) {
     int which = 0;
     for (int k = 1; k < tasks.n; ++k)
         if (blockIdx.x >= tasks.task[k].first) which = k;
@@ -213,7 +284,8 @@ __global__ __launch_bounds__(256) void weight_grad_sum_kernel(SumTasks tasks) {
     f32x4 v = part[0];
 #pragma unroll
     for (int s = 1; s < S; ++s) v += part[s];
-    *reinterpret_cast<f32x4*>(task.out + at) = v;
+    if constexpr (TO_BF16) *reinterpret_cast<u32x2*>(static_cast<bf16_t*>(task.out) + at) = u32x2{pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w)};
+    else *reinterpret_cast<f32x4*>(static_cast<float*>(task.out) + at) = v;
 }
 
 int launched() { return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH; }
@@ -232,6 +304,29 @@ int splits_for(int tiles, int K) {
     if (s > kMaxSplits) s = kMaxSplits;
     return s < 1 ? 1 : s;
 }
+unsigned workgroups_of(const GradTask& t, int splits) {
+    const int inner = t.mtiles < t.ntiles ? t.mtiles : t.ntiles, outer = t.mtiles + t.ntiles - inner;
+    return (unsigned)(ceil_div(outer * splits, 8) * 8 * inner);
+}
+template <bool A_ROWS>
+int launch_products(const GradTasks& tasks, unsigned grid, hipStream_t st) {
+    // four tiles of steps in flight where no compute unit has a second workgroup, else two and two workgroups
+    if (grid <= kWorkgroups) hipLaunchKernelGGL((sum_product_kernel<A_ROWS, 4>), dim3(grid), dim3(kThreads), 0, st, tasks);
+    else hipLaunchKernelGGL((sum_product_kernel<A_ROWS, 2>), dim3(grid), dim3(kThreads), 0, st, tasks);
+    return launched();
+}
+template <bool TO_BF16>
+int launch_sums(const SumTasks& sums, int splits, unsigned grid, hipStream_t st) {
+    switch (splits) {
+#define HAWK_SUM(S) \
+    case S: hipLaunchKernelGGL((sum_partial_kernel<S, TO_BF16>), dim3(grid), dim3(256), 0, st, sums); break;
+        HAWK_SUM(2) HAWK_SUM(3) HAWK_SUM(4) HAWK_SUM(5) HAWK_SUM(6) HAWK_SUM(7) HAWK_SUM(8) HAWK_SUM(16) HAWK_SUM(32)
+#undef HAWK_SUM
+        default: return HAWK_ERR_BAD_SHAPE;
+    }
+    return launched();
+}
+
 int splits_for(int n, int rows, const int* N, const int* K) {
     int tiles = 0;
     for (int k = 0; k < n; ++k) tiles += tiles_of(N[k], K[k]);
@@ -268,21 +363,44 @@ int weight_grads(int n, const void* const* dy, const void* const* x, float* cons
         t = {static_cast<const bf16_t*>(dy[k]), static_cast<const bf16_t*>(x[k]), splits > 1 ? partial : dw[k], N[k], K[k],
              ceil_div(K[k], kTile), ceil_div(N[k], kTile), grid};
         sums.task[k] = {partial, dw[k], values, sum_grid};
-        grid += (unsigned)(ceil_div(t.ntiles * splits, 8) * 8 * t.mtiles);
+        grid += workgroups_of(t, splits);
         sum_grid += (unsigned)((values / 4 + 255) / 256);
         if (splits > 1) partial += splits * values;
     }
-    hipLaunchKernelGGL(weight_grad_kernel, dim3(grid), dim3(kThreads), 0, st, tasks);
-    if (int rc = launched()) return rc;
-    switch (splits) {
-        case 1: return HAWK_OK;
-#define HAWK_SUM(S) \
-    case S: hipLaunchKernelGGL((weight_grad_sum_kernel<S>), dim3(sum_grid), dim3(256), 0, st, sums); break;
-        HAWK_SUM(2) HAWK_SUM(3) HAWK_SUM(4) HAWK_SUM(5) HAWK_SUM(6) HAWK_SUM(7) HAWK_SUM(8)
-#undef HAWK_SUM
-        default: return HAWK_ERR_BAD_SHAPE;
-    }
-    return launched();
+    if (int rc = launch_products<false>(tasks, grid, st)) return rc;
+    return splits > 1 ? launch_sums<false>(sums, splits, sum_grid, st) : HAWK_OK;
+}
+
+
+namespace {
+// Splits of the sum of an input gradient: one workgroup per compute unit, eight steps or more each.
+int input_splits_for(int rows, int N, int K) {
+    const int tiles = tiles_of(rows, K), steps = N / kKT;
+    int s = ceil_div(kWorkgroups, tiles);
+    if (s > steps / kMinSteps) s = steps / kMinSteps;
+    if (s > 8) s = s >= kMaxInputSplits ? kMaxInputSplits : (s >= 16 ? 16 : 8);
+    return s;
+}
+}  // namespace
+
+bool input_grad_supported(int rows, int N, int K) {
+    return rows >= 1 && N >= kKT && N % kKT == 0 && K >= 8 && K % 8 == 0 && N < (1 << 25) && K < (1 << 25) &&
+           (long long)rows * N < (1ll << 30) && (long long)N * K < (1ll << 30) && input_splits_for(rows, N, K) >= 2;
+}
+size_t input_grad_workspace_bytes(int rows, int N, int K) { return (size_t)input_splits_for(rows, N, K) * rows * K * sizeof(float); }
+int input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* ws, hipStream_t st) {
+    const int splits = input_splits_for(rows, N, K);
+    GradTasks tasks;
+    tasks.n = 1, tasks.K = N, tasks.splits = splits;
+    GradTask& t = tasks.task[0];
+    t = {static_cast<const bf16_t*>(dy), static_cast<const bf16_t*>(w), static_cast<float*>(ws), rows, K, ceil_div(K, kTile),
+         ceil_div(rows, kTile), 0};
+    if (int rc = launch_products<true>(tasks, workgroups_of(t, splits), st)) return rc;
+    const size_t values = (size_t)rows * K;
+    SumTasks sums;
+    sums.n = 1;
+    sums.task[0] = {static_cast<const float*>(ws), dx, values, 0};
+    return launch_sums<true>(sums, splits, (unsigned)((values / 4 + 255) / 256), st);
 }
 
 }  // namespace hawk

@@ -351,6 +351,16 @@ int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float*
                       const int* N, const int* K, void* workspace_device, size_t workspace_bytes,
                       void* stream);
 
+/* dx [rows, K] bf16 = dy w for dy [rows, N] and w [N, K] bf16: the input gradient of a linear layer whose sum
+ * over N is long and whose result is few tiles (a head over a vocabulary), summed in fp32 in a fixed order.
+ * Dense and 16-byte aligned, N a multiple of 64, K of 8, both below 2^25, rows * N and N * K below 2^30; results
+ * of so many tiles of 128 x 128 that the sum would not be split (256 and more) are not served.  The workspace
+ * takes the partial sums. */
+int hawk_input_grad_supported(int rows, int N, int K);
+size_t hawk_input_grad_workspace_bytes(int rows, int N, int K);
+int hawk_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* workspace_device,
+                    size_t workspace_bytes, void* stream);
+
 /* Dense projections of a decode step: out [M, N] = x [M, K] w^T for up to 256 rows, bf16 with
  * fp32 sums, w [N, K] as torch.nn.Linear keeps it (upstream: the Linear calls of
  * hawk/hawk.py:70-86, :163-203, :284-303 on one token per sequence).  K must be a multiple of

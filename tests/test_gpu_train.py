@@ -285,6 +285,33 @@ def test_weight_gradients_of_one_launch(rows, sizes):
     assert bool((ws[nbytes:] == 0xA5).all())
 
 
+# one row, ragged rows and columns, one to 32 splits, more and fewer column than row tiles
+@pytest.mark.parametrize("rows,N,K", [(1, 1024, 8), (77, 2048, 136), (300, 4096, 264), (130, 1600, 2048), (1030, 1088, 520),
+                                      (129, 32000, 256)])
+def test_input_gradient_of_a_head(rows, N, K):
+    from hawk_pytorch_amd import _lib
+
+    gen, lib, guard = _gen(rows), _lib.load(), 64
+    dy, w = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, N, K, dtype=torch.bfloat16)
+    dx = torch.full((rows * K + guard,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    assert lib.hawk_input_grad_supported(rows, N, K)
+    nbytes = lib.hawk_input_grad_workspace_bytes(rows, N, K)
+    ws = torch.full((nbytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
+    train_fused._check("hawk_input_grad", dy.data_ptr(), w.data_ptr(), dx.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
+                       _lib.stream_ptr(DEV))
+    want = dy.double() @ w.double()
+    # fp32 sums of exact products, rounded once to bf16
+    _close(dx[:rows * K].view(rows, K), want, (N + 8) * EPS32 * (dy.double().abs() @ w.double().abs()) + 2.0 ** -8 * want.abs())
+    assert bool(dx[rows * K:].isnan().all()) and bool((ws[nbytes:] == 0xA5).all())
+    # a NaN in one row reaches that row alone
+    dy[0, 5] = float("nan")
+    train_fused._check("hawk_input_grad", dy.data_ptr(), w.data_ptr(), dx.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
+                       _lib.stream_ptr(DEV))
+    out = dx[:rows * K].view(rows, K)
+    assert bool(out[0].isnan().all()) and not bool(out[1:].isnan().any())
+    assert not lib.hawk_input_grad_supported(rows, N + 8, K) and not lib.hawk_input_grad_supported(rows, N, K + 1)
+
+
 @pytest.mark.parametrize("where", ["layers.0", "layers.1.mlp", "layers.0.recc.input_xy", "norm", "lm_head", "embed_tokens"])
 def test_backward_hooks_of_modules_are_called(where):
     """Full backward hooks and backward pre-hooks, on every kind of module a node would stand for."""
