@@ -107,6 +107,9 @@ SIGNATURES = {
         _c_int, [_c_int] + [ctypes.POINTER(_c_void_p)] * 3 + [_c_int] + [ctypes.POINTER(_c_int)] * 2
         + [_c_void_p, _c_size_t, _c_void_p]
     ),
+    "hawk_linear_supported": (_c_int, [_c_int] * 3),
+    "hawk_linear_workspace_bytes": (_c_size_t, [_c_int] * 3),
+    "hawk_linear_fwd": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),
     "hawk_input_grad_supported": (_c_int, [_c_int] * 3),
     "hawk_input_grad_workspace_bytes": (_c_size_t, [_c_int] * 3),
     "hawk_input_grad": (_c_int, [_c_void_p] * 3 + [_c_int] * 3 + [_c_void_p, _c_size_t, _c_void_p]),

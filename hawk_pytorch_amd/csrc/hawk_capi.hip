@@ -418,19 +418,34 @@ int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float*
     return hawk::weight_grads(n, dy, x, dw, rows, N, K, workspace_device, as_stream(stream));
 }
 
-int hawk_input_grad_supported(int rows, int N, int K) { return hawk::input_grad_supported(rows, N, K) ? 1 : 0; }
+int hawk_linear_supported(int rows, int N, int K) { return hawk::linear_supported(rows, N, K) ? 1 : 0; }
 
-size_t hawk_input_grad_workspace_bytes(int rows, int N, int K) {
-    return hawk::input_grad_supported(rows, N, K) ? hawk::input_grad_workspace_bytes(rows, N, K) : 0;
+size_t hawk_linear_workspace_bytes(int rows, int N, int K) {
+    return hawk::linear_supported(rows, N, K) ? hawk::linear_workspace_bytes(rows, N, K) : 0;
 }
+
+int hawk_linear_fwd(const void* x, const void* w, void* out, int rows, int N, int K, void* workspace_device,
+                    size_t workspace_bytes, void* stream) {
+    if (!x || !w || !out) return HAWK_ERR_NULL_POINTER;
+    if (!hawk::linear_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
+    if (!aligned16(x) || !aligned16(w) || !aligned16(out) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
+    const size_t need = hawk::linear_workspace_bytes(rows, N, K);
+    if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;
+    return hawk::linear_fwd(x, w, out, rows, N, K, workspace_device, as_stream(stream));
+}
+
+int hawk_input_grad_supported(int rows, int N, int K) { return hawk::linear_supported(rows, K, N) ? 1 : 0; }
+
+size_t hawk_input_grad_workspace_bytes(int rows, int N, int K) { return hawk_linear_workspace_bytes(rows, K, N); }
 
 int hawk_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* workspace_device,
                     size_t workspace_bytes, void* stream) {
     if (!dy || !w || !dx) return HAWK_ERR_NULL_POINTER;
-    if (!hawk::input_grad_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
+    if (!hawk::linear_supported(rows, K, N)) return HAWK_ERR_BAD_SHAPE;
     if (!aligned16(dy) || !aligned16(w) || !aligned16(dx) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
-    if (!workspace_device || workspace_bytes < hawk::input_grad_workspace_bytes(rows, N, K)) return HAWK_ERR_WORKSPACE;
-    return hawk::input_grad(dy, w, dx, rows, N, K, workspace_device, as_stream(stream));
+    const size_t need = hawk::linear_workspace_bytes(rows, K, N);
+    if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;
+    return hawk::linear_input_grad(dy, w, dx, rows, N, K, workspace_device, as_stream(stream));
 }
 
 int hawk_decode_linear_supported(int M, int N, int K) { return hawk::decode_linear_supported(M, N, K) ? 1 : 0; }

@@ -143,9 +143,11 @@ size_t weight_grads_workspace_bytes(int n, int rows, const int* N, const int* K)
 int weight_grads(int n, const void* const* dy, const void* const* x, float* const* dw, int rows, const int* N, const int* K,
                  void* ws, hipStream_t st);
 
-bool input_grad_supported(int rows, int N, int K);
-size_t input_grad_workspace_bytes(int rows, int N, int K);
-int input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* ws, hipStream_t st);
+// x w^T and dy w of a linear layer, [rows, N] over K; the input gradient's sum is the layer's N
+bool linear_supported(int rows, int N, int K);
+size_t linear_workspace_bytes(int rows, int N, int K);
+int linear_fwd(const void* x, const void* w, void* out, int rows, int N, int K, void* ws, hipStream_t st);
+int linear_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* ws, hipStream_t st);
 
 // hawk_probe.hip
 bool stream_probe_shape_ok(size_t bytes, size_t row_pitch, int shape);

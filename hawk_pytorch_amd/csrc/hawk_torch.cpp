@@ -61,7 +61,8 @@ constexpr int64_t kStaggerMinBytes = 16 << 20;   // _lib.activation_empty places
     X(hawk_decode_norm_linear) X(hawk_cast) X(hawk_add_norm_fwd) X(hawk_add_norm_bwd)                                 \
     X(hawk_add_norm_bwd_workspace_bytes) X(hawk_gelu_mul_fwd) X(hawk_gelu_mul_bwd) X(hawk_cross_entropy_fwd)          \
     X(hawk_cross_entropy_bwd) X(hawk_embedding_bwd) X(hawk_weight_grads) X(hawk_weight_grad_supported)                \
-    X(hawk_weight_grads_workspace_bytes) X(hawk_input_grad) X(hawk_input_grad_supported) X(hawk_input_grad_workspace_bytes)
+    X(hawk_weight_grads_workspace_bytes) X(hawk_linear_supported) X(hawk_linear_workspace_bytes)           \
+    X(hawk_linear_fwd) X(hawk_input_grad) X(hawk_input_grad_workspace_bytes)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     HAWK_FUNCTIONS(X)
@@ -692,14 +693,32 @@ std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& p
 }
 Tensor weight_grad(const Tensor& dy, const Tensor& x) { return weight_grads({{dy, x}})[0]; }
 
-// dy w of [n, N] and [N, K] for a head: a long sum and few tiles of results.
-Tensor head_input_grad(const Tensor& dy, const Tensor& w) {
+// x w^T of [n, K] and [N, K], and dy w of [n, N] and [N, K]: by own kernels up to 256 tiles of 128 x 128 of results.
+// There they are ahead of the library's (2048 rows, layers of 512: 6.6, 5.0, 9.3 and 7.0 us against 7.6, 6.3, 10.0 and 7.8,
+// input gradients 7.5, 5.3, 11.9 and 6.9 against 9.3, 7.5, 13.7 and 9.3; a head's over 32000 94 against 201) or, near the
+// line and at a hundred rows of a long sum, within a tenth and 4 us of them, and their launch costs the host 4 us
+// instead of 17; beyond it the library's larger tiles win (4096 x 1024 over 4000 rows 30 against 49).
+bool own_product(int64_t rows, int64_t columns, int64_t sum) {
+    return ((rows + 127) / 128) * ((columns + 127) / 128) <= 256 && lib.hawk_linear_supported(rows, columns, sum);
+}
+Tensor layer_linear(const Tensor& x, const Tensor& w) {
+    const int n = x.size(0), N = w.size(0), K = w.size(1);
+    if (!own_product(n, N, K)) return at::mm(x, w.t());
+    Call c(x.device());
+    Tensor out = c.empty({n, N}, kBF16);
+    const size_t bytes = lib.hawk_linear_workspace_bytes(n, N, K);
+    const Tensor ws = bytes > 0 ? c.empty({(int64_t)bytes}, at::kByte) : Tensor();
+    check("hawk_linear_fwd", lib.hawk_linear_fwd(data(x), data(w), data(out), n, N, K, data_or_null(ws), bytes, c.st));
+    return out;
+}
+Tensor input_grad(const Tensor& dy, const Tensor& w) {
     const int n = dy.size(0), N = w.size(0), K = w.size(1);
-    if (!lib.hawk_input_grad_supported(n, N, K)) return at::mm(dy, w);
+    if (!own_product(n, K, N)) return at::mm(dy, w);
     Call c(dy.device());
     Tensor dx = c.empty({n, K}, kBF16);
-    const Tensor ws = c.empty({(int64_t)lib.hawk_input_grad_workspace_bytes(n, N, K)}, at::kByte);
-    check("hawk_input_grad", lib.hawk_input_grad(data(dy), data(w), data(dx), n, N, K, data(ws), ws.numel(), c.st));
+    const size_t bytes = lib.hawk_input_grad_workspace_bytes(n, N, K);
+    const Tensor ws = bytes > 0 ? c.empty({(int64_t)bytes}, at::kByte) : Tensor();
+    check("hawk_input_grad", lib.hawk_input_grad(data(dy), data(w), data(dx), n, N, K, data_or_null(ws), bytes, c.st));
     return dx;
 }
 
@@ -721,13 +740,13 @@ std::vector<Tensor> layer_fwd(const Tensor& hidden, const std::optional<Tensor>&
     std::optional<Tensor> d;
     if (delta.has_value()) d = delta->view({rows, H});
     auto [total1, x1, rstd1] = add_norm(hidden.view({rows, H}), d, p[0], eps1);
-    const Tensor xy = at::mm(x1, w16[0].t()).view({B, T, 2 * R});
+    const Tensor xy = layer_linear(x1, w16[0]).view({B, T, 2 * R});
     auto [gated, u, xg, ag, h, last] = core_fwd(xy, p[6], p[7], p[8], p[9], p[10], p[11], p[12], want_h, false);
-    const Tensor mixed = at::mm(gated.view({rows, R}), w16[1].t());
+    const Tensor mixed = layer_linear(gated.view({rows, R}), w16[1]);
     auto [total2, x2, rstd2] = add_norm(total1, mixed, p[1], eps2);
-    const Tensor gu = at::mm(x2, w16[2].t());
+    const Tensor gu = layer_linear(x2, w16[2]);
     const Tensor act = gelu_mul(gu, rows, inter);
-    const Tensor out = at::mm(act, w16[3].t());
+    const Tensor out = layer_linear(act, w16[3]);
     return {total2.view({B, T, H}), out.view({B, T, H}), w16[0], w16[1], w16[2], w16[3], total1, x1, rstd1, xy, u, xg, ag, h,
             gated, total2, x2, rstd2, gu, act};
 }
@@ -744,15 +763,15 @@ std::vector<Tensor> layer_bwd(const std::vector<Tensor>& s, const Tensor& d_tota
     const int64_t B = xy.size(0), T = xy.size(1), rows = B * T, H = total1.size(1), R = gated.size(2), inter = act.size(1);
     auto as = [&](const Tensor& t, at::ScalarType type) { return dense16(t.scalar_type() == type ? t : t.to(type)).view({rows, H}); };
     const Tensor d_total = as(d_total_, kF32), d_out = as(d_out_, kBF16);
-    const Tensor d_act = at::mm(d_out, w_dn);
+    const Tensor d_act = input_grad(d_out, w_dn);
     const Tensor d_gu = c.empty(gu.sizes(), kBF16);
     check("hawk_gelu_mul_bwd", lib.hawk_gelu_mul_bwd(data(gu), data(d_act), data(d_gu), rows, inter, c.st));
-    const Tensor d_x2 = at::mm(d_gu, w_gu);
+    const Tensor d_x2 = input_grad(d_gu, w_gu);
     auto [d_total1, d_mixed, g_n2] = add_norm_bwd(d_x2, total2, rstd2, n2, d_total, true);
-    const Tensor d_gated = at::mm(*d_mixed, w_out);
+    const Tensor d_gated = input_grad(*d_mixed, w_out);
     auto [d_xy_, dcw, dcb, dwi, dbi, dwa, dba, dlam] = core_bwd(xy, u, xg, ag, h, cw, wi, wa, lam, d_gated.view({B, T, R}));
     const Tensor d_xy = d_xy_.view({rows, 2 * R});
-    const Tensor d_x1 = at::mm(d_xy, w_in);
+    const Tensor d_x1 = input_grad(d_xy, w_in);
     // (all four at the end: each alone is too few tiles for the chip)
     std::vector<Tensor> g = weight_grads({{d_gu, x2}, {d_out, act}, {d_xy, x1}, {*d_mixed, gated.view({rows, R})}});
     auto [d_hidden, d_delta, g_n1] = add_norm_bwd(d_x1, total1, rstd1, n1, d_total1, want_delta);
@@ -780,7 +799,7 @@ std::vector<Tensor> loss_fwd(const Tensor& hidden, const std::optional<Tensor>& 
     if (delta.has_value()) d = delta->view({rows, H});
     auto [total, x, rstd] = add_norm(hidden.view({rows, H}), d, norm, eps);
     // (every row: the last of a sequence is left out of the loss, not cut out of the tensor)
-    const Tensor logits = at::mm(x, head16.t());
+    const Tensor logits = layer_linear(x, head16);
     const Tensor lse = c.empty({rows}, kF32), each = c.empty({rows}, kF32), mean = c.empty({2}, kF32);
     check("hawk_cross_entropy_fwd", lib.hawk_cross_entropy_fwd(
         data(logits), data<const long long>(labels), data<float>(lse), data<float>(each), data<float>(mean), B, T, V, c.st));
@@ -797,7 +816,7 @@ std::vector<Tensor> loss_bwd(const std::vector<Tensor>& s, const Tensor& labels,
     check("hawk_cross_entropy_bwd", lib.hawk_cross_entropy_bwd(
         data(logits), data<const long long>(labels), data<float>(s[6]), data<float>(s[7]), data<float>(d_loss),
         data(d_logits), shape[0], shape[1], s[1].size(0), c.st));
-    const Tensor d_x = head_input_grad(d_logits, s[1]);
+    const Tensor d_x = input_grad(d_logits, s[1]);
     Tensor d_head = weight_grad(d_logits, s[3]);
     if (d_head.scalar_type() != kF32) d_head = cast_in(c, {d_head}, kF32)[0];
     auto [d_hidden, d_delta, d_norm] = add_norm_bwd(d_x, s[2], s[4], s[0], std::nullopt, want_delta);

@@ -351,11 +351,15 @@ int hawk_weight_grads(int n, const void* const* dy, const void* const* x, float*
                       const int* N, const int* K, void* workspace_device, size_t workspace_bytes,
                       void* stream);
 
-/* dx [rows, K] bf16 = dy w for dy [rows, N] and w [N, K] bf16: the input gradient of a linear layer whose sum
- * over N is long and whose result is few tiles (a head over a vocabulary), summed in fp32 in a fixed order.
- * Dense and 16-byte aligned, N a multiple of 64, K of 8, both below 2^25, rows * N and N * K below 2^30; results
- * of so many tiles of 128 x 128 that the sum would not be split (256 and more) are not served.  The workspace
- * takes the partial sums. */
+/* A linear layer over any number of rows, bf16 with fp32 sums in a fixed order: out [rows, N] = x w^T for
+ * x [rows, K] and w [N, K], and dx [rows, K] = dy w for dy [rows, N].  Dense and 16-byte aligned; the sum (K, and
+ * N for dx) a multiple of 64 and the result's columns of 8, below 2^25, products of two of the sizes below 2^30.
+ * The workspace (NULL where the query says 0) holds partial sums: long sums of few tiles of results, as a head's
+ * input gradient is, are split over workgroups. */
+int hawk_linear_supported(int rows, int N, int K);
+size_t hawk_linear_workspace_bytes(int rows, int N, int K);
+int hawk_linear_fwd(const void* x, const void* w, void* out, int rows, int N, int K, void* workspace_device,
+                    size_t workspace_bytes, void* stream);
 int hawk_input_grad_supported(int rows, int N, int K);
 size_t hawk_input_grad_workspace_bytes(int rows, int N, int K);
 int hawk_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* workspace_device,

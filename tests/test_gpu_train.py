@@ -285,31 +285,40 @@ def test_weight_gradients_of_one_launch(rows, sizes):
     assert bool((ws[nbytes:] == 0xA5).all())
 
 
-# one row, ragged rows and columns, one to 32 splits, more and fewer column than row tiles
-@pytest.mark.parametrize("rows,N,K", [(1, 1024, 8), (77, 2048, 136), (300, 4096, 264), (130, 1600, 2048), (1030, 1088, 520),
-                                      (129, 32000, 256)])
-def test_input_gradient_of_a_head(rows, N, K):
+# the result's rows and columns, the sum's length: one row, ragged tiles of 64 and of 128, one step and several, two to
+# 32 splits, more and fewer column than row tiles, more workgroups than compute units
+@pytest.mark.parametrize("rows,columns,k", [(1, 8, 64), (64, 64, 128), (65, 72, 192), (300, 264, 640), (1030, 520, 1088),
+                                            (2048, 1032, 64), (1, 8, 1024), (77, 136, 2048), (300, 264, 4096), (129, 256, 32000),
+                                            (8200, 520, 128), (130, 2048, 1600)])
+@pytest.mark.parametrize("which", ["fwd", "input_grad"])
+def test_products_of_a_linear_layer(which, rows, columns, k):
     from hawk_pytorch_amd import _lib
 
     gen, lib, guard = _gen(rows), _lib.load(), 64
-    dy, w = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, N, K, dtype=torch.bfloat16)
-    dx = torch.full((rows * K + guard,), float("nan"), device=DEV, dtype=torch.bfloat16)
-    assert lib.hawk_input_grad_supported(rows, N, K)
-    nbytes = lib.hawk_input_grad_workspace_bytes(rows, N, K)
+    a = _randn(gen, rows, k, dtype=torch.bfloat16)
+    w = _randn(gen, *((columns, k) if which == "fwd" else (k, columns)), dtype=torch.bfloat16)
+    b = w.t() if which == "fwd" else w
+    N, K = w.shape
+    out = torch.full((rows * columns + guard,), float("nan"), device=DEV, dtype=torch.bfloat16)
+    name, query = ("hawk_linear_fwd", "hawk_linear") if which == "fwd" else ("hawk_input_grad", "hawk_input_grad")
+    assert getattr(lib, query + "_supported")(rows, N, K)
+    nbytes = getattr(lib, query + "_workspace_bytes")(rows, N, K)
     ws = torch.full((nbytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
-    train_fused._check("hawk_input_grad", dy.data_ptr(), w.data_ptr(), dx.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
-                       _lib.stream_ptr(DEV))
-    want = dy.double() @ w.double()
+
+    def run():
+        train_fused._check(name, a.data_ptr(), w.data_ptr(), out.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
+                           _lib.stream_ptr(DEV))
+        return out[:rows * columns].view(rows, columns)
+
+    want = a.double() @ b.double()
     # fp32 sums of exact products, rounded once to bf16
-    _close(dx[:rows * K].view(rows, K), want, (N + 8) * EPS32 * (dy.double().abs() @ w.double().abs()) + 2.0 ** -8 * want.abs())
-    assert bool(dx[rows * K:].isnan().all()) and bool((ws[nbytes:] == 0xA5).all())
-    # a NaN in one row reaches that row alone
-    dy[0, 5] = float("nan")
-    train_fused._check("hawk_input_grad", dy.data_ptr(), w.data_ptr(), dx.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
-                       _lib.stream_ptr(DEV))
-    out = dx[:rows * K].view(rows, K)
-    assert bool(out[0].isnan().all()) and not bool(out[1:].isnan().any())
-    assert not lib.hawk_input_grad_supported(rows, N + 8, K) and not lib.hawk_input_grad_supported(rows, N, K + 1)
+    _close(run(), want, (k + 8) * EPS32 * (a.double().abs() @ b.double().abs()) + 2.0 ** -8 * want.abs())
+    assert bool(out[rows * columns:].isnan().all()) and bool((ws[nbytes:] == 0xA5).all())
+    a[0, 5] = float("nan")              # a NaN in one row reaches that row alone
+    got = run()
+    assert bool(got[0].isnan().all()) and not bool(got[1:].isnan().any())
+    short = {"fwd": (rows, N, K + 8), "input_grad": (rows, N + 8, K)}[which]      # a sum that is no whole number of steps
+    assert not getattr(lib, query + "_supported")(*short)
 
 
 @pytest.mark.parametrize("where", ["layers.0", "layers.1.mlp", "layers.0.recc.input_xy", "norm", "lm_head", "embed_tokens"])
