@@ -147,6 +147,11 @@ SIGNATURES = {
         _c_int, [_c_void_p, ctypes.c_longlong] + [_c_void_p] * 7 + [_c_int] + [_c_void_p] * 3 + [ctypes.c_longlong]
         + [_c_void_p] * 10 + [_c_int] * 5 + [_c_void_p, _c_size_t] * 3 + [_c_void_p]
     ),
+    "hawk_block_core_grads": (
+        _c_int, [_c_void_p, ctypes.c_longlong] + [_c_void_p] * 7 + [_c_int] + [_c_void_p] * 3 + [ctypes.c_longlong]
+        + [_c_void_p] * 10 + [_c_int] * 5 + [_c_void_p, _c_size_t] * 3 + [_c_void_p]
+    ),
+    "hawk_block_core_grads_conv_workspace_bytes": (_c_size_t, [_c_int] * 4),
 }
 
 

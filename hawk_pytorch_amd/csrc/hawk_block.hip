@@ -3,7 +3,9 @@
 // The kernels are the ones the single entry points launch; what this file adds is the launch
 // sequence with fewer small kernels around them: the fp32 gate weights are rounded to bf16 by
 // one launch for both gates, and the three closing reductions of the backward (dLambda, the
-// conv's dw / db, the projections' dw / db) run as one launch behind the last large kernel.
+// conv's dw / db, the projections' dw / db) run as one launch behind the last large kernel; where
+// the gradient of the conv output is nobody's, the projections' input gradient and the conv's
+// backward are one kernel.
 #include "hawk_scan.h"
 
 namespace hawk {
@@ -71,12 +73,17 @@ int block_core_fwd(const void* xy, long long ld, const float* conv_w, const floa
                           scan_ws_bytes, st);
 }
 
+// The kernel that takes the projections' input gradient through the conv has four taps.
+size_t block_core_grads_conv_workspace_bytes(int B, int T, int D, int W) {
+    return W == 4 ? gate_conv_bwd_workspace_bytes(B * T, D) : conv1d_bwd_workspace_bytes(B, T, D, W);
+}
+
 int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, const void* ag, const void* h,
                    const float* conv_w, const void* w_i, const void* w_a, int w_dtype, const float* lam,
                    const void* gout, void* d_xy, long long ldd, void* du, void* dxg, void* dag, float* d_conv_w,
                    float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* dlam, int B, int T,
                    int D, int nb, int W, void* scan_ws, size_t scan_ws_bytes, void* gate_ws, size_t gate_ws_bytes,
-                   void* conv_ws, size_t conv_ws_bytes, hipStream_t st) {
+                   void* conv_ws, size_t conv_ws_bytes, hipStream_t st, bool keep_du) {
     constexpr int bf = HAWK_DTYPE_BF16;
     const int M = B * T;
     const void* y = static_cast<const bf16_t*>(xy) + D;
@@ -86,13 +93,19 @@ int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, 
     if (int rc = scan_gated_bwd(u, xg, ag, lam, y, ld, h, gout, du, dxg, dag, dy, ldd, dlam, B, T, D, bf, bf, scan_ws,
                                 scan_ws_bytes, st, &r_dlam))
         return rc;
-    // the projections' input gradient accumulates onto the scan's, in place
-    if (int rc = gate_proj_bwd_input(dxg, dag, w_i, w_a, du, du, M, D, nb, bf, w_dtype, bf, st)) return rc;
-    // the conv's backward right behind the kernel that wrote its input gradient (part of that
-    // tensor is then still in the memory-side cache), the weight gradients last
-    if (int rc = conv1d_bwd(du, xy, ld, conv_w, d_xy, ldd, d_conv_w, d_conv_b, B, T, D, W, bf, bf, conv_ws,
-                            conv_ws_bytes, st, &r_conv))
-        return rc;
+    if (!keep_du && W == 4) {
+        if (int rc = gate_conv_bwd(dxg, dag, w_i, w_a, w_dtype, du, xy, ld, conv_w, d_xy, ldd, d_conv_w, d_conv_b, B,
+                                   T, D, nb, conv_ws, conv_ws_bytes, st, &r_conv))
+            return rc;
+    } else {
+        // the projections' input gradient accumulates onto the scan's, in place
+        if (int rc = gate_proj_bwd_input(dxg, dag, w_i, w_a, du, du, M, D, nb, bf, w_dtype, bf, st)) return rc;
+        // the conv's backward right behind the kernel that wrote its input gradient (part of that
+        // tensor is then still in the memory-side cache), the weight gradients last
+        if (int rc = conv1d_bwd(du, xy, ld, conv_w, d_xy, ldd, d_conv_w, d_conv_b, B, T, D, W, bf, bf, conv_ws,
+                                conv_ws_bytes, st, &r_conv))
+            return rc;
+    }
     if (int rc = gate_proj_bwd_weights(u, dxg, dag, dw_i, db_i, dw_a, db_a, M, D, nb, bf, bf, gate_ws, gate_ws_bytes,
                                        st, &r_gates))
         return rc;

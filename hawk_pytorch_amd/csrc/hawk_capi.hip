@@ -601,14 +601,14 @@ int hawk_block_core_fwd(const void* xy, long long xy_row_stride, const float* co
                                 scan_workspace_bytes, as_stream(stream));
 }
 
-int hawk_block_core_bwd(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
-                        const void* a_rg_lru, const void* h_saved, const float* conv_w, const void* w_i,
-                        const void* w_a, int w_dtype, const float* a_param, const void* grad_out, void* d_xy,
-                        long long d_xy_row_stride, void* du, void* d_x_rg_lru, void* d_a_rg_lru, float* d_conv_w,
-                        float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* da_param, int B,
-                        int T, int D, int num_blocks, int temporal_width, void* scan_workspace,
-                        size_t scan_workspace_bytes, void* gate_workspace, size_t gate_workspace_bytes,
-                        void* conv_workspace, size_t conv_workspace_bytes, void* stream) {
+static int core_backward(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
+                         const void* a_rg_lru, const void* h_saved, const float* conv_w, const void* w_i,
+                         const void* w_a, int w_dtype, const float* a_param, const void* grad_out, void* d_xy,
+                         long long d_xy_row_stride, void* du, void* d_x_rg_lru, void* d_a_rg_lru, float* d_conv_w,
+                         float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* da_param, int B,
+                         int T, int D, int num_blocks, int temporal_width, void* scan_workspace,
+                         size_t scan_workspace_bytes, void* gate_workspace, size_t gate_workspace_bytes,
+                         void* conv_workspace, size_t conv_workspace_bytes, void* stream, bool keep_du) {
     if (!xy || !u || !x_rg_lru || !a_rg_lru || !h_saved || !conv_w || !w_i || !w_a || !a_param || !grad_out || !d_xy ||
         !du || !d_x_rg_lru || !d_a_rg_lru || !d_conv_w || !d_conv_b || !dw_i || !dw_a || !da_param)
         return HAWK_ERR_NULL_POINTER;
@@ -630,7 +630,44 @@ int hawk_block_core_bwd(const void* xy, long long xy_row_stride, const void* u, 
                                 grad_out, d_xy, d_xy_row_stride, du, d_x_rg_lru, d_a_rg_lru, d_conv_w, d_conv_b, dw_i,
                                 db_i, dw_a, db_a, da_param, B, T, D, num_blocks, temporal_width, scan_workspace,
                                 scan_workspace_bytes, gate_workspace, gate_workspace_bytes, conv_workspace,
-                                conv_workspace_bytes, as_stream(stream));
+                                conv_workspace_bytes, as_stream(stream), keep_du);
+}
+
+int hawk_block_core_bwd(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
+                        const void* a_rg_lru, const void* h_saved, const float* conv_w, const void* w_i,
+                        const void* w_a, int w_dtype, const float* a_param, const void* grad_out, void* d_xy,
+                        long long d_xy_row_stride, void* du, void* d_x_rg_lru, void* d_a_rg_lru, float* d_conv_w,
+                        float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* da_param, int B,
+                        int T, int D, int num_blocks, int temporal_width, void* scan_workspace,
+                        size_t scan_workspace_bytes, void* gate_workspace, size_t gate_workspace_bytes,
+                        void* conv_workspace, size_t conv_workspace_bytes, void* stream) {
+    return core_backward(xy, xy_row_stride, u, x_rg_lru, a_rg_lru, h_saved, conv_w, w_i, w_a, w_dtype, a_param,
+                         grad_out, d_xy, d_xy_row_stride, du, d_x_rg_lru, d_a_rg_lru,
+                         d_conv_w, d_conv_b, dw_i, db_i, dw_a, db_a, da_param, B, T, D,
+                         num_blocks, temporal_width, scan_workspace, scan_workspace_bytes,
+                         gate_workspace, gate_workspace_bytes, conv_workspace,
+                         conv_workspace_bytes, stream, true);
+}
+
+int hawk_block_core_grads(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
+                          const void* a_rg_lru, const void* h_saved, const float* conv_w, const void* w_i,
+                          const void* w_a, int w_dtype, const float* a_param, const void* grad_out, void* d_xy,
+                          long long d_xy_row_stride, void* du, void* d_x_rg_lru, void* d_a_rg_lru, float* d_conv_w,
+                          float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* da_param, int B,
+                          int T, int D, int num_blocks, int temporal_width, void* scan_workspace,
+                          size_t scan_workspace_bytes, void* gate_workspace, size_t gate_workspace_bytes,
+                          void* conv_workspace, size_t conv_workspace_bytes, void* stream) {
+    return core_backward(xy, xy_row_stride, u, x_rg_lru, a_rg_lru, h_saved, conv_w, w_i, w_a, w_dtype, a_param,
+                         grad_out, d_xy, d_xy_row_stride, du, d_x_rg_lru, d_a_rg_lru,
+                         d_conv_w, d_conv_b, dw_i, db_i, dw_a, db_a, da_param, B, T, D,
+                         num_blocks, temporal_width, scan_workspace, scan_workspace_bytes,
+                         gate_workspace, gate_workspace_bytes, conv_workspace,
+                         conv_workspace_bytes, stream, false);
+}
+
+size_t hawk_block_core_grads_conv_workspace_bytes(int B, int T, int D, int temporal_width) {
+    if (B < 1 || T < 1 || D < 1 || temporal_width < 1 || (long long)B * T > 0x7fffffffLL) return 0;
+    return hawk::block_core_grads_conv_workspace_bytes(B, T, D, temporal_width);
 }
 
 int hawk_stream_probe(const void* const* reads, int n_reads, void* const* writes, int n_writes, size_t bytes,

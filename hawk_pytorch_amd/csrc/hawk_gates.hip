@@ -29,15 +29,13 @@
 
 #include <atomic>
 
-#include "hawk_device.h"
+#include "hawk_tile.h"
 
 namespace hawk {
 
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef bf16x8 bf16x8_t;
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kGroup = 256;                    // channels per workgroup
 constexpr int kTileRows = 32;                  // rows per MFMA tile
@@ -1093,6 +1091,300 @@ __global__ __launch_bounds__(kGateThreads, 1) void gate_proj_bwd_input_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
+// The same input gradient with the temporal conv's backward behind it, all of it bf16:
+//   du[m]  = dxg[m] w_i^T + dag[m] w_a^T + addend[m]               (rounded to bf16, as above)
+//   dx[m]  = sum_s w[W-1-s] du[m+s],   dw[k] = sum_m du[m] x[m-(W-1-k)],   db = sum_m du[m]
+// with rows of other sequences counting as zeros.  Memory traffic bounds both halves; du never
+// leaves the chip here, which saves writing and reading it (2 of 7 passes over the activations).
+//
+// A worker owns a contiguous range of row tiles and walks it from the back, so that the three du
+// rows behind a tile are the first rows of the tile before it in this walk; the three rows behind
+// the whole range are computed once more from their gradients.  The addend and x (with the rows in
+// front of the tile) go straight into LDS while the tile before is worked on, the gradients through
+// registers one tile ahead.  Eight waves of 256 registers rather than sixteen of 128: with 64
+// registers of weights each, the conv's operands would spill in the latter.
+//
+// Measured at [8, 4096, 2560], 10 blocks, in the whole backward (scan, this, weight gradients):
+// 176 us, 4.8 TB/s, where the two kernels take 117 + 92 alone and 128 + 101 in that place; the
+// backward goes from 660 to 604 us, at [2, 32768, 4096] from 1911 to 1748, at [1, 2048, 512]
+// (16 blocks) from 42.3 to 37.5, at [1, 512, 2560] it stays at 51.  Two variants with the conv of
+// one tile between the matrix instructions of the next (a wave both gates of 32 columns, three
+// barriers a tile) took 190 us.
+// ---------------------------------------------------------------------------------------
+template <int N>
+__device__ __forceinline__ void wait_vector_memory() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+constexpr int kBwdThreads = 512;                                   // 8 waves of up to 256 registers
+constexpr int kBwdRows = kBwdThreads / 32;                         // rows that one access of all threads covers
+constexpr int kBwdHalo = kConvTaps - 1;                            // du rows behind a tile
+constexpr int kBwdORow = kGroup * 4 + 16;                          // fp32 sums of one row
+constexpr int kBwdXRows = kTileRows + 4;                           // x rows: 4 in front of the tile
+constexpr int kBwdO = 4 * kATileBytes;
+constexpr int kBwdD = kBwdO + kTileRows * kBwdORow;
+constexpr int kBwdAdd = kBwdD + (kTileRows + kBwdHalo) * kARowBytes;
+constexpr int kBwdX = kBwdAdd + kTileRows * kGroup * 2;
+constexpr int kBwdW = kBwdX + kBwdXRows * kGroup * 2;
+constexpr int kBwdLds = kBwdW + kConvTaps * kGroup * 4;
+static_assert(kBwdLds <= 160 * 1024 && kBwdD % 16 == 0 && kBwdAdd % 16 == 0 && kConvTaps == 4, "LDS layout");
+
+template <typename WT, int BW>
+__global__ __launch_bounds__(kBwdThreads, 1) void gate_conv_bwd_kernel(
+    const bf16_t* __restrict__ dxg, const bf16_t* __restrict__ dag, const WT* __restrict__ w_i,
+    const WT* __restrict__ w_a, const bf16_t* __restrict__ addend, const bf16_t* __restrict__ x,
+    const float* __restrict__ conv_w, bf16_t* __restrict__ dx, float* __restrict__ part, int M, int T, int D, int nb,
+    int ntiles, size_t ldx, size_t lddx) {
+    constexpr int KS = BW / 16;
+    constexpr int G = kGroup / BW;
+    constexpr int kWaves = kBwdThreads / kWave;
+    constexpr bool kOneBlock = BW >= 64;                    // both column halves of a wave read the same A operands
+    extern __shared__ __align__(16) unsigned char smem[];
+    unsigned char* sA = smem;                               // [stage][gate] gradient tiles
+    unsigned char* sO = smem + kBwdO;                       // fp32 partial result, then the sum
+    unsigned char* sD = smem + kBwdD;                       // du, bf16: the tile and the rows behind it
+    unsigned char* sAdd = smem + kBwdAdd;
+    unsigned char* sX = smem + kBwdX;
+    float* sW = reinterpret_cast<float*>(smem + kBwdW);
+
+    const int tid = threadIdx.x;
+    const int lane = tid & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int group = blockIdx.y, worker = blockIdx.x, nworkers = gridDim.x;
+    const int g = w / (kWaves / 2), c = w % (kWaves / 2);   // gate, 64 output columns
+    const int col = lane & 31, khalf = 8 * (lane >> 5);
+    const WT* wsel = g ? w_a : w_i;
+
+    // this worker's tiles [lo, hi); step j works on tile hi - j, step 0 on the rows behind the range
+    const int lo = (int)((long long)worker * ntiles / nworkers);
+    const int hi = (int)((long long)(worker + 1) * ntiles / nworkers);
+    const int steps = hi - lo;
+    const bool open_end = (long long)hi * kTileRows < M && (hi * kTileRows) % T != 0;
+    const int j0 = open_end ? 0 : 1;
+
+    const int lrow = tid >> 5, lc8 = tid & 31;              // this thread's rows: lrow and lrow + kBwdRows
+    const int lcol = group * kGroup + lc8 * 8;
+    const bool col_ok = lcol < D;
+    const uint32_t row_bytes = (uint32_t)D * 2u;
+    const uint32_t g_off = col_ok ? (uint32_t)(lrow * D + lcol) * 2u : 0x80000000u;
+    const uint32_t g_off2 = g_off + kBwdRows * row_bytes;
+    // rows of step j's tile that are read: none past the range
+    auto first_row = [&](int j) { return (hi - min(j, steps)) * kTileRows; };
+    auto rows_read = [&](int j) {
+        return j > steps ? 0 : min(M - first_row(j), j == 0 ? kBwdHalo : kTileRows);
+    };
+    auto load_tile = [&](int j, Row8<bf16_t> (&r)[4]) {
+        const size_t at = (size_t)first_row(j) * D;
+        const uint32_t window = (uint32_t)rows_read(j) * row_bytes;
+        const rsrc_t ri = make_rsrc(dxg + at, window), ra = make_rsrc(dag + at, window);
+        r[0].load_buf(ri, g_off);
+        r[1].load_buf(ri, g_off2);
+        r[2].load_buf(ra, g_off);
+        r[3].load_buf(ra, g_off2);
+    };
+    auto stage_tile = [&](int buf, const Row8<bf16_t> (&r)[4]) {
+        unsigned char* p = sA + (2 * buf) * kATileBytes + lrow * kARowBytes + lc8 * 16;
+        *reinterpret_cast<u32x4*>(p) = r[0].v;
+        *reinterpret_cast<u32x4*>(p + kBwdRows * kARowBytes) = r[1].v;
+        *reinterpret_cast<u32x4*>(p + kATileBytes) = r[2].v;
+        *reinterpret_cast<u32x4*>(p + kATileBytes + kBwdRows * kARowBytes) = r[3].v;
+    };
+    // addend and x of step j: a wave's lanes bring two adjacent rows (of x from 4 rows in front of the
+    // tile on, waves 0 and 1 its last four rows too)
+    auto load_sides = [&](int j) {
+        const int row0 = first_row(j);
+        const rsrc_t re = make_rsrc(addend + (size_t)row0 * D, (uint32_t)rows_read(j) * row_bytes);
+        load_to_lds(re, sAdd + w * 1024, g_off, 0);
+        load_to_lds(re, sAdd + (kWaves + w) * 1024, g_off2, 0);
+        const int back = row0 >= 4 ? 4 : 0;                  // tile 0 has nothing in front of it
+        const int rows = j == 0 || j > steps ? 0 : min(M - row0, kTileRows) + back;
+        const rsrc_t rx = make_rsrc(x + (size_t)(row0 - back) * ldx,
+                                    rows > 0 ? (uint32_t)((rows - 1) * ldx + D) * 2u : 0u);
+        const int xr = lrow - 4 + back;
+        const uint32_t at = col_ok && xr >= 0 ? (uint32_t)(xr * ldx + lcol) * 2u : 0x80000000u;
+        const uint32_t at2 = col_ok ? (uint32_t)((xr + kBwdRows) * ldx + lcol) * 2u : 0x80000000u;
+        load_to_lds(rx, sX + w * 1024, at, 0);
+        load_to_lds(rx, sX + (kWaves + w) * 1024, at2, 0);
+        if (w < 2) load_to_lds(rx, sX + (2 * kWaves + w) * 1024, at2 + (uint32_t)(kBwdRows * ldx) * 2u, 0);
+    };
+
+    Row8<bf16_t> next[4];
+    load_tile(j0, next);
+    __builtin_amdgcn_sched_barrier(0);
+
+    // weights: lane holds row i of w_g[h] and 8 consecutive j per k-step (contiguous)
+    const rsrc_t wres = make_rsrc(wsel, (uint32_t)((size_t)nb * BW * BW * sizeof(WT)));
+    bf16x8 bfrag[2][KS];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        const int blk = (64 * c + 32 * q) / BW, h = group * G + blk;
+        const int i_in = 64 * c + 32 * q - blk * BW + col;  // input channel within the block
+        const float live = (h < nb) ? 1.0f : 0.0f;
+        const uint32_t wlane = (uint32_t)((((size_t)min(h, nb - 1) * BW + i_in) * BW + khalf) * sizeof(WT));
+#pragma unroll
+        for (int s = 0; s < KS; ++s) {
+            bfrag[q][s] = load_weight8(wres, wlane, (uint32_t)(16 * s * sizeof(WT)), live, static_cast<const WT*>(nullptr));
+            if (s % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (int e = tid; e < kConvTaps * kGroup; e += kBwdThreads) {
+        const int ch = group * kGroup + e % kGroup;
+        sW[e] = ch < D ? conv_w[(size_t)(e / kGroup) * D + ch] : 0.0f;
+    }
+
+    stage_tile(0, next);
+    load_tile(j0 + 1, next);
+    load_sides(j0);
+    lds_barrier();
+
+    const int a_off = g * kATileBytes + col * kARowBytes + khalf * 2;
+    unsigned char* o_base = sO + (4 * (lane >> 5)) * kBwdORow + (64 * c + col) * 4;
+
+    // the conv's side: two channels (one pair) of kConvSide rows
+    constexpr int kConvSide = kTileRows * kGroup / 2 / kBwdThreads;
+    const int pair = tid % (kGroup / 2), r0 = kConvSide * (tid / (kGroup / 2));
+    const int ch = group * kGroup + 2 * pair;
+    const uint32_t dx_off = ch < D ? (uint32_t)(r0 * lddx + ch) * 2u : 0x80000000u;
+    float dw[kConvTaps][2] = {}, db[2] = {};
+
+    auto conv_rows = [&](int row0, auto masked) {
+        constexpr bool kMasked = decltype(masked)::value;
+        const unsigned char* pd = sD + r0 * kARowBytes + pair * 4;
+        const unsigned char* px = sX + (r0 + 1) * (kGroup * 2) + pair * 4;
+        const rsrc_t out_rows = make_rsrc(dx + (size_t)row0 * lddx,
+                                          (uint32_t)((min(M - row0, kTileRows) - 1) * lddx + D) * 2u);
+        f32x2 wk[kConvTaps];
+#pragma unroll
+        for (int k = 0; k < kConvTaps; ++k) wk[k] = *reinterpret_cast<const f32x2*>(sW + k * kGroup + 2 * pair);
+        uint32_t d[kConvSide + 3], xv[kConvSide + 3];
+#pragma unroll
+        for (int i = 0; i < kConvSide + 3; ++i) {
+            d[i] = *reinterpret_cast<const uint32_t*>(pd + i * kARowBytes);
+            xv[i] = *reinterpret_cast<const uint32_t*>(px + i * (kGroup * 2));
+        }
+        uint32_t off = dx_off;
+        asm volatile("" : "+v"(off));                        // (eight offsets kept across the loop would spill)
+        int pos = 0;
+        if constexpr (kMasked) pos = (row0 + r0) % T;
+#pragma unroll
+        for (int r = 0; r < kConvSide; ++r) {
+            const float g0 = bf16_lo(d[r]), g1 = bf16_hi(d[r]);
+            float o0 = 0.0f, o1 = 0.0f;
+            db[0] += g0;
+            db[1] += g1;
+#pragma unroll
+            for (int s = 0; s < kConvTaps; ++s) {            // du s rows behind, x s rows in front
+                uint32_t dv = d[r + s], xs = xv[r + 3 - s];
+                if constexpr (kMasked) {
+                    dv = pos + s < T ? dv : 0u;
+                    xs = pos >= s ? xs : 0u;
+                }
+                const int k = kConvTaps - 1 - s;
+                o0 = fmaf(wk[k].x, bf16_lo(dv), o0);
+                o1 = fmaf(wk[k].y, bf16_hi(dv), o1);
+                dw[k][0] = fmaf(g0, bf16_lo(xs), dw[k][0]);
+                dw[k][1] = fmaf(g1, bf16_hi(xs), dw[k][1]);
+            }
+            buffer_store(pack_bf16x2(o0, o1), out_rows, off, 0u);
+            off += (uint32_t)lddx * 2u;
+            if constexpr (kMasked) pos = pos + 1 == T ? 0 : pos + 1;
+        }
+    };
+
+    auto step = [&](int j, int cur) {
+        f32x16 acc[2] = {};
+        const unsigned char* a_base = sA + (2 * cur) * kATileBytes + a_off;
+        constexpr int kBatch = KS < 4 ? KS : 4;
+        const unsigned char* a_half[2] = {a_base + (64 * c) / BW * BW * 2, a_base + (64 * c + 32) / BW * BW * 2};
+#pragma unroll
+        for (int s0 = 0; s0 < KS; s0 += kBatch) {
+            bf16x8 a[kOneBlock ? 1 : 2][kBatch];
+#pragma unroll
+            for (int b = 0; b < (kOneBlock ? 1 : 2); ++b)
+#pragma unroll
+                for (int q = 0; q < kBatch; ++q) a[b][q] = *reinterpret_cast<const bf16x8*>(a_half[b] + (s0 + q) * 32);
+#pragma unroll
+            for (int q = 0; q < kBatch; ++q)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[kOneBlock ? 0 : b][q], bfrag[b][s0 + q], acc[b], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the second gate's waves hand their tile to the first gate's, which add theirs in front
+        if (g == 1) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    *reinterpret_cast<float*>(o_base + (8 * (r / 4) + (r % 4)) * kBwdORow + b * 128) = acc[b][r];
+        }
+        lds_barrier();
+        if (g == 0) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float* p = reinterpret_cast<float*>(o_base + (8 * (r / 4) + (r % 4)) * kBwdORow + b * 128);
+                    *p = acc[b][r] + *p;
+                }
+        }
+        stage_tile(cur ^ 1, next);
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile(j + 2, next);
+        __builtin_amdgcn_sched_barrier(0);
+        // this tile's addend and x are there: only these four loads, issued behind them, are still out
+        wait_vector_memory<4>();
+        lds_barrier();
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int row = lrow + k * kBwdRows;
+            const unsigned char* o_src = sO + row * kBwdORow + lc8 * 32;
+            const f32x4 p0 = *reinterpret_cast<const f32x4*>(o_src), p1 = *reinterpret_cast<const f32x4*>(o_src + 16);
+            Row8<bf16_t> radd;
+            radd.v = *reinterpret_cast<const u32x4*>(sAdd + (row * 32 + lc8) * 16);
+            f32x4 e0, e1;
+            radd.as_f32(e0, e1);
+            const f32x4 s0 = p0 + e0, s1 = p1 + e1;
+            u32x4* du = reinterpret_cast<u32x4*>(sD + row * kARowBytes + lc8 * 16);
+            // the first rows of the tile before this one in the walk are the rows behind it
+            if (k == 0 && row < kBwdHalo) du[kTileRows * kARowBytes / 16] = j > j0 ? *du : u32x4{0u, 0u, 0u, 0u};
+            *du = u32x4{pack_bf16x2(s0.x, s0.y), pack_bf16x2(s0.z, s0.w), pack_bf16x2(s1.x, s1.y),
+                        pack_bf16x2(s1.z, s1.w)};
+        }
+        lds_barrier();
+        if (j > 0) {
+            const int row0 = first_row(j), pos = row0 % T;
+            if (pos >= kBwdHalo && pos + kTileRows + kBwdHalo <= T) conv_rows(row0, std::false_type{});
+            else conv_rows(row0, std::true_type{});
+        }
+        lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        load_sides(j + 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int j = j0, cur = 0; j <= steps; ++j, cur ^= 1) step(j, cur);
+
+    // the worker's sums: several threads hold each channel pair's
+    wait_vector_memory<0>();                                 // the last loads into LDS
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(smem);             // [threads of a pair][taps + 1][kGroup]
+    constexpr int kShare = kBwdThreads / (kGroup / 2);
+    float* mine = red + (tid / (kGroup / 2)) * (kConvTaps + 1) * kGroup + 2 * pair;
+#pragma unroll
+    for (int k = 0; k < kConvTaps; ++k) *reinterpret_cast<f32x2*>(mine + k * kGroup) = f32x2{dw[k][0], dw[k][1]};
+    *reinterpret_cast<f32x2*>(mine + kConvTaps * kGroup) = f32x2{db[0], db[1]};
+    __syncthreads();
+    for (int e = tid; e < (kConvTaps + 1) * kGroup; e += kBwdThreads) {
+        const int at = group * kGroup + e % kGroup;
+        if (at >= D) continue;
+        float sum = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kShare; ++q) sum += red[q * (kConvTaps + 1) * kGroup + e];
+        part[((size_t)worker * (kConvTaps + 1) + e / kGroup) * D + at] = sum;
+    }
+}
+
+// ---------------------------------------------------------------------------------------
 // Weight and bias gradients:
 //   dw_g[h, i, j] = sum_m x[m, h*bw + i] dg[m, h*bw + j],   db_g[c] = sum_m dg[m, c]
 // The contraction runs over the rows, so both operands are needed "column-wise".  A
@@ -1304,7 +1596,6 @@ __global__ void gate_proj_reduce_kernel(GateReduceTask t) {
     gate_reduce_span(t, (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)gridDim.x * blockDim.x);
 }
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // Compute units of the current device (asked once per device): the persistent kernels launch one
 // workgroup per compute unit, and the size of the weight-gradient workspace follows from it.
@@ -1461,6 +1752,39 @@ int gate_bwd_input_out(const void* dxg, const void* dag, const void* w_i, const 
     if (dx_dtype == HAWK_DTYPE_BF16)
         return gate_bwd_input_bw<GT, WT, bf16_t>(dxg, dag, w_i, w_a, addend, dx, M, D, nb, bw, st);
     return gate_bwd_input_bw<GT, WT, float>(dxg, dag, w_i, w_a, addend, dx, M, D, nb, bw, st);
+}
+
+// Workers of the fused backward: one per compute unit, as many as there are row tiles.
+int gate_conv_workers(int M, int D) {
+    const int ngroups = ceil_div(D, kGroup), ntiles = ceil_div(M, kTileRows);
+    int n = num_cu() / ngroups;
+    if (n < 1) n = 1;
+    return n > ntiles ? ntiles : n;
+}
+
+template <typename WT, int BW>
+int launch_gate_conv_bwd(const void* dxg, const void* dag, const void* w_i, const void* w_a, const void* addend,
+                         const void* x, size_t ldx, const float* conv_w, void* dx, size_t lddx, float* part, int M,
+                         int T, int D, int nb, hipStream_t st) {
+    constexpr auto kernel = gate_conv_bwd_kernel<WT, BW>;
+    if (!allow_dynamic_lds<kernel>(kBwdLds)) return HAWK_ERR_LAUNCH;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gate_conv_workers(M, D), (unsigned)ceil_div(D, kGroup)),
+                       dim3(kBwdThreads), kBwdLds, st, static_cast<const bf16_t*>(dxg), static_cast<const bf16_t*>(dag),
+                       static_cast<const WT*>(w_i), static_cast<const WT*>(w_a), static_cast<const bf16_t*>(addend),
+                       static_cast<const bf16_t*>(x), conv_w, static_cast<bf16_t*>(dx), part, M, T, D, nb,
+                       ceil_div(M, kTileRows), ldx, lddx);
+    return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
+}
+
+template <typename WT, typename... Args>
+int gate_conv_bwd_bw(int bw, Args... args) {
+    switch (bw) {
+        case 32: return launch_gate_conv_bwd<WT, 32>(args...);
+        case 64: return launch_gate_conv_bwd<WT, 64>(args...);
+        case 128: return launch_gate_conv_bwd<WT, 128>(args...);
+        case 256: return launch_gate_conv_bwd<WT, 256>(args...);
+        default: return HAWK_ERR_BAD_SHAPE;
+    }
 }
 
 int weight_splits(int M, int D) {
@@ -1639,6 +1963,25 @@ int gate_proj_bwd_input(const void* dxg, const void* dag, const void* w_i, const
     if (w_dtype == HAWK_DTYPE_BF16)
         return gate_bwd_input_out<float, bf16_t>(dxg, dag, w_i, w_a, addend, dx, M, D, nb, bw, dx_dtype, st);
     return gate_bwd_input_out<float, float>(dxg, dag, w_i, w_a, addend, dx, M, D, nb, bw, dx_dtype, st);
+}
+
+size_t gate_conv_bwd_workspace_bytes(int M, int D) {
+    return (size_t)gate_conv_workers(M, D) * (kConvTaps + 1) * D * sizeof(float);
+}
+
+int gate_conv_bwd(const void* dxg, const void* dag, const void* w_i, const void* w_a, int w_dtype, const void* addend,
+                  const void* x, long long ldx, const float* conv_w, void* dx, long long lddx, float* d_conv_w,
+                  float* d_conv_b, int B, int T, int D, int nb, void* ws, size_t ws_bytes, hipStream_t st,
+                  ColsumTask* deferred) {
+    const int M = B * T, bw = D / nb;
+    if (ws == nullptr || ws_bytes < gate_conv_bwd_workspace_bytes(M, D)) return HAWK_ERR_WORKSPACE;
+    float* part = static_cast<float*>(ws);
+    const size_t lx = (size_t)ldx, ld = (size_t)lddx;
+    const int rc = w_dtype == HAWK_DTYPE_BF16
+                       ? gate_conv_bwd_bw<bf16_t>(bw, dxg, dag, w_i, w_a, addend, x, lx, conv_w, dx, ld, part, M, T, D, nb, st)
+                       : gate_conv_bwd_bw<float>(bw, dxg, dag, w_i, w_a, addend, x, lx, conv_w, dx, ld, part, M, T, D, nb, st);
+    *deferred = ColsumTask{part, d_conv_w, d_conv_b, nullptr, gate_conv_workers(M, D), (kConvTaps + 1) * D, kConvTaps * D};
+    return rc;
 }
 
 size_t gate_proj_bwd_weights_workspace_bytes(int M, int D, int nb) {

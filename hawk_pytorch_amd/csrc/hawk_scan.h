@@ -69,6 +69,14 @@ int conv_gate_proj_fwd(const void* x, long long ldx, const float* conv_w, const 
                        int T, int D, int nb, int w_dtype, hipStream_t st);
 int gate_proj_bwd_input(const void* dxg, const void* dag, const void* w_i, const void* w_a, const void* addend,
                         void* dx, int M, int D, int nb, int g_dtype, int w_dtype, int dx_dtype, hipStream_t st);
+// gate_proj_bwd_input (bf16, with the addend) and the backward of a conv of width 4 behind it in one
+// kernel: the gradient between the two is not written.  `deferred` receives d_conv_w's and d_conv_b's
+// closing sum.
+size_t gate_conv_bwd_workspace_bytes(int M, int D);
+int gate_conv_bwd(const void* dxg, const void* dag, const void* w_i, const void* w_a, int w_dtype, const void* addend,
+                  const void* x, long long ldx, const float* conv_w, void* dx, long long lddx, float* d_conv_w,
+                  float* d_conv_b, int B, int T, int D, int nb, void* ws, size_t ws_bytes, hipStream_t st,
+                  ColsumTask* deferred);
 // conv window roll + conv, both projections, state update and output gate of one decode step
 // (bf16 activations and conv window; W <= 8)
 int decode_core_step(void* conv_state, const void* x_new, long long ldx, const float* conv_w, const float* conv_b,
@@ -93,13 +101,16 @@ int block_core_fwd(const void* xy, long long ld, const float* conv_w, const floa
                    const float* b_i, const void* w_a, const float* b_a, int w_dtype, void* w16, const float* lam,
                    void* u, void* xg, void* ag, void* h, void* out, void* h_last, int B, int T, int D, int nb,
                    void* scan_ws, size_t scan_ws_bytes, hipStream_t st);
-// The backward of all of it; du, dxg, dag: [B,T,D] bf16 scratch for the gradients in between.
+// The backward of all of it; du, dxg, dag: [B,T,D] bf16 scratch for the gradients in between.  keep_du: du
+// ends up as the whole gradient of u; otherwise (conv_ws of block_core_grads_conv_workspace_bytes) it is
+// scratch like the others.
+size_t block_core_grads_conv_workspace_bytes(int B, int T, int D, int W);
 int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, const void* ag, const void* h,
                    const float* conv_w, const void* w_i, const void* w_a, int w_dtype, const float* lam,
                    const void* gout, void* d_xy, long long ldd, void* du, void* dxg, void* dag, float* d_conv_w,
                    float* d_conv_b, float* dw_i, float* db_i, float* dw_a, float* db_a, float* dlam, int B, int T,
                    int D, int nb, int W, void* scan_ws, size_t scan_ws_bytes, void* gate_ws, size_t gate_ws_bytes,
-                   void* conv_ws, size_t conv_ws_bytes, hipStream_t st);
+                   void* conv_ws, size_t conv_ws_bytes, hipStream_t st, bool keep_du);
 
 // hawk_decode.hip
 // x w^T for up to kDecodeMaxRows rows; see include/hawk_hip.h for the operands

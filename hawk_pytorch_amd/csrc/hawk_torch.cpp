@@ -56,7 +56,8 @@ constexpr int64_t kStaggerMinBytes = 16 << 20;   // _lib.activation_empty places
     X(hawk_scan_workspace_bytes) X(hawk_rglru_scan_fwd_mixed) X(hawk_rglru_scan_bwd_mixed)                            \
     X(hawk_rglru_scan_gated_fwd) X(hawk_rglru_scan_gated_bwd) X(hawk_conv1d_fwd) X(hawk_conv1d_fwd_strided)           \
     X(hawk_conv1d_bwd) X(hawk_conv1d_bwd_workspace_bytes) X(hawk_gate_proj_fwd) X(hawk_gate_weights_to_bf16)          \
-    X(hawk_gate_proj_bwd_weights_workspace_bytes) X(hawk_block_core_fwd) X(hawk_block_core_bwd)                       \
+    X(hawk_gate_proj_bwd_weights_workspace_bytes) X(hawk_block_core_fwd) X(hawk_block_core_grads)                     \
+    X(hawk_block_core_grads_conv_workspace_bytes)                                                                     \
     X(hawk_decode_core_workspace_bytes) X(hawk_decode_core_step_ws) X(hawk_decode_layer_tail)                         \
     X(hawk_decode_norm_linear) X(hawk_cast) X(hawk_add_norm_fwd) X(hawk_add_norm_bwd)                                 \
     X(hawk_add_norm_bwd_workspace_bytes) X(hawk_gelu_mul_fwd) X(hawk_gelu_mul_bwd) X(hawk_cross_entropy_fwd)          \
@@ -370,10 +371,10 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> core_
            dbi = c.empty({D}, kF32), dba = c.empty({D}, kF32), dcb = c.empty({D}, kF32), dcw = c.empty({W, D}, kF32);
     const Tensor ws = scan_workspaces().get(c, lib.hawk_scan_workspace_bytes(B, T, D, HAWK_DTYPE_BF16));
     const Tensor gws = gate_workspaces().get(c, lib.hawk_gate_proj_bwd_weights_workspace_bytes(B * T, D, nb));
-    const Tensor cws = c.empty({(int64_t)lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W)}, at::kByte);
-    // scan (with the output gate) -> projections' input gradient onto the scan's, in place -> conv ->
+    const Tensor cws = c.empty({(int64_t)lib.hawk_block_core_grads_conv_workspace_bytes(B, T, D, W)}, at::kByte);
+    // scan (with the output gate) -> projections' input gradient onto the scan's and the conv ->
     // projections' weight gradients, and one launch for the three closing reductions
-    check("hawk_block_core_bwd", lib.hawk_block_core_bwd(
+    check("hawk_block_core_grads", lib.hawk_block_core_grads(
         data(xy), row_stride(xy), data(u), data(xg), data(ag), data(h), data<float>(cw), data(wi), data(wa),
         code(wi.scalar_type()), data<float>(lam), data(go), data(d_xy), 2 * D, data(du), data(dxg), data(dag),
         data<float>(dcw), data<float>(dcb), data<float>(dwi), data<float>(dbi), data<float>(dwa), data<float>(dba),

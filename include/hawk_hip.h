@@ -506,6 +506,22 @@ int hawk_block_core_bwd(const void* xy, long long xy_row_stride, const void* u, 
                         size_t gate_workspace_bytes, void* conv_workspace,
                         size_t conv_workspace_bytes, void* stream);
 
+/* The same gradients with the same arguments, where nobody wants the gradient of the conv output:
+ * du is scratch whose contents are unspecified afterwards.  With temporal_width 4 the projections'
+ * input gradient and the conv's backward are one kernel; d_xy has the same bits, d_conv_w and
+ * d_conv_b are added up in another order.  conv_workspace as the size function says. */
+size_t hawk_block_core_grads_conv_workspace_bytes(int B, int T, int D, int temporal_width);
+int hawk_block_core_grads(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
+                          const void* a_rg_lru, const void* h_saved, const float* conv_w,
+                          const void* w_i, const void* w_a, int w_dtype, const float* a_param,
+                          const void* grad_out, void* d_xy, long long d_xy_row_stride, void* du,
+                          void* d_x_rg_lru, void* d_a_rg_lru, float* d_conv_w, float* d_conv_b,
+                          float* dw_i, float* db_i, float* dw_a, float* db_a, float* da_param, int B, int T,
+                          int D, int num_blocks, int temporal_width, void* scan_workspace,
+                          size_t scan_workspace_bytes, void* gate_workspace,
+                          size_t gate_workspace_bytes, void* conv_workspace,
+                          size_t conv_workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * A measurement aid with no counterpart in the reference: copy kernels that move n_reads
  * tensors in and n_writes tensors out (`bytes` each, 16-byte aligned, all distinct) with the scan

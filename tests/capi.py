@@ -352,7 +352,12 @@ def block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, round_weights=Tr
     return out, u, xg, ag, h, h_last, w16
 
 
-def block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, gout, with_bias=True, ws=None):
+def block_core_grads(*args):
+    """block_core_bwd without the gradient of the conv output."""
+    return block_core_bwd(*args, keep_du=False)[:-1]
+
+
+def block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, gout, with_bias=True, ws=None, keep_du=True):
     """Returns (d_xy, d_conv_w, d_conv_b, dw_i, db_i, dw_a, db_a, dlam, du)."""
     B, T, D2 = xy.shape
     D = D2 // 2
@@ -368,8 +373,9 @@ def block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, gout, with_bias=True
         ws = new_workspace(B, T, D, "bf16")
     garbage = lambda n: torch.full((max(n, 16),), 0xAB, dtype=torch.uint8, device="cuda")  # noqa: E731
     gws = garbage(lib.hawk_gate_proj_bwd_weights_workspace_bytes(B * T, D, nb))
-    cws = garbage(lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W))
-    rc = lib.hawk_block_core_bwd(
+    cws = garbage((lib.hawk_conv1d_bwd_workspace_bytes if keep_du else
+                   lib.hawk_block_core_grads_conv_workspace_bytes)(B, T, D, W))
+    rc = (lib.hawk_block_core_bwd if keep_du else lib.hawk_block_core_grads)(
         xy.data_ptr(), xy.stride(1), u.data_ptr(), xg.data_ptr(), ag.data_ptr(), h.data_ptr(), conv_w.data_ptr(),
         w_i.data_ptr(), w_a.data_ptr(), _lib.dtype_code(w_i.dtype), lam.data_ptr(), gout.data_ptr(), d_xy.data_ptr(),
         D2, du.data_ptr(), dxg.data_ptr(), dag.data_ptr(), dcw.data_ptr(), dcb.data_ptr(), dwi.data_ptr(),

@@ -79,6 +79,38 @@ def test_one_call_gives_the_bits_of_the_single_calls(B, T, D, nb, w_dtype, round
     _same_bits(B, T, D, nb, w_dtype, round_weights, seed=B * 1000 + T)
 
 
+# sequences shorter and longer than a row tile and its halo, ends in and between tiles, part of a channel
+# group, fewer and more tiles than workers, several tiles a worker
+@pytest.mark.parametrize("B,T,D,nb,w_dtype", [
+    (1, 32, 256, 1, "bf16"), (70, 1, 64, 2, "bf16"), (23, 3, 128, 1, "f32"), (2, 33, 256, 1, "f32"),
+    (3, 100, 512, 4, "bf16"), (2, 77, 2560, 10, "bf16"), (5, 45, 96, 3, "bf16"), (4, 300, 768, 3, "f32"),
+    (1, 4096, 512, 16, "bf16"), (3, 1024, 2560, 10, "bf16"), (1, 9001, 320, 5, "bf16"), (8, 4096, 2560, 10, "bf16")])
+def test_conv_backward_behind_the_projections(B, T, D, nb, w_dtype):
+    """Without the gradient of the conv output the two run as one kernel: the input gradient keeps its bits;
+    the conv's weight gradients are other orders of the same sums, |error| <= n 2^-24 sum |du x| for n terms
+    in any order."""
+    xy, cw, cb, wi, bi, wa, ba, lam, gout = _inputs(B, T, D, nb, w_dtype, seed=B * 100 + T)
+    x, y = xy[..., :D], xy[..., D:]
+    u = (x.float() + 0.5).to(torch.bfloat16)
+    xg, ag = capi.gate_proj_fwd(u.reshape(-1, D), wi, bi, wa, ba, torch.bfloat16)[:2]
+    xg, ag = xg.reshape(B, T, D), ag.reshape(B, T, D)
+    _, h, _ = capi.scan_gated_fwd(u, xg, ag, lam, y)
+    ref = capi.block_core_bwd(xy, u, xg, ag, h, cw, wi, wa, lam, gout)
+    got = capi.block_core_grads(xy, u, xg, ag, h, cw, wi, wa, lam, gout)
+    again = capi.block_core_grads(xy, u, xg, ag, h, cw, wi, wa, lam, gout)
+    for k in (0, 3, 4, 5, 6, 7):
+        assert torch.equal(got[k], ref[k]), k
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    du, M, W = ref[8].double(), B * T, cw.shape[0]
+    for k in range(W):
+        lag = W - 1 - k
+        terms = du[:, lag:] * x[:, :T - lag].double() if lag < T else du[:, :0]
+        error = (got[1][k].double() - terms.sum((0, 1))).abs()
+        assert (error <= M * 2.0 ** -24 * terms.abs().sum((0, 1))).all(), (k, error.max())
+    error = (got[2].double() - du.sum((0, 1))).abs()
+    assert (error <= M * 2.0 ** -24 * du.abs().sum((0, 1))).all()
+
+
 def test_benchmark_shape_and_twice_on_one_workspace():
     args, first = _same_bits(8, 4096, 2560, 10, "f32", True, seed=5)
     again = _one_call_each_way(*args, True)

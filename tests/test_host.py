@@ -377,6 +377,22 @@ def test_argument_validation_of_the_block_core_entry_points():
     assert lib.hawk_gate_weights_to_bf16(p, p, p + 2, p, 2, 64, None) == E.HAWK_ERR_ALIGNMENT
 
 
+def test_the_two_backwards_of_the_block_core_refuse_the_same():
+    lib, E, p = _lib.load(), _lib, 4096
+    ok = [p, 512, p, p, p, p, p, p, p, 0, p, p, p, 512, p, p, p, p, p, p, None, p, None, p, 2, 64, 256, 1, 4,
+          p, 1 << 20, p, 1 << 20, p, 1 << 20, None]
+    for idx, what in [(28, 9), (1, 511), (13, 516), (27, 3), (26, 252), (24, 70000), (9, 7), (12, p + 4)] + [
+            (i, None) for i in (0, 2, 3, 4, 5, 6, 7, 8, 10, 11, 12, 14, 15, 16, 17, 18, 19, 21, 23, 29, 31, 33)]:
+        bad = list(ok); bad[idx] = what
+        status = lib.hawk_block_core_bwd(*bad)
+        assert status != 0 and lib.hawk_block_core_grads(*bad) == status, (idx, what)
+    # partial sums: one row of taps + 1 per worker, at most one worker per 32 rows; other widths as the conv's own
+    for B, T, D in ((1, 1, 32), (8, 4096, 2560), (3, 1531, 1024)):
+        size = lib.hawk_block_core_grads_conv_workspace_bytes(B, T, D, 4)
+        assert size % (5 * D * 4) == 0 and 1 <= size // (5 * D * 4) <= -(-B * T // 32)
+        assert lib.hawk_block_core_grads_conv_workspace_bytes(B, T, D, 3) == lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, 3)
+
+
 def test_argument_validation_of_the_fused_decode_step():
     lib = _lib.load()
     buf = (ctypes.c_char * 4096)()
