@@ -73,9 +73,16 @@ int block_core_fwd(const void* xy, long long ld, const float* conv_w, const floa
                           scan_ws_bytes, st);
 }
 
-// The kernel that takes the projections' input gradient through the conv has four taps.
+// The projections' input gradient and the conv's backward as one kernel: it has four taps, and pays from 1024 rows
+// on.  Whole backward in us, one kernel against two: 1024 rows 67.0 and 70.6 (2560 channels), 32.9 and 37.4 (512),
+// 91.9 and 97.8 (4096), 2048 rows of 256 channels 50.9 and 54.3; 768 rows of 2560 55.3 and 56.0, 512 rows 50.9 and
+// 51.4 (2560), 31.2 and 31.9 (512), 256 rows 47.3 and 47.1: there a worker has a tile or two, each with its halo,
+// and the conv's weight gradients rather keep the order of the conv's own backward.
+constexpr int kOneKernelRows = 1024;
+bool projections_with_conv(int B, int T, int W) { return W == 4 && B * T >= kOneKernelRows; }
+
 size_t block_core_grads_conv_workspace_bytes(int B, int T, int D, int W) {
-    return W == 4 ? gate_conv_bwd_workspace_bytes(B * T, D) : conv1d_bwd_workspace_bytes(B, T, D, W);
+    return projections_with_conv(B, T, W) ? gate_conv_bwd_workspace_bytes(B * T, D) : conv1d_bwd_workspace_bytes(B, T, D, W);
 }
 
 int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, const void* ag, const void* h,
@@ -93,7 +100,7 @@ int block_core_bwd(const void* xy, long long ld, const void* u, const void* xg, 
     if (int rc = scan_gated_bwd(u, xg, ag, lam, y, ld, h, gout, du, dxg, dag, dy, ldd, dlam, B, T, D, bf, bf, scan_ws,
                                 scan_ws_bytes, st, &r_dlam))
         return rc;
-    if (!keep_du && W == 4) {
+    if (!keep_du && projections_with_conv(B, T, W)) {
         if (int rc = gate_conv_bwd(dxg, dag, w_i, w_a, w_dtype, du, xy, ld, conv_w, d_xy, ldd, d_conv_w, d_conv_b, B,
                                    T, D, nb, conv_ws, conv_ws_bytes, st, &r_conv))
             return rc;

@@ -507,9 +507,10 @@ int hawk_block_core_bwd(const void* xy, long long xy_row_stride, const void* u, 
                         size_t conv_workspace_bytes, void* stream);
 
 /* The same gradients with the same arguments, where nobody wants the gradient of the conv output:
- * du is scratch whose contents are unspecified afterwards.  With temporal_width 4 the projections'
- * input gradient and the conv's backward are one kernel; d_xy has the same bits, d_conv_w and
- * d_conv_b are added up in another order.  conv_workspace as the size function says. */
+ * du is scratch whose contents are unspecified afterwards.  With temporal_width 4 and 1024 rows
+ * (B T) or more the projections' input gradient and the conv's backward are one kernel; all results
+ * have the same bits but d_conv_w and d_conv_b, which are added up in another order there.
+ * conv_workspace as the size function says. */
 size_t hawk_block_core_grads_conv_workspace_bytes(int B, int T, int D, int temporal_width);
 int hawk_block_core_grads(const void* xy, long long xy_row_stride, const void* u, const void* x_rg_lru,
                           const void* a_rg_lru, const void* h_saved, const float* conv_w,

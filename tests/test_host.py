@@ -386,8 +386,10 @@ def test_the_two_backwards_of_the_block_core_refuse_the_same():
         bad = list(ok); bad[idx] = what
         status = lib.hawk_block_core_bwd(*bad)
         assert status != 0 and lib.hawk_block_core_grads(*bad) == status, (idx, what)
-    # partial sums: one row of taps + 1 per worker, at most one worker per 32 rows; other widths as the conv's own
-    for B, T, D in ((1, 1, 32), (8, 4096, 2560), (3, 1531, 1024)):
+    # partial sums: one row of taps + 1 per worker, at most one worker per 32 rows; other widths, and fewer than
+    # 1024 rows, as the conv's own
+    assert lib.hawk_block_core_grads_conv_workspace_bytes(3, 341, 256, 4) == lib.hawk_conv1d_bwd_workspace_bytes(3, 341, 256, 4)
+    for B, T, D in ((1, 1024, 32), (8, 4096, 2560), (3, 1531, 1024)):
         size = lib.hawk_block_core_grads_conv_workspace_bytes(B, T, D, 4)
         assert size % (5 * D * 4) == 0 and 1 <= size // (5 * D * 4) <= -(-B * T // 32)
         assert lib.hawk_block_core_grads_conv_workspace_bytes(B, T, D, 3) == lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, 3)
