@@ -15,7 +15,7 @@
 //   * the four partial tiles meet in LDS at the end and leave in whole rows;
 //   * projections with few columns also split K over workgroups and leave fp32 partial sums, which
 //     the kernel that follows (residual add + norm) adds up in a fixed order on its way.
-// A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 49 / 53 / 63 /
+// A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 45 / 53 / 63 /
 // 79 / 86 / 101 us at 1 / 32 / 64 / 128 / 129 / 256 rows with cold weights (157 MB); the library's four products
 // alone took 121 us at 256 rows, with the norms, additions, GELU and product around them 149.
 // All sums are fp32, in an order that depends on the shape alone, and values are rounded to bf16 where
@@ -498,6 +498,237 @@ int add_norm(void* hidden, const float* partial, int splits, const void* weight,
     return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
 }
 
+// ---------------------------------------------------------------------------------------
+// Products for one or two rows, where a launch's duration is a few memory round trips and not its bytes: a wave takes
+// C weight rows at a time, a lane 16 bytes of each per 512 input channels, and the sums meet in a butterfly over the
+// lanes.  No LDS tile, no loop of staged steps, and the norm in front needs no launch of its own: every workgroup
+// repeats residual add and norm of the few rows into its LDS while its first weights are on their way.
+//   kNoNorm     x [M, K] bf16
+//   kNorm       x = norm(hidden)
+//   kAddNorm    x = norm(hidden + delta), delta [M, K] fp32; the first workgroup writes the sum to hidden_out, which
+//               is not hidden: the others may still be reading that
+// Values are rounded, and squares added up, as in add_norm_kernel.  out as for decode_gemm_kernel, kStorePartial with
+// one split.
+// A layer's four products and two norms at one row, against the tiles and add_norm_kernel: 13.8 us (21.9) at 512
+// channels and an MLP of 1024, 18.6 (29.4) at 1024 and 3072, 45.4 (49.5) at 2560 and 7680 (157 MB, 32 us at the rate
+// of a large copy); a product by itself 7.6 us (9.8) for 5120 x 2560, 31.6 (32.2) for 32000 x 2560.
+// ---------------------------------------------------------------------------------------
+enum Front { kNoNorm = 0, kNorm = 1, kAddNorm = 2 };
+constexpr int kRowsMax = 2;
+// Two rows' arithmetic (16 multiply-adds beside 8 conversions a load, on the vector units) is no longer hidden behind
+// the loads of a large matrix: 5120 x 2560 takes 8.2 us here and 9.9 in tiles, 2560 x 7680 12.8 and 12.4, 32000 x 512
+// 9.9 and 8.3.  At four rows already 5120 x 2560 has little left (9.4), a layer of 2560 loses (68 to 50).
+constexpr size_t kRowsTwoWeights = 14 << 20;
+constexpr int kRowsFourFrom = 4096;
+constexpr int kRowsBlocks = 1024;                  // (512 and 2048 measure the same)
+constexpr int kChunk = 8 * kWave;                  // input channels a wave's lanes cover with one load each
+
+struct NormArgs {
+    const bf16_t* hidden;
+    const float* delta;
+    const bf16_t* weight;
+    float eps;
+    bf16_t* hidden_out;
+};
+
+template <int MR, int C, int EPI, int FRONT>
+__global__ __launch_bounds__(kThreads) void decode_rows_kernel(const bf16_t* __restrict__ x, NormArgs norm,
+                                                               const bf16_t* __restrict__ w, void* __restrict__ out,
+                                                               int M, int N, int K) {
+    // loads of a lane in flight: eight of weights, or twelve with those of x
+    constexpr int kUnroll = FRONT != kNoNorm ? 8 / C : 12 / (C + MR);
+    constexpr int kOut = EPI == kStoreGelu ? C / 2 : C;   // output columns of a wave
+    extern __shared__ __align__(16) unsigned char smem[];  // FRONT: x, bf16 [MR][K]
+    __shared__ float s_sq[MR][kNormMaxThreads / kWave];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint32_t row_bytes = (uint32_t)K * 2u;
+    const int units = (N + kOut - 1) / kOut, stride = (int)gridDim.x * kWaves;
+    int unit = (int)blockIdx.x * kWaves + wv;
+
+    u32x4 rw[kUnroll][C], rx[kUnroll][MR];
+    // weights of `unit`, and x, from input channel k0 on; zeros past K and past N
+    auto load = [&](int u, int k0) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int n = u * kOut + c % kOut;
+            const size_t row = EPI == kStoreGelu && c >= kOut ? (size_t)N + n : (size_t)n;
+            const rsrc_t r = make_rsrc(w + (n < N ? row : 0) * K, u < units && n < N ? row_bytes : 0u);
+#pragma unroll
+            for (int q = 0; q < kUnroll; ++q)
+                rw[q][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                         r, (uint32_t)(k0 + q * kChunk + 8 * lane) * 2u, 0, kAuxDefault));
+        }
+        if constexpr (FRONT == kNoNorm) {
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                const rsrc_t r = make_rsrc(x + (size_t)min(m, M - 1) * K, row_bytes);
+#pragma unroll
+                for (int q = 0; q < kUnroll; ++q)
+                    rx[q][m] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                             r, (uint32_t)(k0 + q * kChunk + 8 * lane) * 2u, 0, kAuxDefault));
+            }
+        }
+    };
+    load(unit, 0);
+    __builtin_amdgcn_sched_barrier(0);
+
+    if constexpr (FRONT != kNoNorm) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const int row = min(m, M - 1);
+            for (int k0 = 0; k0 < K; k0 += 8 * kThreads) {   // (sums per 512 channels, in add_norm_kernel's order)
+                const int k = k0 + 8 * tid;
+                float sq = 0.0f;
+                if (k < K) {
+                    const size_t at = (size_t)row * K + k;
+                    u32x4 r = load_raw<bf16_t, 8>(norm.hidden + at);
+                    float v[8];
+                    unpack(r, v);
+                    if constexpr (FRONT == kAddNorm) {
+                        const f32x4 d0 = *reinterpret_cast<const f32x4*>(norm.delta + at);
+                        const f32x4 d1 = *reinterpret_cast<const f32x4*>(norm.delta + at + 4);
+                        float add[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+                        pack(add, r);                  // rounded where a separate projection rounds its output
+                        unpack(r, add);
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[i] += add[i];
+                        pack(v, r);
+                        if (blockIdx.x == 0 && m < M) *reinterpret_cast<u32x4*>(norm.hidden_out + at) = r;
+                        unpack(r, v);                  // the norm sees the hidden state as it is kept
+                    }
+                    *reinterpret_cast<u32x4*>(smem + (size_t)m * row_bytes + 2 * k) = r;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) sq = fmaf(v[i], v[i], sq);
+                }
+#pragma unroll
+                for (int o = kWave / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+                if (lane == 0) s_sq[m][k0 / kChunk + wv] = sq;
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            float total = 0.0f;
+            for (int q = 0; q < ceil_div(K, kChunk); ++q) total += s_sq[m][q];
+            const float scale = 1.0f / sqrtf(total / (float)K + norm.eps);
+            for (int k = 8 * tid; k < K; k += 8 * kThreads) {
+                u32x4* p = reinterpret_cast<u32x4*>(smem + (size_t)m * row_bytes + 2 * k);
+                float v[8], g[8];
+                unpack(*p, v);
+                unpack(load_raw<bf16_t, 8>(norm.weight + k), g);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) g[i] *= v[i] * scale;
+                pack(g, *p);
+            }
+        }
+        lds_barrier();
+    }
+
+    for (; unit < units; unit += stride) {
+        float acc[C][MR];
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) acc[c][m] = 0.0f;
+        for (int k0 = 0; k0 < K; k0 += kUnroll * kChunk) {
+            u32x4 cw[kUnroll][C], cx[kUnroll][MR];
+#pragma unroll
+            for (int q = 0; q < kUnroll; ++q) {
+#pragma unroll
+                for (int c = 0; c < C; ++c) cw[q][c] = rw[q][c];
+#pragma unroll
+                for (int m = 0; m < MR; ++m)
+                    if constexpr (FRONT == kNoNorm) cx[q][m] = rx[q][m];
+            }
+            const bool last = k0 + kUnroll * kChunk >= K;
+            load(last ? unit + stride : unit, last ? 0 : k0 + kUnroll * kChunk);
+#pragma unroll
+            for (int q = 0; q < kUnroll; ++q) {
+                const int k = k0 + q * kChunk + 8 * lane;
+                if (k0 + q * kChunk >= K) break;   // (the same in every lane)
+                float xv[MR][8];
+#pragma unroll
+                for (int m = 0; m < MR; ++m) {
+                    if constexpr (FRONT == kNoNorm) {
+                        unpack(cx[q][m], xv[m]);
+                    } else {
+                        u32x4 r = {0u, 0u, 0u, 0u};
+                        if (k < K) r = *reinterpret_cast<const u32x4*>(smem + (size_t)m * row_bytes + 2 * k);
+                        unpack(r, xv[m]);
+                    }
+                }
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    float wf[8];
+                    unpack(cw[q][c], wf);
+#pragma unroll
+                    for (int m = 0; m < MR; ++m)
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) acc[c][m] = fmaf(wf[i], xv[m][i], acc[c][m]);
+                }
+            }
+        }
+        // lane c MR + m finishes output column c of row m
+        float mine = 0.0f, up = 0.0f;
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                float v = acc[c][m];
+#pragma unroll
+                for (int o = kWave / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+                if (lane == (c % kOut) * MR + m) {
+                    if (c < kOut) mine = v;
+                    else up = v;
+                }
+            }
+        const int n = unit * kOut + lane / MR, m = lane % MR;
+        if (lane < kOut * MR && n < N && m < M) {
+            if constexpr (EPI == kStorePartial) {
+                static_cast<float*>(out)[(size_t)m * N + n] = mine;
+            } else {
+                float r = mine;
+                if constexpr (EPI == kStoreGelu) {
+                    const uint32_t projected = pack_bf16x2(mine, up);
+                    const float g = gelu_times(bf16_lo(projected), 1.0f);
+                    r = bf16_lo(pack_bf16x2(g, g)) * bf16_hi(projected);
+                }
+                const uint32_t b = pack_bf16x2(r, r);
+                reinterpret_cast<unsigned short*>(out)[(size_t)m * N + n] = (unsigned short)b;
+            }
+        }
+    }
+}
+
+inline bool takes_rows(int M, int N, int K) {
+    return M == 1 || (M <= kRowsMax && (size_t)N * K <= kRowsTwoWeights);
+}
+
+// Workgroups: a wave per C weight rows, C two where four would leave compute units without a wave each.
+template <int EPI, int FRONT>
+int rows_product(const void* x, const NormArgs& norm, const void* w, void* out, int M, int N, int K, hipStream_t st) {
+    const int cols = EPI == kStoreGelu ? 2 * N : N;
+    const bool four = cols > kRowsFourFrom;        // four: a wave per SIMD of the chip
+    const int units = ceil_div(cols, four ? 4 : 2);
+    int blocks = ceil_div(units, kWaves);
+    if (blocks > kRowsBlocks) blocks = kRowsBlocks;
+    const size_t lds = FRONT == kNoNorm ? 0 : (size_t)M * K * 2;
+    const bf16_t* xp = static_cast<const bf16_t*>(x);
+    const bf16_t* wp = static_cast<const bf16_t*>(w);
+#define HAWK_ROWS(MR)                                                                                               \
+    if (four)                                                                                                       \
+        hipLaunchKernelGGL((decode_rows_kernel<MR, 4, EPI, FRONT>), dim3((unsigned)blocks), dim3(kThreads), lds, st, xp, \
+                           norm, wp, out, M, N, K);                                                                 \
+    else                                                                                                            \
+        hipLaunchKernelGGL((decode_rows_kernel<MR, 2, EPI, FRONT>), dim3((unsigned)blocks), dim3(kThreads), lds, st, xp, \
+                           norm, wp, out, M, N, K)
+    if (M == 1) { HAWK_ROWS(1); }
+    else { HAWK_ROWS(2); }
+#undef HAWK_ROWS
+    return hipGetLastError() == hipSuccess ? HAWK_OK : HAWK_ERR_LAUNCH;
+}
+
 // How a product is cut: rows and columns of a tile, tiles in flight, workgroups along K.
 struct Cut {
     int mt, nt, depth, splits;
@@ -584,6 +815,7 @@ size_t decode_layer_workspace_bytes(int M, int H, int R, int I, int n_next) {
 }
 
 int decode_linear(const void* x, const void* w, void* out, int M, int N, int K, void* ws, hipStream_t st) {
+    if (takes_rows(M, N, K)) return rows_product<kStoreBf16, kNoNorm>(x, NormArgs{}, w, out, M, N, K, st);
     const Cut c = cut_for(M, N, K, false, true);
     if (c.splits == 1) return gemm<kStoreBf16>(x, w, out, M, N, K, cut_for(M, N, K, false, false), st);
     if (int rc = gemm<kStorePartial>(x, w, ws, M, N, K, c, st)) return rc;
@@ -592,6 +824,10 @@ int decode_linear(const void* x, const void* w, void* out, int M, int N, int K, 
 
 int decode_norm_linear(void* hidden, const void* norm_w, float eps, const void* w, void* out, int M, int N, int H,
                        void* ws, hipStream_t st) {
+    if (takes_rows(M, N, H)) {
+        const NormArgs norm{static_cast<const bf16_t*>(hidden), nullptr, static_cast<const bf16_t*>(norm_w), eps, nullptr};
+        return rows_product<kStoreBf16, kNorm>(nullptr, norm, w, out, M, N, H, st);
+    }
     if (int rc = add_norm(hidden, nullptr, 0, norm_w, eps, ws, M, H, st)) return rc;
     return decode_linear(ws, w, out, M, N, H, static_cast<char*>(ws) + align256((size_t)M * H * 2), st);
 }
@@ -604,6 +840,17 @@ int decode_layer_tail(const void* gated, const void* w_resid, void* hidden, cons
     void* normed = p;
     void* act = p + align256((size_t)M * H * 2);
     float* partial = reinterpret_cast<float*>(p + align256((size_t)M * H * 2) + align256((size_t)M * I * 2));
+    if (takes_rows(M, H, R) && takes_rows(M, 2 * I, H) && takes_rows(M, H, I) && takes_rows(M, n_next, H)) {
+        // the hidden state between the two norms lies where the wider step keeps its normed rows
+        const NormArgs first{static_cast<const bf16_t*>(hidden), partial, static_cast<const bf16_t*>(norm_w), eps,
+                             static_cast<bf16_t*>(normed)};
+        const NormArgs second{static_cast<const bf16_t*>(normed), partial, static_cast<const bf16_t*>(next_norm_w),
+                              next_eps, static_cast<bf16_t*>(hidden)};
+        if (int rc = rows_product<kStorePartial, kNoNorm>(gated, NormArgs{}, w_resid, partial, M, H, R, st)) return rc;
+        if (int rc = rows_product<kStoreGelu, kAddNorm>(nullptr, first, w_gate_up, act, M, I, H, st)) return rc;
+        if (int rc = rows_product<kStorePartial, kNoNorm>(act, NormArgs{}, w_down, partial, M, H, I, st)) return rc;
+        return rows_product<kStoreBf16, kAddNorm>(nullptr, second, w_next, next_out, M, n_next, H, st);
+    }
     const Cut resid = cut_for(M, H, R, false, true), down = cut_for(M, H, I, false, true);
     if (int rc = gemm<kStorePartial>(gated, w_resid, partial, M, H, R, resid, st)) return rc;
     if (int rc = add_norm(hidden, partial, resid.splits, norm_w, eps, normed, M, H, st)) return rc;

@@ -8,7 +8,7 @@ namespace hawk {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+__host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 // A barrier for what was written to LDS alone: loads from memory stay in flight across it.
 __device__ __forceinline__ void lds_barrier() {

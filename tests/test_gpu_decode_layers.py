@@ -29,7 +29,11 @@ def _exact_linear(x, w):
                                    (64, 136, 640), (65, 328, 640), (128, 520, 256), (129, 5120, 2560), (256, 8, 128),
                                    (255, 264, 7680), (70, 26000, 256), (200, 13064, 384),
                                    # more workgroups than compute units, tiles of 128 and of 64 columns, and one pair of steps
-                                   (200, 17000, 256), (129, 9000, 640), (150, 9000, 128)])
+                                   (200, 17000, 256), (129, 9000, 640), (150, 9000, 128),
+                                   # up to four rows: two and four columns a wave, more columns than waves, ends of
+                                   # the loads of 512 channels, the loop over them
+                                   (1, 4104, 640), (2, 4096, 1152), (3, 20008, 384), (4, 16392, 512), (4, 72, 7680),
+                                   (5, 4104, 640)])
 def test_linear_matches_64_bit_sums(M, N, K):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(M + N + K)
@@ -57,7 +61,11 @@ def test_linear_matches_64_bit_sums(M, N, K):
                                                 (200, 4096, 512, 640, 72), (64, 8192, 512, 1024, 72),
                                                 # gated GELU in 128-wide tiles of ragged rows (its columns, a
                                                 # multiple of 128, are whole tiles), loads 4 and 2 steps ahead
-                                                (200, 256, 256, 13056, 64), (131, 384, 384, 12928, 72)])
+                                                (200, 256, 256, 13056, 64), (131, 384, 384, 12928, 72),
+                                                # up to four rows: either side of what their norm keeps in LDS and
+                                                # of four columns a wave
+                                                (4, 6144, 128, 256, 72), (4, 6272, 128, 256, 72), (2, 8192, 256, 128, 8),
+                                                (1, 2560, 2560, 7680, 5120), (2, 640, 384, 2304, 5000), (4, 512, 512, 1024, 1024)])
 def test_layer_tail_matches_the_separate_operations(M, H, R, inter, n_next):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(H + M)
