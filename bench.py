@@ -15,7 +15,7 @@ forward, input gradient, weight gradients) on 32768 tokens, D = 2560, 10 blocks,
 ``--workload block`` chains the whole recurrent core of one layer at B=8, T=4096, D=2560 (conv and
 both gate projections in one kernel, scan fused with the output gate, and the backward of all of
 them) through the C ABI on the [B,T,2D] output of the block's input projection in place, one host call
-per direction: six large launches that move 30 activation-sized tensors, one that rounds the fp32
+per direction: five large launches that move 28 activation-sized tensors, one that rounds the fp32
 weights of both gates to bf16 (as the Python host does at this size) and one for the three closing
 reductions of the backward; ``--unfused-conv`` runs the single entry points instead (the conv as a
 launch of its own on a copy of the x half, seven large launches and 31 tensors, two weight casts,
@@ -350,7 +350,9 @@ def run_block(args, lib, dev):
     dcw, dcb = torch.empty_like(cw), torch.empty_like(cb)
     ws = torch.zeros(lib.hawk_scan_workspace_bytes(B, T, D, code), dtype=torch.uint8, device=dev)
     gws = torch.empty(lib.hawk_gate_proj_bwd_weights_workspace_bytes(M, D, nb), dtype=torch.uint8, device=dev)
-    cws = torch.empty(lib.hawk_conv1d_bwd_workspace_bytes(B, T, D, W), dtype=torch.uint8, device=dev)
+    cws_bytes = (lib.hawk_conv1d_bwd_workspace_bytes if args.unfused_conv
+                 else lib.hawk_block_core_grads_conv_workspace_bytes)(B, T, D, W)
+    cws = torch.empty(cws_bytes, dtype=torch.uint8, device=dev)
     st = torch.cuda.current_stream(dev).cuda_stream
     p = lambda t: t.data_ptr()  # noqa: E731
 
@@ -379,11 +381,10 @@ def run_block(args, lib, dev):
 
     def bwd():
         if not args.unfused_conv:
-            # one host call: gated scan -> the projections' input gradient onto the scan's, in place
-            # -> conv (right behind the kernel that wrote its input gradient: part of those 168 MB is
-            # then still in the memory-side cache, 1 % of the step) -> the projections' weight
-            # gradients -> one launch for the three closing reductions
-            _lib.check("block_core_bwd", lib.hawk_block_core_bwd(
+            # one host call: gated scan -> the projections' input gradient onto the scan's and the conv's
+            # backward in one kernel -> the projections' weight gradients -> one launch for the three
+            # closing reductions
+            _lib.check("block_core_grads", lib.hawk_block_core_grads(
                 p(xy), 2 * D, p(u), p(xg), p(ag), p(h), p(cw), p(wi16), p(wa16), code, p(lam), p(gout), p(dxy),
                 2 * D, p(du), p(dxg), p(dag), p(dcw), p(dcb), p(dwi), p(dbi), p(dwa), p(dba), p(dlam), B, T, D, nb,
                 W, p(ws), ws.numel(), p(gws), gws.numel(), p(cws), cws.numel(), st))
@@ -423,8 +424,8 @@ def run_block(args, lib, dev):
     bwd_ms = float(np.mean([e_[1].elapsed_time(e_[2]) for e_ in ev]))
     ms_per_step = wall * 1e3 / args.steps
     # tensors moved: conv 2, gates 3 (conv + gates in one kernel: 4), gated scan 6 | gated scan 10,
-    # gate dx 4, gate dw 3, conv 3
-    fwd_bytes, bwd_bytes = (11 if args.unfused_conv else 10) * 2 * N, 20 * 2 * N
+    # gate dx 4, gate dw 3, conv 3 (gate dx + conv in one kernel: 5)
+    fwd_bytes, bwd_bytes = (11 if args.unfused_conv else 10) * 2 * N, (20 if args.unfused_conv else 18) * 2 * N
     step_gbs = (fwd_bytes + bwd_bytes) / (ms_per_step * 1e-3) / 1e9
     return {
         "metric": "Hawk recurrent core (conv, gate projections, gated scan) fwd+bwd tokens/s, 1 GPU",
