@@ -140,23 +140,30 @@ struct Call {
 };
 
 // Workspaces that Python keeps per (device, stream), seen once per stream; inside a capture Python is asked every time.
+// Between Python's answer and the entry here another thread may have it replaced or dropped (clear()): such an answer
+// serves its call, which holds it, and is not kept.
 struct Workspaces {
     const char* name;
     std::mutex mutex;
     std::map<std::pair<int, void*>, Tensor> kept;
+    uint64_t cleared = 0;
 
+    explicit Workspaces(const char* n) : name(n) {}
     Tensor get(const Call& c, size_t bytes) {
         const bool capturing = c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
         const std::pair<int, void*> key{c.dev.index(), c.st};
+        uint64_t before = 0;
         if (!capturing) {
             std::lock_guard<std::mutex> lock(mutex);
             auto it = kept.find(key);
             if (it != kept.end() && (size_t)it->second.numel() >= bytes) return it->second;
+            before = cleared;
         }
+        // (Python clears in here too, where it makes or replaces a buffer: the stream's next call keeps that one)
         Tensor ws = in_python([&] { return callable(name)((int)c.dev.index(), bytes).cast<Tensor>(); });
         if (!capturing) {
             std::lock_guard<std::mutex> lock(mutex);
-            kept[key] = ws;
+            if (cleared == before) kept[key] = ws;
         }
         return ws;
     }
@@ -164,11 +171,12 @@ struct Workspaces {
         std::map<std::pair<int, void*>, Tensor> old;
         std::lock_guard<std::mutex> lock(mutex);
         old.swap(kept);
+        ++cleared;
     }
 };
-Workspaces& scan_workspaces() { static auto* w = new Workspaces{"scan_workspace", {}, {}}; return *w; }
-Workspaces& gate_workspaces() { static auto* w = new Workspaces{"gate_workspace", {}, {}}; return *w; }
-Workspaces& decode_workspaces() { static auto* w = new Workspaces{"decode_workspace", {}, {}}; return *w; }
+Workspaces& scan_workspaces() { static auto* w = new Workspaces("scan_workspace"); return *w; }
+Workspaces& gate_workspaces() { static auto* w = new Workspaces("gate_workspace"); return *w; }
+Workspaces& decode_workspaces() { static auto* w = new Workspaces("decode_workspace"); return *w; }
 
 // ---------------------------------------------------------------------------------------
 // What the nodes take

@@ -123,17 +123,55 @@ def test_other_forms_stay_with_the_python_functions():
         hk.fused_linear_scan(*(torch.randn(1, 9, 64) for _ in range(3)), _lam(64))
 
 
-def test_a_replaced_workspace_is_seen_by_native_code():
+def test_a_replaced_workspace_is_seen_by_native_code(monkeypatch):
+    asked, real = [], _lib.scan_workspace
+    monkeypatch.setattr(_lib, "scan_workspace", lambda dev, n: (asked.append(real(dev, n)), asked[-1])[1])
+    hk.release_workspaces()
     x, xg, ag = (torch.randn(1, 300, 64, device="cuda") for _ in range(3))
     lam = _lam(64)
     want = hk.fused_linear_scan(x, xg, ag, lam)
-    key = next(iter(_lib._workspaces))
-    first = _lib._workspaces[key].data_ptr()
-    big = (torch.randn(4, 4096, 1024, device="cuda") for _ in range(3))
-    hk.fused_linear_scan(*big, _lam(1024))            # needs a larger one
+    hk.fused_linear_scan(x, xg, ag, lam)
+    key, = _lib._workspaces
+    first, calls = _lib._workspaces[key], len(asked)
     assert torch.equal(hk.fused_linear_scan(x, xg, ag, lam), want)
+    assert len(asked) == calls and asked[-1] is first      # kept: Python is not asked again
+    big = (torch.randn(4, 4096, 1024, device="cuda") for _ in range(3))
+    hk.fused_linear_scan(*big, _lam(1024))                 # needs a larger one
+    grown = _lib._workspaces[key]
+    assert grown.numel() > first.numel() and grown.data_ptr() != first.data_ptr()
+    # the small call has the new one too: native code asks for it, or keeps it already
+    assert torch.equal(hk.fused_linear_scan(x, xg, ag, lam), want)
+    assert len(asked) > calls and asked[-1] is grown
     hk.release_workspaces()
     assert not _lib._workspaces
     assert torch.equal(hk.fused_linear_scan(x, xg, ag, lam), want)
-    assert len(_lib._workspaces) == 1 and first is not None
+    assert _lib._workspaces[key] is asked[-1] and asked[-1] is not grown
+    hk.check_scan_status()
+
+
+@pytest.mark.parametrize("other", ["releases", "grows"])
+def test_a_workspace_that_changes_while_native_code_asks_for_it_is_not_kept(other, monkeypatch):
+    """Another thread may release or replace a stream's workspace between Python's answer and native code's note of
+    it; here it does so inside the question."""
+    asked, real = [], _lib.scan_workspace
+
+    def question(dev, nbytes):
+        ws = real(dev, nbytes)
+        if not asked:
+            if other == "releases":
+                hk.release_workspaces()
+            else:
+                real(dev, 4 * ws.numel())
+        asked.append(ws)
+        return ws
+
+    hk.release_workspaces()
+    monkeypatch.setattr(_lib, "scan_workspace", question)
+    x, xg, ag = (torch.randn(1, 300, 64, device="cuda") for _ in range(3))
+    lam = _lam(64)
+    want = hk.fused_linear_scan(x, xg, ag, lam)
+    for _ in range(3):
+        assert torch.equal(hk.fused_linear_scan(x, xg, ag, lam), want)
+    held, = _lib._workspaces.values()
+    assert asked[0] is not held and asked[-1] is held
     hk.check_scan_status()
