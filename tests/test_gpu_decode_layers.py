@@ -30,10 +30,15 @@ def _exact_linear(x, w):
                                    (255, 264, 7680), (70, 26000, 256), (200, 13064, 384),
                                    # more workgroups than compute units, tiles of 128 and of 64 columns, and one pair of steps
                                    (200, 17000, 256), (129, 9000, 640), (150, 9000, 128),
-                                   # up to four rows: two and four columns a wave, more columns than waves, ends of
-                                   # the loads of 512 channels, the loop over them
-                                   (1, 4104, 640), (2, 4096, 1152), (3, 20008, 384), (4, 16392, 512), (4, 72, 7680),
-                                   (5, 4104, 640)])
+                                   # one and two rows without tiles: two and four columns a wave, ends of the loads
+                                   # of 512 channels and the loop over them; more columns than 4096 waves take at
+                                   # once, with a last round of few waves and of all of them
+                                   (1, 4104, 640), (2, 4096, 1152), (1, 72, 7680), (2, 72, 7680), (1, 20008, 384),
+                                   (2, 20008, 384), (1, 32000, 512), (1, 32768, 1152), (2, 16392, 640),
+                                   # two rows: the most weights they take so, and the fewest they leave to the tiles
+                                   (2, 28672, 512), (2, 28680, 512),
+                                   # three to five rows are tiles
+                                   (3, 20008, 384), (4, 16392, 512), (4, 72, 7680), (5, 4104, 640)])
 def test_linear_matches_64_bit_sums(M, N, K):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(M + N + K)
@@ -62,10 +67,17 @@ def test_linear_matches_64_bit_sums(M, N, K):
                                                 # gated GELU in 128-wide tiles of ragged rows (its columns, a
                                                 # multiple of 128, are whole tiles), loads 4 and 2 steps ahead
                                                 (200, 256, 256, 13056, 64), (131, 384, 384, 12928, 72),
-                                                # up to four rows: either side of what their norm keeps in LDS and
-                                                # of four columns a wave
-                                                (4, 6144, 128, 256, 72), (4, 6272, 128, 256, 72), (2, 8192, 256, 128, 8),
-                                                (1, 2560, 2560, 7680, 5120), (2, 640, 384, 2304, 5000), (4, 512, 512, 1024, 1024)])
+                                                # one and two rows without tiles: the widest norm, two and four
+                                                # columns a wave; more of them than 4096 waves take at once, of the
+                                                # next projection and of gate and up
+                                                (2, 8192, 256, 128, 8), (1, 8192, 128, 256, 72),
+                                                (1, 2560, 2560, 7680, 5120), (2, 640, 384, 2304, 5000),
+                                                (1, 512, 512, 1024, 32000), (2, 384, 256, 640, 20008),
+                                                (1, 640, 384, 8448, 72), (2, 256, 384, 9088, 520),
+                                                # two rows, one product of the layer beyond what they take: all tiles
+                                                (2, 512, 512, 1024, 28680),
+                                                # four rows are tiles
+                                                (4, 6144, 128, 256, 72), (4, 6272, 128, 256, 72), (4, 512, 512, 1024, 1024)])
 def test_layer_tail_matches_the_separate_operations(M, H, R, inter, n_next):
     lib = _lib.load()
     gen = torch.Generator("cuda").manual_seed(H + M)
