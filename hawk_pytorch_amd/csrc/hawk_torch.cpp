@@ -28,6 +28,7 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <optional>
@@ -670,11 +671,24 @@ std::tuple<Tensor, std::optional<Tensor>, Tensor> add_norm_bwd(const Tensor& dou
     return {d_sum, d_delta, d_weight};
 }
 
-// dy^T x of [n, N] and [n, K] each: in fp32 and together in one launch, but for large results over many rows, where the
-// library's product is faster, in bf16.  The line is at 256 tiles of 128 x 128 and 2048 rows: up to there the kernel was
-// ahead of the library's product and its conversion at every size measured (4096 x 1024 at 6144 rows 66.4 against
-// 70.6 us, 32000 x 512 at 1000 rows 52.0 against 63.5 and at 2048 90.2 against 89.4); beyond it is behind at most
-// (32000 x 512 at 4000 rows 169 against 149, 8192 x 2048 156 against 146, 2560 x 2560 at 6144 110 against 103).
+// Whether the library's product, with its result in fp32, takes a weight gradient [rows, columns] over a sum of n: results
+// of more than 256 tiles of 128 x 128 over more than 2048 rows, or 4096 and more wide both ways over more than 1024.
+// Kernel / library in us, replayed:
+//   the four weights of a layer in one launch, or those of more than 256 tiles by the library
+//              1024 channels, MLP 2048: 45 / 43 at 1100 rows, 53 / 49 at 1500, 130 / 130 at 4096 (all four by the library
+//              77, 96, 167); 1536 and 4608: 115 / 128, 127 / 160, 292 / 298; 2560 and 7680: 273 / 291, 345 / 364, at 2048
+//              431 / 396, at 3000 618 / 599; 4096 and 12288: 700 / 567, 885 / 708, 1111 / 825, 1532 / 1177; 5120 and 15360
+//              1027 / 945, 1305 / 1187, 1684 / 1352
+//   a head's   32000 x 512 65 / 54 at 1100 rows, 78 / 66 at 1500, 97 / 79 at 2048, 171 / 146 at 4096; 32000 x 768 91 / 87,
+//              111 / 126, 135 / 116; 8192 x 1024 32 / 34, 37 / 43, 52 / 44; 32000 x 4096 462 / 366, 576 / 461, 727 / 538
+// Up to 2048 rows of a narrow head the difference does not show in a pass (two layers, replayed, kernel and library: 512
+// channels 756 / 761 at 1100 rows, 814 / 818 at 1500, 905 / 902 at 2048; 768 921 / 941, 1030 / 1066, 1200 / 1191; 1024
+// 1124 / 1131, 1283 / 1278, 1434 / 1411), and the library's call costs the host 13 us more.
+bool library_weight_grad(int64_t n, int64_t rows, int64_t columns) {
+    const int64_t tiles = ((rows + 127) / 128) * ((columns + 127) / 128);
+    return tiles > 256 && (n > 2048 || (n > 1024 && std::min(rows, columns) >= 4096));
+}
+// dy^T x of [n, N] and [n, K] each, in fp32: together in one launch, but for those that the library takes.
 std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& products) {
     Call c(products[0].first.device());
     const int n = products[0].first.size(0);
@@ -685,9 +699,8 @@ std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& p
     for (size_t k = 0; k < products.size(); ++k) {
         const auto& [g, in] = products[k];
         const int rows = g.size(1), cols = in.size(1);
-        const bool large = (int64_t)((rows + 127) / 128) * ((cols + 127) / 128) > 256 && n > 2048;
-        if (large || !lib.hawk_weight_grad_supported(n, rows, cols)) {
-            out[k] = at::mm(g.t(), in);
+        if (library_weight_grad(n, rows, cols) || !lib.hawk_weight_grad_supported(n, rows, cols)) {
+            out[k] = at::mm(g.t(), in, kF32);
             continue;
         }
         out[k] = c.empty({rows, cols}, kF32);
@@ -702,17 +715,27 @@ std::vector<Tensor> weight_grads(const std::vector<std::pair<Tensor, Tensor>>& p
 }
 Tensor weight_grad(const Tensor& dy, const Tensor& x) { return weight_grads({{dy, x}})[0]; }
 
-// x w^T of [n, K] and [N, K], and dy w of [n, N] and [N, K]: by own kernels up to 256 tiles of 128 x 128 of results.
-// There they are ahead of the library's (2048 rows, layers of 512: 6.6, 5.0, 9.3 and 7.0 us against 7.6, 6.3, 10.0 and 7.8,
-// input gradients 7.5, 5.3, 11.9 and 6.9 against 9.3, 7.5, 13.7 and 9.3; a head's over 32000 94 against 201) or, near the
-// line and at a hundred rows of a long sum, within a tenth and 4 us of them, and their launch costs the host 4 us
-// instead of 17; beyond it the library's larger tiles win (4096 x 1024 over 4000 rows 30 against 49).
+// x w^T of [n, K] and [N, K], and dy w of [n, N] and [N, K]: by own kernels up to 256 tiles of 128 x 128 of results; their
+// launch costs the host 4 us, a library product 17.
+// An input gradient's operand lies across the sum, and the library's products of that kind are the slower ones: of 120
+// sizes of 512 to 4096 channels and heads of 32000 at 100 to 4096 rows the kernels are ahead at 98 (dx of 15360 x 2560 at
+// 1024 rows 146 / 204 us, 9216 x 1536 at 512 41 / 61, 32000 x 512 at 2048 107 / 210), level within 9 % at 17 and behind at
+// five (4096 x 1024 at 1500 and 3000 rows 33 / 28 and 47 / 41, 2560 x 2560 at 1500 41 / 29).
 bool own_product(int64_t rows, int64_t columns, int64_t sum) {
     return ((rows + 127) / 128) * ((columns + 127) / 128) <= 256 && lib.hawk_linear_supported(rows, columns, sum);
 }
+// An output's operands lie along the sum.  The kernels are ahead up to 2^31 multiply-adds (own / library in us: 1024 x 1024 at
+// 1024 rows 7.1 / 9.0 and at 2048 10.3 / 10.6, 4096 x 1024 at 512 10.0 / 10.7, 1024 x 512 at 4096 9.7 / 11.1, 9216 x 1536
+// at 100 16.3 / 18.7) and behind beyond (1024 x 1024 at 4096 14.7 / 12.9, 2048 x 1024 at 2048 15.2 / 13.1, 1536 x 4608 at
+// 1024 37.7 / 28.0, 15360 x 2560 at 100 30.6 / 25.0), but for one tile of rows over a sum longer than the row of results,
+// which they split (4096 x 12288 at 100 32.4 / 41.6).  Short of the line they are up to 3 us behind at a hundred rows
+// (1536 x 4608 13.4 / 10.8, 2560 x 2560 12.3 / 10.7), less than their launch saves the host.
+bool own_output(int64_t rows, int64_t columns, int64_t sum) {
+    return own_product(rows, columns, sum) && (rows * columns * sum <= (int64_t)1 << 31 || (rows <= 128 && sum > columns));
+}
 Tensor layer_linear(const Tensor& x, const Tensor& w) {
     const int n = x.size(0), N = w.size(0), K = w.size(1);
-    if (!own_product(n, N, K)) return at::mm(x, w.t());
+    if (!own_output(n, N, K)) return at::mm(x, w.t());
     Call c(x.device());
     Tensor out = c.empty({n, N}, kBF16);
     const size_t bytes = lib.hawk_linear_workspace_bytes(n, N, K);
@@ -782,17 +805,8 @@ std::vector<Tensor> layer_bwd(const std::vector<Tensor>& s, const Tensor& d_tota
     const Tensor d_xy = d_xy_.view({rows, 2 * R});
     const Tensor d_x1 = input_grad(d_xy, w_in);
     // (all four at the end: each alone is too few tiles for the chip)
-    std::vector<Tensor> g = weight_grads({{d_gu, x2}, {d_out, act}, {d_xy, x1}, {*d_mixed, gated.view({rows, R})}});
+    const std::vector<Tensor> g = weight_grads({{d_gu, x2}, {d_out, act}, {d_xy, x1}, {*d_mixed, gated.view({rows, R})}});
     auto [d_hidden, d_delta, g_n1] = add_norm_bwd(d_x1, total1, rstd1, n1, d_total1, want_delta);
-    // gradients that the library's products left in bf16, converted by one launch
-    std::vector<Tensor*> narrow;
-    std::vector<Tensor> in;
-    for (Tensor& t : g)
-        if (t.scalar_type() != kF32) narrow.push_back(&t), in.push_back(t);
-    if (!in.empty()) {
-        const std::vector<Tensor> wide = cast_in(c, in, kF32);
-        for (size_t k = 0; k < wide.size(); ++k) *narrow[k] = wide[k];
-    }
     const int64_t nb = wi.size(0), bw = wi.size(1);
     return {d_hidden.view({B, T, H}), d_delta.has_value() ? d_delta->view({B, T, H}) : Tensor(), g_n1, g_n2, g[2], g[3], g[0],
             g[1], dcw, dcb, dwi, dbi.view({nb, bw}), dwa, dba.view({nb, bw}), dlam};
@@ -826,8 +840,7 @@ std::vector<Tensor> loss_bwd(const std::vector<Tensor>& s, const Tensor& labels,
         data(logits), data<const long long>(labels), data<float>(s[6]), data<float>(s[7]), data<float>(d_loss),
         data(d_logits), shape[0], shape[1], s[1].size(0), c.st));
     const Tensor d_x = input_grad(d_logits, s[1]);
-    Tensor d_head = weight_grad(d_logits, s[3]);
-    if (d_head.scalar_type() != kF32) d_head = cast_in(c, {d_head}, kF32)[0];
+    const Tensor d_head = weight_grad(d_logits, s[3]);
     auto [d_hidden, d_delta, d_norm] = add_norm_bwd(d_x, s[2], s[4], s[0], std::nullopt, want_delta);
     return {d_hidden.view(shape), d_delta.has_value() ? d_delta->view(shape) : Tensor(), d_norm, d_head};
 }

@@ -247,9 +247,11 @@ def test_second_derivatives_frozen_parameters_and_saved_tensor_hooks():
         assert float((g - w).norm()) <= 2e-2 * float(w.norm())
 
 
-# a single value, ragged edges of a tile in all three sizes, rows that end inside a step, one and several splits
+# a single value, ragged edges of a tile in all three sizes, rows that end inside a step, one and several splits; the
+# library's product: more than 256 tiles beyond 2048 rows, 4096 wide beyond 1024, sizes the kernel refuses
 @pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (64, 128, 128), (77, 136, 120), (513, 264, 136), (1024, 128, 256),
-                                      (2047, 1024, 512), (4593, 8, 1032), (130, 2048, 1024)])
+                                      (2047, 1024, 512), (4593, 8, 1032), (130, 2048, 1024), (2048, 2056, 2048),
+                                      (2049, 2056, 2048), (1024, 4096, 4096), (1025, 4096, 4096), (33, 12, 20)])
 def test_weight_gradient(rows, N, K):
     gen = _gen(rows)
     dy, x = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, rows, K, dtype=torch.bfloat16)
