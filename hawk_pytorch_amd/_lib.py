@@ -209,7 +209,7 @@ def native():
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_hawk_torch", loader))
         loader.exec_module(module)
         module.bind({name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in module.functions()},
-                    _native_callables())
+                    _native_callables(), _STAGGER_MIN_BYTES)
         _native = module
         return module
 

@@ -441,7 +441,7 @@ size_t hawk_input_grad_workspace_bytes(int rows, int N, int K) { return hawk_lin
 int hawk_input_grad(const void* dy, const void* w, void* dx, int rows, int N, int K, void* workspace_device,
                     size_t workspace_bytes, void* stream) {
     if (!dy || !w || !dx) return HAWK_ERR_NULL_POINTER;
-    if (!hawk::linear_supported(rows, K, N)) return HAWK_ERR_BAD_SHAPE;
+    if (!hawk_input_grad_supported(rows, N, K)) return HAWK_ERR_BAD_SHAPE;
     if (!aligned16(dy) || !aligned16(w) || !aligned16(dx) || !aligned16(workspace_device)) return HAWK_ERR_ALIGNMENT;
     const size_t need = hawk::linear_workspace_bytes(rows, K, N);
     if (need > 0 && (!workspace_device || workspace_bytes < need)) return HAWK_ERR_WORKSPACE;

@@ -48,7 +48,6 @@ namespace py = pybind11;
 
 constexpr auto kBF16 = at::kBFloat16;
 constexpr auto kF32 = at::kFloat;
-constexpr int64_t kStaggerMinBytes = 16 << 20;   // _lib.activation_empty places tensors from this size on
 
 // ---------------------------------------------------------------------------------------
 // The library and Python's part
@@ -71,6 +70,7 @@ struct Library {
 #undef X
 };
 Library lib;
+int64_t placed_from_bytes = 0;   // _lib.activation_empty places tensors from this size on
 
 // Python callables by name; never destroyed (the interpreter may be gone before this library is).
 py::dict* python = nullptr;
@@ -133,7 +133,7 @@ struct Call {
     }
     // as _lib.activation_empty, which places large ones
     Tensor activation(at::IntArrayRef shape, at::ScalarType t) const {
-        if (c10::multiply_integers(shape) * (int64_t)c10::elementSize(t) < kStaggerMinBytes) return empty(shape, t);
+        if (c10::multiply_integers(shape) * (int64_t)c10::elementSize(t) < placed_from_bytes) return empty(shape, t);
         return in_python([&] {
             return callable("activation_empty")(shape.vec(), t == kBF16, (int)dev.index()).cast<Tensor>();
         });
@@ -201,7 +201,7 @@ bool dense(const Tensor& t, at::Device dev, at::ScalarType type, at::IntArrayRef
     return dense(t, dev, type) && t.sizes() == shape;
 }
 // Elements between consecutive rows of a [B, T, D] tensor whose row b * T + t starts at (b * T + t) times that; 0 if
-// it is not laid out like this.
+// it is not laid out like this.  (scan_fused._row_stride is the same in Python, which a tracing compiler sees through.)
 int64_t row_stride(const Tensor& t) {
     const int64_t b = t.size(0), sq = t.size(1), d = t.size(2);
     if (t.stride(2) != 1 && d > 1) return 0;
@@ -638,9 +638,6 @@ std::vector<Tensor> cast_in(const Call& c, const std::vector<Tensor>& in, at::Sc
     check("hawk_cast", lib.hawk_cast(src.data(), dst.data(), counts.data(), (int)in.size(), type == kBF16, c.st));
     return out;
 }
-std::vector<Tensor> cast(const std::vector<Tensor>& in, bool to_bf16) {
-    return cast_in(Call(in[0].device()), in, to_bf16 ? kBF16 : kF32);
-}
 
 // (hidden + delta, its norm in bf16, 1 / rms) of [n, D] rows.
 std::tuple<Tensor, Tensor, Tensor> add_norm(const Tensor& hidden, const std::optional<Tensor>& delta, const Tensor& weight,
@@ -870,11 +867,12 @@ auto bound(R (*f)(A...)) {
 }  // namespace
 
 PYBIND11_MODULE(_hawk_torch, m) {
-    m.def("bind", [](const py::dict& addresses, const py::dict& callables) {
+    m.def("bind", [](const py::dict& addresses, const py::dict& callables, int64_t placed_from) {
 #define X(name) lib.name = reinterpret_cast<decltype(lib.name)>(addresses[#name].cast<uintptr_t>());
         HAWK_FUNCTIONS(X)
 #undef X
         python = new py::dict(callables);
+        placed_from_bytes = placed_from;
     });
     m.def("functions", [] {
         std::vector<std::string> names;
@@ -908,7 +906,6 @@ PYBIND11_MODULE(_hawk_torch, m) {
     m.def("decode_core", decode_core);
     m.def("decode_first", bound(decode_first));
     m.def("decode_tail", bound(decode_tail));
-    m.def("cast", bound(cast));
     m.def("add_norm", bound(add_norm));
     m.def("add_norm_bwd", bound(add_norm_bwd));
     m.def("weight_grad", bound(weight_grad));

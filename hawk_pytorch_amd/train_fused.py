@@ -28,25 +28,6 @@ EMBEDDING_MAX_ROWS = 8192
 LOSS_MAX_ROWS = (1 << 23) - 1   # hawk_cross_entropy_fwd's: a workgroup of 512 threads per row
 
 
-def _check(name: str, *args) -> None:
-    _lib.check(name, getattr(_lib.load(), name)(*args))
-
-
-def _add_norm(hidden, delta, weight, eps: float):
-    """(hidden + delta, its norm in bf16, 1 / rms) of [n, D] rows."""
-    return _lib.native().add_norm(hidden, delta, weight, eps)
-
-
-def _add_norm_backward(dout, total, rstd, weight, d_direct, want_delta: bool):
-    """(gradient of the sum in fp32, its bf16 rounding, gradient of the weight)."""
-    return _lib.native().add_norm_bwd(dout, total, rstd, weight, d_direct, want_delta)
-
-
-def _weight_grad(dy: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """dy^T x of [n, N] and [n, K]: fp32 by the kernel that splits the rows, or the library's product in bf16."""
-    return _lib.native().weight_grad(dy, x)
-
-
 def _replayed(fn, inputs, grads, needs):
     """Gradients of fn(*inputs) as a differentiable graph, for a backward pass that is itself recorded.
 

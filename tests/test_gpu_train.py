@@ -1,12 +1,14 @@
 """The kernels around the recurrent core in a training pass (hawk_train.hip) against 64-bit references,
 and the model's loss and gradients with one autograd node per layer against the modules' own."""
 
+import ctypes
+
 import pytest
 import torch
 import torch.nn.functional as F
 
 import hawk_pytorch_amd as hk
-from hawk_pytorch_amd import train_fused
+from hawk_pytorch_amd import _lib, train_fused
 
 pytestmark = pytest.mark.gpu
 
@@ -22,6 +24,10 @@ def _randn(gen, *shape, dtype=torch.float32):
     return torch.randn(*shape, generator=gen, device=DEV).to(dtype)
 
 
+def _check(name, *args):
+    _lib.check(name, getattr(_lib.load(), name)(*args))
+
+
 def _close(got, want, bound):
     assert bool(((got.double() - want).abs() <= bound).all())
 
@@ -35,14 +41,14 @@ def test_add_norm(rows, D, with_delta):
     hidden, w = _randn(gen, rows, D), _randn(gen, D) * 0.1 + 1
     delta = _randn(gen, rows, D, dtype=torch.bfloat16) if with_delta else None
     dout, direct = _randn(gen, rows, D, dtype=torch.bfloat16), _randn(gen, rows, D)
-    total, out, rstd = train_fused._add_norm(hidden, delta, w, 1e-6)
+    total, out, rstd = _lib.native().add_norm(hidden, delta, w, 1e-6)
     want = hidden + delta.float() if with_delta else hidden
     assert torch.equal(total, want)
     x, wd, dy = want.double().requires_grad_(), w.double().requires_grad_(), dout.double()
     y = x / torch.sqrt((x * x).mean(-1, keepdim=True) + 1e-6) * wd
     _close(out, y.detach(), 2.0 ** -8 * y.detach().abs() + 1e-6)
     dx, dw = torch.autograd.grad(y, (x, wd), dy)
-    d_sum, d_delta, dweight = train_fused._add_norm_backward(dout, total, rstd, w, direct, with_delta)
+    d_sum, d_delta, dweight = _lib.native().add_norm_bwd(dout, total, rstd, w, direct, with_delta)
     want_d = dx + direct.double()
     # sums of D (rows) products in fp32, over terms whose sizes the second factors bound
     _close(d_sum, want_d, 64 * EPS32 * (want_d.abs() + dx.abs().mean(-1, keepdim=True) + (dy * wd).abs().detach() + 1))
@@ -54,15 +60,13 @@ def test_add_norm(rows, D, with_delta):
 
 @pytest.mark.parametrize("rows,inter", [(1, 8), (3, 264), (257, 1024)])
 def test_gelu_mul_rounds_like_the_separate_operations(rows, inter):
-    from hawk_pytorch_amd import _lib
-
     gen = _gen(inter)
     gu = _randn(gen, rows, 2 * inter, dtype=torch.bfloat16) * 2
     dact = _randn(gen, rows, inter, dtype=torch.bfloat16)
     act, dgu = torch.empty_like(dact), torch.empty_like(gu)
     st = _lib.stream_ptr(DEV)
-    train_fused._check("hawk_gelu_mul_fwd", gu.data_ptr(), act.data_ptr(), rows, inter, st)
-    train_fused._check("hawk_gelu_mul_bwd", gu.data_ptr(), dact.data_ptr(), dgu.data_ptr(), rows, inter, st)
+    _check("hawk_gelu_mul_fwd", gu.data_ptr(), act.data_ptr(), rows, inter, st)
+    _check("hawk_gelu_mul_bwd", gu.data_ptr(), dact.data_ptr(), dgu.data_ptr(), rows, inter, st)
     leaf = gu.clone().requires_grad_()
     gate, up = leaf.chunk(2, dim=-1)
     want = F.gelu(gate) * up
@@ -151,8 +155,6 @@ def test_embedding_gradient(rows, V, D):
                                     (100, 16648)])
 @pytest.mark.parametrize("ids", ["distinct", "equal", "padded", "few", "outside"])
 def test_embedding_gradient_over_the_ways_tokens_repeat(rows, D, ids):
-    from hawk_pytorch_amd import _lib
-
     gen = _gen(rows + D)
     V = rows
     t = dict(distinct=torch.randperm(V, generator=gen, device=DEV), equal=torch.full((rows,), V - 1, device=DEV),
@@ -164,7 +166,7 @@ def test_embedding_gradient_over_the_ways_tokens_repeat(rows, D, ids):
     guard = 1024
     whole = torch.zeros(1 + V * D + guard, device=DEV)
     got = whole[1:1 + V * D].view(V, D)      # (no more than a 4-byte boundary is asked of it)
-    train_fused._check("hawk_embedding_bwd", t.data_ptr(), d.data_ptr(), got.data_ptr(), rows, V, D, _lib.stream_ptr(DEV))
+    _check("hawk_embedding_bwd", t.data_ptr(), d.data_ptr(), got.data_ptr(), rows, V, D, _lib.stream_ptr(DEV))
     known = (t >= 0) & (t < V)
     want = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, t[known], d[known].double())
     scale = torch.zeros(V, D, dtype=torch.float64, device=DEV).index_add_(0, t[known], d[known].double().abs())
@@ -255,21 +257,39 @@ def test_second_derivatives_frozen_parameters_and_saved_tensor_hooks():
 def test_weight_gradient(rows, N, K):
     gen = _gen(rows)
     dy, x = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, rows, K, dtype=torch.bfloat16)
-    got = train_fused._weight_grad(dy, x)
+    got = _lib.native().weight_grad(dy, x)
     assert got.dtype == torch.float32
     want = dy.double().t() @ x.double()
     _close(got, want, (rows + 8) * EPS32 * (dy.double().abs().t() @ x.double().abs()))   # fp32 sums of exact products
-    assert torch.equal(train_fused._weight_grad(dy, x), got)
+    assert torch.equal(_lib.native().weight_grad(dy, x), got)
+
+
+@pytest.mark.parametrize("rows,N,K", [(2049, 2056, 2048), (1025, 4096, 4096), (2500, 32000, 256)])
+def test_the_librarys_weight_gradients_replay_from_a_graph(rows, N, K):
+    """Every replay gives the eager result, with new values and eager work in between."""
+    gen = _gen(K)
+    dy, x = _randn(gen, rows, N, dtype=torch.bfloat16), _randn(gen, rows, K, dtype=torch.bfloat16)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        _lib.native().weight_grad(dy, x)
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = _lib.native().weight_grad(dy, x)
+    for k in range(4):
+        dy.copy_(_randn(gen, rows, N, dtype=torch.bfloat16))
+        want = _lib.native().weight_grad(dy, x)
+        torch.cuda.synchronize()
+        got.fill_(float("nan"))
+        graph.replay()
+        assert torch.equal(got, want), k
 
 
 @pytest.mark.parametrize("rows,sizes", [(70, [(8, 8), (136, 120), (128, 264)]), (520, [(256, 128), (8, 520), (264, 136), (128, 128)]),
                                         (3100, [(512, 256), (256, 256), (1024, 256), (256, 512)]), (1, [(264, 8)] * 8)])
 def test_weight_gradients_of_one_launch(rows, sizes):
     """Several products share a launch's workgroups: every one against 64 bits, one and several splits."""
-    import ctypes
-
-    from hawk_pytorch_amd import _lib
-
     gen, lib, n = _gen(rows), _lib.load(), len(sizes)
     dy, x = ([_randn(gen, rows, s[k], dtype=torch.bfloat16) for s in sizes] for k in (0, 1))
     guard = 64
@@ -278,7 +298,7 @@ def test_weight_gradients_of_one_launch(rows, sizes):
     nbytes = lib.hawk_weight_grads_workspace_bytes(n, rows, Ns, Ks)
     ws = torch.full((nbytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
     ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])   # noqa: E731
-    train_fused._check("hawk_weight_grads", n, ptrs(dy), ptrs(x), ptrs(dw), rows, Ns, Ks, ws.data_ptr(), nbytes,
+    _check("hawk_weight_grads", n, ptrs(dy), ptrs(x), ptrs(dw), rows, Ns, Ks, ws.data_ptr(), nbytes,
                        _lib.stream_ptr(DEV))
     for g, a, b, (N, K) in zip(dw, dy, x, sizes):
         want = a.double().t() @ b.double()
@@ -294,8 +314,6 @@ def test_weight_gradients_of_one_launch(rows, sizes):
                                             (8200, 520, 128), (130, 2048, 1600)])
 @pytest.mark.parametrize("which", ["fwd", "input_grad"])
 def test_products_of_a_linear_layer(which, rows, columns, k):
-    from hawk_pytorch_amd import _lib
-
     gen, lib, guard = _gen(rows), _lib.load(), 64
     a = _randn(gen, rows, k, dtype=torch.bfloat16)
     w = _randn(gen, *((columns, k) if which == "fwd" else (k, columns)), dtype=torch.bfloat16)
@@ -308,7 +326,7 @@ def test_products_of_a_linear_layer(which, rows, columns, k):
     ws = torch.full((nbytes + guard,), 0xA5, dtype=torch.uint8, device=DEV)
 
     def run():
-        train_fused._check(name, a.data_ptr(), w.data_ptr(), out.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
+        _check(name, a.data_ptr(), w.data_ptr(), out.data_ptr(), rows, N, K, ws.data_ptr(), nbytes,
                            _lib.stream_ptr(DEV))
         return out[:rows * columns].view(rows, columns)
 
