@@ -34,14 +34,11 @@ constexpr int kThreads = kWaves * kWave;
 constexpr int kNT = 64;          // output columns of a workgroup
 constexpr int kKT = 64;          // input channels of a step: 128 bytes of a row
 constexpr int kRowBytes = kKT * 2;
+static_assert(kRowBytes == kPieceRowBytes, "piece_offset's rows");
 
 enum Epilogue { kStoreBf16 = 0, kStorePartial = 1, kStoreGelu = 2 };
 
 inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
-
-// 16-byte piece `c` of row `r` of a staged tile.  The pieces of a row are permuted by the row's
-// number, so that the 8 rows one LDS cycle reads the same piece of cover all banks.
-__device__ __forceinline__ int piece_offset(int r, int c) { return r * kRowBytes + ((c ^ (r & 7)) << 4); }
 
 // One thread's share of a finished row: 8 adjacent columns a, c, or 4 gate columns a and the up
 // columns c beside them.
@@ -240,12 +237,6 @@ struct WideLds {
 constexpr int kWideWaves = 8;
 constexpr int kWideThreads = kWideWaves * kWave;
 
-// Until at most N of this wave's loads are in flight (they arrive in order).
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 template <int NT, int STAGES, int EPI>
 __global__ __launch_bounds__(kWideThreads, STAGES == 4 ? 2 : 4) void decode_gemm_wide_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
@@ -328,30 +319,7 @@ __global__ __launch_bounds__(kWideThreads, STAGES == 4 ? 2 : 4) void decode_gemm
                 acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[ks], fx[ks][mb], acc[mb], 0, 0, 0);
     };
 
-    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
-    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
-#pragma unroll
-    for (int d = 0; d < S - 1; ++d)
-        if (d < steps) load(d, d);
-    int i = 0, slot = 0;
-    for (; i + S - 1 < steps; ++i) {
-        wait_loads<(S - 2) * L>();
-        lds_barrier();
-        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    for (; i < steps; ++i) {
-        switch (steps - 1 - i) {
-            case 0: wait_loads<0>(); break;
-            case 1: wait_loads<L>(); break;
-            default: wait_loads<2 * L>(); break;       // (no more than S - 2 = 2)
-        }
-        lds_barrier();
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    lds_barrier();
+    staged_steps<S, L>(steps, load, multiply);
 
     // the tile through LDS, [128 rows][NT / 4 pieces of 4 columns] with the pieces permuted by the row,
     // so that it leaves in whole rows

@@ -1111,11 +1111,6 @@ __global__ __launch_bounds__(kGateThreads, 1) void gate_proj_bwd_input_kernel(
 // one tile between the matrix instructions of the next (a wave both gates of 32 columns, three
 // barriers a tile) took 190 us.
 // ---------------------------------------------------------------------------------------
-template <int N>
-__device__ __forceinline__ void wait_vector_memory() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 constexpr int kBwdThreads = 512;                                   // 8 waves of up to 256 registers
 constexpr int kBwdRows = kBwdThreads / 32;                         // rows that one access of all threads covers
 constexpr int kBwdHalo = kConvTaps - 1;                            // du rows behind a tile

@@ -90,16 +90,8 @@ __device__ __forceinline__ void read_transposed(uint32_t at0, uint32_t at1, uint
 #endif
 }
 #undef HAWK_TR
+// (An operand whose rows are the result's, [T rows][64 values of the sum], is read by piece_offset.)
 __device__ __forceinline__ bf16x8 operand(u32x2 lo, u32x2 hi) { return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}); }
-// One whose rows are the result's ([T rows][64 values of the sum], 128 bytes a row): the 16-byte pieces of a row are
-// permuted by its number.
-__device__ __forceinline__ int piece_offset(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
-
-template <int N>
-__device__ __forceinline__ void wait_loads() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 // One product of a launch: out [M, N] (or partial sums [splits, M, N]) = a^T b for a [K, M] and b [K, N], a b for
 // a [M, K], a b^T for b [N, K].  Its workgroups start at first; the launch's tasks share K and the number of splits.
 struct GradTask {
@@ -242,30 +234,7 @@ __global__ __launch_bounds__(T / 16 * kWave, STAGES == 2 ? 4 : 2) void sum_produ
         half(std::integral_constant<int, 2>{}, s);
     };
 
-    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
-    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
-#pragma unroll
-    for (int d = 0; d < S - 1; ++d)
-        if (d < steps) load(d, d);
-    int i = 0, slot = 0;
-    for (; i + S - 1 < steps; ++i) {
-        wait_loads<(S - 2) * 2 * L>();
-        lds_barrier();
-        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    for (; i < steps; ++i) {
-        switch (steps - 1 - i) {
-            case 0: wait_loads<0>(); break;
-            case 1: wait_loads<2 * L>(); break;
-            default: wait_loads<4 * L>(); break;       // (no more than S - 2 = 2)
-        }
-        lds_barrier();
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    lds_barrier();
+    staged_steps<S, 2 * L>(steps, load, multiply);
 
     // the tile through LDS, [T rows][T / 4 pieces of 4 columns], so that it leaves in whole rows
     constexpr int PR = T / 4;
