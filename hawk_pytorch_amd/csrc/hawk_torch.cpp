@@ -118,6 +118,11 @@ Tensor dense16(const Tensor& t) {
     Tensor d = t.contiguous();
     return aligned(d) ? d : d.clone(at::MemoryFormat::Contiguous);
 }
+std::vector<Tensor> dense16(const std::vector<Tensor>& ts) {
+    std::vector<Tensor> out;
+    for (const Tensor& t : ts) out.push_back(dense16(t));
+    return out;
+}
 
 // Device and stream of a call, and the guards of its body: no autograd, no autocast.
 struct Call {
@@ -366,13 +371,15 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> core_fwd(
     return {out, u, xg, ag, h, last};
 }
 
-// (d_xy, d_conv_w, d_conv_b, dw_i, db_i, dw_a, db_a, dlam)
+// (d_xy, d_conv_w, d_conv_b, dw_i, db_i, dw_a, db_a, dlam).  What the forward pass saved may come back in another layout:
+// hooks that pack saved tensors return what they like.
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> core_bwd(
-    const Tensor& xy_, const Tensor& u, const Tensor& xg, const Tensor& ag, const Tensor& h, const Tensor& cw_,
+    const Tensor& xy_, const Tensor& u_, const Tensor& xg_, const Tensor& ag_, const Tensor& h_, const Tensor& cw_,
     const Tensor& wi_, const Tensor& wa_, const Tensor& lam_, const Tensor& go_) {
     Call c(xy_.device());
-    const Tensor xy = aligned(xy_) ? xy_ : xy_.clone(at::MemoryFormat::Contiguous);
-    const Tensor cw = dense16(cw_), wi = dense16(wi_), wa = dense16(wa_), lam = dense16(lam_), go = dense16(go_);
+    const Tensor xy = aligned(xy_) && row_stride(xy_) % 8 == 0 && row_stride(xy_) > 0 ? xy_ : xy_.clone(at::MemoryFormat::Contiguous);
+    const Tensor u = dense16(u_), xg = dense16(xg_), ag = dense16(ag_), h = dense16(h_), cw = dense16(cw_),
+                 wi = dense16(wi_), wa = dense16(wa_), lam = dense16(lam_), go = dense16(go_);
     const int64_t B = xy.size(0), T = xy.size(1), D = xy.size(2) / 2, W = cw.size(0), nb = wi.size(0), bw = wi.size(1);
     Tensor d_xy = c.activation(xy.sizes(), kBF16), du = c.activation({B, T, D}, kBF16), dxg = c.activation({B, T, D}, kBF16),
            dag = c.activation({B, T, D}, kBF16);
@@ -783,8 +790,9 @@ std::vector<Tensor> layer_fwd(const Tensor& hidden, const std::optional<Tensor>&
 // Its backward pass.  s: n1, n2, cw, lam, wi, wa and what layer_fwd returned behind (total2, out), in its order.
 // Returns d_hidden, d_delta (undefined without want_delta), d_n1, d_n2, d_w_in, d_w_out, d_w_gu, d_w_dn, d_cw, d_cb,
 // d_wi, d_bi, d_wa, d_ba, d_lam, all in fp32 but d_delta.
-std::vector<Tensor> layer_bwd(const std::vector<Tensor>& s, const Tensor& d_total_, const Tensor& d_out_, bool want_delta) {
+std::vector<Tensor> layer_bwd(const std::vector<Tensor>& saved, const Tensor& d_total_, const Tensor& d_out_, bool want_delta) {
     Call c(d_total_.device());
+    const std::vector<Tensor> s = dense16(saved);
     const Tensor &n1 = s[0], &n2 = s[1], &cw = s[2], &lam = s[3], &wi = s[4], &wa = s[5], &w_in = s[6], &w_out = s[7],
                  &w_gu = s[8], &w_dn = s[9], &total1 = s[10], &x1 = s[11], &rstd1 = s[12], &xy = s[13], &u = s[14],
                  &xg = s[15], &ag = s[16], &h = s[17], &gated = s[18], &total2 = s[19], &x2 = s[20], &rstd2 = s[21],
@@ -827,9 +835,11 @@ std::vector<Tensor> loss_fwd(const Tensor& hidden, const std::optional<Tensor>& 
 }
 
 // s: norm, head16, total, x, rstd, logits, lse, mean.  Returns d_hidden, d_delta, d_norm, d_head.
-std::vector<Tensor> loss_bwd(const std::vector<Tensor>& s, const Tensor& labels, const Tensor& d_loss_, at::IntArrayRef shape,
-                             bool want_delta) {
-    Call c(s[0].device());
+std::vector<Tensor> loss_bwd(const std::vector<Tensor>& saved, const Tensor& labels_, const Tensor& d_loss_,
+                             at::IntArrayRef shape, bool want_delta) {
+    Call c(saved[0].device());
+    const std::vector<Tensor> s = dense16(saved);
+    const Tensor labels = labels_.contiguous();
     const Tensor d_loss = d_loss_.scalar_type() == kF32 ? d_loss_ : d_loss_.to(kF32);
     const Tensor &logits = s[5];
     const Tensor d_logits = c.empty(logits.sizes(), kBF16);
@@ -842,8 +852,9 @@ std::vector<Tensor> loss_bwd(const std::vector<Tensor>& s, const Tensor& labels,
     return {d_hidden.view(shape), d_delta.has_value() ? d_delta->view(shape) : Tensor(), d_norm, d_head};
 }
 
-Tensor embedding_bwd(const Tensor& ids, const Tensor& d_out_, int64_t V) {
+Tensor embedding_bwd(const Tensor& ids_, const Tensor& d_out_, int64_t V) {
     Call c(d_out_.device());
+    const Tensor ids = ids_.contiguous();
     const Tensor d_out = dense16(d_out_.scalar_type() == kF32 ? d_out_ : d_out_.to(kF32));
     const int64_t D = d_out.size(-1);
     Tensor dweight = at::zeros({V, D}, at::TensorOptions().dtype(kF32).device(c.dev));

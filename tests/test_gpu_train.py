@@ -249,6 +249,40 @@ def test_second_derivatives_frozen_parameters_and_saved_tensor_hooks():
         assert float((g - w).norm()) <= 2e-2 * float(w.norm())
 
 
+def _strided(t):
+    """The same values in another order of memory: no kernel reads it as it is."""
+    if t.dim() < 2:
+        return torch.stack([t, t], -1)[..., 0]
+    return t.transpose(-1, 0).contiguous().transpose(-1, 0)
+
+
+def _shifted(t):
+    """The same values one element behind a 16-byte boundary."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    return buf[1:].copy_(t.reshape(-1)).view(t.shape)
+
+
+@pytest.mark.parametrize("unpack", [_strided, _shifted], ids=["strided", "shifted"])
+@pytest.mark.parametrize("what", ["model", "core"])
+def test_saved_tensors_may_come_back_in_another_layout(what, unpack):
+    """Hooks that pack saved tensors (compress them, keep them on the host) return their own."""
+    if what == "model":
+        model = _model()
+        ids = torch.randint(0, 1000, (2, 70), generator=_gen(1), device=DEV)
+        run = lambda: _grads(model, ids, ids)[1]   # noqa: E731
+    else:
+        conv, gates = hk.Conv1D(256, 4, w_init_variance_scale=1.0).cuda(), [hk.BlockDiagonalLinear(256, 4, device=DEV) for _ in range(2)]
+        xy = _randn(_gen(2), 2, 70, 512, dtype=torch.bfloat16).requires_grad_()
+        lam = torch.nn.Parameter(hk.rnn_param_init(torch.empty(256, device=DEV), 0.9, 0.999))
+        wrt = [xy, lam, *conv.parameters(), *gates[0].parameters(), *gates[1].parameters()]
+        run = lambda: torch.autograd.grad(hk.recurrent_block_core(xy, conv, *gates, lam).float().square().sum(), wrt)   # noqa: E731
+    want = run()
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        got = run()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 # a single value, ragged edges of a tile in all three sizes, rows that end inside a step, one and several splits; the
 # library's product: more than 256 tiles beyond 2048 rows, 4096 wide beyond 1024, sizes the kernel refuses
 @pytest.mark.parametrize("rows,N,K", [(1, 8, 8), (64, 128, 128), (77, 136, 120), (513, 264, 136), (1024, 128, 256),
