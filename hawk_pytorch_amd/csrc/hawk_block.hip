@@ -77,7 +77,9 @@ int block_core_fwd(const void* xy, long long ld, const float* conv_w, const floa
 // on.  Whole backward in us, one kernel against two: 1024 rows 67.0 and 70.6 (2560 channels), 32.9 and 37.4 (512),
 // 91.9 and 97.8 (4096), 2048 rows of 256 channels 50.9 and 54.3; 768 rows of 2560 55.3 and 56.0, 512 rows 50.9 and
 // 51.4 (2560), 31.2 and 31.9 (512), 256 rows 47.3 and 47.1: there a worker has a tile or two, each with its halo,
-// and the conv's weight gradients rather keep the order of the conv's own backward.
+// and the conv's weight gradients rather keep the order of the conv's own backward.  (Many
+// short sequences gain least: of up to 256 positions each they are level to 2 us behind at 1024 rows and, up to 768
+// channels, at 4096, 45.1 and 43.2 for 40 of 33 positions of 256 channels, 63.8 and 62.1 for 16 of 64 of 2560.)
 constexpr int kOneKernelRows = 1024;
 bool projections_with_conv(int B, int T, int W) { return W == 4 && B * T >= kOneKernelRows; }
 

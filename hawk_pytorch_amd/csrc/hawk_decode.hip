@@ -15,8 +15,8 @@
 //   * the four partial tiles meet in LDS at the end and leave in whole rows;
 //   * projections with few columns also split K over workgroups and leave fp32 partial sums, which
 //     the kernel that follows (residual add + norm) adds up in a fixed order on its way.
-// A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 45 / 53 / 63 /
-// 79 / 86 / 101 us at 1 / 32 / 64 / 128 / 129 / 256 rows with cold weights (157 MB); the library's four products
+// A layer of 2560 channels and an MLP of 7680, next layer's input projection included, takes 44 / 53 / 64 /
+// 78 / 83 / 98 us at 1 / 32 / 64 / 128 / 129 / 256 rows with cold weights (157 MB); the library's four products
 // alone took 121 us at 256 rows, with the norms, additions, GELU and product around them 149.
 // All sums are fp32, in an order that depends on the shape alone, and values are rounded to bf16 where
 // the separate operations round them, so both routes differ by the order of the sums only.
@@ -701,13 +701,13 @@ int rows_product(const void* x, const NormArgs& norm, const void* w, void* out, 
 struct Cut {
     int mt, nt, depth, splits;
 };
-// Workgroups a product that is split over K is cut into: one per compute unit.  Measured on a layer
-// of 2560 x 7680 (four products, two norms): 240 to 266 (the same cuts there) give 49 / 53 / 63 / 82 / 104 us
-// at 1 / 32 / 64 / 128 / 256 rows, 320 gives 52 / 59 / 71 / 95 / 121 (the partial sums of more splits cost more
-// than the second workgroup on a compute unit brings), 160 gives 49 / 55 / 67 / 84 / 114.  With 240 the 128
-// tiles of 4096 columns at 129 rows and more, and of 8192 at 33 to 128, were not split and left half of the
-// chip idle: steps of two and four such layers took 999 and 1094 us at 64 and 256 rows, in two splits 887 and
-// 908.  From 129 tiles on one split stays: 160 tiles over K = 2560 in two take 2 % more of a layer's time.
+// Workgroups a product that is split over K is cut into: one per compute unit.  A layer of 2560 channels (MLP 7680;
+// 240 to 266 are the same cuts there) takes 49 / 53 / 64 / 78 / 83 / 98 us at 3 / 32 / 64 / 128 / 129 / 256 rows, with 320
+// workgroups 53 / 60 / 73 / 91 / 93 / 119 (the partial sums of more splits cost more than the second workgroup on a
+// compute unit brings), with 160 50 / 56 / 68 / 81 / 88 / 106.  With 240 the 128 tiles of 4096 columns at 129 rows and more,
+// and of 8192 at 33 to 128, are not split and half of the chip is idle: a layer of 4096 (MLP 12288) takes 199 and 231 us
+// at 129 and 256 rows, in two splits 171 and 190, one of 8192 (MLP 24576) 400 / 436 / 512 at 33 / 64 / 128, in two splits
+// 356 / 381 / 452.  From 129 tiles on one split stays: 160 tiles over K = 2560 in two take 2 % more of a layer's time.
 constexpr int kComputeUnits = 256;
 constexpr int kSplitWorkgroups = kComputeUnits;
 // Tiles of 128 x 128 from this many of them on; with fewer, part of the chip would be idle.

@@ -13,7 +13,8 @@
 // parentheses the library's (with its conversion for dw): four weights of a layer of 512 (MLP 1024) over 2048 rows 26.3
 // in one launch (97), 62.6 in four; with operands turned in registers by byte permutes 33.4.  2048 x 1024 x 512 6.6 (7.6),
 // in tiles of 128 8.1; 2048 x 512 x 512 5.0 (6.3), dx 2048 x 512 over 2048 11.9 (13.7), in tiles of 128 21.2; over
-// 32000 94 (201, on 60 workgroups).  6144 x 4096 x 1024 75 (50): callers leave more than 256 tiles to the library.
+// 32000 94 (201, on 60 workgroups).  6144 x 4096 x 1024 75 (50): callers leave to the library what
+// it is faster at, large outputs and weight gradients (hawk_torch.cpp has the lines and both sides' figures).
 #include "hawk_scan.h"
 
 #include <stdint.h>

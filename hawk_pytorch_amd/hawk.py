@@ -17,9 +17,9 @@ What differs from upstream is the recurrent block and how a whole pass is launch
   of twice;
 * a decode step of bf16 weights without gradients (``HawkModel._decode_step``) and a training pass of
   fp32 weights under bf16 autocast (``HawkModel._train_step``) run the norms, residual additions, gated
-  GELU, loss and, in decode, the projections as this package's kernels, with the modules' parameters and
-  roundings.  Where a module is not what the constructor made, or something watches its call, the
-  modules run.
+  GELU, loss and the projections (in training up to the sizes from which the library is faster) as this
+  package's kernels, with the modules' parameters and roundings.  Where a module is not what the
+  constructor made, or something watches its call, the modules run.
 """
 
 from __future__ import annotations

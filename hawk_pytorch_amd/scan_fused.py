@@ -6,7 +6,7 @@ Public surface mirrors the upstream operator boundary (hawk/scan_fused.py:319-44
     sequential_scan_backward(x, x_rg_lru, a_rg_lru, a_param, h_saved, grad_out)
         -> (dx, dx_rg_lru, da_rg_lru, da_param)
     DiagonalRecurrence            torch.autograd.Function
-    fused_linear_scan             = DiagonalRecurrence.apply
+    fused_linear_scan             DiagonalRecurrence.apply, in native code where it can be
 
 and, beyond upstream, the scan fused with the block's gate (hawk/hawk.py:134-135, :186):
 

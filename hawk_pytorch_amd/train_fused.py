@@ -1,6 +1,7 @@
 """A training pass of the model with one autograd node per layer (hawk/hawk.py:53-58, :70-86, :163-203,
 :222-303 upstream): residual add + RMSNorm, the gated GELU, the loss, the embedding's gradient and the
-weights' conversions are one kernel each, around the library GEMMs and the recurrent core's own kernels.
+weights' conversions are one kernel each, around the matrix products (own kernels or the library's, by size)
+and the recurrent core's own kernels.
 
 Module by module a layer is about sixty launches and as many autograd nodes per pass, 1 ms of host time at
 any size; the values that reach memory here are the ones that bf16 autocast rounds and stores there.
