@@ -319,7 +319,30 @@ __global__ __launch_bounds__(kWideThreads, STAGES == 4 ? 2 : 4) void decode_gemm
                 acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[ks], fx[ks][mb], acc[mb], 0, 0, 0);
     };
 
-    staged_steps<S, L>(steps, load, multiply);
+    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
+    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
+#pragma unroll
+    for (int d = 0; d < S - 1; ++d)
+        if (d < steps) load(d, d);
+    int i = 0, slot = 0;
+    for (; i + S - 1 < steps; ++i) {
+        wait_vector_memory<(S - 2) * L>();
+        lds_barrier();
+        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    for (; i < steps; ++i) {
+        switch (steps - 1 - i) {
+            case 0: wait_vector_memory<0>(); break;
+            case 1: wait_vector_memory<L>(); break;
+            default: wait_vector_memory<2 * L>(); break;       // (no more than S - 2 = 2)
+        }
+        lds_barrier();
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    lds_barrier();
 
     // the tile through LDS, [128 rows][NT / 4 pieces of 4 columns] with the pieces permuted by the row,
     // so that it leaves in whole rows

@@ -38,35 +38,4 @@ __device__ __forceinline__ void wait_vector_memory() {
 constexpr int kPieceRowBytes = 128;
 __device__ __forceinline__ int piece_offset(int r, int c) { return r * kPieceRowBytes + ((c ^ (r & 7)) << 4); }
 
-// A ring of S tiles in LDS, `steps` of them worked on one after the other, S - 1 loads ahead, one barrier a step.
-// load(slot, step) issues LOADS loads into LDS per wave.  Step i: its tile has arrived when at most S - 2 younger ones
-// are in flight; behind the barrier everyone's part has, and everyone is done with the tile of step i - 1, whose place
-// the tile of step i + S - 1 takes.
-template <int S, int LOADS, typename Load, typename Multiply>
-__device__ __forceinline__ void staged_steps(int steps, const Load& load, const Multiply& multiply) {
-    static_assert(S >= 2 && S <= 4, "the last steps' waits");
-#pragma unroll
-    for (int d = 0; d < S - 1; ++d)
-        if (d < steps) load(d, d);
-    int i = 0, slot = 0;
-    for (; i + S - 1 < steps; ++i) {
-        wait_vector_memory<(S - 2) * LOADS>();
-        lds_barrier();
-        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    for (; i < steps; ++i) {
-        switch (steps - 1 - i) {
-            case 0: wait_vector_memory<0>(); break;
-            case 1: wait_vector_memory<LOADS>(); break;
-            default: wait_vector_memory<2 * LOADS>(); break;       // (no more than S - 2 = 2)
-        }
-        lds_barrier();
-        multiply(slot);
-        slot = slot == S - 1 ? 0 : slot + 1;
-    }
-    lds_barrier();
-}
-
 }  // namespace hawk

@@ -235,7 +235,30 @@ __global__ __launch_bounds__(T / 16 * kWave, STAGES == 2 ? 4 : 2) void sum_produ
         half(std::integral_constant<int, 2>{}, s);
     };
 
-    staged_steps<S, 2 * L>(steps, load, multiply);
+    // Step i: its tile has arrived when at most S - 2 younger ones are in flight; behind the barrier everyone's part
+    // has, and everyone is done with the tile of step i - 1, whose place the tile of step i + S - 1 takes.
+#pragma unroll
+    for (int d = 0; d < S - 1; ++d)
+        if (d < steps) load(d, d);
+    int i = 0, slot = 0;
+    for (; i + S - 1 < steps; ++i) {
+        wait_vector_memory<(S - 2) * 2 * L>();
+        lds_barrier();
+        load(slot == 0 ? S - 1 : slot - 1, i + S - 1);
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    for (; i < steps; ++i) {
+        switch (steps - 1 - i) {
+            case 0: wait_vector_memory<0>(); break;
+            case 1: wait_vector_memory<2 * L>(); break;
+            default: wait_vector_memory<4 * L>(); break;       // (no more than S - 2 = 2)
+        }
+        lds_barrier();
+        multiply(slot);
+        slot = slot == S - 1 ? 0 : slot + 1;
+    }
+    lds_barrier();
 
     // the tile through LDS, [T rows][T / 4 pieces of 4 columns], so that it leaves in whole rows
     constexpr int PR = T / 4;
