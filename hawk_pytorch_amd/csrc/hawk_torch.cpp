@@ -730,12 +730,13 @@ bool own_product(int64_t rows, int64_t columns, int64_t sum) {
 }
 // An output's operands lie along the sum.  The kernels are ahead up to 2^31 multiply-adds (own / library in us: 1024 x 1024 at
 // 1024 rows 7.1 / 9.0 and at 2048 10.3 / 10.6, 4096 x 1024 at 512 10.0 / 10.7, 1024 x 512 at 4096 9.7 / 11.1, 9216 x 1536
-// at 100 16.3 / 18.7) and behind beyond (1024 x 1024 at 4096 14.7 / 12.9, 2048 x 1024 at 2048 15.2 / 13.1, 1536 x 4608 at
-// 1024 37.7 / 28.0, 15360 x 2560 at 100 30.6 / 25.0), but for one tile of rows over a sum longer than the row of results,
-// which they split (4096 x 12288 at 100 32.4 / 41.6).  Short of the line they are up to 3 us behind at a hundred rows
-// (1536 x 4608 13.4 / 10.8, 2560 x 2560 12.3 / 10.7), less than their launch saves the host.
+// at 100 16.3 / 18.7), 1 to 4 us behind from there to 2^32 (2048 x 1024 at 2048 15.2 / 13.1, 2560 x 2560 at 512 18.5 / 15.5,
+// 15360 x 2560 at 100 30.6 / 25.0), less than their launch saves the host (with the line at 2^31 passes of three layers
+// of 768 over 2000 rows took 1430 us instead of 1414, of 1024 over 1500 rows 1567 instead of 1551), and further beyond
+// (1536 x 4608 at 1024 37.7 / 28.0, 2560 x 7680 at 1024 79.0 / 63.4, 32000 x 4096 at 100 72.8 / 57.4), but for one tile of
+// rows over a sum longer than the row of results, which they split (4096 x 12288 at 100 32.4 / 41.6).
 bool own_output(int64_t rows, int64_t columns, int64_t sum) {
-    return own_product(rows, columns, sum) && (rows * columns * sum <= (int64_t)1 << 31 || (rows <= 128 && sum > columns));
+    return own_product(rows, columns, sum) && (rows * columns * sum <= (int64_t)1 << 32 || (rows <= 128 && sum > columns));
 }
 Tensor layer_linear(const Tensor& x, const Tensor& w) {
     const int n = x.size(0), N = w.size(0), K = w.size(1);
