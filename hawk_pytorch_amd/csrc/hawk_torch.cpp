@@ -337,6 +337,20 @@ std::tuple<Tensor, Tensor, Tensor> conv_bwd(const Tensor& gy_, const Tensor& x_,
     return {dx, dw, db};
 }
 
+// The core's kernels are told sizes and one type for both gates' weights: everything else they read has to agree with that.
+void check_core_sizes(int64_t D, const Tensor& cw, const Tensor& wi, const Tensor& wa, const Tensor& lam) {
+    TORCH_CHECK(wi.dim() == 3 && wi.size(1) == wi.size(2) && wi.size(0) * wi.size(1) == D && wa.sizes() == wi.sizes(),
+                "gate weights must be [num_blocks, width, width] of ", D, " channels, got ", wi.sizes(), " and ", wa.sizes());
+    TORCH_CHECK(wi.scalar_type() == kBF16 || wi.scalar_type() == kF32, "gate weights must be bf16 or fp32, got ", wi.scalar_type());
+    TORCH_CHECK(cw.dim() == 2 && cw.size(1) == D && cw.scalar_type() == kF32, "the conv's weight must be fp32 [width, ", D,
+                "], got ", cw.sizes());
+    TORCH_CHECK(lam.numel() == D && lam.scalar_type() == kF32, "a_param must be fp32 [", D, "], got ", lam.sizes());
+}
+void check_core_vector(const char* what, const Tensor& t, int64_t D) {
+    TORCH_CHECK(t.numel() == D && t.scalar_type() == kF32, what, " must hold ", D, " fp32 values, got ", t.sizes());
+}
+Tensor as_type(const Tensor& t, at::ScalarType type) { return t.scalar_type() == type ? t : t.to(type); }
+
 constexpr int kFusedConvMinT = 32;   // hawk_block_core_fwd needs T >= 32 and a temporal width of 4
 
 // (out, u, xg, ag, h, h_last)
@@ -345,9 +359,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> core_fwd(
     const Tensor& ba_, const Tensor& lam_, bool want_h, bool want_last) {
     Call c(xy_.device());
     const Tensor xy = aligned(xy_) ? xy_ : xy_.clone(at::MemoryFormat::Contiguous);
-    const Tensor cw = dense16(cw_), cb = dense16(cb_), wi = dense16(wi_), bi = dense16(bi_), wa = dense16(wa_),
-                 ba = dense16(ba_), lam = dense16(lam_);
     const int64_t B = xy.size(0), T = xy.size(1), D = xy.size(2) / 2, ld = row_stride(xy);
+    TORCH_CHECK(xy.scalar_type() == kBF16, "xy must be bf16");
+    check_core_sizes(D, cw_, wi_, wa_, lam_);
+    check_core_vector("the conv's bias", cb_, D);
+    check_core_vector("a gate's bias", bi_, D);
+    check_core_vector("a gate's bias", ba_, D);
+    const Tensor cw = dense16(cw_), cb = dense16(cb_), wi = dense16(wi_), bi = dense16(bi_),
+                 wa = dense16(as_type(wa_, wi_.scalar_type())), ba = dense16(ba_), lam = dense16(lam_);
     const int W = cw.size(0), nb = wi.size(0), wt = code(wi.scalar_type()), bf = HAWK_DTYPE_BF16;
     Tensor u = c.activation({B, T, D}, kBF16), xg = c.activation({B, T, D}, kBF16), ag = c.activation({B, T, D}, kBF16),
            out = c.activation({B, T, D}, kBF16), h = want_h ? c.activation({B, T, D}, kBF16) : c.empty({0}, kBF16),
@@ -378,9 +397,14 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> core_
     const Tensor& wi_, const Tensor& wa_, const Tensor& lam_, const Tensor& go_) {
     Call c(xy_.device());
     const Tensor xy = aligned(xy_) && row_stride(xy_) % 8 == 0 && row_stride(xy_) > 0 ? xy_ : xy_.clone(at::MemoryFormat::Contiguous);
-    const Tensor u = dense16(u_), xg = dense16(xg_), ag = dense16(ag_), h = dense16(h_), cw = dense16(cw_),
-                 wi = dense16(wi_), wa = dense16(wa_), lam = dense16(lam_), go = dense16(go_);
-    const int64_t B = xy.size(0), T = xy.size(1), D = xy.size(2) / 2, W = cw.size(0), nb = wi.size(0), bw = wi.size(1);
+    const int64_t B = xy.size(0), T = xy.size(1), D = xy.size(2) / 2;
+    check_core_sizes(D, cw_, wi_, wa_, lam_);
+    const at::IntArrayRef states[] = {u_.sizes(), xg_.sizes(), ag_.sizes(), h_.sizes(), go_.sizes()};
+    for (const auto& size : states) TORCH_CHECK(size == at::IntArrayRef({B, T, D}), "expected [", B, ", ", T, ", ", D, "], got ", size);
+    for (const Tensor* t : {&xy_, &u_, &xg_, &ag_, &h_, &go_}) TORCH_CHECK(t->scalar_type() == kBF16, "the core's tensors must be bf16");
+    const Tensor u = dense16(u_), xg = dense16(xg_), ag = dense16(ag_), h = dense16(h_), cw = dense16(cw_), wi = dense16(wi_),
+                 wa = dense16(as_type(wa_, wi_.scalar_type())), lam = dense16(lam_), go = dense16(go_);
+    const int64_t W = cw.size(0), nb = wi.size(0), bw = wi.size(1);
     Tensor d_xy = c.activation(xy.sizes(), kBF16), du = c.activation({B, T, D}, kBF16), dxg = c.activation({B, T, D}, kBF16),
            dag = c.activation({B, T, D}, kBF16);
     Tensor dlam = c.empty({D}, kF32), dwi = c.empty({nb, bw, bw}, kF32), dwa = c.empty({nb, bw, bw}, kF32),

@@ -178,6 +178,7 @@ def temporal_conv1d_step(conv_state, x_new, w, b, out_dtype: Optional[torch.dtyp
         f"conv_state must be [B, W-1, D] = {(B, W - 1, D)}, got {tuple(conv_state.shape)}"
     )
     assert conv_state.is_contiguous(), "conv_state is updated in place and must be contiguous"
+    assert b.numel() == D, "conv bias does not match the channel count"
     dev = _lib.require_cuda(conv_state, xn, w, b)
     xn = _lib.dense16(xn.to(conv_state.dtype))
     if out_dtype is None:
@@ -200,7 +201,7 @@ def rglru_step(x, x_rg_lru, a_rg_lru, a_param, recc_state):
     D = x.shape[-1]
     shape = x.shape
     B = x.numel() // D
-    assert recc_state.numel() == B * D and recc_state.is_contiguous()
+    assert recc_state.numel() == B * D and recc_state.is_contiguous() and a_param.numel() == D
     dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, recc_state)
     run_dtype = x.dtype if x.dtype in (torch.bfloat16, torch.float32) else torch.float32
     xs = [_lib.dense16(t.reshape(B, D).to(run_dtype)) for t in (x, x_rg_lru, a_rg_lru)]
@@ -225,7 +226,7 @@ def rglru_step_gated(x, x_rg_lru, a_rg_lru, a_param, recc_state, y, bias_i=None,
     D = x.shape[-1]
     shape = x.shape
     B = x.numel() // D
-    assert recc_state.numel() == B * D and recc_state.is_contiguous()
+    assert recc_state.numel() == B * D and recc_state.is_contiguous() and a_param.numel() == D
     dev = _lib.require_cuda(x, x_rg_lru, a_rg_lru, a_param, recc_state, y)
     run_dtype = x.dtype if x.dtype in (torch.bfloat16, torch.float32) else torch.float32
     xs = [_lib.dense16(t.reshape(B, D).to(run_dtype)) for t in (x, x_rg_lru, a_rg_lru)]
@@ -310,12 +311,16 @@ def decode_core_step(conv_state, x_new, conv: "Conv1D", input_gate: "BlockDiagon
     b_i, b_a = input_gate.b, a_gate.b
     if b_i.numel() != D or b_a.numel() != D:
         b_i, b_a = b_i.reshape(D), b_a.reshape(D)   # raises for the one of another size
+    if w_a.dtype != w_i.dtype:
+        w_a = w_a.detach().to(w_i.dtype)
+    nb, bw = input_gate.num_blocks, D // input_gate.num_blocks
+    assert w_i.shape == w_a.shape == (nb, bw, bw) and conv.b.numel() == D and a_param.numel() == D, (
+        f"gate weights, conv bias or a_param do not match {D} channels in {nb} blocks"
+    )
     w32, b32, b_i, b_a, lam = (
         t if t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
         else _lib.dense16(t.detach().float()) for t in (conv_w, conv.b, b_i, b_a, a_param))
     w_i, w_a = (t if t.is_contiguous() and t.data_ptr() % 16 == 0 else _lib.dense16(t.detach()) for t in (w_i, w_a))
-    if w_a.dtype != w_i.dtype:
-        w_a = w_a.detach().to(w_i.dtype)
     out = torch.empty(shape, dtype=torch.bfloat16, device=dev)
     lib = _lib.load()
     with _lib.on_device(dev):
@@ -454,11 +459,22 @@ def _gate_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     return ws
 
 
+def _same_gates(w_i, w_a):
+    """The kernels take one type and one shape for both gates' weights."""
+    nb, bw, cols = w_i.shape
+    assert w_a.shape == w_i.shape and cols == bw, (
+        f"gate weights must be [num_blocks, width, width] alike, got {tuple(w_i.shape)} and {tuple(w_a.shape)}"
+    )
+    return w_i, (w_a if w_a.dtype == w_i.dtype else w_a.to(w_i.dtype))
+
+
 def _launch_gate_fwd(x, w_i, b_i, w_a, b_a, out_bf16: bool):
     dev = _lib.require_cuda(x, w_i, b_i, w_a, b_a)
+    w_i, w_a = _same_gates(w_i, w_a)
     nb, bw, _ = w_i.shape
     D = nb * bw
     M = x.numel() // D
+    assert b_i.numel() == D and b_a.numel() == D, "gate biases do not match the channel count"
     x2, w_i, w_a, b_i, b_a = (_lib.dense16(t) for t in (x.reshape(M, D), w_i, w_a, b_i, b_a))
     out_dtype = torch.bfloat16 if out_bf16 else torch.float32
     xg = _lib.activation_empty(x.shape, out_dtype, dev)
@@ -475,6 +491,7 @@ def _launch_gate_fwd(x, w_i, b_i, w_a, b_a, out_bf16: bool):
 
 def _launch_gate_bwd(x, d_xg, d_ag, w_i, w_a, addend=None):
     dev = _lib.require_cuda(x, d_xg, d_ag, w_i, w_a)
+    w_i, w_a = _same_gates(w_i, w_a)
     nb, bw, _ = w_i.shape
     D = nb * bw
     M = x.numel() // D
@@ -559,9 +576,13 @@ _CAST_WEIGHTS_MIN_ROWS = 8192
 
 
 def kernel_weights(w_i: torch.Tensor, w_a: torch.Tensor, rows: int):
+    """Both gates' weights as the kernels read them: of one type, bf16 or fp32."""
+    _lib.dtype_code(w_i.dtype)
+    if w_a.dtype != w_i.dtype:
+        return w_i.detach().to(torch.bfloat16), w_a.detach().to(torch.bfloat16)
     if w_i.dtype == torch.float32 and rows >= _CAST_WEIGHTS_MIN_ROWS:
         nb, bw, _ = w_i.shape
-        if w_i.is_cuda and w_a.dtype == torch.float32 and w_a.shape == w_i.shape and bw % 4 == 0:
+        if w_i.is_cuda and w_a.shape == w_i.shape and bw % 4 == 0:
             # both gates in one launch
             return _lib.native().gate_weights_to_bf16(w_i.detach(), w_a.detach())
         return w_i.detach().to(torch.bfloat16), w_a.detach().to(torch.bfloat16)

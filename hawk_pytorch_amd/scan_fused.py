@@ -455,11 +455,13 @@ def block_core_layout_ok(xy: torch.Tensor) -> bool:
 
 def _launch_block_core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, want_h: bool, want_last: bool):
     _lib.require_cuda(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam)
+    _lib.dtype_code(w_i.dtype)
     return _lib.native().core_fwd(xy, conv_w, conv_b, w_i, b_i, w_a, b_a, lam, want_h, want_last)
 
 
 def _launch_block_core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out):
     _lib.require_cuda(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out)
+    _lib.dtype_code(w_i.dtype)
     return _lib.native().core_bwd(xy, u, xg, ag, h, conv_w, w_i, w_a, lam, grad_out)
 
 

@@ -32,7 +32,7 @@ def _exact_linear(x, w):
                                    (200, 17000, 256), (129, 9000, 640), (150, 9000, 128),
                                    # one and two rows without tiles: two and four columns a wave, ends of the loads
                                    # of 512 channels and the loop over them; more columns than 4096 waves take at
-                                   # once, with a last round of few waves and of all of them
+                                   # once, with a last turn of few waves and of all of them
                                    (1, 4104, 640), (2, 4096, 1152), (1, 72, 7680), (2, 72, 7680), (1, 20008, 384),
                                    (2, 20008, 384), (1, 32000, 512), (1, 32768, 1152), (2, 16392, 640),
                                    # two rows: the most weights they take so, and the fewest they leave to the tiles

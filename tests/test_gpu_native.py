@@ -175,3 +175,66 @@ def test_a_workspace_that_changes_while_native_code_asks_for_it_is_not_kept(othe
     held, = _lib._workspaces.values()
     assert asked[0] is not held and asked[-1] is held
     hk.check_scan_status()
+
+
+@pytest.mark.parametrize("types", [(F32, BF), (BF, F32), (BF, torch.float16)], ids=lambda t: "-".join(str(x).split(".")[1] for x in t))
+@pytest.mark.parametrize("which", ["core", "recurrent_core", "projections", "decode"])
+def test_gates_whose_weights_differ_in_type(which, types):
+    """The kernels read both gates' weights as one type: as if both had been bf16, which they are rounded to anyway."""
+    B, T, D, nb = 2, 40, 256, 2
+    torch.manual_seed(5)
+    conv = hk.Conv1D(D, 4, w_init_variance_scale=1.0).cuda()
+    gates = [hk.BlockDiagonalLinear(D, nb, device="cuda") for _ in range(2)]
+    same = [hk.BlockDiagonalLinear(D, nb, device="cuda") for _ in range(2)]
+    for g, s, t in zip(gates, same, types):
+        g.w.data = g.w.data.to(t)
+        s.w.data = g.w.data.to(BF)
+    lam, xy = _lam(D), torch.randn(B, T, 2 * D, device="cuda").to(BF)
+    u, y = xy.chunk(2, -1)
+    state, window = torch.randn(B, 1, D, device="cuda"), torch.randn(B, 3, D, device="cuda").to(BF)
+
+    def run(i, a):
+        if which == "core":
+            return hk.recurrent_block_core(xy, conv, i, a, lam)
+        if which == "recurrent_core":
+            return scan_fused.recurrent_core(u, i, a, lam, y)
+        if which == "projections":
+            return external.gate_projections(u, i, a)[1]
+        with torch.no_grad():
+            return external.decode_core_step(window.clone(), u[:, :1], conv, i, a, lam, state.clone(), y[:, :1])
+
+    got, want = run(*gates), run(*same)
+    assert torch.equal(got, want)
+    if which == "decode":
+        return
+    go, used = torch.randn_like(got), (1,) if which == "projections" else (0, 1)
+    grads = [torch.autograd.grad(out, [ms[k].w for k in used], go) for out, ms in ((got, gates), (want, same))]
+    for k, x, r in zip(used, *grads):
+        assert x.dtype == types[k]
+        if types[k] != torch.float16:
+            assert torch.equal(x.to(BF), r)
+
+
+def test_operands_that_do_not_fit_are_refused_before_a_launch():
+    D, nb = 128, 2
+    conv = hk.Conv1D(D, 4).cuda()
+    gate, wide, half = (hk.BlockDiagonalLinear(d, nb, device="cuda", dtype=t) for d, t in ((D, F32), (2 * D, F32), (D, torch.float16)))
+    xy, lam, state, window = (torch.zeros(s, device="cuda", dtype=BF) for s in ((1, 40, 2 * D), (D,), (1, 1, D), (1, 3, D)))
+    u, y = xy.chunk(2, -1)
+    short = torch.zeros(D // 2, device="cuda")
+    with pytest.raises(TypeError):
+        hk.recurrent_block_core(xy, conv, half, half, lam)
+    with pytest.raises(TypeError):
+        scan_fused.recurrent_core(u, half, half, lam, y)
+    for args in ((hk.Conv1D(2 * D, 4).cuda(), gate, gate, lam), (conv, wide, wide, lam), (conv, gate, wide, lam), (conv, gate, gate, short)):
+        with pytest.raises((RuntimeError, AssertionError)):
+            hk.recurrent_block_core(xy, *args)
+    with pytest.raises((RuntimeError, AssertionError)):
+        scan_fused.recurrent_core(u, gate, wide, lam, y)
+    for i, a, l in ((wide, wide, lam), (gate, wide, lam), (gate, gate, short)):
+        with pytest.raises((RuntimeError, AssertionError)):
+            external.decode_core_step(window, u[:, :1], conv, i, a, l, state, y[:, :1])
+    with pytest.raises(AssertionError):
+        external.temporal_conv1d_step(window, u[:, 0], conv.w, short)
+    with pytest.raises(AssertionError):
+        external.rglru_step(u[:, 0], u[:, 0], u[:, 0], short, state)
